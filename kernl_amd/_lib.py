@@ -1,9 +1,11 @@
-"""ctypes binding of libkernl_hip.so (C ABI: include/kernl_hip.h).
+"""Binding of libkernl_hip.so (C ABI: include/kernl_hip.h): ctypes, and for the calls made per token or per layer the
+CPython module `_host` (csrc/host_ops.cpp), which costs 2 us a call where ctypes and its conversions cost 10.
 
-The library is built in-tree by `kernl_amd/csrc/Makefile` (see `kernl_amd.build`).  There is no fallback:
-if the shared object is missing or a call fails, the error is raised to the caller.
+Both are built in-tree by `kernl_amd/csrc/Makefile` (see `kernl_amd.build`).  There is no fallback:
+if a shared object is missing or a call fails, the error is raised to the caller.
 """
 import ctypes
+import importlib
 import os
 from typing import Optional, Sequence
 
@@ -11,6 +13,7 @@ import torch
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libkernl_hip.so")
 _lib: Optional[ctypes.CDLL] = None
+_host = None
 
 KERNL_F16, KERNL_BF16, KERNL_F32 = 0, 1, 2
 DTYPE_CODE = {torch.float16: KERNL_F16, torch.bfloat16: KERNL_BF16, torch.float32: KERNL_F32}
@@ -176,6 +179,20 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def host():
+    """The CPython module over the library, loaded once; raises KernlLibraryError if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            module = importlib.import_module("kernl_amd._host")
+        except ImportError as exc:
+            raise KernlLibraryError(f"kernl_amd/_host.so cannot be loaded ({exc}): build it with `python -m kernl_amd.build`") from exc
+        module.set_error_type(KernlLibraryError)
+        _host = module
+    return _host
+
+
 def _arr(values: Sequence[int]):
     return (ctypes.c_int64 * len(values))(*values)
 
@@ -197,44 +214,12 @@ def _require_gpu(*tensors: torch.Tensor) -> None:
 
 
 def attention_fwd(q, k, v, out, mask, sm_scale: float, is_causal: bool, mask_min_clamp: float) -> None:
-    _require_gpu(q, k, v, out, mask)
-    B, H, M, D = q.shape
-    N = k.shape[2]
-    lib = load()
-    if mask is not None:
-        msizes, mstrides, mdtype, mptr = _arr(mask.shape), _arr(mask.stride()), DTYPE_CODE[mask.dtype], mask.data_ptr()
-    else:
-        msizes, mstrides, mdtype, mptr = None, None, KERNL_F32, None
-    with torch.cuda.device(q.device):
-        st = lib.kernl_attention_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mptr,
-            B, H, M, N, D,
-            _arr(q.stride()), _arr(k.stride()), _arr(v.stride()), _arr(out.stride()),
-            msizes, mstrides, mdtype,
-            float(sm_scale), int(bool(is_causal)), float(mask_min_clamp), DTYPE_CODE[q.dtype], _stream(q),
-        )
-    _check(st, "kernl_attention_fwd")
+    (_host or host()).attention_fwd(q, k, v, out, mask, sm_scale, is_causal, mask_min_clamp)
 
 
 def attention_cached_fwd(q, k, v, out, mask, sm_scale: float, start_position: int, mask_min_clamp: float) -> None:
     """Causal attention of the rows of q, which sit at positions start_position.. of the sequence held in k / v."""
-    _require_gpu(q, k, v, out, mask)
-    B, H, M, D = q.shape
-    N = k.shape[2]
-    lib = load()
-    if mask is not None:
-        msizes, mstrides, mdtype, mptr = _arr(mask.shape), _arr(mask.stride()), DTYPE_CODE[mask.dtype], mask.data_ptr()
-    else:
-        msizes, mstrides, mdtype, mptr = None, None, KERNL_F32, None
-    with torch.cuda.device(q.device):
-        st = lib.kernl_attention_cached_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mptr,
-            B, H, M, N, D,
-            _arr(q.stride()), _arr(k.stride()), _arr(v.stride()), _arr(out.stride()),
-            msizes, mstrides, mdtype,
-            float(sm_scale), int(start_position), float(mask_min_clamp), DTYPE_CODE[q.dtype], _stream(q),
-        )
-    _check(st, "kernl_attention_cached_fwd")
+    (_host or host()).attention_cached_fwd(q, k, v, out, mask, sm_scale, start_position, mask_min_clamp)
 
 
 def attention_kv8_fwd(q, k8, v8, out, mask, sm_scale: float, is_causal: bool, start_position: int, mask_min_clamp: float) -> None:
@@ -263,27 +248,7 @@ def attention_skinny_workspace_bytes(B: int, H: int, M: int, N: int, D: int) -> 
 
 
 def attention_skinny_fwd(q, k, v, out, mask, workspace, sm_scale: float, is_causal: bool, mask_min_clamp: float) -> None:
-    _require_gpu(q, k, v, out, mask, workspace)
-    B, H, M, D = q.shape
-    N = k.shape[2]
-    lib = load()
-    if mask is not None:
-        msizes, mstrides, mdtype, mptr = _arr(mask.shape), _arr(mask.stride()), DTYPE_CODE[mask.dtype], mask.data_ptr()
-    else:
-        msizes, mstrides, mdtype, mptr = None, None, KERNL_F32, None
-    ws_ptr = None if workspace is None else workspace.data_ptr()
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    with torch.cuda.device(q.device):
-        one_byte = k.dtype in (torch.int8, torch.uint8, torch.float8_e5m2)
-        entry = lib.kernl_attention_skinny_kv8_fwd if one_byte else lib.kernl_attention_skinny_fwd
-        st = entry(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mptr, ws_ptr, ws_bytes,
-            B, H, M, N, D,
-            _arr(q.stride()), _arr(k.stride()), _arr(v.stride()), _arr(out.stride()),
-            msizes, mstrides, mdtype,
-            float(sm_scale), int(bool(is_causal)), float(mask_min_clamp), DTYPE_CODE[q.dtype], _stream(q),
-        )
-    _check(st, "kernl_attention_skinny_fwd")
+    (_host or host()).attention_skinny_fwd(q, k, v, out, mask, workspace, sm_scale, is_causal, mask_min_clamp)
 
 
 def attention_skinny_static_init(device=None) -> None:
@@ -341,19 +306,7 @@ def linear_wide_kind(M: int, N: int, K: int) -> int:
 
 
 def linear_fwd(x2d, weight, bias, out2d, act_in2d, activation: int) -> None:
-    _require_gpu(x2d, weight, bias, out2d, act_in2d)
-    M, K = x2d.shape
-    N = weight.shape[0]
-    lib = load()
-    with torch.cuda.device(x2d.device):
-        st = lib.kernl_linear_fwd(
-            x2d.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out2d.data_ptr(),
-            None if act_in2d is None else act_in2d.data_ptr(),
-            M, N, K,
-            _arr(x2d.stride()), _arr(out2d.stride()), None if act_in2d is None else _arr(act_in2d.stride()),
-            int(activation), DTYPE_CODE[x2d.dtype], _stream(x2d),
-        )
-    _check(st, "kernl_linear_fwd")
+    (_host or host()).linear_fwd(x2d, weight, bias, out2d, act_in2d, activation)
 
 
 def linear_w8_supported(x2d, weight8) -> bool:
@@ -393,18 +346,7 @@ def linear_rms_supported(x2d) -> bool:
 
 
 def linear_rms_fwd(x2d, rms_weight, eps: float, weight, bias, out2d, activation: int, gated: bool) -> None:
-    _require_gpu(x2d, rms_weight, weight, bias, out2d)
-    M, K = x2d.shape
-    N = out2d.shape[1]
-    lib = load()
-    with torch.cuda.device(x2d.device):
-        st = lib.kernl_linear_rms_fwd(
-            x2d.data_ptr(), rms_weight.data_ptr(), float(eps), weight.data_ptr(),
-            None if bias is None else bias.data_ptr(), out2d.data_ptr(), M, N, K,
-            _arr(x2d.stride()), _arr(out2d.stride()), int(activation), int(bool(gated)), DTYPE_CODE[x2d.dtype],
-            _stream(x2d),
-        )
-    _check(st, "kernl_linear_rms_fwd")
+    (_host or host()).linear_rms_fwd(x2d, rms_weight, eps, weight, bias, out2d, activation, gated)
 
 
 def linear_scaled_supported(x2d, weight) -> bool:
@@ -508,24 +450,7 @@ def linear_decode_fwd(x2d, rms_weight, eps: float, weight, bias, residual2d, out
                       rope_cols: int = 0, rows_per_batch: int = 1) -> None:
     """cos / sin: [batch | 1, positions, head_dim] tables (unit feature stride) or None; row m of x2d is position
     m % rows_per_batch of batch entry m / rows_per_batch."""
-    _require_gpu(x2d, rms_weight, weight, bias, residual2d, out2d, cos, sin)
-    M, K = x2d.shape
-    N = out2d.shape[1]
-    lib = load()
-    if cos is not None:
-        tstrides = _arr((0 if cos.shape[0] == 1 else cos.stride(0), cos.stride(1), cos.stride(2)))
-        tdtype, cptr, sptr = DTYPE_CODE[cos.dtype], cos.data_ptr(), sin.data_ptr()
-    else:
-        tstrides, tdtype, cptr, sptr = None, KERNL_F32, None, None
-    with torch.cuda.device(x2d.device):
-        st = lib.kernl_linear_decode_fwd(
-            x2d.data_ptr(), None if rms_weight is None else rms_weight.data_ptr(), float(eps), weight.data_ptr(),
-            None if bias is None else bias.data_ptr(), None if residual2d is None else residual2d.data_ptr(),
-            out2d.data_ptr(), M, N, K, _arr(x2d.stride()), _arr(out2d.stride()),
-            None if residual2d is None else _arr(residual2d.stride()), cptr, sptr, int(head_dim), int(rope_cols),
-            int(rows_per_batch), tstrides, tdtype, DTYPE_CODE[x2d.dtype], _stream(x2d),
-        )
-    _check(st, "kernl_linear_decode_fwd")
+    (_host or host()).linear_decode_fwd(x2d, rms_weight, eps, weight, bias, residual2d, out2d, cos, sin, head_dim, rope_cols, rows_per_batch)
 
 
 def linear_splitk_workspace_bytes(x2d, weight) -> int:
@@ -577,34 +502,11 @@ def linear_fewrow_workspace_bytes(M: int, N: int, K: int, gated: bool = False, r
 def linear_fewrow_fwd(x2d, weight, bias, residual2d, out2d, activation: int, workspace=None, rms_weight=None,
                       eps: float = 0.0, gated: bool = False, cos=None, sin=None, head_dim: int = 0, rope_cols: int = 0,
                       rows_per_batch: int = 1) -> None:
-    """`workspace`: device tensor of at least `linear_fewrow_workspace_bytes` bytes; allocated here when None (a fresh
-    allocation per call: stream-ordered, so calls on different streams never share one).  cos / sin as for
+    """`workspace`: device tensor of at least `linear_fewrow_workspace_bytes` bytes; allocated in the call when None (a
+    fresh allocation per call: stream-ordered, so calls on different streams never share one).  cos / sin as for
     `linear_decode_fwd`; `gated`: weight and bias interleaved as for `linear_glu_fwd`, out2d half as wide."""
-    _require_gpu(x2d, weight, bias, residual2d, out2d, workspace, rms_weight, cos, sin)
-    M, K = x2d.shape
-    N = out2d.shape[1]
-    lib = load()
-    if workspace is None:
-        need = linear_fewrow_workspace_bytes(M, N, K, gated, cos is not None)
-        if need:
-            workspace = torch.empty(need, dtype=torch.uint8, device=x2d.device)
-    ws_ptr = None if workspace is None else workspace.data_ptr()
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    if cos is not None:
-        tstrides = _arr((0 if cos.shape[0] == 1 else cos.stride(0), cos.stride(1), cos.stride(2)))
-        tdtype, cptr, sptr = DTYPE_CODE[cos.dtype], cos.data_ptr(), sin.data_ptr()
-    else:
-        tstrides, tdtype, cptr, sptr = None, KERNL_F32, None, None
-    entry = lib.kernl_linear_fewrow_fwd if weight.element_size() == 2 else lib.kernl_linear_fewrow_w8_fwd
-    with torch.cuda.device(x2d.device):
-        st = entry(
-            x2d.data_ptr(), None if rms_weight is None else rms_weight.data_ptr(), float(eps), weight.data_ptr(),
-            None if bias is None else bias.data_ptr(), None if residual2d is None else residual2d.data_ptr(),
-            out2d.data_ptr(), ws_ptr, ws_bytes, M, N, K, _arr(x2d.stride()), _arr(out2d.stride()),
-            None if residual2d is None else _arr(residual2d.stride()), cptr, sptr, int(head_dim), int(rope_cols),
-            int(rows_per_batch), tstrides, tdtype, int(activation), int(bool(gated)), DTYPE_CODE[x2d.dtype], _stream(x2d),
-        )
-    _check(st, "kernl_linear_fewrow_fwd")
+    (_host or host()).linear_fewrow_fwd(x2d, weight, bias, residual2d, out2d, activation, workspace, rms_weight, eps, gated, cos, sin,
+                                        head_dim, rope_cols, rows_per_batch)
 
 
 def linear_glu_fwd(x2d, weight_interleaved, bias_interleaved, out2d, activation: int) -> None:
@@ -622,24 +524,4 @@ def linear_glu_fwd(x2d, weight_interleaved, bias_interleaved, out2d, activation:
 
 
 def layernorm_fwd(x2d, weight, bias, out2d, mean, rstd, eps: float, is_rms: bool, residual2d=None) -> None:
-    _require_gpu(x2d, weight, bias, out2d, mean, rstd, residual2d)
-    M, N = x2d.shape
-    lib = load()
-    with torch.cuda.device(x2d.device):
-        if residual2d is None:
-            st = lib.kernl_layernorm_fwd(
-                x2d.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out2d.data_ptr(),
-                None if mean is None else mean.data_ptr(), None if rstd is None else rstd.data_ptr(),
-                M, N, x2d.stride(0), x2d.stride(1), out2d.stride(0), out2d.stride(1),
-                float(eps), int(bool(is_rms)), DTYPE_CODE[x2d.dtype], _stream(x2d),
-            )
-            _check(st, "kernl_layernorm_fwd")
-        else:
-            st = lib.kernl_add_layernorm_fwd(
-                x2d.data_ptr(), residual2d.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(),
-                out2d.data_ptr(), None if mean is None else mean.data_ptr(), None if rstd is None else rstd.data_ptr(),
-                M, N, x2d.stride(0), x2d.stride(1), residual2d.stride(0), residual2d.stride(1),
-                out2d.stride(0), out2d.stride(1),
-                float(eps), int(bool(is_rms)), DTYPE_CODE[x2d.dtype], _stream(x2d),
-            )
-            _check(st, "kernl_add_layernorm_fwd")
+    (_host or host()).layernorm_fwd(x2d, weight, bias, out2d, mean, rstd, eps, is_rms, residual2d)

@@ -126,4 +126,7 @@ def attention_forward(
 ):
     """Reference: attention.py:532-541; `start_position` as in `triton_fa` of
     experimental/llama-v2/kernel/fused_kernel_attention.py:113-146."""
+    out = _lib.host().op_attention(q, k, v, output, attention_mask, sm_scale, is_causal, start_position)  # None: not a plain call
+    if out is not None:
+        return out
     return Attention.apply(q, k, v, output, sm_scale, is_causal, attention_mask, start_position)

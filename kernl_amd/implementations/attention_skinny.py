@@ -83,4 +83,7 @@ def skinny_attention_forward(
     attention_mask: Optional[torch.Tensor] = None,
 ):
     """Reference: attention_skinny.py:539-548."""
+    out = _lib.host().op_skinny_attention(q, k, v, output, attention_mask, sm_scale, is_causal)  # None: not a plain call
+    if out is not None:
+        return out
     return SkinnyAttention.apply(q, k, v, output, sm_scale, is_causal, attention_mask)

@@ -68,6 +68,9 @@ def layer_norm(
     use_rms_norm: bool = False,
 ):
     """Reference: layer_norm.py:338-346."""
+    out = _lib.host().op_layer_norm(x, weight, bias, eps, use_rms_norm, None)  # None: not a plain call
+    if out is not None:
+        return out
     return LayerNorm.apply(x, weight, bias, eps, implementation, use_rms_norm)
 
 
@@ -81,6 +84,9 @@ def add_layer_norm(
 ):
     """LayerNorm(x + residual) in one pass over HBM.  No reference counterpart: there the add is a separate
     eager op in front of every LayerNorm."""
+    out = _lib.host().op_layer_norm(x, weight, bias, eps, use_rms_norm, residual)
+    if out is not None:
+        return out
     return LayerNorm.apply(x, weight, bias, eps, None, use_rms_norm, residual)
 
 

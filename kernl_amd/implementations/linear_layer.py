@@ -136,6 +136,14 @@ def linear_layer(
     act_inputs: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """Reference: linear_layer.py:285-292."""
+    code = ACTIVATIONS.get(activation, _lib.ACT_NONE)
+    out = _lib.host().op_linear(x, weight, bias, code, act_inputs, SMALL_PROBLEM_KERNELS)  # None: not a plain call
+    if out is not None:
+        if type(out) is not tuple:
+            return out
+        x2d, out2d, out = out
+        _lib.linear_fewrow_fwd(x2d, weight, bias, None, out2d, code)
+        return out
     return LinearLayer.apply(x, weight, bias, activation, act_inputs)
 
 
@@ -215,6 +223,15 @@ def rms_linear_layer(
     RMSNorm kernel and multiplied by the linear kernels."""
     from kernl_amd.implementations.layer_norm import layer_norm
 
+    plan = None if rms_weight is None else _lib.host().plan_few_rows(x, weight, bias, rms_weight, None, gated, None, None, 0, 0)
+    if plan is not None:  # the checks and allocations of the few-row paths below, made in one native call
+        x_, _, out2d, out, stream_k, _ = plan
+        eps, code = rms_eps(x.dtype, eps), ACTIVATIONS.get(activation, _lib.ACT_NONE)
+        if stream_k:
+            _lib.linear_fewrow_fwd(x_, weight, bias, None, out2d, code, rms_weight=rms_weight, eps=eps, gated=gated)
+        else:
+            _lib.linear_rms_fwd(x_, rms_weight, eps, weight, bias, out2d, code, gated)
+        return out
     assert x.dtype == weight.dtype == rms_weight.dtype and x.dtype in (torch.float16, torch.bfloat16)
     assert weight.is_contiguous() and rms_weight.is_contiguous() and rms_weight.shape[0] == x.shape[-1]
     x_ = x if x.ndim == 2 else x.reshape(-1, x.shape[-1])
@@ -372,6 +389,16 @@ def decode_linear_layer(
     counts as one batch entry); residual of the output's shape.  Reference: `rms_matmul_rbe_qkv_wrapper`,
     experimental/llama-v2/kernel/fused_kernel_proj_qkv.py:289-344 (RMSNorm prologue + query/key/value projection +
     rotation of the query and key columns in one kernel)."""
+    plan = _lib.host().plan_few_rows(x, weight, bias, rms_weight, residual, False, cos, sin, head_dim, rope_cols)
+    if plan is not None:  # the checks and allocations below, made in one native call
+        x_, res_, out2d, out, stream_k, rows_per_batch = plan
+        eps = eps if rms_weight is None else rms_eps(x.dtype, eps)
+        if stream_k:
+            _lib.linear_fewrow_fwd(x_, weight, bias, res_, out2d, _lib.ACT_NONE, rms_weight=rms_weight, eps=eps, cos=cos, sin=sin,
+                                   head_dim=head_dim, rope_cols=rope_cols, rows_per_batch=rows_per_batch)
+        else:
+            _lib.linear_decode_fwd(x_, rms_weight, eps, weight, bias, res_, out2d, cos, sin, head_dim, rope_cols, rows_per_batch)
+        return out
     assert decode_linear_supported(x, weight, head_dim if cos is not None else None), \
         "decode_linear_layer: at most 64 rows of 16-bit x (128 against a large weight), K a multiple of 64"
     assert (cos is None) == (sin is None)
