@@ -275,6 +275,27 @@ int kernl_linear_residual_fwd(const void *x, const void *w, const void *bias, co
                               const int64_t residual_strides[2], int dtype, void *stream);
 
 /*
+ * A LayerNorm between linear layers without a launch of its own, for small problems (a few hundred rows; widths that are a
+ * multiple of 32, up to 1024).  The layer in front of the norm,
+ *     kernl_linear_norm_add_fwd:    out = s = round(x @ w^T + bias + residual),
+ *                                   out_stats[m][n / 32] = (sum, sum of squared deviations from their mean) of s[m][n .. n + 31],
+ * leaves the rows un-normalised; the layer behind,
+ *     kernl_linear_norm_apply_fwd:  out = act(LN(x) @ w^T + bias) = act(rstd (x @ w_folded^T - mean colsum) + bias32),
+ * with w_folded = w * gamma (columns), colsum[n] = sum_k w_folded[n][k], bias32 = bias + w @ beta, normalises its sums.  A
+ * residual that is such a deferred norm itself (residual_stats given) is normalised on the fly: residual stands for
+ * (residual - mean) * rstd * gamma + beta.  kernl_linear_norm_kind: 0 where the small-problem kernels do not take M x N x K.
+ * The reference runs a LayerNorm kernel between its linear kernels (src/kernl/implementations/layer_norm.py:279-335).
+ */
+int kernl_linear_norm_kind(int64_t M, int64_t N, int64_t K);
+int kernl_linear_norm_add_fwd(const void *x, const void *w, const void *bias, const void *residual, const float *residual_stats,
+                              const void *gamma, const void *beta, float eps, void *out, float *out_stats, int64_t M, int64_t N,
+                              int64_t K, int64_t x_row_stride, int64_t out_row_stride, int64_t residual_row_stride, int dtype,
+                              void *stream);
+int kernl_linear_norm_apply_fwd(const void *x, const float *x_stats, float eps, const void *w_folded, const float *colsum,
+                                const float *bias32, void *out, int64_t M, int64_t N, int64_t K, int64_t x_row_stride,
+                                int64_t out_row_stride, int activation, int dtype, void *stream);
+
+/*
  * Whether kernl_linear_fwd runs M x N x K (16-bit, plain epilogue, x with unit feature stride) on one of its
  * small-problem kernels, and which: 0 = no; otherwise the kernl_linear_force_tile value of the kernel (10 .. 15).  A
  * caller that would otherwise route such a shape to the stream-K or split-K entry points (kernl_linear_fewrow_fwd,

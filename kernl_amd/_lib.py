@@ -41,6 +41,9 @@ EXPORTED_SYMBOLS = (
     "kernl_linear_scaled_fwd",
     "kernl_linear_residual_fwd",
     "kernl_linear_wide_kind",
+    "kernl_linear_norm_kind",
+    "kernl_linear_norm_add_fwd",
+    "kernl_linear_norm_apply_fwd",
     "kernl_embedding_layernorm_fwd",
     "kernl_linear_decode_fwd",
     "kernl_linear_splitk_workspace_bytes",
@@ -161,6 +164,12 @@ def load() -> ctypes.CDLL:
     lib.kernl_linear_small_kind.argtypes = [_i64] * 3
     lib.kernl_linear_wide_kind.restype = ctypes.c_int
     lib.kernl_linear_wide_kind.argtypes = [_i64] * 3
+    lib.kernl_linear_norm_kind.restype = ctypes.c_int
+    lib.kernl_linear_norm_kind.argtypes = [_i64] * 3
+    lib.kernl_linear_norm_add_fwd.restype = ctypes.c_int
+    lib.kernl_linear_norm_add_fwd.argtypes = [_vp] * 7 + [ctypes.c_float, _vp, _vp] + [_i64] * 6 + [ctypes.c_int, _vp]
+    lib.kernl_linear_norm_apply_fwd.restype = ctypes.c_int
+    lib.kernl_linear_norm_apply_fwd.argtypes = [_vp, _vp, ctypes.c_float] + [_vp] * 4 + [_i64] * 5 + [ctypes.c_int, ctypes.c_int, _vp]
     lib.kernl_linear_glu_fwd.restype = ctypes.c_int
     lib.kernl_linear_glu_fwd.argtypes = [_vp] * 4 + [_i64] * 3 + [_i64p] * 2 + [ctypes.c_int, ctypes.c_int, _vp]
     lib.kernl_layernorm_fwd.restype = ctypes.c_int
@@ -307,6 +316,50 @@ def linear_wide_kind(M: int, N: int, K: int) -> int:
 
 def linear_fwd(x2d, weight, bias, out2d, act_in2d, activation: int) -> None:
     (_host or host()).linear_fwd(x2d, weight, bias, out2d, act_in2d, activation)
+
+
+def linear_norm_kind(M: int, N: int, K: int) -> int:
+    """Non-zero when both deferred-norm entry points take an M x N x K problem."""
+    return int(load().kernl_linear_norm_kind(int(M), int(N), int(K)))
+
+
+def linear_norm_add_fwd(x2d, weight, bias, residual2d, residual_stats, gamma, beta, eps: float, out2d, out_stats) -> None:
+    """out = x @ w^T + bias + residual with the statistics of its rows; with `residual_stats` the residual is the
+    un-normalised rows of a deferred LayerNorm (gamma, beta, eps)."""
+    _require_gpu(x2d, weight, bias, residual2d, residual_stats, gamma, beta, out2d, out_stats)
+    M, K = x2d.shape
+    N = weight.shape[0]
+    if any(t is not None and (t.dtype != torch.float32 or t.numel() != M * N // 16 or not t.is_contiguous()) for t in (residual_stats, out_stats)):
+        raise ValueError("statistics are contiguous fp32 [rows, columns / 32, 2]")
+    if x2d.stride(1) != 1 or residual2d.stride(1) != 1 or out2d.stride(1) != 1 or not weight.is_contiguous():
+        raise ValueError("unit feature strides and a contiguous weight")
+    with torch.cuda.device(x2d.device):
+        st = load().kernl_linear_norm_add_fwd(
+            x2d.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), residual2d.data_ptr(),
+            None if residual_stats is None else residual_stats.data_ptr(), None if gamma is None else gamma.data_ptr(),
+            None if beta is None else beta.data_ptr(), float(eps), out2d.data_ptr(), out_stats.data_ptr(), M, N, K, x2d.stride(0),
+            out2d.stride(0), residual2d.stride(0), DTYPE_CODE[x2d.dtype], _stream(x2d),
+        )
+    _check(st, "kernl_linear_norm_add_fwd")
+
+
+def linear_norm_apply_fwd(x2d, x_stats, eps: float, weight_folded, colsum, bias32, out2d, activation: int) -> None:
+    """out = act(LN(x) @ w^T + bias) of un-normalised rows x with their statistics and the folded parameters."""
+    _require_gpu(x2d, x_stats, weight_folded, colsum, bias32, out2d)
+    M, K = x2d.shape
+    N = weight_folded.shape[0]
+    if x_stats.dtype != torch.float32 or x_stats.numel() != M * K // 16 or not x_stats.is_contiguous():
+        raise ValueError("statistics are contiguous fp32 [rows, columns / 32, 2]")
+    if any(t.dtype != torch.float32 or t.numel() != N or not t.is_contiguous() for t in (colsum, bias32)):
+        raise ValueError("colsum and bias32 are contiguous fp32 vectors with one entry per column")
+    if x2d.stride(1) != 1 or out2d.stride(1) != 1 or not weight_folded.is_contiguous():
+        raise ValueError("unit feature strides and a contiguous weight")
+    with torch.cuda.device(x2d.device):
+        st = load().kernl_linear_norm_apply_fwd(
+            x2d.data_ptr(), x_stats.data_ptr(), float(eps), weight_folded.data_ptr(), colsum.data_ptr(), bias32.data_ptr(),
+            out2d.data_ptr(), M, N, K, x2d.stride(0), out2d.stride(0), int(activation), DTYPE_CODE[x2d.dtype], _stream(x2d),
+        )
+    _check(st, "kernl_linear_norm_apply_fwd")
 
 
 def linear_w8_supported(x2d, weight8) -> bool:

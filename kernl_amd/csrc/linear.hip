@@ -1,5 +1,6 @@
 // Fused linear layer: dispatch and C entry points (kernels and launchers: linear_kernels.h).
 #include "linear_kernels.h"
+#include "norm_fold.h"
 
 namespace kernl {
 
@@ -19,11 +20,11 @@ static int linear_mfma_dispatch(const LinearArgs &a) {
     // small problems: one launch of small tiles over the whole K (10 / 11 / 15 force its 32 x 64 / 64 x 64 / 64 x 128 form)
     if (pick == 0 && !(a.act & kGluBit)) pick = small_problem_kind(a.M, a.N, a.K);
     if ((pick == 12 || pick == 13 || pick == 14) && !(a.act & kGluBit)) {
-        run_small_dealt(a, kDtype, pick == 12 ? 16 : pick == 13 ? 32 : 64);
+        run_small_dealt(a, kDtype, pick == 12 ? 16 : pick == 13 ? 32 : 64, kNormNone, NormFold());
         return check_launch("linear (small tiles, dealt k-tiles)");
     }
     if ((pick == 10 || pick == 11 || pick == 15) && !(a.act & kGluBit)) {
-        run_small(a, kDtype, pick == 10 ? 32 : 64, pick == 15 ? 128 : 64);
+        run_small(a, kDtype, pick == 10 ? 32 : 64, pick == 15 ? 128 : 64, kNormNone, NormFold());
         return check_launch("linear (small tiles)");
     }
     if (pick == 0 || pick == 9) pick = pick_tile(a.M, a.N, a.K, (a.act & kGluBit) != 0);
@@ -277,6 +278,84 @@ extern "C" int kernl_linear_residual_fwd(const void *x, const void *w, const voi
     else if (pick == 7) run_wide_half(a, dtype, 256);
     else run_wide_half(a, dtype, 192);
     return check_launch("linear + residual");
+}
+
+// Both sides of a deferred LayerNorm run on the small-problem kernels (10 .. 15).
+static void run_norm_small(const kernl::LinearArgs &a, int dtype, int mode, const kernl::NormFold &nf) {
+    using namespace kernl;
+    const int pick = g_linear_force_tile >= 10 && g_linear_force_tile <= 15 ? g_linear_force_tile : small_problem_kind(a.M, a.N, a.K);
+    if (pick == 12 || pick == 13 || pick == 14) run_small_dealt(a, dtype, pick == 12 ? 16 : pick == 13 ? 32 : 64, mode, nf);
+    else run_small(a, dtype, pick == 10 ? 32 : 64, pick == 15 ? 128 : 64, mode, nf);
+}
+
+extern "C" int kernl_linear_norm_kind(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || N % kernl::kNormGroup != 0 || K % 8 != 0) return 0;
+    return kernl::small_problem_kind(M, N, K);
+}
+
+static int norm_arguments_bad(const char *what, const void *x, const void *w, const void *out, int64_t M, int64_t N, int64_t K, int64_t x_rs,
+                              int64_t out_rs, int dtype) {
+    using namespace kernl;
+    if (x == nullptr || w == nullptr || out == nullptr) return set_error(KERNL_ERR_INVALID_ARG, "%s: x, w and out must not be NULL", what);
+    if (M < 0 || N <= 0 || K <= 0)
+        return set_error(KERNL_ERR_INVALID_ARG, "%s: bad sizes M=%lld N=%lld K=%lld", what, (long long)M, (long long)N, (long long)K);
+    if (dtype != KERNL_F16 && dtype != KERNL_BF16) return set_error(KERNL_ERR_UNSUPPORTED, "%s: only f16 and bf16 are supported, got dtype %d", what, dtype);
+    if (!aligned16(x) || !aligned16(w) || x_rs % 8 != 0 || x_rs < K || x_rs >= (1 << 22) || K >= (1 << 22) || ((uintptr_t)out & 7) != 0 || out_rs % 4 != 0 || out_rs < N)
+        return set_error(KERNL_ERR_UNSUPPORTED, "%s: x and w need 16-byte aligned rows, out 8-byte aligned ones", what);
+    if (M > 0 && kernl_linear_norm_kind(M, N, K) == 0)
+        return set_error(KERNL_ERR_UNSUPPORTED, "%s: M=%lld N=%lld K=%lld is not a small problem (kernl_linear_norm_kind)", what, (long long)M,
+                         (long long)N, (long long)K);
+    return KERNL_OK;
+}
+
+extern "C" int kernl_linear_norm_apply_fwd(const void *x, const float *x_stats, float eps, const void *w_folded, const float *colsum,
+                                           const float *bias32, void *out, int64_t M, int64_t N, int64_t K, int64_t x_row_stride,
+                                           int64_t out_row_stride, int activation, int dtype, void *stream) {
+    using namespace kernl;
+    if (x_stats == nullptr || colsum == nullptr || bias32 == nullptr || !aligned16(x_stats) || !aligned16(colsum) || !aligned16(bias32))
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (deferred norm): x_stats, colsum and bias32 must be 16-byte aligned fp32 arrays");
+    if (activation < KERNL_ACT_NONE || activation > KERNL_ACT_SILU)
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (deferred norm): unknown activation %d", activation);
+    const int bad = norm_arguments_bad("linear (deferred norm)", x, w_folded, out, M, N, K, x_row_stride, out_row_stride, dtype);
+    if (bad != KERNL_OK) return bad;
+    if (K % kNormGroup != 0 || K > kNormGroup * kNormMaxGroups)
+        return set_error(KERNL_ERR_UNSUPPORTED, "linear (deferred norm): normalised width %lld is no multiple of 32 up to 1024", (long long)K);
+    if (M == 0) return KERNL_OK;
+    LinearArgs a;
+    a.x = x; a.w = w_folded; a.bias = nullptr; a.out = out; a.act_in = nullptr;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K;
+    a.x_rs = x_row_stride; a.x_cs = 1; a.out_rs = out_row_stride; a.out_cs = 1; a.ai_rs = a.ai_cs = 0;
+    a.act = activation; a.st = static_cast<hipStream_t>(stream);
+    NormFold nf;
+    nf.in_stats = x_stats; nf.in_groups = (int)(K / kNormGroup); nf.eps = eps; nf.colsum = colsum; nf.bias32 = bias32;
+    run_norm_small(a, dtype, kNormApply, nf);
+    return check_launch("linear (deferred norm)");
+}
+
+extern "C" int kernl_linear_norm_add_fwd(const void *x, const void *w, const void *bias, const void *residual, const float *residual_stats,
+                                         const void *gamma, const void *beta, float eps, void *out, float *out_stats, int64_t M, int64_t N,
+                                         int64_t K, int64_t x_row_stride, int64_t out_row_stride, int64_t residual_row_stride, int dtype,
+                                         void *stream) {
+    using namespace kernl;
+    if (residual == nullptr || out_stats == nullptr || ((uintptr_t)residual & 7) != 0 || residual_row_stride % 4 != 0 || !aligned16(out_stats))
+        return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: residual needs 8-byte aligned rows, out_stats a 16-byte aligned array");
+    if (residual_stats != nullptr && (gamma == nullptr || !aligned16(residual_stats) || ((uintptr_t)gamma & 7) != 0 || ((uintptr_t)beta & 7) != 0))
+        return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: a deferred residual comes with its statistics and aligned norm parameters");
+    const int bad = norm_arguments_bad("linear + addition + statistics", x, w, out, M, N, K, x_row_stride, out_row_stride, dtype);
+    if (bad != KERNL_OK) return bad;
+    if (N > kNormGroup * kNormMaxGroups)
+        return set_error(KERNL_ERR_UNSUPPORTED, "linear + addition + statistics: width %lld exceeds 1024", (long long)N);
+    if (M == 0) return KERNL_OK;
+    LinearArgs a;
+    a.x = x; a.w = w; a.bias = bias; a.out = out; a.act_in = nullptr;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K;
+    a.x_rs = x_row_stride; a.x_cs = 1; a.out_rs = out_row_stride; a.out_cs = 1; a.ai_rs = a.ai_cs = 0;
+    a.act = KERNL_ACT_NONE; a.st = static_cast<hipStream_t>(stream);
+    NormFold nf;
+    nf.in_stats = residual_stats; nf.in_groups = (int)(N / kNormGroup); nf.eps = eps;
+    nf.residual = residual; nf.res_rs = residual_row_stride; nf.gamma = gamma; nf.beta = beta; nf.out_stats = out_stats;
+    run_norm_small(a, dtype, kNormAdd, nf);
+    return check_launch("linear + addition + statistics");
 }
 
 extern "C" int kernl_linear_w8_fwd(const void *x, const void *w8, const void *bias, void *out, void *act_in, int64_t M,

@@ -31,8 +31,9 @@ void run_wide_w8(const LinearArgs &a);                               // fp8 e5m2
 void run_wide_half(const LinearArgs &a, int dtype, int cols);        // 128-row tiles
 void run_wide_half_w8(const LinearArgs &a);
 void run_half_split(const LinearArgs &a, const HalfSplitPlan &p, float *part, int dtype);
-void run_small(const LinearArgs &a, int dtype, int rows, int cols);  // 32 x 64, 64 x 64 or 64 x 128 tiles over the whole K (linear_small.hip)
-void run_small_dealt(const LinearArgs &a, int dtype, int rows);      // 16-, 32- or 64-row, 32-column tiles, k-tiles dealt to the waves
+struct NormFold;
+void run_small(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf);  // mode: norm_fold.h; 32 x 64, 64 x 64 or 64 x 128 tiles over the whole K (linear_small.hip)
+void run_small_dealt(const LinearArgs &a, int dtype, int rows, int mode, const NormFold &nf);      // 16-, 32- or 64-row, 32-column tiles, k-tiles dealt to the waves
 
 
 // ----------------------------------------------------------------------------------------------------

@@ -12,6 +12,7 @@
 // ahead, one barrier per k-tile and waits by count.  A last k-tile that reaches beyond K has the chunks that
 // start there pointed out of range (zeros, in both operands).
 #include "linear_kernels.h"
+#include "norm_fold.h"
 
 namespace kernl {
 
@@ -19,26 +20,39 @@ namespace kernl {
 template <typename T>
 __device__ __forceinline__ void load_bias4(const T *__restrict__ bias, int n, int N, bool vec_ok, float (&dst)[4]) {
     if (bias != nullptr && vec_ok && n + 4 <= N) {
-        const u32x2 raw = *reinterpret_cast<const u32x2 *>(bias + n);
-        typedef T pair_t __attribute__((ext_vector_type(2)));
-        const uint32_t r0 = raw[0], r1 = raw[1];  // (a bit cast straight from a vector ELEMENT reads the vector's first one)
-        const pair_t lo = __builtin_bit_cast(pair_t, r0), hi = __builtin_bit_cast(pair_t, r1);
-        dst[0] = to_float(lo[0]); dst[1] = to_float(lo[1]); dst[2] = to_float(hi[0]); dst[3] = to_float(hi[1]);
+        unpack4<T>(*reinterpret_cast<const u32x2 *>(bias + n), dst);
         return;
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) dst[e] = (bias != nullptr && n + e < N) ? to_float(bias[n + e]) : 0.0f;
 }
 
+// Row statistics on their way to the epilogue: the pairs of a row tile lie in one piece of memory and travel to LDS in
+// front of the first k-tile, `per_wave` KB-sized loads per wave (pieces past the end arrive as zeros or are not asked for).
+template <int BM>
+__device__ __forceinline__ void request_norm_stats(const NormFold &nf, int m0, int rows, uint32_t lds, int wave, int lane) {
+    constexpr int PER_WAVE = BM * kNormMaxGroups * 8 / 4096;
+    static_assert(PER_WAVE >= 1, "whole KB per wave");
+    const uint64_t addr = (uint64_t)(uintptr_t)(nf.in_stats + (int64_t)m0 * nf.in_groups * 2);
+    const u32x4 rsrc = {(uint32_t)addr, (uint32_t)(addr >> 32) & 0xFFFFu, (uint32_t)(rows * nf.in_groups * 8), 0x00020000u};
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; ++i) {
+        const int piece = wave * PER_WAVE + i;
+        if (piece * 1024 < rows * nf.in_groups * 8)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                         :: "s"(lds + piece * 1024), "v"(piece * 1024 + lane * 16), "s"(rsrc) : "memory", "m0");
+    }
+}
+
 constexpr int kSmallBK = 64;  // measured against 128-wide k-tiles in 6 / 4 stages: 5-10 % faster
 // ring stages of the shared-tile kernel: 8 of them, or as many as fit 144 KB
 constexpr int small_stages(int bm, int bn) { return (bm + bn) * kSmallBK * 2 * 8 <= 144 * 1024 ? 8 : (144 * 1024) / ((bm + bn) * kSmallBK * 2); }
 
-template <typename T, int BM, int BN>
+template <typename T, int BM, int BN, int MODE>
 __global__ void __launch_bounds__(256, 1)
 linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
                     T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs, int64_t out_cs,
-                    int64_t ai_rs, int64_t ai_cs, int act, int tiles_m) {
+                    int64_t ai_rs, int64_t ai_cs, int act, int tiles_m, NormFold nf) {
     typedef typename Vec8<T>::type vec8;
     constexpr int BK = kSmallBK, RB = BK * 2, CPR = BK / 8, S = small_stages(BM, BN), KSTEPS = BK / 32;
     static_assert(RB == SmallTileMap::ROW_BYTES && CPR == SmallTileMap::CHUNKS_PER_ROW, "tile rows as the tile map lays them out");
@@ -137,15 +151,38 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
     for (int i = 0; i < NBM; ++i)
 #pragma unroll
         for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
-    // the bias of the lane's columns, requested before anything else: fetched where it is used, every block of the
-    // epilogue would cost the wave a memory round trip of its own
+    // what the epilogue needs of the lane's rows and columns, requested before anything else: fetched where it is used,
+    // every block of the epilogue would cost the wave a memory round trip of its own
     float bz[NBN][4];
+    f32x4 cs[MODE == kNormApply ? NBN : 1];
+    u32x2 res[MODE == kNormAdd ? NBM : 1][MODE == kNormAdd ? NBN : 1], gam[MODE == kNormAdd ? NBN : 1], bet[MODE == kNormAdd ? NBN : 1];
     const bool bias_vec = ((uintptr_t)bias & 7) == 0;
 #pragma unroll
     for (int j = 0; j < NBN; ++j) {
         const int n = n0 + wave_n * (BN / 2) + 16 * j + 4 * g;
-        load_bias4<T>(bias, n, N, bias_vec, bz[j]);
+        if (MODE == kNormApply) {
+            const bool in = n < N;  // (N is a multiple of 32 with a norm)
+            const f32x4 b32 = in ? *reinterpret_cast<const f32x4 *>(nf.bias32 + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            cs[j] = in ? *reinterpret_cast<const f32x4 *>(nf.colsum + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bz[j][e] = b32[e];
+        } else {
+            load_bias4<T>(bias, n, N, bias_vec, bz[j]);
+        }
+        if (MODE == kNormAdd) {
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) {
+                const int m = m0 + wave_m * (BM / 2) + 16 * i + r;
+                res[i][j] = m < M && n < N ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + (int64_t)m * nf.res_rs + n) : u32x2{0, 0};
+            }
+            if (nf.in_stats != nullptr) {
+                gam[j] = n < N ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.gamma) + n) : u32x2{0, 0};
+                bet[j] = n < N && nf.beta != nullptr ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.beta) + n) : u32x2{0, 0};
+            }
+        }
     }
+    const bool row_stats = MODE == kNormApply || (MODE == kNormAdd && nf.in_stats != nullptr);
+    if (MODE != kNormNone && row_stats) request_norm_stats<BM>(nf, m0, rows_x, lds_base + S * STAGE, wave, lane);
 
 #pragma unroll
     for (int kt = 0; kt < S - 1; ++kt) request(kt, kt);
@@ -174,6 +211,89 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
         stage = stage == S - 1 ? 0 : stage + 1;
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the out-of-range requests of the last rounds are done with before the LDS goes away
+
+    if (MODE != kNormNone) {
+        // mean and 1 / std of the lane's rows: the four lanes of a row take a quarter of its statistics pairs each
+        float mean[NBM], rstd[NBM];
+        if (row_stats) {
+            const unsigned char *st = smem + S * STAGE;
+            const int groups = nf.in_groups;
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) {
+                const f32x2 *row = reinterpret_cast<const f32x2 *>(st) + (wave_m * (BM / 2) + 16 * i + r) * groups;
+                const float pivot = row[0][0] * (1.0f / kNormGroup);
+                NormMerge mg;
+                for (int p = g; p < groups; p += 4) mg.take(row[p], pivot);
+                mg.d = halves32_sum(mg.d + __shfl_xor(mg.d, 16));
+                mg.dd = halves32_sum(mg.dd + __shfl_xor(mg.dd, 16));
+                mg.m2 = halves32_sum(mg.m2 + __shfl_xor(mg.m2, 16));
+                mg.finish(pivot, groups, nf.eps, mean[i], rstd[i]);
+            }
+        }
+        auto finish_norm = [&](auto act_c) __attribute__((always_inline)) {
+            constexpr int ACT = decltype(act_c)::value;
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) {
+                const int m = m0 + wave_m * (BM / 2) + 16 * i + r;
+                float y[NBN][4];
+#pragma unroll
+                for (int j = 0; j < NBN; ++j) {
+                    const int n = n0 + wave_n * (BN / 2) + 16 * j + 4 * g;
+                    float h[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if (MODE == kNormAdd) {
+                        unpack4<T>(res[i][j], h);
+                        if (row_stats) {
+                            float gm[4], bt[4];
+                            unpack4<T>(gam[j], gm);
+                            unpack4<T>(bet[j], bt);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) h[e] = fmaf((h[e] - mean[i]) * rstd[i], gm[e], bt[e]);
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (MODE == kNormApply) y[j][e] = apply_act16(fmaf(fmaf(-mean[i], cs[j][e], acc[i][j][e]), rstd[i], bz[j][e]), ACT);
+                        else y[j][e] = to_float(from_float<T>(acc[i][j][e] + bz[j][e] + h[e]));
+                    }
+                    if (m < M && n < N)
+                        *reinterpret_cast<u32x2 *>(out + (int64_t)m * out_rs + n) = u32x2{pack2<T>(y[j][0], y[j][1]), pack2<T>(y[j][2], y[j][3])};
+                }
+                if (MODE == kNormAdd) {
+                    // statistics of the stored values: 32 columns are two blocks of the row's four lanes
+#pragma unroll
+                    for (int j = 0; j < NBN; j += 2) {
+                        float sum = 0.0f, m2 = 0.0f;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) sum += y[j][e] + y[j + 1][e];
+                        sum = halves32_sum(sum + __shfl_xor(sum, 16));
+                        const float mu = sum * (1.0f / kNormGroup);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float a = y[j][e] - mu, b = y[j + 1][e] - mu;
+                            m2 = fmaf(a, a, fmaf(b, b, m2));
+                        }
+                        m2 = halves32_sum(m2 + __shfl_xor(m2, 16));
+                        const int n = n0 + wave_n * (BN / 2) + 16 * j;
+                        if (g == 0 && m < M && n < N)
+                            *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / kNormGroup) + n / kNormGroup) * 2) = f32x2{sum, m2};
+                    }
+                }
+            }
+        };
+        if (MODE == kNormAdd) {
+            finish_norm(IntC<KERNL_ACT_NONE>());
+            return;
+        }
+        switch (act) {
+            case KERNL_ACT_RELU: finish_norm(IntC<KERNL_ACT_RELU>()); break;
+            case KERNL_ACT_TANH: finish_norm(IntC<KERNL_ACT_TANH>()); break;
+            case KERNL_ACT_GELU_ERF: finish_norm(IntC<KERNL_ACT_GELU_ERF>()); break;
+            case KERNL_ACT_GELU_TANH: finish_norm(IntC<KERNL_ACT_GELU_TANH>()); break;
+            case KERNL_ACT_SILU: finish_norm(IntC<KERNL_ACT_SILU>()); break;
+            default: finish_norm(IntC<KERNL_ACT_NONE>()); break;
+        }
+        return;
+    }
 
     // ---- epilogue: bias, optional pre-activation, activation, one rounding; 4 consecutive columns per lane and block
     const bool out_vec = out_cs == 1 && (out_rs & 3) == 0 && ((uintptr_t)out & 7) == 0;
@@ -233,11 +353,11 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
 // a wave's ring: 32 KB, 36 KB for the 12 KB stages of 64 x 32 tiles (three of them)
 constexpr int small_ring_bytes(int bm, int bn) { return (bm + bn) == 96 ? 36 * 1024 : 32 * 1024; }
 
-template <typename T, int BM, int BN>
+template <typename T, int BM, int BN, int MODE>
 __global__ void __launch_bounds__(256, 1)
 linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias,
                           T *__restrict__ out, T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs,
-                          int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int act, int tiles_m) {
+                          int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int act, int tiles_m, NormFold nf) {
     typedef typename Vec8<T>::type vec8;
     constexpr int BK = 64, RB = BK * 2, CPR = BK / 8, WAVES = 4;
     static_assert(RB == SmallTileMap::ROW_BYTES && CPR == SmallTileMap::CHUNKS_PER_ROW, "tile rows as the tile map lays them out");
@@ -322,15 +442,37 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
 #pragma unroll
         for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // the bias of the columns this wave finishes in the epilogue, requested before anything else
-    constexpr int OWN = (NBM * NBN + WAVES - 1) / WAVES;  // blocks per wave in the epilogue: wave, wave + 4, ...
-    float bz[OWN][4];
-    const bool bias_vec = ((uintptr_t)bias & 7) == 0;
+    // In the epilogue thread t finishes columns 4 (t % 8) .. + 3 of the tile's rows t / 8, t / 8 + 32, ...: whole 64-byte row
+    // pieces per store, and a row's 32 columns meet in eight neighbouring lanes (statistics).  What it needs of them is
+    // requested before anything else.
+    static_assert(BN == kNormGroup, "a tile row is one statistics group");
+    constexpr int OWN = (BM + 31) / 32;
+    const int own_row = tid >> 3, n_own = n0 + 4 * (tid & 7);
+    float bz[4];
+    f32x4 cs = {0.0f, 0.0f, 0.0f, 0.0f};
+    u32x2 res[OWN], gam = {0, 0}, bet = {0, 0};
+    if (MODE == kNormApply) {  // (N is a multiple of 32 with a norm: every column of the tile exists)
+        const f32x4 b32 = *reinterpret_cast<const f32x4 *>(nf.bias32 + n_own);
+        cs = *reinterpret_cast<const f32x4 *>(nf.colsum + n_own);
 #pragma unroll
-    for (int t = 0; t < OWN; ++t) {
-        const int n = n0 + 16 * ((wave + WAVES * t) % NBN) + 4 * g;
-        load_bias4<T>(bias, n, N, bias_vec, bz[t]);
+        for (int e = 0; e < 4; ++e) bz[e] = b32[e];
+    } else {
+        load_bias4<T>(bias, n_own, N, ((uintptr_t)bias & 7) == 0, bz);
     }
+    const bool row_stats = MODE == kNormApply || (MODE == kNormAdd && nf.in_stats != nullptr);
+    if (MODE == kNormAdd) {
+#pragma unroll
+        for (int t = 0; t < OWN; ++t) {
+            const int m = m0 + own_row + 32 * t;
+            res[t] = own_row + 32 * t < rows_x ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + (int64_t)m * nf.res_rs + n_own) : u32x2{0, 0};
+        }
+        if (row_stats) {
+            gam = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.gamma) + n_own);
+            if (nf.beta != nullptr) bet = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.beta) + n_own);
+        }
+    }
+    if (MODE != kNormNone && row_stats)
+        request_norm_stats<BM>(nf, m0, rows_x, (uint32_t)(uintptr_t)(lds_void *)smem + WAVES * RING, wave, lane);
     const int mine = nk > wave ? (nk - wave + WAVES - 1) / WAVES : 0;  // k-tiles of this wave
 #pragma unroll
     for (int j = 0; j < S - 1; ++j) request(j, j);
@@ -375,20 +517,55 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     constexpr int ACT = decltype(act_c)::value;
 #pragma unroll
     for (int t = 0; t < OWN; ++t) {
-        const int b = wave + WAVES * t;
-        if (b >= NBM * NBN) break;
-        const int i = b / NBN, j = b % NBN;
-        const int m = m0 + 16 * i + r, n = n0 + 16 * j + 4 * g;
-        f32x4_acc sum = *reinterpret_cast<const f32x4_acc *>(red + (b * 64 + lane) * 4);
+        const int row = own_row + 32 * t;
+        if (BM < 32 && row >= BM) break;
+        // block (row / 16, (tid & 7) / 4), its lane (row % 16, tid & 3)
+        const int at = (((row >> 4) * NBN + ((tid & 7) >> 2)) * 64 + (tid & 3) * 16 + (row & 15)) * 4;
+        f32x4_acc sum = *reinterpret_cast<const f32x4_acc *>(red + at);
 #pragma unroll
-        for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_acc *>(red + ((w * (NBM * NBN) + b) * 64 + lane) * 4);
-        if (m >= M || n >= N) continue;
-        float v[4], y[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = sum[e] + bz[t][e];
-            y[e] = apply_act16(v[e], ACT);
+        for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_acc *>(red + w * (NBM * NBN) * 256 + at);
+        const int m = m0 + row, n = n_own;
+        float v[4], y[4], mean = 0.0f, rstd = 0.0f;
+        if (MODE != kNormNone && row_stats) {
+            const f32x2 *pairs = reinterpret_cast<const f32x2 *>(smem + WAVES * RING) + row * nf.in_groups;
+            const float pivot = pairs[0][0] * (1.0f / kNormGroup);
+            NormMerge mg;
+            for (int p = tid & 7; p < nf.in_groups; p += 8) mg.take(pairs[p], pivot);
+            mg.d = oct_sum(mg.d);
+            mg.dd = oct_sum(mg.dd);
+            mg.m2 = oct_sum(mg.m2);
+            mg.finish(pivot, nf.in_groups, nf.eps, mean, rstd);
         }
+        if (MODE == kNormAdd) {
+            float h[4], gm[4], bt[4];
+            unpack4<T>(res[t], h);
+            if (row_stats) {
+                unpack4<T>(gam, gm);
+                unpack4<T>(bet, bt);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) h[e] = fmaf((h[e] - mean) * rstd, gm[e], bt[e]);
+            }
+            float total = 0.0f, m2 = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                y[e] = to_float(from_float<T>(sum[e] + bz[e] + h[e]));
+                total += y[e];
+            }
+            total = oct_sum(total);
+            const float mu = total * (1.0f / kNormGroup);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m2 = fmaf(y[e] - mu, y[e] - mu, m2);
+            m2 = oct_sum(m2);
+            if ((tid & 7) == 0 && m < M)
+                *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / kNormGroup) + n0 / kNormGroup) * 2) = f32x2{total, m2};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = MODE == kNormApply ? fmaf(fmaf(-mean, cs[e], sum[e]), rstd, bz[e]) : sum[e] + bz[e];
+                y[e] = apply_act16(v[e], ACT);
+            }
+        }
+        if (m >= M || n >= N) continue;
         if (n + 4 <= N && out_vec) {
             const u32x2 p = {pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
             *reinterpret_cast<u32x2 *>(out + (int64_t)m * out_rs + n) = p;
@@ -397,7 +574,7 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
             for (int e = 0; e < 4; ++e)
                 if (n + e < N) out[(int64_t)m * out_rs + (int64_t)(n + e) * out_cs] = from_float<T>(y[e]);
         }
-        if (act_in != nullptr) {
+        if (MODE == kNormNone && act_in != nullptr) {
             if (n + 4 <= N && ai_vec) {
                 const u32x2 p = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
                 *reinterpret_cast<u32x2 *>(act_in + (int64_t)m * ai_rs + n) = p;
@@ -409,6 +586,10 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
         }
     }
     };
+    if (MODE == kNormAdd) {
+        finish(IntC<KERNL_ACT_NONE>());
+        return;
+    }
     switch (act) {
         case KERNL_ACT_RELU: finish(IntC<KERNL_ACT_RELU>()); break;
         case KERNL_ACT_TANH: finish(IntC<KERNL_ACT_TANH>()); break;
@@ -419,10 +600,10 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     }
 }
 
-template <typename T, int BM, int BN>
-static void launch_small_dealt(const LinearArgs &a) {
-    auto kern = linear_small_dealt_kernel<T, BM, BN>;
-    constexpr int LDS_BYTES = 4 * small_ring_bytes(BM, BN);
+template <typename T, int BM, int BN, int MODE>
+static void launch_small_dealt_mode(const LinearArgs &a, const NormFold &nf) {
+    auto kern = linear_small_dealt_kernel<T, BM, BN, MODE>;
+    constexpr int LDS_BYTES = 4 * small_ring_bytes(BM, BN) + (MODE != kNormNone ? BM * kNormMaxGroups * 8 : 0);
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
@@ -432,26 +613,33 @@ static void launch_small_dealt(const LinearArgs &a) {
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), LDS_BYTES, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out),
                        static_cast<T *>(a.act_in), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs, a.act,
-                       tiles_m);
+                       tiles_m, nf);
+}
+
+template <typename T, int BM, int BN>
+static void launch_small_dealt(const LinearArgs &a, int mode, const NormFold &nf) {
+    if (mode == kNormApply) launch_small_dealt_mode<T, BM, BN, kNormApply>(a, nf);
+    else if (mode == kNormAdd) launch_small_dealt_mode<T, BM, BN, kNormAdd>(a, nf);
+    else launch_small_dealt_mode<T, BM, BN, kNormNone>(a, nf);
 }
 
 // rows: 16, 32 or 64 per tile (32 columns)
-void run_small_dealt(const LinearArgs &a, int dtype, int rows) {
+void run_small_dealt(const LinearArgs &a, int dtype, int rows, int mode, const NormFold &nf) {
     if (dtype == KERNL_F16) {
-        if (rows == 16) launch_small_dealt<f16, 16, 32>(a);
-        else if (rows == 32) launch_small_dealt<f16, 32, 32>(a);
-        else launch_small_dealt<f16, 64, 32>(a);
+        if (rows == 16) launch_small_dealt<f16, 16, 32>(a, mode, nf);
+        else if (rows == 32) launch_small_dealt<f16, 32, 32>(a, mode, nf);
+        else launch_small_dealt<f16, 64, 32>(a, mode, nf);
     } else {
-        if (rows == 16) launch_small_dealt<bf16, 16, 32>(a);
-        else if (rows == 32) launch_small_dealt<bf16, 32, 32>(a);
-        else launch_small_dealt<bf16, 64, 32>(a);
+        if (rows == 16) launch_small_dealt<bf16, 16, 32>(a, mode, nf);
+        else if (rows == 32) launch_small_dealt<bf16, 32, 32>(a, mode, nf);
+        else launch_small_dealt<bf16, 64, 32>(a, mode, nf);
     }
 }
 
-template <typename T, int BM, int BN>
-static void launch_small(const LinearArgs &a) {
-    auto kern = linear_small_kernel<T, BM, BN>;
-    constexpr int LDS_BYTES = small_stages(BM, BN) * (BM + BN) * kSmallBK * 2;
+template <typename T, int BM, int BN, int MODE>
+static void launch_small_mode(const LinearArgs &a, const NormFold &nf) {
+    auto kern = linear_small_kernel<T, BM, BN, MODE>;
+    constexpr int LDS_BYTES = small_stages(BM, BN) * (BM + BN) * kSmallBK * 2 + (MODE != kNormNone ? BM * kNormMaxGroups * 8 : 0);
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
@@ -461,19 +649,26 @@ static void launch_small(const LinearArgs &a) {
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), LDS_BYTES, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out),
                        static_cast<T *>(a.act_in), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs, a.act,
-                       tiles_m);
+                       tiles_m, nf);
+}
+
+template <typename T, int BM, int BN>
+static void launch_small(const LinearArgs &a, int mode, const NormFold &nf) {
+    if (mode == kNormApply) launch_small_mode<T, BM, BN, kNormApply>(a, nf);
+    else if (mode == kNormAdd) launch_small_mode<T, BM, BN, kNormAdd>(a, nf);
+    else launch_small_mode<T, BM, BN, kNormNone>(a, nf);
 }
 
 // tile shapes: 32 x 64, 64 x 64, 64 x 128 (rows x columns; the last in a ring of 6 stages)
-void run_small(const LinearArgs &a, int dtype, int rows, int cols) {
+void run_small(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf) {
     if (dtype == KERNL_F16) {
-        if (cols == 128) launch_small<f16, 64, 128>(a);
-        else if (rows == 32) launch_small<f16, 32, 64>(a);
-        else launch_small<f16, 64, 64>(a);
+        if (cols == 128) launch_small<f16, 64, 128>(a, mode, nf);
+        else if (rows == 32) launch_small<f16, 32, 64>(a, mode, nf);
+        else launch_small<f16, 64, 64>(a, mode, nf);
     } else {
-        if (cols == 128) launch_small<bf16, 64, 128>(a);
-        else if (rows == 32) launch_small<bf16, 32, 64>(a);
-        else launch_small<bf16, 64, 64>(a);
+        if (cols == 128) launch_small<bf16, 64, 128>(a, mode, nf);
+        else if (rows == 32) launch_small<bf16, 32, 64>(a, mode, nf);
+        else launch_small<bf16, 64, 64>(a, mode, nf);
     }
 }
 

@@ -19,6 +19,7 @@ from kernl_amd.optimizer.layer_norm import (
     replace_layer_norm_rms,
 )
 from kernl_amd.optimizer.linear import (
+    defer_layer_norms,
     fuse_linears_into_add_layer_norms,
     fuse_residual_into_linears,
     fuse_rms_norm_into_linears,
@@ -66,4 +67,5 @@ def dynamo_backend_ofi(gm: torch.fx.GraphModule, assume_causal=False):
     fuse_residual_into_linears(gm)
     fuse_linears_into_add_layer_norms(gm)
     fuse_rms_stats_into_residual_adds(gm)
+    defer_layer_norms(gm)
     return gm
