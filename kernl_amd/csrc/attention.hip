@@ -1122,6 +1122,15 @@ static int attention_entry(const void *q, const void *k, const void *v, void *ou
         else launch_stream_kv8<128>(p, mask_mode, causal, st);
         return check_launch("attention (mfma, fp8 keys/values)");
     }
+    // Short key sequences: a wave keeps all of its 16 queries' scores (attention_short.hip).
+    {
+        const int64_t wgs = B * H * ((M + 63) / 64);
+        const bool applies = mfma_ok && mask_mode != MASK_MATRIX && N <= kShortMaxKeys && wgs < (1ll << 31);
+        if (applies && (g_attention_variant == 6 || (g_attention_variant == 0 && attention_short_pays(wgs, (int)N, (int)D)))) {
+            run_attention_short(p, (int)D, dtype, mask_mode == MASK_VECTOR, causal, st);
+            return check_launch("attention (mfma, short key sequences)");
+        }
+    }
     // Small grids (BERT-base at batch 1: 12 heads x 4 query tiles on 256 CUs, each walking all key tiles): 32-row
     // workgroups whose four waves split the key tiles, where that still is a single round of workgroups (one per CU:
     // 130 KB of LDS) and every wave gets a tile.  Measured over 4 .. 64 heads x 64 .. 1536 rows x 256 .. 2048 keys: ahead of

@@ -60,4 +60,19 @@ static constexpr int kPipeMaxMaskKeys = 2048;
 static constexpr int kPipeMinKeys = 1024;
 bool launch_attention_pipe(const AttnParams &p, int D, int dtype, int mask_mode, bool causal, bool force, hipStream_t st);
 
+// Kernel for short key sequences (attention_short.hip): up to kShortMaxKeys keys, no mask or a per-key mask, causal or not.
+static constexpr int kShortMaxKeys = 256;
+// Where it is the fastest (graph replay, us, before -> with it; [batch, heads, keys, head size], per-key mask unless said):
+//   [1,12,16,64] 4.8 -> 2.6   [3,12,77,64] 6.1 -> 3.4   [8,12,128,64] 6.0 -> 3.9   [32,12,128,64] 7.8 -> 5.9   [4,12,256,64] 7.6 -> 5.1
+//   [512,12,16,64] 40 -> 10.6   [1,32,128,128] causal 7.4 -> 5.1   [4,16,256,128] 10.7 -> 8.5   [64,32,30,128] 26 -> 12.8
+// Every wave reads all keys of its head from LDS, so with enough workgroups to fill the chip several times over the kernels
+// whose waves share 128-row tiles win: [64,12,128,64] 12.3 -> 12.3, [16,12,256,64] 8.5 -> 9.6 without a mask, [8,32,160,128] 15.0
+// -> 17.6.  The limits lie at the last grid of each size where it was ahead with and without a mask.
+static inline bool attention_short_pays(int64_t workgroups, int N, int D) {
+    if (N <= 64) return true;
+    if (D == 64) return workgroups <= (N <= 128 ? 1024 : N <= 192 ? 512 : 384);
+    return workgroups <= (N <= 128 ? 384 : 256);
+}
+void run_attention_short(const AttnParams &p, int D, int dtype, bool masked, bool causal, hipStream_t st);
+
 }  // namespace kernl

@@ -1,0 +1,183 @@
+// Flash attention for SHORT key sequences (up to 256 keys): encoder batches of sentences, short prompts.
+//
+// What bounds such a launch is latency, not work: [1,12,16,64] is 0.4 MFLOP, and the streaming kernel spends 4.8 us on it (3.7
+// without a mask) in a chain of tile classification, key-tile stages and an online softmax; the launch itself is 1.6.  Here a
+// wave owns 16 query rows and ALL their scores: one round trip to memory (keys and values HBM -> LDS), S^T = K Q^T into
+// registers, one plain softmax, O^T = V^T P^T, store.  No tile loop, no running maximum, no vote: 2.6 us.  The keys go through
+// LDS although every wave reads all of them: fetched straight into MFMA operands (16 rows of 64 bytes per load, by every wave)
+// they cost 5.1 us instead of 3.6 at 128 keys.
+//
+// Key terms (the mask scaled to the base-2 domain; -inf past the last key) are built by one thread per key and read back four
+// at a time.  A lane ends the score products with keys 16 b + 4 g .. + 3 of its query; the value products use the same order
+// of keys inside a 32-key step, so the probabilities never move between lanes.
+#include "attention_common.h"
+
+namespace kernl {
+
+template <typename T, int D, int NB, bool CAUSAL>
+__global__ void __launch_bounds__(256, 1) attention_short_kernel(const AttnParams p, int masked) {
+    typedef typename Vec8<T>::type vec8;
+    constexpr int KS = D / 32, FB = D / 16, ROW = D * 2, CPR = D / 8;  // k-steps of a score product, 16-feature blocks, value rows in LDS
+    constexpr int TILE = NB * 16 * ROW;
+    extern __shared__ __attribute__((aligned(16))) unsigned char tiles[];  // keys, values
+    __shared__ __attribute__((aligned(16))) float terms[NB * 16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const int bh = blockIdx.x % (p.B * p.H), tile = blockIdx.x / (p.B * p.H), b = bh / p.H, h = bh % p.H;
+    const int N = p.N, M = p.M, m0 = tile * 64 + wave * 16, m = min(m0 + r, M - 1);
+    const T *kp = static_cast<const T *>(p.k) + b * p.ks[0] + h * p.ks[1];
+
+    // ---- everything this workgroup reads, requested at once
+    float term = 0.0f;
+    if (tid < NB * 16) {
+        if (tid >= N) term = -INFINITY;
+        else if (masked) term = scale_mask(load_mask_value(p.mask, p.mask_dtype, b * p.ms[0] + h * p.ms[1] + tid * p.ms[3]), p.clamp);
+    }
+    // (buffer loads: an address is one 32-bit offset, and keys past N lie outside the resource and arrive as zeros)
+    const T *qp = static_cast<const T *>(p.q) + b * p.qs[0] + h * p.qs[1], *vp = static_cast<const T *>(p.v) + b * p.vs[0] + h * p.vs[1];
+    const uint32_t k_step = (uint32_t)p.ks[2] * 2, v_step = (uint32_t)p.vs[2] * 2;
+    vec8 qf[KS];
+    const bool work = m0 < M;
+    if (work) {
+        const T *qrow = qp + (int64_t)m * p.qs[2];
+#pragma unroll
+        for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const vec8 *>(qrow + 32 * s + 8 * g);
+    }
+    // LDS chunk q of 16 bytes holds chunk q % CPR of row q / CPR, swizzled: keys for whole-row fragment reads, values by one bit
+    typedef __attribute__((address_space(3))) void lds_void;
+    const uint32_t lds = (uint32_t)(uintptr_t)(lds_void *)tiles;
+    {
+        constexpr int ROWS = 64 / CPR;  // per load
+        const uint64_t ka = (uint64_t)(uintptr_t)kp, va = (uint64_t)(uintptr_t)vp;
+        const u32x4 krsrc = {(uint32_t)ka, (uint32_t)(ka >> 32) & 0xFFFFu, (N - 1) * k_step + D * 2, 0x00020000u};
+        const u32x4 vrsrc = {(uint32_t)va, (uint32_t)(va >> 32) & 0xFFFFu, (N - 1) * v_step + D * 2, 0x00020000u};
+        const int row = wave * ROWS + lane / CPR, c = lane % CPR;
+        const uint32_t k_at = row * k_step, v_at = row * v_step + ((c ^ ((row >> 1) & 1)) * 16);
+#pragma unroll
+        for (int i = 0; i < NB * 16 / (4 * ROWS); ++i)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                         :: "s"(lds + wave * 1024 + i * 4096), "v"(k_at + i * 4 * ROWS * k_step + swz_chunk<ROW>(row + i * 4 * ROWS, c) * 16), "s"(krsrc) : "memory", "m0");
+#pragma unroll
+        for (int i = 0; i < NB * 16 / (4 * ROWS); ++i)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                         :: "s"(lds + TILE + wave * 1024 + i * 4096), "v"(v_at + i * 4 * ROWS * v_step), "s"(vrsrc) : "memory", "m0");
+    }
+    if (tid < NB * 16) terms[tid] = term;
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    if (!work) return;
+
+    // ---- scores: lane (r, g) gets keys 16 n + 4 g .. + 3 of query r
+    vec8 kf[NB][KS];
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int k = 0; k < KS; ++k) kf[n][k] = *reinterpret_cast<const vec8 *>(tiles + swz_offset<ROW>(16 * n + r, 4 * k + g));
+    f32x4_acc s[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+        s[n] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < KS; ++k) s[n] = mfma16(kf[n][k], qf[k], s[n]);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+        const f32x4 t = *reinterpret_cast<const f32x4 *>(terms + 16 * n + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float v = fmaf(s[n][e], p.scale_log2, t[e]);
+            if (CAUSAL) v = 16 * n + 4 * g + e > m + p.causal_off ? -INFINITY : v;
+            s[n][e] = v;
+            mx = fmaxf(mx, v);
+        }
+    }
+    mx = halves32_max(fmaxf(mx, __shfl_xor(mx, 16)));
+    float l = 0.0f;
+    vec8 pf[NB / 2];
+#pragma unroll
+    for (int t = 0; t < NB / 2; ++t) {
+        float e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            e[j] = __builtin_amdgcn_exp2f(s[2 * t + (j >> 2)][j & 3] - mx);
+            l += e[j];
+        }
+        const u32x4 packed = {pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3]), pack2<T>(e[4], e[5]), pack2<T>(e[6], e[7])};
+        pf[t] = __builtin_bit_cast(vec8, packed);
+    }
+    l = halves32_sum(l + __shfl_xor(l, 16));
+
+    // ---- values: block f of the result carries features 4 FB g' + 4 f + e in row 4 g' + e, so a lane ends with 4 FB features in
+    // a row.  Transposing reads: lane i of a 16-lane group hands in 4 features of key i / 4 and receives 4 keys of one feature.
+    f32x4_acc o[FB];
+#pragma unroll
+    for (int f = 0; f < FB; ++f) o[f] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t vbase = lds + TILE;
+    const int key = 4 * g + (r >> 2), flip = (key >> 1) & 1;  // (32- and 16-key steps leave the flip alone)
+#pragma unroll
+    for (int t = 0; t < NB / 2; ++t) {
+        u32x2 lo[FB], hi[FB];
+#pragma unroll
+        for (int f = 0; f < FB; ++f) {
+            const uint32_t chunk = (uint32_t)((((r & 3) * FB + f) >> 1) ^ flip);
+            const uint32_t at = vbase + key * ROW + chunk * 16 + (f & 1) * 8;
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo[f]) : "v"(at), "n"(t * 32 * ROW));
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(hi[f]) : "v"(at), "n"(t * 32 * ROW + 16 * ROW));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int f = 0; f < FB; ++f) {
+            asm volatile("" : "+v"(lo[f]), "+v"(hi[f]));
+            const u32x4 v4 = {lo[f][0], lo[f][1], hi[f][0], hi[f][1]};
+            o[f] = mfma16(__builtin_bit_cast(vec8, v4), pf[t], o[f]);
+        }
+    }
+    if (m0 + r < M) {
+        const float inv = 1.0f / l;
+        T *orow = static_cast<T *>(p.o) + b * p.os[0] + h * p.os[1] + (int64_t)(m0 + r) * p.os[2] + 4 * FB * g;
+#pragma unroll
+        for (int f = 0; f < FB; f += 2) {
+            const u32x4 w = {pack2<T>(o[f][0] * inv, o[f][1] * inv), pack2<T>(o[f][2] * inv, o[f][3] * inv),
+                             pack2<T>(o[f + 1][0] * inv, o[f + 1][1] * inv), pack2<T>(o[f + 1][2] * inv, o[f + 1][3] * inv)};
+            *reinterpret_cast<u32x4 *>(orow + 4 * f) = w;
+        }
+    }
+}
+
+template <typename T, int D>
+static void launch_short(const AttnParams &p, bool masked, bool causal, hipStream_t st) {
+    const dim3 grid((unsigned)(p.B * p.H * ((p.M + 63) / 64))), block(256);
+    const int blocks = (p.N + 15) / 16;
+#define KERNL_SHORT(NB)                                                                                            \
+    do {                                                                                                           \
+        constexpr int LDS = 2 * NB * 16 * D * 2;                                                                       \
+        auto kc = attention_short_kernel<T, D, NB, true>;                                                              \
+        auto kn = attention_short_kernel<T, D, NB, false>;                                                             \
+        static bool attr_done = false; /* benign race: the attribute calls are idempotent */                           \
+        if (!attr_done && LDS > 65536 - 2048) {                                                                        \
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kc), hipFuncAttributeMaxDynamicSharedMemorySize, LDS); \
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kn), hipFuncAttributeMaxDynamicSharedMemorySize, LDS); \
+        }                                                                                                              \
+        attr_done = true;                                                                                              \
+        hipLaunchKernelGGL(causal ? kc : kn, grid, block, LDS, st, p, (int)masked);                                    \
+    } while (0)
+    if (blocks <= 2) KERNL_SHORT(2);
+    else if (blocks <= 4) KERNL_SHORT(4);
+    else if (blocks <= 6) KERNL_SHORT(6);
+    else if (blocks <= 8) KERNL_SHORT(8);
+    else if (blocks <= 12) KERNL_SHORT(12);
+    else KERNL_SHORT(16);
+#undef KERNL_SHORT
+}
+
+void run_attention_short(const AttnParams &p, int D, int dtype, bool masked, bool causal, hipStream_t st) {
+    if (dtype == KERNL_F16) {
+        if (D == 64) launch_short<f16, 64>(p, masked, causal, st);
+        else launch_short<f16, 128>(p, masked, causal, st);
+    } else {
+        if (D == 64) launch_short<bf16, 64>(p, masked, causal, st);
+        else launch_short<bf16, 128>(p, masked, causal, st);
+    }
+}
+
+}  // namespace kernl
