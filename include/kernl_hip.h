@@ -278,7 +278,8 @@ int kernl_linear_residual_fwd(const void *x, const void *w, const void *bias, co
  * A LayerNorm between linear layers without a launch of its own, for small problems (a few hundred rows; widths that are a
  * multiple of 32, up to 1024).  The layer in front of the norm,
  *     kernl_linear_norm_add_fwd:    out = s = round(x @ w^T + bias + residual),
- *                                   out_stats[m][n / 32] = (sum, sum of squared deviations from their mean) of s[m][n .. n + 31],
+ *                                   out_stats[m][n / g] = (sum, sum of squared deviations from their mean) of s[m][n .. n + g - 1],
+ *                                   g = kernl_linear_norm_group(M) columns (16 or 32),
  * leaves the rows un-normalised; the layer behind,
  *     kernl_linear_norm_apply_fwd:  out = act(LN(x) @ w^T + bias) = act(rstd (x @ w_folded^T - mean colsum) + bias32),
  * with w_folded = w * gamma (columns), colsum[n] = sum_k w_folded[n][k], bias32 = bias + w @ beta, normalises its sums.  A
@@ -287,6 +288,7 @@ int kernl_linear_residual_fwd(const void *x, const void *w, const void *bias, co
  * The reference runs a LayerNorm kernel between its linear kernels (src/kernl/implementations/layer_norm.py:279-335).
  */
 int kernl_linear_norm_kind(int64_t M, int64_t N, int64_t K);
+int kernl_linear_norm_group(int64_t M);
 int kernl_linear_norm_add_fwd(const void *x, const void *w, const void *bias, const void *residual, const float *residual_stats,
                               const void *gamma, const void *beta, float eps, void *out, float *out_stats, int64_t M, int64_t N,
                               int64_t K, int64_t x_row_stride, int64_t out_row_stride, int64_t residual_row_stride, int dtype,
@@ -306,13 +308,20 @@ int kernl_linear_norm_apply_fwd(const void *x, const float *x_stats, float eps, 
 int kernl_linear_small_kind(int64_t M, int64_t N, int64_t K);
 
 /*
- * Whether kernl_linear_fwd runs M x N x K (16-bit, plain epilogue) on one of its wide tile kernels, and which: 0 = no,
- * otherwise the kernl_linear_force_tile value of the kernel (5 .. 8).  kernl_linear_residual_fwd and
+ * Whether kernl_linear_fwd runs M x N x K (16-bit, plain epilogue) on one of its wide or 8-wave tile kernels, and which: 0 = no,
+ * otherwise the kernl_linear_force_tile value of the kernel.  kernl_linear_residual_fwd and
  * kernl_linear_scaled_fwd exist on those kernels only and run them whatever the shape: a caller asks here first and
  * keeps the separate addition (or normalisation) where another kernel is the faster one.  No counterpart in the
  * reference (one kernel and an autotuner, src/kernl/implementations/linear_layer.py:47-91).
  */
 int kernl_linear_wide_kind(int64_t M, int64_t N, int64_t K);
+
+/*
+ * Whether kernl_linear_fwd (gated: kernl_linear_glu_fwd, N = rows of the interleaved weight) runs M x N x K, more than 64 rows and
+ * no small problem, on one of its 8-wave tiles over the whole K, and which (the kernl_linear_force_tile value).  A caller that
+ * would otherwise route such a shape to the stream-K or split-K entry points should call kernl_linear_fwd instead.
+ */
+int kernl_linear_mid_kind(int64_t M, int64_t N, int64_t K, int gated);
 
 /*
  * kernl_linear_fwd for row counts between the two regimes (129 to a few hundred rows against a few thousand columns),

@@ -41,7 +41,9 @@ EXPORTED_SYMBOLS = (
     "kernl_linear_scaled_fwd",
     "kernl_linear_residual_fwd",
     "kernl_linear_wide_kind",
+    "kernl_linear_mid_kind",
     "kernl_linear_norm_kind",
+    "kernl_linear_norm_group",
     "kernl_linear_norm_add_fwd",
     "kernl_linear_norm_apply_fwd",
     "kernl_embedding_layernorm_fwd",
@@ -164,8 +166,12 @@ def load() -> ctypes.CDLL:
     lib.kernl_linear_small_kind.argtypes = [_i64] * 3
     lib.kernl_linear_wide_kind.restype = ctypes.c_int
     lib.kernl_linear_wide_kind.argtypes = [_i64] * 3
+    lib.kernl_linear_mid_kind.restype = ctypes.c_int
+    lib.kernl_linear_mid_kind.argtypes = [_i64] * 3 + [ctypes.c_int]
     lib.kernl_linear_norm_kind.restype = ctypes.c_int
     lib.kernl_linear_norm_kind.argtypes = [_i64] * 3
+    lib.kernl_linear_norm_group.restype = ctypes.c_int
+    lib.kernl_linear_norm_group.argtypes = [_i64]
     lib.kernl_linear_norm_add_fwd.restype = ctypes.c_int
     lib.kernl_linear_norm_add_fwd.argtypes = [_vp] * 7 + [ctypes.c_float, _vp, _vp] + [_i64] * 6 + [ctypes.c_int, _vp]
     lib.kernl_linear_norm_apply_fwd.restype = ctypes.c_int
@@ -309,6 +315,12 @@ def linear_small_kind(M: int, N: int, K: int) -> int:
     return int(load().kernl_linear_small_kind(int(M), int(N), int(K)))
 
 
+def linear_mid_kind(M: int, N: int, K: int, gated: bool = False) -> int:
+    """Non-zero when `kernl_linear_fwd` (`kernl_linear_glu_fwd`) runs the problem on one of its 8-wave tiles: such shapes are not
+    handed to the stream-K or split-K entry points."""
+    return int(load().kernl_linear_mid_kind(int(M), int(N), int(K), int(bool(gated))))
+
+
 def linear_wide_kind(M: int, N: int, K: int) -> int:
     """Non-zero when `kernl_linear_fwd` runs a plain 16-bit M x N x K problem on one of its wide tile kernels."""
     return int(load().kernl_linear_wide_kind(int(M), int(N), int(K)))
@@ -323,14 +335,19 @@ def linear_norm_kind(M: int, N: int, K: int) -> int:
     return int(load().kernl_linear_norm_kind(int(M), int(N), int(K)))
 
 
+def linear_norm_group(M: int) -> int:
+    """Columns per statistics pair of a deferred norm over M rows."""
+    return int(load().kernl_linear_norm_group(int(M)))
+
+
 def linear_norm_add_fwd(x2d, weight, bias, residual2d, residual_stats, gamma, beta, eps: float, out2d, out_stats) -> None:
     """out = x @ w^T + bias + residual with the statistics of its rows; with `residual_stats` the residual is the
     un-normalised rows of a deferred LayerNorm (gamma, beta, eps)."""
     _require_gpu(x2d, weight, bias, residual2d, residual_stats, gamma, beta, out2d, out_stats)
     M, K = x2d.shape
     N = weight.shape[0]
-    if any(t is not None and (t.dtype != torch.float32 or t.numel() != M * N // 16 or not t.is_contiguous()) for t in (residual_stats, out_stats)):
-        raise ValueError("statistics are contiguous fp32 [rows, columns / 32, 2]")
+    if any(t is not None and (t.dtype != torch.float32 or t.numel() != M * N // linear_norm_group(M) * 2 or not t.is_contiguous()) for t in (residual_stats, out_stats)):
+        raise ValueError("statistics are contiguous fp32 [rows, columns / linear_norm_group(rows), 2]")
     if x2d.stride(1) != 1 or residual2d.stride(1) != 1 or out2d.stride(1) != 1 or not weight.is_contiguous():
         raise ValueError("unit feature strides and a contiguous weight")
     with torch.cuda.device(x2d.device):
@@ -348,8 +365,8 @@ def linear_norm_apply_fwd(x2d, x_stats, eps: float, weight_folded, colsum, bias3
     _require_gpu(x2d, x_stats, weight_folded, colsum, bias32, out2d)
     M, K = x2d.shape
     N = weight_folded.shape[0]
-    if x_stats.dtype != torch.float32 or x_stats.numel() != M * K // 16 or not x_stats.is_contiguous():
-        raise ValueError("statistics are contiguous fp32 [rows, columns / 32, 2]")
+    if x_stats.dtype != torch.float32 or x_stats.numel() != M * K // linear_norm_group(M) * 2 or not x_stats.is_contiguous():
+        raise ValueError("statistics are contiguous fp32 [rows, columns / linear_norm_group(rows), 2]")
     if any(t.dtype != torch.float32 or t.numel() != N or not t.is_contiguous() for t in (colsum, bias32)):
         raise ValueError("colsum and bias32 are contiguous fp32 vectors with one entry per column")
     if x2d.stride(1) != 1 or out2d.stride(1) != 1 or not weight_folded.is_contiguous():

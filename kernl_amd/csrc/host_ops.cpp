@@ -492,7 +492,8 @@ PyObject *op_linear(PyObject *const *a, Py_ssize_t n) {
         Py_RETURN_NONE;
     const int act = (int)integer(a[3]);
     const bool vectors = r.vectors() && aligned16(*x) && aligned16(*w);
-    const bool small = truth(a[5]) && vectors && kernl_linear_small_kind(M, N, K) != 0;
+    const bool small = vectors && ((truth(a[5]) && kernl_linear_small_kind(M, N, K) != 0) ||
+                                   (M > 64 && r.strides[0] < (1 << 22) && kernl_linear_mid_kind(M, N, K, 0) != 0));
     const at::Tensor out = output_for(*x, N);
     const int64_t os[2] = {N, 1};
     if (!small && vectors && K % 64 == 0) {

@@ -6,6 +6,28 @@ namespace kernl {
 
 int g_linear_force_tile = 0;
 
+// Runs the kernel a value of small_problem_kind / mid_kind (or of the hook) names; 0: it does not take this epilogue.
+static int run_one_launch(const LinearArgs &a, int dtype, int kind, int mode, const NormFold &nf) {
+    if (kind == 11 || kind == 15 || kind >= 17) return run_mid(a, dtype, kind, mode, nf);
+    if ((a.act & kGluBit) || a.row_scale != nullptr || a.residual != nullptr) return 0;
+    if (kind == 10) {
+        run_small(a, dtype, mode, nf);
+        return 1;
+    }
+    // Dealt k-tiles: time is what a workgroup pulls from memory, so the smallest tiles that are still one round (us, 32 x 32 -> 16 x 16
+    // tiles): 17 x 768 x 3072 6.9 -> 5.6, 64 x 768 x 3072 7.8 -> 5.9, 64 x 768 x 768 4.5 -> 4.0, 64 x 1024 x 4096 8.6 -> 6.5; 16 x 32:
+    // 96 x 768 x 3072 7.8 -> 6.7, 48 x 2304 x 768 5.0 -> 4.7.
+    auto tiles = [&](int bm, int bn) { return (int64_t)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
+    int rows = kind == 12 || kind == 16 ? 16 : kind == 13 ? 32 : 64, cols = kind == 16 ? 16 : 32;
+    if (kind == 12 || kind == 13) {
+        const bool narrow = mode != kNormAdd || nf.group == kNormGroupFew;  // (a tile row holds whole statistics groups)
+        if (narrow && tiles(16, 16) <= 256) rows = cols = 16;
+        else if (a.M <= 96 && tiles(16, 32) <= 256) rows = 16;
+    }
+    run_small_dealt(a, dtype, rows, cols, mode, nf);
+    return 1;
+}
+
 template <typename T>
 static int linear_mfma_dispatch(const LinearArgs &a) {
     constexpr int kDtype = std::is_same<T, f16>::value ? KERNL_F16 : KERNL_BF16;
@@ -17,17 +39,11 @@ static int linear_mfma_dispatch(const LinearArgs &a) {
         else launch_skinny<T, false>(a);
         return check_launch("linear (skinny)");
     }
-    // small problems: one launch of small tiles over the whole K (10 / 11 / 15 force its 32 x 64 / 64 x 64 / 64 x 128 form)
-    if (pick == 0 && !(a.act & kGluBit)) pick = small_problem_kind(a.M, a.N, a.K);
-    if ((pick == 12 || pick == 13 || pick == 14) && !(a.act & kGluBit)) {
-        run_small_dealt(a, kDtype, pick == 12 ? 16 : pick == 13 ? 32 : 64, kNormNone, NormFold());
-        return check_launch("linear (small tiles, dealt k-tiles)");
-    }
-    if ((pick == 10 || pick == 11 || pick == 15) && !(a.act & kGluBit)) {
-        run_small(a, kDtype, pick == 10 ? 32 : 64, pick == 15 ? 128 : 64, kNormNone, NormFold());
-        return check_launch("linear (small tiles)");
-    }
-    if (pick == 0 || pick == 9) pick = pick_tile(a.M, a.N, a.K, (a.act & kGluBit) != 0);
+    // one launch of small or middling tiles over the whole K (the hook forces any of them)
+    if (pick == 0) pick = (a.act & kGluBit) ? 0 : small_problem_kind(a.M, a.N, a.K);
+    if (pick == 0) pick = mid_kind(a.M, a.N, a.K, (a.act & kGluBit) != 0);
+    if (pick >= 10 && run_one_launch(a, kDtype, pick, kNormNone, NormFold())) return check_launch("linear (one launch over the whole K)");
+    if (pick == 0 || pick >= 9) pick = pick_tile(a.M, a.N, a.K, (a.act & kGluBit) != 0);
     if (a.act & kGluBit) {
         if (pick == 5) run_wide(a, kDtype, 256);
         else if (pick == 3) launch_mfma_glu<T, Tile128x128>(a);
@@ -62,10 +78,16 @@ extern "C" int kernl_linear_small_kind(int64_t M, int64_t N, int64_t K) {
     return kernl::small_problem_kind(M, N, K);
 }
 
+extern "C" int kernl_linear_mid_kind(int64_t M, int64_t N, int64_t K, int gated) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    return kernl::mid_kind(M, N, K, gated != 0);
+}
+
 extern "C" int kernl_linear_wide_kind(int64_t M, int64_t N, int64_t K) {
     using namespace kernl;
     if (M <= 64 || N <= 0 || K <= 0 || K % 8 != 0 || M > INT32_MAX || N > INT32_MAX || K >= (1 << 22)) return 0;
     if (small_problem_kind(M, N, K) != 0) return 0;
+    if (const int mid = mid_kind(M, N, K, false)) return mid == 14 ? 0 : mid;
     const int pick = pick_tile((int)M, (int)N, (int)K, false);
     return pick >= 5 && pick <= 8 ? pick : 0;
 }
@@ -231,7 +253,10 @@ extern "C" int kernl_linear_scaled_fwd(const void *x, const void *w, const void 
     a.act = gated ? (kGluBit | activation) : activation;
     a.st = static_cast<hipStream_t>(stream);
     a.row_scale = row_scale;
-    // only the wide kernels take per-row factors (5 / 6: 256-row tiles, 7 / 8: 128-row tiles; gated: 256 x 256 only)
+    // the wide kernels take per-row factors (5 / 6: 256-row tiles, 7 / 8: 128-row tiles; gated: 256 x 256 only), and the 8-wave tiles
+    if (g_linear_force_tile == 0 && small_problem_kind(a.M, a.N, a.K) == 0)
+        if (const int mid = mid_kind(a.M, a.N, a.K, gated != 0))
+            if (run_one_launch(a, dtype, mid, kNormNone, NormFold())) return check_launch("scaled linear (8-wave tiles)");
     int pick = g_linear_force_tile >= 5 && g_linear_force_tile <= 8 ? g_linear_force_tile : pick_tile(a.M, a.N, a.K, gated != 0, true);
     if (gated) pick = 5;
     if (pick == 5) run_wide(a, dtype, 256);
@@ -271,7 +296,10 @@ extern "C" int kernl_linear_residual_fwd(const void *x, const void *w, const voi
     a.st = static_cast<hipStream_t>(stream);
     a.residual = residual;
     a.res_rs = residual_strides[0]; a.res_cs = residual_strides[1];
-    // only the wide kernels add a residual (5 / 6: 256-row tiles, 7 / 8: 128-row tiles)
+    // the wide kernels add a residual (5 / 6: 256-row tiles, 7 / 8: 128-row tiles), and the 8-wave tiles
+    if (g_linear_force_tile == 0 && small_problem_kind(a.M, a.N, a.K) == 0)
+        if (const int mid = mid_kind(a.M, a.N, a.K, false))
+            if (run_one_launch(a, dtype, mid, kNormNone, NormFold())) return check_launch("linear + residual (8-wave tiles)");
     const int pick = g_linear_force_tile >= 5 && g_linear_force_tile <= 8 ? g_linear_force_tile : pick_tile(a.M, a.N, a.K, false, true);
     if (pick == 5) run_wide(a, dtype, 256);
     else if (pick == 6) run_wide(a, dtype, 192);
@@ -280,18 +308,24 @@ extern "C" int kernl_linear_residual_fwd(const void *x, const void *w, const voi
     return check_launch("linear + residual");
 }
 
-// Both sides of a deferred LayerNorm run on the small-problem kernels (10 .. 15).
-static void run_norm_small(const kernl::LinearArgs &a, int dtype, int mode, const kernl::NormFold &nf) {
+// Both sides of a deferred LayerNorm run on the small-problem kernels or the 8-wave tiles whose waves own 32 columns.
+static int norm_kind(int64_t M, int64_t N, int64_t K) {
     using namespace kernl;
-    const int pick = g_linear_force_tile >= 10 && g_linear_force_tile <= 15 ? g_linear_force_tile : small_problem_kind(a.M, a.N, a.K);
-    if (pick == 12 || pick == 13 || pick == 14) run_small_dealt(a, dtype, pick == 12 ? 16 : pick == 13 ? 32 : 64, mode, nf);
-    else run_small(a, dtype, pick == 10 ? 32 : 64, pick == 15 ? 128 : 64, mode, nf);
+    int pick = g_linear_force_tile >= 10 ? g_linear_force_tile : small_problem_kind(M, N, K);
+    if (M <= kNormFewRows) return pick == 12 || pick == 13 || pick == 16 ? pick : 0;  // (16-column groups: tiles that stage that many)
+    if (pick == 0) pick = mid_kind(M, N, K, false);
+    return pick <= 17 && pick != 16 ? pick : 0;
 }
 
+// (128 x 64 tiles stage the statistics of up to 24 groups)
+static bool norm_groups_fit(int kind, int64_t groups) { return kind != 15 || groups <= 24; }
+
 extern "C" int kernl_linear_norm_kind(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0 || N % kernl::kNormGroup != 0 || K % 8 != 0) return 0;
-    return kernl::small_problem_kind(M, N, K);
+    if (M <= 0 || N <= 0 || K <= 0 || N % kernl::kNormGroup != 0 || K % 8 != 0 || M > INT32_MAX || N > INT32_MAX) return 0;
+    return norm_kind(M, N, K);
 }
+
+extern "C" int kernl_linear_norm_group(int64_t M) { return kernl::norm_group_of(M); }
 
 static int norm_arguments_bad(const char *what, const void *x, const void *w, const void *out, int64_t M, int64_t N, int64_t K, int64_t x_rs,
                               int64_t out_rs, int dtype) {
@@ -300,8 +334,8 @@ static int norm_arguments_bad(const char *what, const void *x, const void *w, co
     if (M < 0 || N <= 0 || K <= 0)
         return set_error(KERNL_ERR_INVALID_ARG, "%s: bad sizes M=%lld N=%lld K=%lld", what, (long long)M, (long long)N, (long long)K);
     if (dtype != KERNL_F16 && dtype != KERNL_BF16) return set_error(KERNL_ERR_UNSUPPORTED, "%s: only f16 and bf16 are supported, got dtype %d", what, dtype);
-    if (!aligned16(x) || !aligned16(w) || x_rs % 8 != 0 || x_rs < K || x_rs >= (1 << 22) || K >= (1 << 22) || ((uintptr_t)out & 7) != 0 || out_rs % 4 != 0 || out_rs < N)
-        return set_error(KERNL_ERR_UNSUPPORTED, "%s: x and w need 16-byte aligned rows, out 8-byte aligned ones", what);
+    if (!aligned16(x) || !aligned16(w) || x_rs % 8 != 0 || x_rs < K || x_rs >= (1 << 22) || K >= (1 << 22) || !aligned16(out) || out_rs % 8 != 0 || out_rs < N)
+        return set_error(KERNL_ERR_UNSUPPORTED, "%s: x, w and out need 16-byte aligned rows", what);
     if (M > 0 && kernl_linear_norm_kind(M, N, K) == 0)
         return set_error(KERNL_ERR_UNSUPPORTED, "%s: M=%lld N=%lld K=%lld is not a small problem (kernl_linear_norm_kind)", what, (long long)M,
                          (long long)N, (long long)K);
@@ -327,8 +361,9 @@ extern "C" int kernl_linear_norm_apply_fwd(const void *x, const float *x_stats, 
     a.x_rs = x_row_stride; a.x_cs = 1; a.out_rs = out_row_stride; a.out_cs = 1; a.ai_rs = a.ai_cs = 0;
     a.act = activation; a.st = static_cast<hipStream_t>(stream);
     NormFold nf;
-    nf.in_stats = x_stats; nf.in_groups = (int)(K / kNormGroup); nf.eps = eps; nf.colsum = colsum; nf.bias32 = bias32;
-    run_norm_small(a, dtype, kNormApply, nf);
+    nf.stats_of(M, K); nf.in_stats = x_stats; nf.eps = eps; nf.colsum = colsum; nf.bias32 = bias32;
+    const int kind = norm_kind(M, N, K);
+    run_one_launch(a, dtype, norm_groups_fit(kind, nf.in_groups) ? kind : 11, kNormApply, nf);
     return check_launch("linear (deferred norm)");
 }
 
@@ -337,9 +372,9 @@ extern "C" int kernl_linear_norm_add_fwd(const void *x, const void *w, const voi
                                          int64_t K, int64_t x_row_stride, int64_t out_row_stride, int64_t residual_row_stride, int dtype,
                                          void *stream) {
     using namespace kernl;
-    if (residual == nullptr || out_stats == nullptr || ((uintptr_t)residual & 7) != 0 || residual_row_stride % 4 != 0 || !aligned16(out_stats))
-        return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: residual needs 8-byte aligned rows, out_stats a 16-byte aligned array");
-    if (residual_stats != nullptr && (gamma == nullptr || !aligned16(residual_stats) || ((uintptr_t)gamma & 7) != 0 || ((uintptr_t)beta & 7) != 0))
+    if (residual == nullptr || out_stats == nullptr || !aligned16(residual) || residual_row_stride % 8 != 0 || !aligned16(out_stats))
+        return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: residual needs 16-byte aligned rows, out_stats a 16-byte aligned array");
+    if (residual_stats != nullptr && (gamma == nullptr || !aligned16(residual_stats) || !aligned16(gamma) || !aligned16(beta)))
         return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: a deferred residual comes with its statistics and aligned norm parameters");
     const int bad = norm_arguments_bad("linear + addition + statistics", x, w, out, M, N, K, x_row_stride, out_row_stride, dtype);
     if (bad != KERNL_OK) return bad;
@@ -352,9 +387,10 @@ extern "C" int kernl_linear_norm_add_fwd(const void *x, const void *w, const voi
     a.x_rs = x_row_stride; a.x_cs = 1; a.out_rs = out_row_stride; a.out_cs = 1; a.ai_rs = a.ai_cs = 0;
     a.act = KERNL_ACT_NONE; a.st = static_cast<hipStream_t>(stream);
     NormFold nf;
-    nf.in_stats = residual_stats; nf.in_groups = (int)(N / kNormGroup); nf.eps = eps;
+    nf.stats_of(M, N); nf.in_stats = residual_stats; nf.eps = eps;
     nf.residual = residual; nf.res_rs = residual_row_stride; nf.gamma = gamma; nf.beta = beta; nf.out_stats = out_stats;
-    run_norm_small(a, dtype, kNormAdd, nf);
+    const int kind = norm_kind(M, N, K);
+    run_one_launch(a, dtype, norm_groups_fit(kind, nf.in_groups) ? kind : 11, kNormAdd, nf);
     return check_launch("linear + addition + statistics");
 }
 

@@ -32,8 +32,10 @@ void run_wide_half(const LinearArgs &a, int dtype, int cols);        // 128-row 
 void run_wide_half_w8(const LinearArgs &a);
 void run_half_split(const LinearArgs &a, const HalfSplitPlan &p, float *part, int dtype);
 struct NormFold;
-void run_small(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf);  // mode: norm_fold.h; 32 x 64, 64 x 64 or 64 x 128 tiles over the whole K (linear_small.hip)
-void run_small_dealt(const LinearArgs &a, int dtype, int rows, int mode, const NormFold &nf);      // 16-, 32- or 64-row, 32-column tiles, k-tiles dealt to the waves
+void run_small(const LinearArgs &a, int dtype, int mode, const NormFold &nf);  // mode: norm_fold.h; 32 x 64 tiles over the whole K (linear_small.hip)
+// 8-wave tiles over the whole K (linear_mid.hip), by hook value 11, 15, 17 .. 21; 0: that tile does not take the epilogue asked for
+int run_mid(const LinearArgs &a, int dtype, int kind, int mode, const NormFold &nf);
+void run_small_dealt(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf);      // 16- to 64-row, 16- or 32-column tiles, k-tiles dealt to the waves
 
 
 // ----------------------------------------------------------------------------------------------------
@@ -1954,8 +1956,9 @@ static int pick_tile(int M, int N, int K, bool gated, bool wide_only = false) {
 }
 
 // Which of the small-problem kernels (linear_small.hip) takes M x N x K, as the value of the tile hook that forces it
-// (10 / 11 / 15: 32 x 64 / 64 x 64 / 64 x 128 tiles shared by the waves; 12 / 13 / 14: 16 x 32 / 32 x 32 / 64 x 32 tiles with
-// the k-tiles dealt to the waves), or 0 when the problem is not their kind.  One round of workgroups is the condition for all of them.
+// (10: 32 x 64 tiles shared by four waves; 11 / 15: 64 x 64 / 128 x 64 tiles of linear_mid.hip; 12 / 13 / 14: up to 16 / 32 / 64 rows
+// by 16 or 32 columns with the k-tiles dealt to the waves), or 0 when the problem is not their kind.  One round of workgroups is
+// the condition for all of them.
 //  - dealt k-tiles: weights of up to 8 M elements, 8 rows or more (fewer stream the weight faster), at most 256 tiles.
 //    Graph replay, us, against what ran before: 16 x 768 x 3072 6.7 (9.0), 64 x 768 x 3072 8.0 (11.6), 128 x 768 x 3072
 //    8.4 (14.3), 256 x 768 x 3072 9.8 (15.8), 128 x 768 x 768 5.1 (7.3), 64 x 2304 x 768 5.4 (7.6), 128 x 2048 x 2048 9.0
@@ -1985,7 +1988,71 @@ static int small_problem_kind(int64_t M, int64_t N, int64_t K) {
     return 0;
 }
 
-extern int g_linear_force_tile;  // test / tuning hook (defined in linear.hip): 0 = heuristic, 1 = 256x256, 2 = 256x192, 3 = 128x128, 4 = 256x128 k32, 5 = wide 256x256, 6 = wide 256x192, 7 = wide 128x256, 8 = wide 128x192, 10 .. 15 = the small-problem kernels
+// Which 8-wave tile (linear_mid.hip) takes M x N x K beyond what small_problem_kind names, as its hook value, or 0 where another
+// kernel is faster.  `N`: rows of the weight (gated: twice the output columns).
+//  - short K: by tile counts, from a sweep of 65 .. 4096 rows over BERT's and wider weights (us, before -> with it): 768 x 3072 x 768
+//    12.9 -> 11.2, 1024 x 2304 x 768 12.1 -> 11.0, 1024 x 4096 x 1024 16.9 -> 15.5, 3072 x 768 x 768 12.0 -> 11.2.
+//  - long K: time = launch + k-tiles x rounds x the tile's measured time per k-tile (weights from HBM), or the weight's bytes at
+//    the HBM rate, against the same estimate for what would run otherwise: 1024 x 2048 x 2048 23.2 -> 15.3, 130 x 22016 x 4096 gated
+//    85 -> 53, 333 x 22016 x 4096 gated 88 -> 77, 160 x 12288 x 4096 44 -> 37, 768 x 4096 x 4096 50 -> 40, 768 x 4096 x 11008 126 -> 106,
+//    128 x 22016 x 4096 gated 64 -> 51 (few-row kernel), 1536 x 4096 x 11008 154 -> 139.  The kernels are within 5 % of the best tile
+//    of that sweep nearly everywhere.
+static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
+    if (M <= 64 || N < 64 || K % 8 != 0 || K < 64 || M > 4096 || N > INT32_MAX / 64 || K >= (1 << 22) || (gated && N % 64 != 0)) return 0;
+    auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const bool short_k = K < 1536;
+    if (short_k && !gated) {
+        if (N * K > (1 << 23)) return 0;
+        if (tiles(128, 64) <= 256 || (tiles(128, 64) <= 512 && M <= 1280)) return 15;
+        return tiles(128, 128) <= 256 && M <= 3072 ? 17 : 0;
+    }
+    if (short_k || (M <= 128 && N * K < 12 * (1 << 20))) return 0;
+    const double nk = (double)((K + 63) / 64), hbm = 4.0 + (double)(N * K) * 2.0 / 4.6e6;  // us at 4.6 TB/s
+    auto cost = [&](int bm, int bn, double per_k) {
+        const int64_t t = tiles(bm, bn);
+        double rounds = (double)((t + 255) / 256);
+        if (bn == 64 && t > 256 && t <= 512) rounds = 1.6;  // two workgroups per CU
+        const double c = 3.5 + nk * per_k * rounds;
+        return c > hbm ? c : hbm;
+    };
+    int best = 0;
+    double best_cost = 1e30;
+    auto offer = [&](int kind, double c) {
+        if (c < best_cost) { best_cost = c; best = kind; }
+    };
+    offer(11, cost(64, 64, 0.285));
+    offer(15, cost(128, 64, 0.45));
+    offer(17, cost(128, 128, 0.62));
+    offer(18, cost(192, 128, 0.83));
+    offer(19, cost(192, 192, 1.15));
+    offer(20, cost(128, 256, 0.98));
+    offer(21, cost(256, 128, 0.97));
+    double other = cost(256, 256, 1.38);
+    if (!gated) {
+        const double c6 = cost(256, 192, 1.34), c7 = cost(128, 256, 0.90), c8 = cost(128, 192, 0.755);
+        other = other < c6 ? other : c6;
+        other = other < c7 ? other : c7;
+        other = other < c8 ? other : c8;
+        if (M > 128 && K % 64 == 0) {
+            const HalfSplitPlan p = half_split_plan(M, N, K);
+            const double per = (double)(((int64_t)nk + p.splits - 1) / p.splits);
+            const double c = 6.5 + per * 0.755 + (double)p.splits * (double)(M * N) * 8.0 / 4e6;
+            if (p.splits > 1 && c < other) other = c;
+        }
+    }
+    if (M <= 128 && K % 64 == 0) {
+        const double few = 10.0 + (double)(N * K) * 2.0 / 3.7e6;
+        other = other < few ? other : few;
+        // 64 x 32 tiles with dealt k-tiles, one round of them: 128 x 4096 x 4096 20.8 -> 17.3
+        if (!gated && tiles(64, 32) <= 256) {
+            const double c = 3.5 + nk * 0.2;
+            offer(14, c > hbm ? c : hbm);
+        }
+    }
+    return best_cost < 0.97 * other ? best : 0;
+}
+
+extern int g_linear_force_tile;  // test / tuning hook (defined in linear.hip): 0 = heuristic, 1 = 256x256, 2 = 256x192, 3 = 128x128, 4 = 256x128 k32, 5 = wide 256x256, 6 = wide 256x192, 7 = wide 128x256, 8 = wide 128x192, 10 = 32 x 64, 12 .. 14 and 16 = dealt k-tiles, 11, 15, 17 .. 21 = the 8-wave tiles of linear_mid.hip
 
 template <typename T, bool GATED, int MB, int NR, bool W8, bool RMS = false, bool ROPE = false>
 static void launch_skinny_blocks(const LinearArgs &a, const void *rms_w = nullptr, float eps = 0.0f,

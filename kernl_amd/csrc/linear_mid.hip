@@ -1,0 +1,449 @@
+// Linear layer for MIDDLING problems — 65 to some 3000 rows —, which give the big tile kernels less than a round of workgroups.
+//
+// What bounds such a launch: a CU's tile loads.  A CU takes 45 to 58 bytes per clock from L2 through its direct-to-LDS loads
+// whatever the depth of the ring (1024 x 4096 x 4096 with the matrix instructions and LDS reads taken out: 27 us with the weight
+// in the memory-side cache, 40 us from HBM; with the loads taken out: 28; whole: 42), so time is (BM + BN) x K x rounds, and
+// latency: barrier, LDS read and matrix instruction of a k-tile form a chain that four waves do not hide.  Hence
+//   - tiles of 64 x 64 to 256 x 128, as large as still put a tile on (nearly) every CU;
+//   - eight waves, two per SIMD, and LDS fragments read one k-step ahead ACROSS the barrier (while k-step 1 of a k-tile is
+//     multiplied, k-step 0 of the next is read): 231 x 2304 x 768 in 64 x 64 tiles 7.6 -> 6.7 us against four waves that read, then
+//     multiply; sched_barrier keeps the compiler from moving the reads back behind the multiplications;
+//   - the small tiles in rings of 64 to 72 KB, so that two workgroups share a CU where there are more tiles than CUs (512 x 3072 x 768
+//     in 128 x 64 tiles 10.5 -> 8.4 us, 1024 x 3072 x 768 13.1 -> 12.0).
+// Weight rows are placed in LDS so that a lane's blocks are consecutive output columns: 16-byte stores.
+#include "linear_kernels.h"
+#include "norm_fold.h"
+
+namespace kernl {
+
+// tile shape, wave grid and ring depth of one build of the kernel
+template <int BM_, int BN_, int WM_, int WN_, int S_>
+struct MidTile {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_;
+    static constexpr int BK = 64, RB = BK * 2;
+    static constexpr int TM = BM / WM, TN = BN / WN, NBM = TM / 16, NBN = TN / 16;
+    static constexpr int X_BYTES = BM * RB, STAGE = (BM + BN) * RB, LDS = S * STAGE;
+    static constexpr int LX = BM / 64, LW = BN / 64, L = LX + LW;
+    static_assert(WM * WN == 8 && BM % 64 == 0 && BN % 64 == 0 && LDS <= 160 * 1024 && S >= 3 && (S - 1) * L <= 63, "tile shape");
+};
+
+// How the tile grid is dealt to the 8 XCDs, each with an L2 of its own: as 2^xm_shift x 8 / 2^xm_shift blocks of per_m x per_n tiles,
+// so that an XCD reads a part of x AND a part of the weight (1024 x 768 x 3072 in 64 x 64 tiles: 32 MB from the memory side instead of
+// the 55 that a run of 24 tiles per XCD, which spans all of x, asks for).  per_m = 0: runs of tiles, the row tile fastest.
+struct MidGrid {
+    int xm_mask = 0, xm_shift = 0, per_m = 0, per_n = 0;
+};
+
+// which weight row of the tile LDS row `row` carries: the lane's blocks become consecutive output columns
+template <bool GATED, int TN>
+__device__ __forceinline__ int mid_weight_row(int row) {
+    constexpr int NBN = TN / 16;
+    const int wt = row / TN, rem = row % TN, j = rem / 16, rr = rem % 16;
+    if (!GATED) return wt * TN + 4 * NBN * (rr >> 2) + 4 * j + (rr & 3);
+    constexpr int H = NBN / 2;
+    const int c = wt * (TN / 2) + 4 * H * (rr >> 2) + 4 * (j % (H > 0 ? H : 1)) + (rr & 3);
+    return 64 * (c >> 5) + (c & 31) + 32 * (j / (H > 0 ? H : 1));
+}
+
+template <typename T, typename Cfg, bool GATED, int MODE>
+__global__ void __launch_bounds__(512, 2)
+linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
+                  T *__restrict__ act_in, const float *__restrict__ row_scale, const T *__restrict__ residual, int M, int N, int K,
+                  int64_t ldx, int64_t out_rs, int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int64_t res_rs, int64_t res_cs, int act,
+                  int tiles_m, MidGrid grid, NormFold nf) {
+    typedef typename Vec8<T>::type vec8;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, S = Cfg::S, NBM = Cfg::NBM, NBN = Cfg::NBN, STAGE = Cfg::STAGE, L = Cfg::L;
+    constexpr int LX = Cfg::LX, LW = Cfg::LW, BK = Cfg::BK;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_m = wave % Cfg::WM, wave_n = wave / Cfg::WM;
+    const int r = lane & 15, g = lane >> 4;
+    // workgroup b runs on XCD b % 8, which works on a block of the tile grid of its own (or on a contiguous run of tiles)
+    int tile_m, tile_n;
+    if (grid.per_m != 0) {
+        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+        tile_m = (xcd & grid.xm_mask) * grid.per_m + slot % grid.per_m;
+        tile_n = (xcd >> grid.xm_shift) * grid.per_n + slot / grid.per_m;
+        if (tile_m >= tiles_m || tile_n * BN >= N) return;
+    } else {
+        const int tile = xcd_contiguous_index((int)blockIdx.x, (int)gridDim.x);
+        tile_m = tile % tiles_m;
+        tile_n = tile / tiles_m;
+    }
+    const int m0 = tile_m * BM, n0 = tile_n * BN;
+
+    constexpr uint32_t kOutOfRange = 0x80000000u;
+    const int rows_x = min(BM, M - m0), rows_w = min(BN, N - n0);
+    const uint64_t xaddr = (uint64_t)(uintptr_t)(X + (int64_t)m0 * ldx);
+    const uint64_t waddr = (uint64_t)(uintptr_t)(W + (int64_t)n0 * K);
+    const u32x4 xrsrc = {(uint32_t)xaddr, (uint32_t)(xaddr >> 32) & 0xFFFFu, (uint32_t)((((int64_t)rows_x - 1) * ldx + K) * 2), 0x00020000u};
+    const u32x4 wrsrc = {(uint32_t)waddr, (uint32_t)(waddr >> 32) & 0xFFFFu, (uint32_t)((int64_t)rows_w * K * 2), 0x00020000u};
+    const int nk = (K + BK - 1) / BK, k_last = K - (nk - 1) * BK;
+    // load i of a wave fills the 1 KB (8 rows) piece i * 8 + wave of the operand tile
+    uint32_t xd[LX], wd[LW], tail_bits = 0;
+#pragma unroll
+    for (int i = 0; i < LX; ++i) {
+        const int q = (i * 8 + wave) * 64 + lane, row = SmallTileMap::load_row(q), c = SmallTileMap::load_chunk(q);
+        xd[i] = row < rows_x ? (uint32_t)(((int64_t)row * ldx + c * 8) * 2) : kOutOfRange;
+        if (c * 8 < k_last) tail_bits |= 1u << i;
+    }
+#pragma unroll
+    for (int i = 0; i < LW; ++i) {
+        const int q = (i * 8 + wave) * 64 + lane, row = mid_weight_row<GATED, Cfg::TN>(SmallTileMap::load_row(q)), c = SmallTileMap::load_chunk(q);
+        wd[i] = row < rows_w ? (uint32_t)(((int64_t)row * K + c * 8) * 2) : kOutOfRange;
+        if (c * 8 < k_last) tail_bits |= 1u << (LX + i);
+    }
+    typedef __attribute__((address_space(3))) void lds_void;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_void *)smem + wave * 1024;
+    auto load1 = [&](const u32x4 &rsrc, uint32_t off, uint32_t lds, int kbytes) __attribute__((always_inline)) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                     :: "s"(lds), "v"(off), "s"(rsrc), "s"(kbytes) : "memory", "m0");
+    };
+    auto clip = [&](uint32_t keep) __attribute__((always_inline)) {
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < LX; ++i) xd[i] = ((keep >> i) & 1u) != 0 ? xd[i] : kOutOfRange;
+#pragma unroll
+        for (int i = 0; i < LW; ++i) wd[i] = ((keep >> (LX + i)) & 1u) != 0 ? wd[i] : kOutOfRange;
+    };
+    auto request = [&](int kt, int stage) __attribute__((always_inline)) {
+        if (kt == nk - 1 || kt == nk) clip(kt == nk ? 0u : tail_bits);
+        const uint32_t base = lds_base + (uint32_t)stage * STAGE;
+        const int kbytes = kt < nk ? kt * BK * 2 : 0;
+#pragma unroll
+        for (int i = 0; i < LX; ++i) load1(xrsrc, xd[i], base + i * 8192, kbytes);
+#pragma unroll
+        for (int i = 0; i < LW; ++i) load1(wrsrc, wd[i], base + Cfg::X_BYTES + i * 8192, kbytes);
+    };
+    int xoff[2][NBM], woff[2][NBN];
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+#pragma unroll
+        for (int i = 0; i < NBM; ++i) xoff[st][i] = SmallTileMap::frag_offset(wave_m * Cfg::TM + 16 * i + r, st, g);
+#pragma unroll
+        for (int j = 0; j < NBN; ++j) woff[st][j] = Cfg::X_BYTES + SmallTileMap::frag_offset(wave_n * Cfg::TN + 16 * j + r, st, g);
+    }
+    f32x4_acc acc[NBM][NBN];
+#pragma unroll
+    for (int i = 0; i < NBM; ++i)
+#pragma unroll
+        for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // what the epilogue needs of the lane's rows and columns, requested before anything else: where it is used it would cost
+    // a memory round trip
+    constexpr int C = GATED ? 2 * NBN : 4 * NBN;  // consecutive output columns of a lane
+    constexpr int V = C % 8 == 0 ? 8 : 4;         // columns per access
+    typedef uint32_t words __attribute__((ext_vector_type(V / 2)));
+    const int out_n = GATED ? N / 2 : N;
+    const int n_first = (GATED ? n0 / 2 : n0) + wave_n * (GATED ? Cfg::TN / 2 : Cfg::TN) + C * g;
+    float bz[NBN][4];
+    f32x4 cs[MODE == kNormApply ? NBN : 1];
+    const bool bias_vec = ((uintptr_t)bias & 7) == 0;
+#pragma unroll
+    for (int j = 0; j < NBN; ++j) {
+        const int n = n0 + mid_weight_row<GATED, Cfg::TN>(wave_n * Cfg::TN + 16 * j + 4 * g);
+        if (MODE == kNormApply) {
+            const bool in = n < N;  // (N is a multiple of 32 with a norm)
+            const f32x4 b32 = in ? *reinterpret_cast<const f32x4 *>(nf.bias32 + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            cs[j] = in ? *reinterpret_cast<const f32x4 *>(nf.colsum + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bz[j][e] = b32[e];
+        } else {
+            load_bias4<T>(bias, n, N, bias_vec, bz[j]);
+        }
+    }
+    static_assert(MODE == kNormNone || (!GATED && Cfg::TN == kNormGroup), "with a norm a wave's columns are one statistics group");
+    const bool row_stats = MODE == kNormApply || (MODE == kNormAdd && nf.in_stats != nullptr);
+    words res[MODE == kNormAdd ? NBM : 1], gam = {}, bet = {};
+    if (MODE == kNormAdd) {
+#pragma unroll
+        for (int i = 0; i < NBM; ++i) {
+            const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
+            res[i] = m < M && n_first < N ? *reinterpret_cast<const words *>(static_cast<const T *>(nf.residual) + (int64_t)m * nf.res_rs + n_first) : words{};
+        }
+        if (row_stats && n_first < N) {
+            gam = *reinterpret_cast<const words *>(static_cast<const T *>(nf.gamma) + n_first);
+            if (nf.beta != nullptr) bet = *reinterpret_cast<const words *>(static_cast<const T *>(nf.beta) + n_first);
+        }
+    }
+    auto wait_loads = [&](auto n_c) __attribute__((always_inline)) {
+        constexpr int n = decltype(n_c)::value;
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
+    };
+    // Row statistics: the pairs of the tile's rows lie in one piece of memory.  They travel to the last stage of the ring, in front of
+    // the tiles, are merged by 512 / BM threads a row while the first k-tiles are on their way, and leave (mean, 1 / std) in LDS.
+    __shared__ f32x2 row_norm[MODE != kNormNone ? BM : 1];
+    if (MODE != kNormNone && row_stats) {
+        const uint64_t addr = (uint64_t)(uintptr_t)(nf.in_stats + (int64_t)m0 * nf.in_groups * 2);
+        const int bytes = rows_x * nf.in_groups * 8;
+        const u32x4 rsrc = {(uint32_t)addr, (uint32_t)(addr >> 32) & 0xFFFFu, (uint32_t)bytes, 0x00020000u};
+        for (int piece = wave; piece * 1024 < bytes; piece += 8)
+            load1(rsrc, piece * 1024 + lane * 16, lds_base - wave * 1024 + (S - 1) * STAGE + piece * 1024, 0);
+    }
+#pragma unroll
+    for (int kt = 0; kt < S - 1; ++kt) request(kt, kt);
+    if (MODE != kNormNone && row_stats) {
+        wait_loads(IntC<(S - 1) * L>());
+        __syncthreads();
+        constexpr int LPR = 512 / BM;  // lanes of a row: 4 or 8
+        constexpr int PER = kNormMaxGroups / LPR;
+        const int row = tid / LPR, c = tid % LPR;
+        const f32x2 *pairs = reinterpret_cast<const f32x2 *>(smem + (S - 1) * STAGE) + row * nf.in_groups;
+        f32x2 v[PER];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) v[i] = pairs[c + LPR * i < nf.in_groups ? c + LPR * i : 0];
+        const float pivot = pairs[0][0] * nf.inv_group;
+        NormMerge mg;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (c + LPR * i < nf.in_groups) mg.take(v[i], pivot, nf.inv_group);
+        auto lpr_sum = [](float x) __attribute__((always_inline)) { return LPR == 8 ? oct_sum(x) : quad_sum(x); };
+        mg.d = lpr_sum(mg.d);
+        mg.dd = lpr_sum(mg.dd);
+        mg.m2 = lpr_sum(mg.m2);
+        const f32x2 norm = mg.finish(pivot, nf);
+        if (c == 0) row_norm[row] = norm;
+        __syncthreads();  // the stage is free
+    }
+    request(S - 1, S - 1);
+
+    vec8 xf[2][NBM], wf[2][NBN];
+    auto read = [&](int st, int stage) __attribute__((always_inline)) {
+        const unsigned char *sb = smem + stage * STAGE;
+#pragma unroll
+        for (int i = 0; i < NBM; ++i) xf[st][i] = *reinterpret_cast<const vec8 *>(sb + xoff[st][i]);
+#pragma unroll
+        for (int j = 0; j < NBN; ++j) wf[st][j] = *reinterpret_cast<const vec8 *>(sb + woff[st][j]);
+    };
+    auto multiply = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NBM; ++i)
+#pragma unroll
+            for (int j = 0; j < NBN; ++j) acc[i][j] = mfma16(wf[st][j], xf[st][i], acc[i][j]);
+    };
+    wait_loads(IntC<(S - 1) * L>());
+    __syncthreads();
+    read(0, 0);
+    int stage = 0;
+    for (int kt = 0; kt < nk; ++kt) {
+        const int next = stage == S - 1 ? 0 : stage + 1;
+        read(1, stage);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        wait_loads(IntC<(S - 2) * L>());
+        __syncthreads();  // k-tile kt + 1 has landed for everyone, and nobody reads k-tile kt any more
+        request(kt + S, stage);
+        read(0, next);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1);
+        __builtin_amdgcn_sched_barrier(0);
+        stage = next;
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+
+    // ---- epilogue
+    if (MODE != kNormNone) {
+        auto finish_norm = [&](auto act_c) __attribute__((always_inline)) {
+            constexpr int ACT = decltype(act_c)::value;
+            float gm[8], bt[8];
+            if (MODE == kNormAdd) {
+                unpack4<T>(u32x2{gam[0], gam[1]}, gm);
+                unpack4<T>(u32x2{gam[2 % (V / 2)], gam[3 % (V / 2)]}, gm + 4);
+                unpack4<T>(u32x2{bet[0], bet[1]}, bt);
+                unpack4<T>(u32x2{bet[2 % (V / 2)], bet[3 % (V / 2)]}, bt + 4);
+            }
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) {
+                const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
+                float mean = 0.0f, rstd = 0.0f;
+                if (row_stats) {
+                    const f32x2 norm = row_norm[wave_m * Cfg::TM + 16 * i + r];
+                    mean = norm[0];
+                    rstd = norm[1];
+                }
+                float y[8], h[8] = {};
+                if (MODE == kNormAdd) {
+                    unpack4<T>(u32x2{res[i][0], res[i][1]}, h);
+                    unpack4<T>(u32x2{res[i][2 % (V / 2)], res[i][3 % (V / 2)]}, h + 4);
+                    if (row_stats)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) h[e] = fmaf((h[e] - mean) * rstd, gm[e], bt[e]);
+                }
+                float sum = 0.0f, m2 = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float a = acc[i][(e >> 2) % NBN][e & 3];
+                    if (MODE == kNormApply) y[e] = apply_act16(fmaf(fmaf(-mean, cs[(e >> 2) % NBN][e & 3], a), rstd, bz[(e >> 2) % NBN][e & 3]), ACT);
+                    else y[e] = to_float(from_float<T>(a + bz[(e >> 2) % NBN][e & 3] + h[e]));
+                    sum += y[e];
+                }
+                const bool in = m < M && n_first < N;
+                if (in)
+                    *reinterpret_cast<u32x4 *>(out + (int64_t)m * out_rs + n_first) =
+                        u32x4{pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3]), pack2<T>(y[4], y[5]), pack2<T>(y[6], y[7])};
+                if (MODE == kNormAdd) {
+                    sum = halves32_sum(sum + __shfl_xor(sum, 16));
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) m2 = fmaf(y[e] - sum * (1.0f / kNormGroup), y[e] - sum * (1.0f / kNormGroup), m2);
+                    m2 = halves32_sum(m2 + __shfl_xor(m2, 16));
+                    if (g == 0 && in)
+                        *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / kNormGroup) + n_first / kNormGroup) * 2) = f32x2{sum, m2};
+                }
+            }
+        };
+        if (MODE == kNormAdd) {
+            finish_norm(IntC<KERNL_ACT_NONE>());
+            return;
+        }
+        switch (act) {
+            case KERNL_ACT_RELU: finish_norm(IntC<KERNL_ACT_RELU>()); break;
+            case KERNL_ACT_TANH: finish_norm(IntC<KERNL_ACT_TANH>()); break;
+            case KERNL_ACT_GELU_ERF: finish_norm(IntC<KERNL_ACT_GELU_ERF>()); break;
+            case KERNL_ACT_GELU_TANH: finish_norm(IntC<KERNL_ACT_GELU_TANH>()); break;
+            case KERNL_ACT_SILU: finish_norm(IntC<KERNL_ACT_SILU>()); break;
+            default: finish_norm(IntC<KERNL_ACT_NONE>()); break;
+        }
+        return;
+    }
+    const bool out_vec = out_cs == 1 && (out_rs & (V - 1)) == 0 && ((uintptr_t)out & (2 * V - 1)) == 0;
+    const bool ai_vec = act_in != nullptr && ai_cs == 1 && (ai_rs & (V - 1)) == 0 && ((uintptr_t)act_in & (2 * V - 1)) == 0;
+    const bool res_vec = residual != nullptr && res_cs == 1 && (res_rs & (V - 1)) == 0 && ((uintptr_t)residual & (2 * V - 1)) == 0;
+    auto store = [&](T *p, int64_t cs, bool vec, int n, const float *y) __attribute__((always_inline)) {
+        if (vec && n + V <= out_n) {
+            words w;
+#pragma unroll
+            for (int e = 0; e < V / 2; ++e) w[e] = pack2<T>(y[2 * e], y[2 * e + 1]);
+            *reinterpret_cast<words *>(p) = w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+                if (n + e < out_n) p[e * cs] = from_float<T>(y[e]);
+        }
+    };
+    auto finish = [&](auto act_c) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_c)::value;
+#pragma unroll
+        for (int i = 0; i < NBM; ++i) {
+            const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
+            if (m >= M) continue;
+            const float scale = row_scale != nullptr ? row_scale[m] : 1.0f;
+            float y[C], v[C];
+#pragma unroll
+            for (int j = 0; j < (GATED ? NBN / 2 : NBN); ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float a = fmaf(acc[i][j][e], scale, bz[j][e]);
+                    if (GATED) {
+                        constexpr int H = GATED ? NBN / 2 : 0;
+                        y[4 * j + e] = apply_act16(a, ACT) * fmaf(acc[i][(j + H) % NBN][e], scale, bz[(j + H) % NBN][e]);
+                    } else {
+                        v[4 * j + e] = a;
+                        y[4 * j + e] = apply_act16(a, ACT);
+                    }
+                }
+#pragma unroll
+            for (int c = 0; c < C; c += V) {
+                const int n = n_first + c;
+                if (residual != nullptr) {
+                    const T *rp = residual + (int64_t)m * res_rs + (int64_t)n * res_cs;
+                    T rv[V];
+                    if (res_vec && n + V <= out_n) *reinterpret_cast<words *>(rv) = *reinterpret_cast<const words *>(rp);
+                    else
+#pragma unroll
+                        for (int e = 0; e < V; ++e) rv[e] = n + e < out_n ? rp[e * res_cs] : from_float<T>(0.0f);
+#pragma unroll
+                    for (int e = 0; e < V; ++e) y[c + e] = to_float(from_float<T>(y[c + e])) + to_float(rv[e]);
+                }
+                store(out + (int64_t)m * out_rs + (int64_t)n * out_cs, out_cs, out_vec, n, y + c);
+                if (!GATED && act_in != nullptr) store(act_in + (int64_t)m * ai_rs + (int64_t)n * ai_cs, ai_cs, ai_vec, n, v + c);
+            }
+        }
+    };
+    switch (act) {
+        case KERNL_ACT_RELU: finish(IntC<KERNL_ACT_RELU>()); break;
+        case KERNL_ACT_TANH: finish(IntC<KERNL_ACT_TANH>()); break;
+        case KERNL_ACT_GELU_ERF: finish(IntC<KERNL_ACT_GELU_ERF>()); break;
+        case KERNL_ACT_GELU_TANH: finish(IntC<KERNL_ACT_GELU_TANH>()); break;
+        case KERNL_ACT_SILU: finish(IntC<KERNL_ACT_SILU>()); break;
+        default: finish(IntC<KERNL_ACT_NONE>()); break;
+    }
+}
+
+template <typename T, typename Cfg, bool GATED, int MODE = kNormNone>
+static void launch_mid_cfg(const LinearArgs &a, const NormFold &nf = NormFold()) {
+    auto kern = linear_mid_kernel<T, Cfg, GATED, MODE>;
+    static bool attr_done = false;  // benign race: the attribute call is idempotent
+    if (!attr_done) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);
+        attr_done = true;
+    }
+    const int tiles_m = (a.M + Cfg::BM - 1) / Cfg::BM, tiles_n = (a.N + Cfg::BN - 1) / Cfg::BN;
+    // the XCD blocks: as square in bytes as 8 blocks can be, where they take no more rounds than the tiles themselves
+    MidGrid grid;
+    int blocks = tiles_m * tiles_n;
+    int64_t least = INT64_MAX;
+    for (int s = 0; s <= 3; ++s) {
+        const int xm = 1 << s, xn = 8 >> s, pm = (tiles_m + xm - 1) / xm, pn = (tiles_n + xn - 1) / xn;
+        const int64_t bytes = (int64_t)pm * Cfg::BM + (int64_t)pn * Cfg::BN;
+        if ((int64_t)pm * pn > (int64_t)(tiles_m * tiles_n + 255) / 256 * 32 || bytes >= least) continue;
+        least = bytes;
+        grid.xm_mask = xm - 1; grid.xm_shift = s; grid.per_m = pm; grid.per_n = pn;
+        blocks = 8 * pm * pn;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(512), Cfg::LDS, a.st, static_cast<const T *>(a.x),
+                       static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out), static_cast<T *>(a.act_in),
+                       a.row_scale, static_cast<const T *>(a.residual), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs,
+                       a.res_rs, a.res_cs, a.act & (kGluBit - 1), tiles_m, grid, nf);
+}
+
+// the tiles, by the kernl_linear_force_tile value that forces them
+typedef MidTile<64, 64, 4, 2, 4> Mid64x64;      // 11   64 KB: two workgroups per CU
+typedef MidTile<128, 64, 4, 2, 3> Mid128x64;    // 15   72 KB: two workgroups per CU
+typedef MidTile<128, 128, 2, 4, 4> Mid128x128;  // 17
+typedef MidTile<192, 128, 4, 2, 4> Mid192x128;  // 18
+typedef MidTile<192, 192, 4, 2, 3> Mid192x192;  // 19
+typedef MidTile<128, 256, 2, 4, 3> Mid128x256;  // 20
+typedef MidTile<256, 128, 4, 2, 3> Mid256x128;  // 21
+
+template <typename T, typename Cfg>
+static int launch_mid(const LinearArgs &a, int mode, const NormFold &nf) {
+    if (mode != kNormNone) {
+        if constexpr (Cfg::TN == kNormGroup) {
+            if (mode == kNormApply) launch_mid_cfg<T, Cfg, false, kNormApply>(a, nf);
+            else launch_mid_cfg<T, Cfg, false, kNormAdd>(a, nf);
+            return 1;
+        }
+        return 0;
+    }
+    if (a.act & kGluBit) {
+        if constexpr (Cfg::NBN % 2 == 0) {
+            launch_mid_cfg<T, Cfg, true>(a);
+            return 1;
+        }
+        return 0;
+    }
+    launch_mid_cfg<T, Cfg, false>(a);
+    return 1;
+}
+
+template <typename T>
+static int run_mid_t(const LinearArgs &a, int kind, int mode, const NormFold &nf) {
+    switch (kind) {
+        case 11: return launch_mid<T, Mid64x64>(a, mode, nf);
+        case 15: return launch_mid<T, Mid128x64>(a, mode, nf);
+        case 17: return launch_mid<T, Mid128x128>(a, mode, nf);
+        case 18: return launch_mid<T, Mid192x128>(a, mode, nf);
+        case 19: return launch_mid<T, Mid192x192>(a, mode, nf);
+        case 20: return launch_mid<T, Mid128x256>(a, mode, nf);
+        case 21: return launch_mid<T, Mid256x128>(a, mode, nf);
+        default: return 0;
+    }
+}
+
+int run_mid(const LinearArgs &a, int dtype, int kind, int mode, const NormFold &nf) {
+    return dtype == KERNL_F16 ? run_mid_t<f16>(a, kind, mode, nf) : run_mid_t<bf16>(a, kind, mode, nf);
+}
+
+}  // namespace kernl

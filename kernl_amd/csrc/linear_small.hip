@@ -6,7 +6,7 @@
 // C = act(A @ W^T + bias), optional store of the pre-activation); what differs is the shape of the work.  A workgroup of
 // 4 waves (2 x 2) owns a 64 x 64 or 32 x 64 output tile over the WHOLE of K: one launch, no partial sums in memory,
 // 50 to 256 workgroups.  Such a tile is 4 or 8 MFMAs per wave and 64-wide k-tile — the loop is bound by how fast the
-// CU can pull its operand tiles (12 or 16 KB per k-tile) out of L2, i.e. by latency unless many k-tiles are in
+// CU can pull its operand tiles (12 KB per k-tile) out of L2, i.e. by latency unless many k-tiles are in
 // flight: operand tiles travel HBM/L2 -> LDS directly (buffer loads with the LDS flag, every lane fetching the 16-byte
 // chunk that belongs at its LDS position under the XOR swizzle) through a ring of 8 stages, 7 k-tiles requested
 // ahead, one barrier per k-tile and waits by count.  A last k-tile that reaches beyond K has the chunks that
@@ -16,22 +16,12 @@
 
 namespace kernl {
 
-// bias[n .. n + 3] as floats (zeros past N or without a bias): one 8-byte load where the four are inside and aligned
-template <typename T>
-__device__ __forceinline__ void load_bias4(const T *__restrict__ bias, int n, int N, bool vec_ok, float (&dst)[4]) {
-    if (bias != nullptr && vec_ok && n + 4 <= N) {
-        unpack4<T>(*reinterpret_cast<const u32x2 *>(bias + n), dst);
-        return;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) dst[e] = (bias != nullptr && n + e < N) ? to_float(bias[n + e]) : 0.0f;
-}
-
 // Row statistics on their way to the epilogue: the pairs of a row tile lie in one piece of memory and travel to LDS in
 // front of the first k-tile, `per_wave` KB-sized loads per wave (pieces past the end arrive as zeros or are not asked for).
-template <int BM>
+constexpr int norm_stats_bytes(int bm) { return bm * 8 * (bm <= 32 ? 2 * kNormMaxGroups : kNormMaxGroups); }
+template <int BM, int WAVES>
 __device__ __forceinline__ void request_norm_stats(const NormFold &nf, int m0, int rows, uint32_t lds, int wave, int lane) {
-    constexpr int PER_WAVE = BM * kNormMaxGroups * 8 / 4096;
+    constexpr int PER_WAVE = norm_stats_bytes(BM) / 1024 / WAVES;
     static_assert(PER_WAVE >= 1, "whole KB per wave");
     const uint64_t addr = (uint64_t)(uintptr_t)(nf.in_stats + (int64_t)m0 * nf.in_groups * 2);
     const u32x4 rsrc = {(uint32_t)addr, (uint32_t)(addr >> 32) & 0xFFFFu, (uint32_t)(rows * nf.in_groups * 8), 0x00020000u};
@@ -182,7 +172,7 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
         }
     }
     const bool row_stats = MODE == kNormApply || (MODE == kNormAdd && nf.in_stats != nullptr);
-    if (MODE != kNormNone && row_stats) request_norm_stats<BM>(nf, m0, rows_x, lds_base + S * STAGE, wave, lane);
+    if (MODE != kNormNone && row_stats) request_norm_stats<BM, 4>(nf, m0, rows_x, lds_base + S * STAGE, wave, lane);
 
 #pragma unroll
     for (int kt = 0; kt < S - 1; ++kt) request(kt, kt);
@@ -221,13 +211,20 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
 #pragma unroll
             for (int i = 0; i < NBM; ++i) {
                 const f32x2 *row = reinterpret_cast<const f32x2 *>(st) + (wave_m * (BM / 2) + 16 * i + r) * groups;
-                const float pivot = row[0][0] * (1.0f / kNormGroup);
+                const float pivot = row[0][0] * nf.inv_group;
                 NormMerge mg;
-                for (int p = g; p < groups; p += 4) mg.take(row[p], pivot);
+                f32x2 pairs[kNormMaxGroups / 2];  // (read together: one after the other each costs an LDS round trip)
+#pragma unroll
+                for (int q = 0; q < kNormMaxGroups / 2; ++q) pairs[q] = row[4 * q + g < groups ? 4 * q + g : 0];
+#pragma unroll
+                for (int q = 0; q < kNormMaxGroups / 2; ++q)
+                    if (4 * q + g < groups) mg.take(pairs[q], pivot, nf.inv_group);
                 mg.d = halves32_sum(mg.d + __shfl_xor(mg.d, 16));
                 mg.dd = halves32_sum(mg.dd + __shfl_xor(mg.dd, 16));
                 mg.m2 = halves32_sum(mg.m2 + __shfl_xor(mg.m2, 16));
-                mg.finish(pivot, groups, nf.eps, mean[i], rstd[i]);
+                const f32x2 norm = mg.finish(pivot, nf);
+                mean[i] = norm[0];
+                rstd[i] = norm[1];
             }
         }
         auto finish_norm = [&](auto act_c) __attribute__((always_inline)) {
@@ -347,22 +344,22 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
 
 // The same problem class with a LONG K (BERT-base's feed-forward down projection at batch 1: 128 x 768 x 3072): time per
 // workgroup is latency x (bytes the workgroup pulls) / (bytes the CU keeps in flight), so the tiles get smaller still
-// — 32 x 32 or 16 x 32, up to 256 workgroups — and the four waves no longer share a tile's k-tiles but deal them out:
+// — 16 x 16 to 64 x 32, up to 256 workgroups — and the four waves no longer share a tile's k-tiles but deal them out:
 // wave w multiplies k-tiles w, w + 4, ... of the WHOLE tile out of a ring of its own (no barrier in the loop, program
 // order and the load counter are all the synchronisation), and the four partial tiles meet in LDS at the end.
 // a wave's ring: 32 KB, 36 KB for the 12 KB stages of 64 x 32 tiles (three of them)
-constexpr int small_ring_bytes(int bm, int bn) { return (bm + bn) == 96 ? 36 * 1024 : 32 * 1024; }
+constexpr int small_ring_bytes(int bm, int bn, int waves) { return waves == 8 ? 16 * 1024 : (bm + bn) == 96 ? 36 * 1024 : 32 * 1024; }
 
-template <typename T, int BM, int BN, int MODE>
-__global__ void __launch_bounds__(256, 1)
+template <typename T, int BM, int BN, int WAVES, int MODE>
+__global__ void __launch_bounds__(64 * WAVES, 1)
 linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias,
                           T *__restrict__ out, T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs,
                           int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int act, int tiles_m, NormFold nf) {
     typedef typename Vec8<T>::type vec8;
-    constexpr int BK = 64, RB = BK * 2, CPR = BK / 8, WAVES = 4;
+    constexpr int BK = 64, RB = BK * 2, CPR = BK / 8;
     static_assert(RB == SmallTileMap::ROW_BYTES && CPR == SmallTileMap::CHUNKS_PER_ROW, "tile rows as the tile map lays them out");
     constexpr int X_BYTES = BM * RB, W_BYTES = BN * RB, STAGE = X_BYTES + W_BYTES;
-    constexpr int RING = small_ring_bytes(BM, BN), S = RING / STAGE;  // a wave's ring and its stages
+    constexpr int RING = small_ring_bytes(BM, BN, WAVES), S = RING / STAGE;  // a wave's ring and its stages
     constexpr int LX = BM * CPR / 64, LW = BN * CPR / 64, L = LX + LW;  // 1 KB loads per wave and stage
     constexpr int NBM = BM / 16, NBN = BN / 16;
     static_assert(S >= 3 && (S - 2) * L <= 63, "ring depth and wait count");
@@ -442,12 +439,12 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
 #pragma unroll
         for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // In the epilogue thread t finishes columns 4 (t % 8) .. + 3 of the tile's rows t / 8, t / 8 + 32, ...: whole 64-byte row
-    // pieces per store, and a row's 32 columns meet in eight neighbouring lanes (statistics).  What it needs of them is
-    // requested before anything else.
-    static_assert(BN == kNormGroup, "a tile row is one statistics group");
-    constexpr int OWN = (BM + 31) / 32;
-    const int own_row = tid >> 3, n_own = n0 + 4 * (tid & 7);
+    // In the epilogue LPR = BN / 4 neighbouring lanes finish a row of the tile, 4 columns each: whole row pieces per store, and
+    // a row's columns meet in neighbouring lanes (statistics).  What a thread needs of its row and columns is requested before
+    // anything else.
+    constexpr int LPR = BN / 4, ROWS = 64 * WAVES / LPR, OWN = (BM + ROWS - 1) / ROWS;
+    const int own_row = tid / LPR, own_c = tid % LPR, n_own = n0 + 4 * own_c;
+    auto lpr_sum = [](float v) __attribute__((always_inline)) { return LPR == 8 ? oct_sum(v) : quad_sum(v); };
     float bz[4];
     f32x4 cs = {0.0f, 0.0f, 0.0f, 0.0f};
     u32x2 res[OWN], gam = {0, 0}, bet = {0, 0};
@@ -463,8 +460,8 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     if (MODE == kNormAdd) {
 #pragma unroll
         for (int t = 0; t < OWN; ++t) {
-            const int m = m0 + own_row + 32 * t;
-            res[t] = own_row + 32 * t < rows_x ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + (int64_t)m * nf.res_rs + n_own) : u32x2{0, 0};
+            const int m = m0 + own_row + ROWS * t;
+            res[t] = own_row + ROWS * t < rows_x ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + (int64_t)m * nf.res_rs + n_own) : u32x2{0, 0};
         }
         if (row_stats) {
             gam = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.gamma) + n_own);
@@ -472,7 +469,7 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
         }
     }
     if (MODE != kNormNone && row_stats)
-        request_norm_stats<BM>(nf, m0, rows_x, (uint32_t)(uintptr_t)(lds_void *)smem + WAVES * RING, wave, lane);
+        request_norm_stats<BM, WAVES>(nf, m0, rows_x, (uint32_t)(uintptr_t)(lds_void *)smem + WAVES * RING, wave, lane);
     const int mine = nk > wave ? (nk - wave + WAVES - 1) / WAVES : 0;  // k-tiles of this wave
 #pragma unroll
     for (int j = 0; j < S - 1; ++j) request(j, j);
@@ -503,6 +500,33 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the out-of-range requests of the last rounds are done with
     __syncthreads();                     // every ring is free: the partial tiles take their place
 
+    // row statistics (staged behind the rings) merged by up to 16 threads a row, beside the stores of the partial tiles
+    f32x2 *row_norm = reinterpret_cast<f32x2 *>(smem + WAVES * RING) - BM;  // (the end of the rings, which the partial tiles leave free)
+    static_assert(WAVES * NBM * NBN * 1024 + BM * 8 <= WAVES * RING, "room behind the partial tiles");
+    if (MODE != kNormNone && row_stats) {
+        constexpr int SPAN = 64 * WAVES / BM < 16 ? 64 * WAVES / BM : 16, PER = norm_stats_bytes(BM) / BM / 8 / SPAN;
+        const int row = tid / SPAN, c = tid % SPAN;
+        if (row < BM) {
+            const f32x2 *pairs = reinterpret_cast<const f32x2 *>(smem + WAVES * RING) + row * nf.in_groups;
+            const float pivot = pairs[0][0] * nf.inv_group;
+            NormMerge mg;
+            auto merge = [&](int first, int last) __attribute__((always_inline)) {
+                f32x2 v[PER];  // (read together: one after the other each costs an LDS round trip)
+#pragma unroll
+                for (int q = first; q < last; ++q) v[q] = pairs[SPAN * q + c < nf.in_groups ? SPAN * q + c : 0];
+#pragma unroll
+                for (int q = first; q < last; ++q)
+                    if (SPAN * q + c < nf.in_groups) mg.take(v[q], pivot, nf.inv_group);
+            };
+            merge(0, PER / 2);
+            if (SPAN * (PER / 2) < nf.in_groups) merge(PER / 2, PER);
+            auto span_sum = [](float x) __attribute__((always_inline)) { return SPAN == 16 ? row16_sum(x) : SPAN == 8 ? oct_sum(x) : quad_sum(x); };
+            mg.d = span_sum(mg.d);
+            mg.dd = span_sum(mg.dd);
+            mg.m2 = span_sum(mg.m2);
+            if (c == 0) row_norm[row] = mg.finish(pivot, nf);
+        }
+    }
     float *red = reinterpret_cast<float *>(smem);  // [wave][block][lane][4]
 #pragma unroll
     for (int i = 0; i < NBM; ++i)
@@ -517,24 +541,19 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     constexpr int ACT = decltype(act_c)::value;
 #pragma unroll
     for (int t = 0; t < OWN; ++t) {
-        const int row = own_row + 32 * t;
-        if (BM < 32 && row >= BM) break;
-        // block (row / 16, (tid & 7) / 4), its lane (row % 16, tid & 3)
-        const int at = (((row >> 4) * NBN + ((tid & 7) >> 2)) * 64 + (tid & 3) * 16 + (row & 15)) * 4;
+        const int row = own_row + ROWS * t;
+        if (BM < ROWS && row >= BM) break;
+        // block (row / 16, own_c / 4), its lane (row % 16, own_c % 4)
+        const int at = (((row >> 4) * NBN + (own_c >> 2)) * 64 + (own_c & 3) * 16 + (row & 15)) * 4;
         f32x4_acc sum = *reinterpret_cast<const f32x4_acc *>(red + at);
 #pragma unroll
         for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_acc *>(red + w * (NBM * NBN) * 256 + at);
         const int m = m0 + row, n = n_own;
-        float v[4], y[4], mean = 0.0f, rstd = 0.0f;
+        float pre[4], y[4], mean = 0.0f, rstd = 0.0f;
         if (MODE != kNormNone && row_stats) {
-            const f32x2 *pairs = reinterpret_cast<const f32x2 *>(smem + WAVES * RING) + row * nf.in_groups;
-            const float pivot = pairs[0][0] * (1.0f / kNormGroup);
-            NormMerge mg;
-            for (int p = tid & 7; p < nf.in_groups; p += 8) mg.take(pairs[p], pivot);
-            mg.d = oct_sum(mg.d);
-            mg.dd = oct_sum(mg.dd);
-            mg.m2 = oct_sum(mg.m2);
-            mg.finish(pivot, nf.in_groups, nf.eps, mean, rstd);
+            const f32x2 norm = row_norm[row];
+            mean = norm[0];
+            rstd = norm[1];
         }
         if (MODE == kNormAdd) {
             float h[4], gm[4], bt[4];
@@ -551,18 +570,21 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
                 y[e] = to_float(from_float<T>(sum[e] + bz[e] + h[e]));
                 total += y[e];
             }
-            total = oct_sum(total);
-            const float mu = total * (1.0f / kNormGroup);
+            // statistics of the stored values: the row's lanes, or with 16-column groups in 32-column tiles half of them
+            const bool halves = LPR == 8 && nf.group == kNormGroupFew;
+            const int cols = halves ? kNormGroupFew : BN;
+            total = halves ? quad_sum(total) : lpr_sum(total);
+            const float mu = total / (float)cols;
 #pragma unroll
             for (int e = 0; e < 4; ++e) m2 = fmaf(y[e] - mu, y[e] - mu, m2);
-            m2 = oct_sum(m2);
-            if ((tid & 7) == 0 && m < M)
-                *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / kNormGroup) + n0 / kNormGroup) * 2) = f32x2{total, m2};
+            m2 = halves ? quad_sum(m2) : lpr_sum(m2);
+            if (own_c % (cols / 4) == 0 && m < M)
+                *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / cols) + n_own / cols) * 2) = f32x2{total, m2};
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v[e] = MODE == kNormApply ? fmaf(fmaf(-mean, cs[e], sum[e]), rstd, bz[e]) : sum[e] + bz[e];
-                y[e] = apply_act16(v[e], ACT);
+                pre[e] = MODE == kNormApply ? fmaf(fmaf(-mean, cs[e], sum[e]), rstd, bz[e]) : sum[e] + bz[e];
+                y[e] = apply_act16(pre[e], ACT);
             }
         }
         if (m >= M || n >= N) continue;
@@ -576,12 +598,12 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
         }
         if (MODE == kNormNone && act_in != nullptr) {
             if (n + 4 <= N && ai_vec) {
-                const u32x2 p = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+                const u32x2 p = {pack2<T>(pre[0], pre[1]), pack2<T>(pre[2], pre[3])};
                 *reinterpret_cast<u32x2 *>(act_in + (int64_t)m * ai_rs + n) = p;
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (n + e < N) act_in[(int64_t)m * ai_rs + (int64_t)(n + e) * ai_cs] = from_float<T>(v[e]);
+                    if (n + e < N) act_in[(int64_t)m * ai_rs + (int64_t)(n + e) * ai_cs] = from_float<T>(pre[e]);
             }
         }
     }
@@ -600,46 +622,50 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     }
 }
 
-template <typename T, int BM, int BN, int MODE>
+template <typename T, int BM, int BN, int WAVES, int MODE>
 static void launch_small_dealt_mode(const LinearArgs &a, const NormFold &nf) {
-    auto kern = linear_small_dealt_kernel<T, BM, BN, MODE>;
-    constexpr int LDS_BYTES = 4 * small_ring_bytes(BM, BN) + (MODE != kNormNone ? BM * kNormMaxGroups * 8 : 0);
+    auto kern = linear_small_dealt_kernel<T, BM, BN, WAVES, MODE>;
+    constexpr int LDS_BYTES = WAVES * small_ring_bytes(BM, BN, WAVES) + (MODE != kNormNone ? norm_stats_bytes(BM) : 0);
+    static_assert(LDS_BYTES <= 160 * 1024, "one workgroup per CU");
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
         attr_done = true;
     }
     const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), LDS_BYTES, a.st, static_cast<const T *>(a.x),
+    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * WAVES), LDS_BYTES, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out),
                        static_cast<T *>(a.act_in), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs, a.act,
                        tiles_m, nf);
 }
 
-template <typename T, int BM, int BN>
+template <typename T, int BM, int BN, int WAVES = 4>
 static void launch_small_dealt(const LinearArgs &a, int mode, const NormFold &nf) {
-    if (mode == kNormApply) launch_small_dealt_mode<T, BM, BN, kNormApply>(a, nf);
-    else if (mode == kNormAdd) launch_small_dealt_mode<T, BM, BN, kNormAdd>(a, nf);
-    else launch_small_dealt_mode<T, BM, BN, kNormNone>(a, nf);
+    if (mode == kNormApply) launch_small_dealt_mode<T, BM, BN, WAVES, kNormApply>(a, nf);
+    else if (mode == kNormAdd) launch_small_dealt_mode<T, BM, BN, WAVES, kNormAdd>(a, nf);
+    else launch_small_dealt_mode<T, BM, BN, WAVES, kNormNone>(a, nf);
 }
 
-// rows: 16, 32 or 64 per tile (32 columns)
-void run_small_dealt(const LinearArgs &a, int dtype, int rows, int mode, const NormFold &nf) {
-    if (dtype == KERNL_F16) {
-        if (rows == 16) launch_small_dealt<f16, 16, 32>(a, mode, nf);
-        else if (rows == 32) launch_small_dealt<f16, 32, 32>(a, mode, nf);
-        else launch_small_dealt<f16, 64, 32>(a, mode, nf);
-    } else {
-        if (rows == 16) launch_small_dealt<bf16, 16, 32>(a, mode, nf);
-        else if (rows == 32) launch_small_dealt<bf16, 32, 32>(a, mode, nf);
-        else launch_small_dealt<bf16, 64, 32>(a, mode, nf);
-    }
+template <typename T>
+static void run_small_dealt_t(const LinearArgs &a, int rows, int cols, int mode, const NormFold &nf) {
+    if (cols == 16) {
+        if (a.K >= 24 * 64) launch_small_dealt<T, 16, 16, 8>(a, mode, nf);  // three k-tiles a wave or more
+        else launch_small_dealt<T, 16, 16>(a, mode, nf);
+    } else if (rows == 16) launch_small_dealt<T, 16, 32>(a, mode, nf);
+    else if (rows == 32) launch_small_dealt<T, 32, 32>(a, mode, nf);
+    else launch_small_dealt<T, 64, 32>(a, mode, nf);
+}
+
+// rows x cols of a tile: 16 x 16, 16 x 32, 32 x 32 or 64 x 32
+void run_small_dealt(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf) {
+    if (dtype == KERNL_F16) run_small_dealt_t<f16>(a, rows, cols, mode, nf);
+    else run_small_dealt_t<bf16>(a, rows, cols, mode, nf);
 }
 
 template <typename T, int BM, int BN, int MODE>
 static void launch_small_mode(const LinearArgs &a, const NormFold &nf) {
     auto kern = linear_small_kernel<T, BM, BN, MODE>;
-    constexpr int LDS_BYTES = small_stages(BM, BN) * (BM + BN) * kSmallBK * 2 + (MODE != kNormNone ? BM * kNormMaxGroups * 8 : 0);
+    constexpr int LDS_BYTES = small_stages(BM, BN) * (BM + BN) * kSmallBK * 2 + (MODE != kNormNone ? norm_stats_bytes(BM) : 0);
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
@@ -659,17 +685,10 @@ static void launch_small(const LinearArgs &a, int mode, const NormFold &nf) {
     else launch_small_mode<T, BM, BN, kNormNone>(a, nf);
 }
 
-// tile shapes: 32 x 64, 64 x 64, 64 x 128 (rows x columns; the last in a ring of 6 stages)
-void run_small(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf) {
-    if (dtype == KERNL_F16) {
-        if (cols == 128) launch_small<f16, 64, 128>(a, mode, nf);
-        else if (rows == 32) launch_small<f16, 32, 64>(a, mode, nf);
-        else launch_small<f16, 64, 64>(a, mode, nf);
-    } else {
-        if (cols == 128) launch_small<bf16, 64, 128>(a, mode, nf);
-        else if (rows == 32) launch_small<bf16, 32, 64>(a, mode, nf);
-        else launch_small<bf16, 64, 64>(a, mode, nf);
-    }
+// 32 x 64 tiles
+void run_small(const LinearArgs &a, int dtype, int mode, const NormFold &nf) {
+    if (dtype == KERNL_F16) launch_small<f16, 32, 64>(a, mode, nf);
+    else launch_small<bf16, 32, 64>(a, mode, nf);
 }
 
 }  // namespace kernl

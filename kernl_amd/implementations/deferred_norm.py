@@ -10,7 +10,7 @@ import torch
 from kernl_amd import _lib
 from kernl_amd.implementations.linear_layer import ACTIVATIONS
 
-MAX_WIDTH = 1024  # statistics of a row that the kernels stage (32 columns a pair)
+MAX_WIDTH = 1024  # statistics of a row that the kernels stage
 
 
 class FoldedParams(NamedTuple):
@@ -89,7 +89,8 @@ def linear_add_deferred(x: torch.Tensor, weight: torch.Tensor, bias, residual, g
     """linear(x, weight, bias) + residual with its row statistics, in one launch; `residual` may be a deferred norm."""
     n = weight.shape[0]
     out = torch.empty((*x.shape[:-1], n), device=x.device, dtype=x.dtype)
-    stats = torch.empty((x.numel() // x.shape[-1], n // 32, 2), device=x.device, dtype=torch.float32)
+    rows = x.numel() // x.shape[-1]
+    stats = torch.empty((rows, n // _lib.linear_norm_group(rows), 2), device=x.device, dtype=torch.float32)
     if isinstance(residual, DeferredNorm):
         args = (_rows(residual.rows), residual.stats, residual.gamma, residual.beta, residual.kernel_eps)
     else:

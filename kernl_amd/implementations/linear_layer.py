@@ -61,6 +61,16 @@ def takes_small_problem_kernel(x2d: torch.Tensor, weight: torch.Tensor) -> bool:
     )
 
 
+def takes_mid_kernel(x2d: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
+    """Whether the product runs on one of the 8-wave tiles over the whole K (65 to some 3000 rows): faster there than the
+    stream-K and split-K kernels the shape would otherwise qualify for."""
+    return (
+        x2d.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x2d.dtype
+        and x2d.stride(1) == 1 and x2d.stride(0) % 8 == 0 and x2d.stride(0) < (1 << 22) and x2d.data_ptr() % 16 == 0
+        and weight.data_ptr() % 16 == 0 and _lib.linear_mid_kind(x2d.shape[0], weight.shape[0], x2d.shape[1], gated) != 0
+    )
+
+
 def takes_few_row_kernel(x2d: torch.Tensor, weight: torch.Tensor) -> bool:
     return few_row_rule(x2d.shape[0], weight.shape[0], weight.shape[1]) and _lib.linear_fewrow_supported(x2d, weight)
 
@@ -111,7 +121,7 @@ class LinearLayer(torch.autograd.Function):
         outputs = torch.empty((M, N), device=x.device, dtype=x.dtype)
         if act_inputs is not None:
             assert act_inputs.shape == (M, N) and act_inputs.dtype == x.dtype
-        small = takes_small_problem_kernel(x_, weight)
+        small = takes_small_problem_kernel(x_, weight) or takes_mid_kernel(x_, weight)
         split_bytes = 0
         if not small and FEW_ROW_MAX_ROWS < M <= SPLIT_K_MAX_ROWS:
             split_bytes = _lib.linear_splitk_workspace_bytes(x_, weight)
@@ -181,7 +191,7 @@ class LinearGLU(torch.autograd.Function):
             x_ = x_.contiguous()
         M, N = x_.shape[0], weight.shape[0] // 2
         out = torch.empty((M, N), device=x.device, dtype=x.dtype)
-        if takes_few_row_kernel(x_, weight):
+        if takes_few_row_kernel(x_, weight) and not takes_mid_kernel(x_, weight, gated=True):
             _lib.linear_fewrow_fwd(x_, weight, bias, None, out, ACTIVATIONS.get(activation, _lib.ACT_NONE), gated=True)
         else:
             _lib.linear_glu_fwd(x_, weight, bias, out, ACTIVATIONS.get(activation, _lib.ACT_NONE))
@@ -258,7 +268,9 @@ def rms_linear_layer(
         and (bias is None or bias.dtype == x.dtype)
         # only where the plain product would run the wide tile kernels anyway (not the small-tile or split-K forms)
         and not takes_small_problem_kernel(x_, folded_weight)
-        and (x_.shape[0] > SPLIT_K_MAX_ROWS or _lib.linear_splitk_workspace_bytes(x_, folded_weight) == 0)
+        # (8-wave tiles take the row factors too: a large weight's product then saves the norm's launch and pass)
+        and (x_.shape[0] > SPLIT_K_MAX_ROWS or _lib.linear_splitk_workspace_bytes(x_, folded_weight) == 0
+             or (folded_weight.numel() >= 1 << 24 and takes_mid_kernel(x_, folded_weight, gated)))
     ):
         if rstd is None:
             rstd = rms_stats(x_, eps, clamp=False)
@@ -337,7 +349,7 @@ def residual_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optio
     x_ = x if x.ndim == 2 else x.reshape(-1, x.shape[-1])
     if not _lib.linear_scaled_supported(x_, weight):
         return False
-    if rows <= SPLIT_K_MAX_ROWS and _lib.linear_splitk_workspace_bytes(x_, weight) != 0:
+    if rows <= SPLIT_K_MAX_ROWS and not takes_mid_kernel(x_, weight) and _lib.linear_splitk_workspace_bytes(x_, weight) != 0:
         return False
     return _lib.linear_wide_kind(rows, weight.shape[0], weight.shape[1]) != 0
 

@@ -45,9 +45,10 @@ def test_both_sides_of_a_deferred_norm(rows, n, k, offset, dtype):
     s = x.double() @ w.double().T + b.double() + res.double()
     assert _error(norm.rows, s) <= unit
     # statistics of the stored rows, group by group
-    groups = norm.rows.double().view(rows, n // 32, 32)
+    group = _lib.linear_norm_group(rows)
+    groups = norm.rows.double().view(rows, n // group, group)
     assert torch.allclose(norm.stats[..., 0].double(), groups.sum(-1), rtol=1e-5, atol=1e-3)
-    assert torch.allclose(norm.stats[..., 1].double(), groups.var(-1, unbiased=False) * 32, rtol=1e-4, atol=1e-4)
+    assert torch.allclose(norm.stats[..., 1].double(), groups.var(-1, unbiased=False) * group, rtol=1e-4, atol=1e-4)
     # a second addition on top of the deferred residual
     eps = norm.kernel_eps
     h = _ln(norm.rows, gamma, beta, eps)
@@ -66,7 +67,7 @@ def test_both_sides_of_a_deferred_norm(rows, n, k, offset, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("force, rows", [(10, 70), (11, 70), (15, 70), (12, 21), (13, 45), (14, 70)], ids=str)
+@pytest.mark.parametrize("force, rows", [(10, 70), (11, 70), (15, 70), (12, 21), (13, 45), (14, 70), (16, 40), (17, 130)], ids=str)
 def test_every_tile_form_takes_both_modes(force, rows):
     from kernl_amd.implementations.deferred_norm import FoldedParams, linear_add_deferred
 
