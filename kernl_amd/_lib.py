@@ -47,6 +47,9 @@ EXPORTED_SYMBOLS = (
     "kernl_linear_norm_add_fwd",
     "kernl_linear_norm_apply_fwd",
     "kernl_embedding_layernorm_fwd",
+    "kernl_embedding_layernorm_via_fwd",
+    "kernl_copy_many",
+    "kernl_select_mask_fwd",
     "kernl_linear_decode_fwd",
     "kernl_linear_splitk_workspace_bytes",
     "kernl_linear_splitk_fwd",
@@ -160,6 +163,14 @@ def load() -> ctypes.CDLL:
     lib.kernl_embedding_layernorm_fwd.restype = ctypes.c_int
     lib.kernl_embedding_layernorm_fwd.argtypes = [_vp, _vp, _i64, _i64, _i64] * 3 + [_vp, _vp, _vp, _i64, _i64, _i64,
                                                                                       ctypes.c_float, ctypes.c_int, _vp]
+    lib.kernl_embedding_layernorm_via_fwd.restype = ctypes.c_int
+    lib.kernl_embedding_layernorm_via_fwd.argtypes = (
+        [_vp, _vp, _i64, _i64, _i64] * 3 + [ctypes.c_int, _vp, _i64] + [_vp, _vp, _vp, _i64, _i64, _i64, ctypes.c_float, ctypes.c_int, _vp]
+    )
+    lib.kernl_copy_many.restype = ctypes.c_int
+    lib.kernl_copy_many.argtypes = [ctypes.c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _i64p, _vp]
+    lib.kernl_select_mask_fwd.restype = ctypes.c_int
+    lib.kernl_select_mask_fwd.argtypes = [_vp, ctypes.c_int, ctypes.c_float, ctypes.c_float, _vp, _i64, ctypes.c_int, _vp]
     lib.kernl_add_rms_stats_fwd.restype = ctypes.c_int
     lib.kernl_add_rms_stats_fwd.argtypes = [_vp] * 4 + [_i64] * 5 + [ctypes.c_float, ctypes.c_int, _vp]
     lib.kernl_linear_small_kind.restype = ctypes.c_int
@@ -464,9 +475,10 @@ def linear_residual_fwd(x2d, weight, bias, residual2d, out2d) -> None:
     _check(st, "kernl_linear_residual_fwd")
 
 
-def embedding_layernorm_fwd(tables, ids, weight, bias, out, eps: float) -> None:
+def embedding_layernorm_fwd(tables, ids, weight, bias, out, eps: float, via=None) -> None:
     """out[b, s] = LayerNorm(sum of tables[i][ids[i][b, s]]) (rows added one after the other in the tables' dtype).
-    tables: 1 to 3 contiguous [rows, N] matrices; ids: int64 [batch, seq] views (stride 0 allowed); out [batch, seq, N]."""
+    tables: 1 to 3 contiguous [rows, N] matrices; ids: int64 [batch, seq] views (stride 0 allowed); out [batch, seq, N].
+    via: None or (slot, vector): the ids of table `slot` are vector[ids[slot]]."""
     _require_gpu(*tables, *ids, weight, bias, out)
     batch, seq, n = out.shape
     if not 1 <= len(tables) <= 3 or len(ids) != len(tables):
@@ -483,9 +495,27 @@ def embedding_layernorm_fwd(tables, ids, weight, bias, out, eps: float) -> None:
             args += [None, None, 0, 0, 0]
     lib = load()
     with torch.cuda.device(out.device):
-        st = lib.kernl_embedding_layernorm_fwd(*args, weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(),
-                                               batch, seq, n, float(eps), DTYPE_CODE[out.dtype], _stream(out))
+        rest = (weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(), batch, seq, n, float(eps),
+                DTYPE_CODE[out.dtype], _stream(out))
+        if via is None:
+            st = lib.kernl_embedding_layernorm_fwd(*args, *rest)
+        else:
+            slot, source = via
+            if source.dtype != torch.int64 or source.dim() != 1 or not source.is_contiguous() or not source.is_cuda:
+                raise ValueError("the vector that ids go through is a contiguous int64 vector on the GPU")
+            st = lib.kernl_embedding_layernorm_via_fwd(*args, int(slot), source.data_ptr(), source.numel(), *rest)
     _check(st, "kernl_embedding_layernorm_fwd")
+
+
+def select_mask_fwd(mask, on: float, off: float, out) -> None:
+    """out = where(mask != 0, on, off) of a contiguous integer or boolean mask."""
+    _require_gpu(mask, out)
+    if not mask.is_contiguous() or not out.is_contiguous() or mask.numel() != out.numel() or mask.is_floating_point():
+        raise ValueError("a contiguous integer mask and an output of its size")
+    with torch.cuda.device(mask.device):
+        st = load().kernl_select_mask_fwd(mask.data_ptr(), mask.element_size(), float(on), float(off), out.data_ptr(), mask.numel(),
+                                          DTYPE_CODE[out.dtype], _stream(mask))
+    _check(st, "kernl_select_mask_fwd")
 
 
 def add_rms_stats_fwd(a2d, b2d, sum2d, rstd, eps: float) -> None:

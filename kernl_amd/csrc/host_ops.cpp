@@ -565,6 +565,37 @@ PyObject *plan_few_rows(PyObject *const *a, Py_ssize_t n) {
     return Py_BuildValue("(NNNNOL)", x2d, res2d, y2d, y, stream_k ? Py_True : Py_False, (long long)per_batch);
 }
 
+// Copies src[i] into dst[i] (lists of tensors of equal shapes and dtypes), all in one launch; None where some pair needs torch's copy.
+PyObject *copy_many(PyObject *const *a, Py_ssize_t n) {
+    count(n, 2);
+    if (!PyList_Check(a[0]) || !PyList_Check(a[1])) Py_RETURN_NONE;
+    const Py_ssize_t pairs = PyList_GET_SIZE(a[0]);
+    if (pairs == 0 || pairs > 8 || PyList_GET_SIZE(a[1]) != pairs) Py_RETURN_NONE;
+    void *dst[8];
+    const void *src[8];
+    int64_t bytes[8];
+    const at::Tensor *first = nullptr;
+    for (Py_ssize_t i = 0; i < pairs; ++i) {
+        PyObject *d = PyList_GET_ITEM(a[0], i), *s = PyList_GET_ITEM(a[1], i);
+        if (!THPVariable_Check(d) || !THPVariable_Check(s)) Py_RETURN_NONE;
+        const at::Tensor &D = THPVariable_Unpack(d), &S = THPVariable_Unpack(s);
+        if (first == nullptr) first = &D;
+        if (!D.is_cuda() || D.device() != first->device() || S.device() != D.device() || S.scalar_type() != D.scalar_type() || S.sizes() != D.sizes() ||
+            !S.is_contiguous() || !D.is_contiguous() || !aligned16(S) || !aligned16(D) || S.is_conj() || S.is_neg())
+            Py_RETURN_NONE;
+        dst[i] = D.data_ptr();
+        src[i] = S.data_ptr();
+        bytes[i] = (int64_t)S.nbytes();
+    }
+    for (Py_ssize_t i = 0; i < pairs; ++i)  // one after the other where one's source is another's destination
+        for (Py_ssize_t j = 0; j < pairs; ++j) {
+            const char *s = static_cast<const char *>(src[i]), *d = static_cast<const char *>(dst[j]);
+            if (!(i == j && s == d) && s < d + bytes[j] && d < s + bytes[i]) Py_RETURN_NONE;
+        }
+    Py_DECREF(launched(*first, "kernl_copy_many", [&](void *stream) { return kernl_copy_many((int)pairs, src, dst, bytes, stream); }));
+    Py_RETURN_TRUE;
+}
+
 PyObject *set_error_type(PyObject *, PyObject *type) {
     Py_XINCREF(type);
     Py_XSETREF(g_error, type);
@@ -575,7 +606,7 @@ PyObject *set_error_type(PyObject *, PyObject *type) {
 PyMethodDef kMethods[] = {
     ENTRY(attention_fwd), ENTRY(attention_cached_fwd), ENTRY(attention_skinny_fwd), ENTRY(linear_fwd), ENTRY(linear_rms_fwd),
     ENTRY(linear_decode_fwd), ENTRY(linear_fewrow_fwd), ENTRY(layernorm_fwd), ENTRY(op_layer_norm), ENTRY(op_attention),
-    ENTRY(op_skinny_attention), ENTRY(op_linear), ENTRY(plan_few_rows),
+    ENTRY(op_skinny_attention), ENTRY(op_linear), ENTRY(plan_few_rows), ENTRY(copy_many),
     {"set_error_type", set_error_type, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -16,6 +16,7 @@ from typing import Callable, Iterable, List, Optional, Sequence, Union
 import torch
 from torch._subclasses import FakeTensor
 
+from kernl_amd import _lib
 from kernl_amd.optimizer.linear import refresh_fused_parameters
 from kernl_amd.optimizer.pool_cuda_graphs import CudaGraphPool, get_aligned_size
 
@@ -133,8 +134,10 @@ class _CapturedGraph:
         if self.dynamic_idx and self._same_layout(args):
             # the placement is a function of the input signature (see prepare_inputs): inputs of the captured shapes go
             # straight to the slots the graph reads
-            for i in self.dynamic_idx:
-                self.graph_inputs[i].copy_(args[i])
+            slots, values = [self.graph_inputs[i] for i in self.dynamic_idx], [args[i] for i in self.dynamic_idx]
+            if not _lib.host().copy_many(slots, values):  # one launch for all of them, where they are plain
+                for slot, value in zip(slots, values):
+                    slot.copy_(value)
         elif self.dynamic_idx:
             copies = prepare_inputs([args[i] for i in self.dynamic_idx], self.pools)
             for i, c in zip(self.dynamic_idx, copies):

@@ -14,6 +14,7 @@ from kernl_amd.optimizer.dropout import remove_dropout
 from kernl_amd.optimizer.kv_cache import drop_empty_cat_operands
 from kernl_amd.optimizer.layer_norm import (
     fuse_embeddings_into_layer_norm,
+    gather_ids_in_embeddings,
     replace_layer_norm,
     replace_layer_norm_fn,
     replace_layer_norm_rms,
@@ -31,6 +32,7 @@ from kernl_amd.optimizer.mask import (
     constant_causal_masks_to_flag,
     drop_all_true_conjuncts,
     full_range_index_to_view,
+    fuse_mask_selection,
     merge_nested_expands,
     scalar_tensors_to_full,
     sink_expand_below_where,
@@ -57,11 +59,13 @@ def dynamo_backend_ofi(gm: torch.fx.GraphModule, assume_causal=False):
     fuse_attention_sdpa(gm, assume_causal)
     constant_causal_masks_to_flag(gm)
     share_mask_conversion(gm)
+    fuse_mask_selection(gm)
     replace_all_linear(gm)
     replace_layer_norm(gm)
     replace_layer_norm_fn(gm)
     replace_layer_norm_rms(gm)
     fuse_embeddings_into_layer_norm(gm)
+    gather_ids_in_embeddings(gm)
     fuse_rms_norm_into_linears(gm)
     fuse_rotary_into_projections(gm)
     fuse_residual_into_linears(gm)

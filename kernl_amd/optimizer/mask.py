@@ -12,6 +12,8 @@ import operator
 import torch
 from torch.fx import Node
 
+from kernl_amd import _lib
+
 
 def _is_scalar(value) -> bool:
     if isinstance(value, (int, float)):
@@ -267,6 +269,84 @@ def constant_causal_masks_to_flag(gm: torch.fx.GraphModule):
         args[mask_idx] = None
         args[5] = True  # is_causal, same position in both wrappers
         node.args = tuple(args)
+        changed = True
+    if changed:
+        gm.graph.eliminate_dead_code()
+        gm.graph.lint()
+        gm.recompile()
+
+
+def select_mask(mask: torch.Tensor, on: float, off: float, dtype: torch.dtype) -> torch.Tensor:
+    """where(mask != 0, on, off) in `dtype`, in one launch."""
+    if mask.is_cuda and mask.dtype in (torch.bool, torch.uint8, torch.int8, torch.int32, torch.int64) and mask.is_contiguous():
+        out = torch.empty(mask.shape, dtype=dtype, device=mask.device)
+        _lib.select_mask_fwd(mask, on, off, out)
+        return out
+    on_off = torch.tensor([on, off], dtype=dtype, device=mask.device)
+    return torch.where(mask.to(torch.bool), on_off[0], on_off[1])
+
+
+torch.fx.wrap("select_mask")
+
+_SHAPE_METHODS = ("reshape", "view", "unsqueeze", "expand", "contiguous")
+
+
+def fuse_mask_selection(gm: torch.fx.GraphModule):
+    """`where(shape_ops(mask.to(bool)), a, b)` with numbers a and b — the additive mask of a padding mask, made by a conversion, a fill,
+    a scalar tensor and a selection — becomes `shape_ops(select_mask(mask, a, b))`, one launch; so does the boolean mask handed to
+    `additive_mask` (0 and -inf).  Only where the converted mask goes nowhere else.  No counterpart in the reference."""
+    from kernl_amd.optimizer.attention import additive_mask
+
+    def number(value):
+        """(number, dtype or None) of a Python number or a 0-d torch.full"""
+        if isinstance(value, (int, float)) and not isinstance(value, bool):
+            return float(value), None
+        if isinstance(value, Node) and value.op == "call_function" and value.target is torch.full and len(value.args) == 2 and value.args[0] == ():
+            if isinstance(value.args[1], (int, float)) and value.kwargs.get("dtype") in (torch.float16, torch.bfloat16, torch.float32):
+                return float(value.args[1]), value.kwargs["dtype"]
+        return None
+
+    def to_bool(node):
+        if not (isinstance(node, Node) and node.op == "call_method" and node.target == "to" and node.args):
+            return False
+        rest = list(node.args[1:]) + list(node.kwargs.values())
+        source = getattr(node.args[0], "meta", {}).get("example_value")
+        whole = source is not None and not source.is_floating_point() and not source.is_complex()
+        return whole and torch.bool in rest and set(node.kwargs) <= {"dtype", "device"}
+
+    def shape_only(node):
+        if node.op != "call_method":
+            return False
+        if node.target == "to":  # a move to the device it is on
+            return len(node.args) == 2 and isinstance(node.args[1], torch.device) and not node.kwargs
+        return node.target in _SHAPE_METHODS
+
+    changed = False
+    for start in list(gm.graph.nodes):
+        if not to_bool(start):
+            continue
+        end = start
+        while len(end.users) == 1 and shape_only(next(iter(end.users))) and next(iter(end.users)).args[0] is end:
+            end = next(iter(end.users))
+        if len(end.users) != 1:
+            continue
+        user = next(iter(end.users))
+        if user.op == "call_function" and user.target is torch.where and len(user.args) == 3 and user.args[0] is end and not user.kwargs:
+            on, off = number(user.args[1]), number(user.args[2])
+            if on is None or off is None or (on[1] is not None and off[1] is not None and on[1] != off[1]):
+                continue
+            dtype, final = on[1] or off[1] or torch.get_default_dtype(), user
+        elif user.op == "call_function" and user.target is additive_mask and len(user.args) == 1 and not user.kwargs:
+            on, off, dtype, final = (0.0, None), (float("-inf"), None), torch.get_default_dtype(), None
+        else:
+            continue
+        with gm.graph.inserting_before(start):
+            selected = gm.graph.call_function(select_mask, (start.args[0], on[0], off[0], dtype))
+        start.replace_all_uses_with(selected)
+        gm.graph.erase_node(start)
+        if final is not None:  # (`additive_mask` passes masks that are additive already through)
+            final.replace_all_uses_with(selected if end is start else end)
+            gm.graph.erase_node(final)
         changed = True
     if changed:
         gm.graph.eliminate_dead_code()

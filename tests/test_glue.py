@@ -1,0 +1,84 @@
+"""What surrounds the kernels of a captured encoder (csrc/glue.hip): the copies of its inputs, its mask and its token types."""
+import pytest
+import torch
+
+from kernl_amd import _lib
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[1], [15, 16, 17], [16384, 16383, 16385, 3], [40000, 1, 0, 4096, 5, 6, 7, 70001]], ids=str)
+def test_copies_of_all_inputs_in_one_launch(sizes):
+    src = [torch.randint(0, 255, (n,), dtype=torch.uint8, device="cuda") for n in sizes]
+    dst = [torch.zeros(n + 16, dtype=torch.uint8, device="cuda")[:n] for n in sizes]
+    assert _lib.host().copy_many(dst, src) is True
+    for d, s, n in zip(dst, src, sizes):
+        assert torch.equal(d, s)
+        assert not d.as_strided((16,), (1,), n).any()
+
+
+@pytest.mark.gpu
+def test_inputs_that_need_more_than_a_plain_copy_are_left_to_torch():
+    x = torch.arange(64, device="cuda")
+    for dst, src in (([x.clone()], [x.int()]), ([x.clone()], [x.cpu()]), ([x.clone()[:32]], [x[::2]]), ([x[:32], x[32:]], [x[32:], x[:32]]),
+                     ([x.clone()[1:]], [x[1:]]), ([torch.empty_like(x)] * 9, [x] * 9)):
+        before = [d.clone() for d in dst]
+        assert _lib.host().copy_many(dst, src) is None
+        assert all(torch.equal(d, b) for d, b in zip(dst, before))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=str)
+@pytest.mark.parametrize("mask_dtype", [torch.bool, torch.uint8, torch.int32, torch.int64], ids=str)
+@pytest.mark.parametrize("shape", [(1, 1), (3, 85), (2, 128), (0, 4), (7, 513)], ids=str)
+def test_mask_selection(shape, mask_dtype, dtype):
+    from kernl_amd.optimizer.mask import select_mask
+
+    mask = torch.randint(0, 2, shape).to(mask_dtype)
+    if mask_dtype == torch.int64:
+        mask = mask << 32  # no look at the low half only
+    for off in (float("-inf"), torch.finfo(dtype).min):
+        out = select_mask(mask.cuda(), 0.0, off, dtype)
+        want = torch.where(mask.bool(), torch.zeros((), dtype=dtype), torch.full((), off, dtype=dtype))
+        assert out.dtype == dtype and torch.equal(out.cpu(), want)
+        assert torch.equal(select_mask(mask, 0.0, off, dtype), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slot", [0, 1, 2])
+def test_embedding_ids_through_a_vector(slot):
+    from kernl_amd.implementations.layer_norm import embedding_layer_norm
+
+    gen = torch.Generator().manual_seed(slot)
+    tables = [torch.randn(r, 96, generator=gen).half().cuda() for r in (50, 3, 70)]
+    ids = [torch.randint(0, t.shape[0], (2, 19), generator=gen).cuda() for t in tables]
+    vector = torch.randint(0, tables[slot].shape[0], (64,), generator=gen).cuda()
+    w = torch.randn(96, generator=gen).half().cuda()
+    index = torch.randint(0, 64, (1, 19), generator=gen).cuda()
+    through = list(ids)
+    ids[slot], through[slot] = vector[index].expand(2, 19), index
+    assert torch.equal(embedding_layer_norm(tables, through, w, None, 1e-5, via=(slot, vector)), embedding_layer_norm(tables, ids, w, None, 1e-5))
+
+
+def test_mask_selection_pass_leaves_other_readers_alone():
+    from kernl_amd.optimizer.mask import fuse_mask_selection, select_mask
+
+    class Model(torch.nn.Module):
+        def __init__(self, shared):
+            super().__init__()
+            self.shared = shared
+
+        def forward(self, mask):
+            keep = mask.to(torch.bool)
+            additive = torch.where(keep.reshape(2, 1, 1, 5), 0.0, -65504.0)
+            return (additive, keep) if self.shared else additive
+
+    mask = torch.tensor([[1, 1, 0, 1, 0], [0, 1, 1, 1, 3]])
+    for shared in (False, True):
+        model = Model(shared)
+        gm = torch.fx.symbolic_trace(model)
+        next(n for n in gm.graph.nodes if n.op == "placeholder").meta["example_value"] = mask
+        fuse_mask_selection(gm)
+        assert any(n.target is select_mask for n in gm.graph.nodes) == (not shared)
+        got, want = gm(mask), model(mask)
+        for g, w in zip((got if shared else (got,)), (want if shared else (want,))):
+            assert g.dtype == w.dtype and torch.equal(g, w)
