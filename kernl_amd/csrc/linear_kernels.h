@@ -14,6 +14,7 @@
 // "B" side, i.e. the instruction produces a 32(n) x 32(m) block of outᵀ; together with the row permutation
 // rowperm16 on the weight tile this leaves every lane holding 16 consecutive output columns of one output
 // row, so bias loads and output stores are 16-byte vectors without any shuffle through LDS.
+#include <algorithm>
 #include <type_traits>
 
 #include "activations.h"
@@ -1346,7 +1347,22 @@ struct SkinnyExtra {
     int rows_per_batch;     // row m of x is position m % rows_per_batch of batch entry m / rows_per_batch
 };
 
-template <typename T, int MB, bool GATED, int WAVES, int NR, bool W8 = false, bool RMS = false, bool ROPE = false>
+// XL (with RMS): x times the norm's weight is made once per workgroup and kept in LDS (dynamic, M rows
+// `skinny_staged_stride` bytes apart).  The kernel is bound by the weight stream; x and the norm's weight, fetched chunk by
+// chunk, put four more loads and some 40 vector instructions of a wave between two batches of weights and leave it the
+// registers for half as large a batch (gated pairs keep the smaller one: 33.2 us against 34.5 below).  Here x is requested
+// first, the first batch of weights behind it, and staging runs while those arrive.  One row, K = 4096, weights from HBM, fp16: 12288 columns 23.2 -> 20.2 us (5.0 TB/s),
+// 32000 columns 51.1 -> 46.2 (5.7), 11008 gated pairs 35.1 -> 33.2 (5.4), 12288 rotated 23.7 -> 22.7.
+// x rows in LDS lie 144 bytes further apart than they are long, so that neighbouring rows start in other banks.
+__host__ __device__ constexpr int skinny_staged_stride(int K) { return 2 * K + 144; }
+// Every workgroup stages all of x, which costs about 0.7 us a row of 4096: one row gains (also 5632 x 2048 gated
+// 13.9 -> 12.5 us, 5120 x 4096 plain 15.2 -> 13.7), three rows still where a workgroup has one block of columns
+// (12288 x 4096 plain 23.4 -> 21.8; twelve rows of 1024 6.2 -> 7.1), but not where it has two and streams twice as long
+// anyway (three rows, 8192 x 4096 gated 26.5 -> 28.0, rotated 16.9 -> 17.8).
+constexpr int kSkinnyStagedElements = 12288;  // 24 KB of x, with three workgroups on a CU
+
+template <typename T, int MB, bool GATED, int WAVES, int NR, bool W8 = false, bool RMS = false, bool ROPE = false,
+          bool XL = false>
 __global__ void __launch_bounds__(64 * WAVES)
 linear_skinny_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
                      T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs, int64_t out_cs,
@@ -1355,10 +1371,14 @@ linear_skinny_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *
     typedef typename Vec8<T>::type vec8;
     constexpr int NA = GATED ? 2 : 1;        // weight fragments per 16 output columns: plain, or gate and value
     constexpr int NF = NA * NR;              // weight fragments per step (NR blocks of 16 output columns)
-    constexpr int U = (MB <= 2 && NF <= 2 && !RMS) ? 4 : 2;  // chunks requested together
+    static_assert(!XL || (RMS && MB == 1 && !W8), "the staged form is the normalising one with at most 16 rows of x");
+    constexpr int U = (MB <= 2 && NF <= 2 && (!RMS || (XL && !GATED))) ? 4 : 2;  // chunks requested together
     static_assert(WAVES * NF * MB <= 64, "partial sums fit 64 KB of LDS");
-    __shared__ __attribute__((aligned(16))) float red[WAVES][NF * MB][64][4];
+    __shared__ __attribute__((aligned(16))) float red_own[XL ? 1 : WAVES][NF * MB][64][4];
     __shared__ float red_sq[RMS ? WAVES : 1][MB][16];
+    extern __shared__ __attribute__((aligned(16))) unsigned char staged_x[];
+    // the partial sums take the place of the staged x when every wave is done with it
+    float(*red)[NF * MB][64][4] = XL ? reinterpret_cast<float(*)[NF * MB][64][4]>(staged_x) : red_own;
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int r = lane & 15, g = lane >> 4;
@@ -1418,8 +1438,8 @@ linear_skinny_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *
     }
     const int nchunks = K / 64;
     const int rot = (int)((blockIdx.x * 13u) % (unsigned)nchunks);
-    for (int c0 = wave; c0 < nchunks; c0 += WAVES * U) {
-        vec8 wf[U][NF][2], xf[U][MB][2], gf[RMS ? U : 1][2];
+    vec8 wf[U][NF][2], xf[U][MB][2], gf[RMS ? U : 1][2];
+    auto request = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             // chunks past the end are neither fetched nor multiplied (the test is uniform over the wave); only the
@@ -1450,20 +1470,29 @@ linear_skinny_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *
                     wf[u][f][1] = *reinterpret_cast<const vec8 *>(wp[f] + k0 + 8);
                 }
             }
+            if constexpr (XL) continue;
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) {
                 xf[u][mb][0] = *reinterpret_cast<const vec8 *>(xp[mb] + k0);
                 xf[u][mb][1] = *reinterpret_cast<const vec8 *>(xp[mb] + k0 + 8);
             }
-            if constexpr (RMS) {
+            if constexpr (RMS && !XL) {
                 gf[u][0] = *reinterpret_cast<const vec8 *>(rms_w + k0 + 16 * g);
                 gf[u][1] = *reinterpret_cast<const vec8 *>(rms_w + k0 + 16 * g + 8);
             }
         }
+    };
+    auto multiply = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (c0 + WAVES * u < nchunks) {
-                if constexpr (RMS) {
+                if constexpr (XL) {
+                    int cc = c0 + WAVES * u + rot;
+                    cc = cc >= nchunks ? cc - nchunks : cc;
+                    const vec8 *src = reinterpret_cast<const vec8 *>(staged_x + min(r, M - 1) * skinny_staged_stride(K) + (cc * 64 + 16 * g) * 2);
+                    xf[u][0][0] = src[0];
+                    xf[u][0][1] = src[1];
+                } else if constexpr (RMS) {
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -1485,15 +1514,64 @@ linear_skinny_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *
                     }
             }
         }
+    };
+    int c0 = wave;
+    if constexpr (XL) {
+        // 16-byte pieces of x, two at a time per thread; a wave's 64 pieces belong to one row (K is a multiple of 512)
+        constexpr int THREADS = 64 * WAVES;
+        const int ppr = K / 8, pieces = M * ppr;
+        if (lane < 16) red_sq[wave][0][lane] = 0.0f;
+        vec8 px[2], pg[2];
+        auto fetch = [&](int q0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int q = min(q0 + THREADS * i, pieces - 1), row = q / ppr, p = q - row * ppr;
+                px[i] = *reinterpret_cast<const vec8 *>(X + (int64_t)row * ldx + p * 8);
+                pg[i] = *reinterpret_cast<const vec8 *>(rms_w + p * 8);
+            }
+        };
+        auto stage = [&](int q0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int q = q0 + THREADS * i;
+                if (__builtin_amdgcn_readfirstlane(q) >= pieces) continue;  // pieces is a multiple of 64: whole waves
+                const int row = q / ppr, p = q - row * ppr;
+                float t = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float xv = to_float(px[i][e]);
+                    t = fmaf(xv, xv, t);
+                }
+#pragma unroll
+                for (int off = 1; off < 64; off <<= 1) t += __shfl_xor(t, off, 64);
+                if (lane == 0) red_sq[wave][0][row] += t;
+                *reinterpret_cast<vec8 *>(staged_x + row * skinny_staged_stride(K) + p * 16) = px[i] * pg[i];
+            }
+        };
+        fetch((int)threadIdx.x);
+        request(c0);
+        stage((int)threadIdx.x);
+        for (int q0 = (int)threadIdx.x + 2 * THREADS; q0 - (int)threadIdx.x < pieces; q0 += 2 * THREADS) {
+            fetch(q0);
+            stage(q0);
+        }
+        __syncthreads();
+        multiply(c0);
+        c0 += WAVES * U;
+    }
+    for (; c0 < nchunks; c0 += WAVES * U) {
+        request(c0);
+        multiply(c0);
     }
 
+    if constexpr (XL) __syncthreads();
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int e = 0; e < 4; ++e) red[wave][f * MB + mb][lane][e] = acc[f][mb][e];
-    if constexpr (RMS) {
+    if constexpr (RMS && !XL) {
         // a row's squares are spread over the 4 lanes r, r + 16, r + 32, r + 48 of every wave
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
@@ -2054,7 +2132,7 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
 
 extern int g_linear_force_tile;  // test / tuning hook (defined in linear.hip): 0 = heuristic, 1 = 256x256, 2 = 256x192, 3 = 128x128, 4 = 256x128 k32, 5 = wide 256x256, 6 = wide 256x192, 7 = wide 128x256, 8 = wide 128x192, 10 = 32 x 64, 12 .. 14 and 16 = dealt k-tiles, 11, 15, 17 .. 21 = the 8-wave tiles of linear_mid.hip
 
-template <typename T, bool GATED, int MB, int NR, bool W8, bool RMS = false, bool ROPE = false>
+template <typename T, bool GATED, int MB, int NR, bool W8, bool RMS = false, bool ROPE = false, bool XL = false>
 static void launch_skinny_blocks(const LinearArgs &a, const void *rms_w = nullptr, float eps = 0.0f,
                                  const SkinnyExtra *extra = nullptr) {
     const int n_out = GATED ? a.N / 2 : a.N;
@@ -2067,7 +2145,7 @@ static void launch_skinny_blocks(const LinearArgs &a, const void *rms_w = nullpt
     // there are chunks, and no more than the LDS for their partial sums allows
     const int nchunks = a.K / 64;
     // (the normalising form also keeps a few more loads per chunk in flight: half the waves for it)
-    constexpr int kUnits = (GATED ? 2 : 1) * NR * MB * (RMS ? 2 : 1);
+    constexpr int kUnits = (GATED ? 2 : 1) * NR * MB * (RMS && !XL ? 2 : 1);
     constexpr int kMaxWaves = kUnits > 8 ? 4 : kUnits > 4 ? 8 : 16;
     // ... and few enough that the workgroups one CU gets (256 CUs) are resident together: a 1024-thread workgroup
     // fills half a CU, and 344 of them would leave a third of the chip idle
@@ -2075,8 +2153,14 @@ static void launch_skinny_blocks(const LinearArgs &a, const void *rms_w = nullpt
     int waves = nchunks >= 64 ? 16 : nchunks >= 24 ? 8 : 4;
     if (per_cu >= 3) waves = 4;
     else if (per_cu == 2 && waves > 8) waves = 8;
+    // Staged x and two column blocks (several workgroups a CU, below): the weights in flight are enough with 4 waves each, and
+    // more only lengthen the merge (one row, 12288 x 4096 rotated: 22.0 us with 4 waves, 23.3 with 8, 26.9 with 16;
+    // 8192 x 4096 gated: 25.5 with 4, 26.0 with 8).
+    if (XL && (GATED || ROPE)) waves = 4;
+    const int sums = waves * (GATED ? 2 : 1) * NR * MB * 1024;  // partial sums, 1 KB per wave and block
+    const unsigned lds = XL ? (unsigned)std::max(a.M * skinny_staged_stride(a.K), sums) : 0;
 #define KERNL_SKINNY(WV)                                                                                                \
-    hipLaunchKernelGGL((linear_skinny_kernel<T, MB, GATED, WV, NR, W8, RMS, ROPE>), grid, dim3(64 * WV), 0, a.st,                \
+    hipLaunchKernelGGL((linear_skinny_kernel<T, MB, GATED, WV, NR, W8, RMS, ROPE, XL>), grid, dim3(64 * WV), lds, a.st,          \
                        static_cast<const T *>(a.x), static_cast<const T *>(a.w), static_cast<const T *>(a.bias),       \
                        static_cast<T *>(a.out), static_cast<T *>(a.act_in), a.M, n_out, a.K, a.x_rs, a.out_rs, a.out_cs, \
                        a.ai_rs, a.ai_cs, act, static_cast<const T *>(rms_w), eps, ex)
@@ -2136,11 +2220,21 @@ static void launch_skinny(const LinearArgs &a) {
     else { if (two) launch_skinny_blocks<T, GATED, 4, 2, W8>(a); else launch_skinny_blocks<T, GATED, 4, 1, W8>(a); }
 }
 
+// Whether the normalising form keeps x in LDS: whole waves of 16-byte pieces per row (K % 512) and few rows.
+// paired_blocks: workgroups of a grid whose workgroups take two column blocks (gated, rotated), 0 for one block.  Those gain
+// with one row, and only where a CU has a second workgroup that streams while this one stages: with 256 workgroups the
+// barrier is waited for (8192 x 4096 rotated 16.8 -> 17.4 us, 4096 x 2048 gated 9.6 -> 10.1; with 384 23.8 -> 22.6).
+static bool skinny_stages_x(const LinearArgs &a, int paired_blocks) {
+    if (paired_blocks > 0 && (a.M > 1 || paired_blocks <= 256)) return false;
+    return a.M <= 3 && a.K % 512 == 0 && a.M * (int64_t)a.K <= kSkinnyStagedElements;
+}
+
 // RMS-normalised input: 16 output columns per workgroup, 16-bit weights
 template <typename T, bool GATED>
 static void launch_skinny_rms(const LinearArgs &a, const void *rms_w, float eps) {
     const int mb = (a.M + 15) / 16;
-    if (mb <= 1) launch_skinny_blocks<T, GATED, 1, 1, false, true>(a, rms_w, eps);
+    if (skinny_stages_x(a, GATED ? a.N / 32 : 0)) launch_skinny_blocks<T, GATED, 1, 1, false, true, false, true>(a, rms_w, eps);
+    else if (mb <= 1) launch_skinny_blocks<T, GATED, 1, 1, false, true>(a, rms_w, eps);
     else if (mb <= 2) launch_skinny_blocks<T, GATED, 2, 1, false, true>(a, rms_w, eps);
     else launch_skinny_blocks<T, GATED, 4, 1, false, true>(a, rms_w, eps);
 }
@@ -2150,11 +2244,13 @@ template <typename T>
 static void launch_skinny_decode(const LinearArgs &a, const void *rms_w, float eps, const SkinnyExtra &ex) {
     const int mb = (a.M + 15) / 16;
     if (ex.half > 0) {  // rotating form: two column blocks per workgroup, always with the normalising prologue
-        if (mb <= 1) launch_skinny_blocks<T, false, 1, 2, false, true, true>(a, rms_w, eps, &ex);
+        if (skinny_stages_x(a, (a.N + 31) / 32)) launch_skinny_blocks<T, false, 1, 2, false, true, true, true>(a, rms_w, eps, &ex);
+        else if (mb <= 1) launch_skinny_blocks<T, false, 1, 2, false, true, true>(a, rms_w, eps, &ex);
         else if (mb <= 2) launch_skinny_blocks<T, false, 2, 2, false, true, true>(a, rms_w, eps, &ex);
         else launch_skinny_blocks<T, false, 4, 2, false, true, true>(a, rms_w, eps, &ex);
     } else if (rms_w != nullptr) {
-        if (mb <= 1) launch_skinny_blocks<T, false, 1, 1, false, true>(a, rms_w, eps, &ex);
+        if (skinny_stages_x(a, 0)) launch_skinny_blocks<T, false, 1, 1, false, true, false, true>(a, rms_w, eps, &ex);
+        else if (mb <= 1) launch_skinny_blocks<T, false, 1, 1, false, true>(a, rms_w, eps, &ex);
         else if (mb <= 2) launch_skinny_blocks<T, false, 2, 1, false, true>(a, rms_w, eps, &ex);
         else launch_skinny_blocks<T, false, 4, 1, false, true>(a, rms_w, eps, &ex);
     } else {

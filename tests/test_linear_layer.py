@@ -516,6 +516,43 @@ def test_rms_norm_fused_into_the_linear_layer(shape, kind, dtype, close):
     close(out, ref, dtype, what=f"rms + linear {shape} {kind}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("kind", ["plain", "gated", "rotated"])
+# x kept in LDS (one row, plain products up to three): fewer pieces than threads, the largest x in one row and in three, several
+# staging rounds, one to three workgroups a CU; and just beyond
+@pytest.mark.parametrize("shape", [(1, 64, 512), (1, 64, 12288), (1, 4096, 1024), (1, 4160, 1024), (1, 9216, 1536), (1, 12352, 512), (1, 8256, 12288), (2, 9216, 1536), (3, 128, 4096),
+                                   (3, 12352, 512), (4, 64, 1024), (1, 64, 12800), (1, 64, 576)], ids=str)
+def test_rms_linear_with_staged_rows(shape, kind, dtype, close):
+    """Decoding-step products whose normalised rows are kept in LDS, at the edges of that form: rows far apart in scale (each
+    needs its own sum of squares), x with a row stride of its own."""
+    from kernl_amd.implementations.linear_layer import decode_linear_layer, interleave_glu_rows, rms_linear_layer
+    from oracle import glu_oracle, rms_norm_oracle, rotary_oracle
+
+    M, N, K = shape
+    gen = torch.Generator().manual_seed(M * K)
+    x = torch.randn((M, K), generator=gen) * torch.logspace(-1, 1, M)[:, None]
+    x = x.to(dtype)
+    xd = torch.full((M, K + 24), float("nan"), dtype=dtype, device="cuda")[:, :K]
+    xd.copy_(x)
+    g = (1.0 + 0.2 * torch.randn((K,), generator=gen)).to(dtype)
+    w, w2 = ((torch.randn((N, K), generator=gen) * K ** -0.5).to(dtype) for _ in range(2))
+    normed = rms_norm_oracle(x, g, 1.6e-5)
+    if kind == "gated":
+        out = rms_linear_layer(xd, g.cuda(), 1.6e-5, interleave_glu_rows(w, w2).cuda(), None, "silu", gated=True)
+        ref = glu_oracle(normed, w, None, w2, None, "silu")
+    elif kind == "plain":
+        out = rms_linear_layer(xd, g.cuda(), 1.6e-5, w.cuda(), None, "")
+        ref = linear_oracle(normed, w, None, "")
+    else:
+        angles = torch.rand((1, M, 64), generator=gen) * 6.28
+        out = decode_linear_layer(xd, w.cuda(), None, g.cuda(), 1.6e-5, None, angles.cos().cuda(), angles.sin().cuda(), head_dim=64, rope_cols=64)
+        heads = linear_oracle(normed, w, None, "").reshape(1, M, N // 64, 64)
+        turned = rotary_oracle(heads[:, :, :1], angles.cos()[:, :, None, :], angles.sin()[:, :, None, :])
+        ref = torch.cat((turned, heads[:, :, 1:]), dim=2).reshape(M, N)
+    torch.cuda.synchronize()
+    close(out, ref, dtype, scale="magnitude", what=f"staged rows {shape} {kind}")
+
+
 def test_linear_few_rows_strided_output_and_batched_input(close):
     gen = torch.Generator().manual_seed(18)
     x, w, b = _inputs(2, 640, 256, torch.float16, gen, w_std=1 / 16, batch=3)  # [3, 2, 256] -> 6 rows
