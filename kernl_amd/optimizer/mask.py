@@ -298,9 +298,10 @@ def fuse_mask_selection(gm: torch.fx.GraphModule):
     from kernl_amd.optimizer.attention import additive_mask
 
     def number(value):
-        """(number, dtype or None) of a Python number or a 0-d torch.full"""
-        if isinstance(value, (int, float)) and not isinstance(value, bool):
-            return float(value), None
+        """(number, dtype or None) of a Python float or a 0-d torch.full of floating type.  (An integer is no mask value: a
+        selection between integers has an integer type, which is counted and indexed with.)"""
+        if isinstance(value, float):
+            return value, None
         if isinstance(value, Node) and value.op == "call_function" and value.target is torch.full and len(value.args) == 2 and value.args[0] == ():
             if isinstance(value.args[1], (int, float)) and value.kwargs.get("dtype") in (torch.float16, torch.bfloat16, torch.float32):
                 return float(value.args[1]), value.kwargs["dtype"]

@@ -82,3 +82,27 @@ def test_mask_selection_pass_leaves_other_readers_alone():
         got, want = gm(mask), model(mask)
         for g, w in zip((got if shared else (got,)), (want if shared else (want,))):
             assert g.dtype == w.dtype and torch.equal(g, w)
+
+
+def _fused_selection(forward, mask):
+    """The graph of `forward` after the pass, and whether the pass took the selection."""
+    from kernl_amd.optimizer.mask import fuse_mask_selection, select_mask
+
+    class Model(torch.nn.Module):
+        def forward(self, mask):
+            return forward(mask)
+
+    gm = torch.fx.symbolic_trace(Model())
+    next(n for n in gm.graph.nodes if n.op == "placeholder").meta["example_value"] = mask
+    fuse_mask_selection(gm)
+    return gm, any(n.target is select_mask for n in gm.graph.nodes)
+
+
+@pytest.mark.parametrize("on, off, fused", [(0.0, -65504.0, True), (1, 0, False), (16777217, 0, False), (0, -65504.0, False),
+                                            (True, False, False)], ids=str)
+def test_only_selections_between_floats_are_fused(on, off, fused):
+    """A selection between integers keeps its integer type (positions are counted with such masks) and all their bits."""
+    mask = torch.tensor([[1, 1, 0, 1, 0], [0, 1, 1, 1, 3]])
+    gm, taken = _fused_selection(lambda m: torch.where(m.to(torch.bool), on, off), mask)
+    want = torch.where(mask.to(torch.bool), on, off)
+    assert taken == fused and gm(mask).dtype == want.dtype and torch.equal(gm(mask), want)
