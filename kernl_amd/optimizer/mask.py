@@ -308,12 +308,16 @@ def fuse_mask_selection(gm: torch.fx.GraphModule):
         return None
 
     def to_bool(node):
+        """x.to(torch.bool) of an integer x that stays on its device and asks for nothing else"""
         if not (isinstance(node, Node) and node.op == "call_method" and node.target == "to" and node.args):
             return False
-        rest = list(node.args[1:]) + list(node.kwargs.values())
         source = getattr(node.args[0], "meta", {}).get("example_value")
-        whole = source is not None and not source.is_floating_point() and not source.is_complex()
-        return whole and torch.bool in rest and set(node.kwargs) <= {"dtype", "device"}
+        if source is None or source.is_floating_point() or source.is_complex():
+            return False
+        rest = [v for v in node.args[1:] + tuple(node.kwargs.values()) if v is not torch.bool]
+        if len(rest) != len(node.args) - 2 + len(node.kwargs) or not set(node.kwargs) <= {"dtype", "device"}:
+            return False
+        return not rest or (len(rest) == 1 and isinstance(rest[0], (str, torch.device)) and torch.device(rest[0]) == source.device)
 
     def shape_only(node):
         if node.op != "call_method":

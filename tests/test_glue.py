@@ -106,3 +106,22 @@ def test_only_selections_between_floats_are_fused(on, off, fused):
     gm, taken = _fused_selection(lambda m: torch.where(m.to(torch.bool), on, off), mask)
     want = torch.where(mask.to(torch.bool), on, off)
     assert taken == fused and gm(mask).dtype == want.dtype and torch.equal(gm(mask), want)
+
+
+@pytest.mark.parametrize("convert, fused", [
+    (lambda m: m.to(torch.bool), True),
+    (lambda m: m.to(dtype=torch.bool), True),
+    (lambda m: m.to(device=torch.device("cpu"), dtype=torch.bool), True),
+    (lambda m: m.to("cpu", torch.bool), True),
+    (lambda m: m.to(device=torch.device("meta"), dtype=torch.bool), False),
+    (lambda m: m.to("meta", torch.bool), False),
+    (lambda m: m.to(torch.bool, False), False),
+    (lambda m: m.to(torch.bool, copy=True), False),
+], ids=str)
+def test_conversions_that_move_the_mask_are_left_alone(convert, fused):
+    mask = torch.tensor([[1, 1, 0, 1, 0], [0, 1, 1, 1, 3]])
+    gm, taken = _fused_selection(lambda m: torch.where(convert(m).reshape(2, 1, 1, 5), 0.0, -65504.0), mask)
+    want = torch.where(convert(mask).reshape(2, 1, 1, 5), 0.0, -65504.0)
+    got = gm(mask)
+    assert taken == fused and got.device == want.device and got.dtype == want.dtype and got.shape == want.shape
+    assert want.is_meta or torch.equal(got, want)
