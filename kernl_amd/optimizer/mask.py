@@ -277,13 +277,15 @@ def constant_causal_masks_to_flag(gm: torch.fx.GraphModule):
 
 
 def select_mask(mask: torch.Tensor, on: float, off: float, dtype: torch.dtype) -> torch.Tensor:
-    """where(mask != 0, on, off) in `dtype`, in one launch."""
-    if mask.is_cuda and mask.dtype in (torch.bool, torch.uint8, torch.int8, torch.int32, torch.int64) and mask.is_contiguous():
-        out = torch.empty(mask.shape, dtype=dtype, device=mask.device)
-        _lib.select_mask_fwd(mask, on, off, out)
-        return out
-    on_off = torch.tensor([on, off], dtype=dtype, device=mask.device)
-    return torch.where(mask.to(torch.bool), on_off[0], on_off[1])
+    """where(mask != 0, on, off) in `dtype`: one launch, two for a mask sliced out of a longer one.  Nothing here copies from
+    the host (stream capture refuses that), and the result has the layout the selection by `mask.to(torch.bool)` has."""
+    if mask.is_cuda and mask.dtype in (torch.bool, torch.uint8, torch.int8, torch.int32, torch.int64) and dtype in _lib.DTYPE_CODE:
+        dense = mask if mask.is_contiguous() else mask.clone()
+        if dense.is_contiguous():
+            out = torch.empty(mask.shape, dtype=dtype, device=mask.device)
+            _lib.select_mask_fwd(dense, on, off, out)
+            return out
+    return torch.where(mask.to(torch.bool), *(torch.full((), value, dtype=dtype, device=mask.device) for value in (on, off)))
 
 
 torch.fx.wrap("select_mask")
@@ -324,7 +326,8 @@ def fuse_mask_selection(gm: torch.fx.GraphModule):
             return False
         if node.target == "to":  # a move to the device it is on
             return len(node.args) == 2 and isinstance(node.args[1], torch.device) and not node.kwargs
-        return node.target in _SHAPE_METHODS
+        # (a view as another type looks at the bits of the bool)
+        return node.target in _SHAPE_METHODS and not any(isinstance(v, torch.dtype) for v in node.args + tuple(node.kwargs.values()))
 
     changed = False
     for start in list(gm.graph.nodes):
@@ -344,6 +347,8 @@ def fuse_mask_selection(gm: torch.fx.GraphModule):
         elif user.op == "call_function" and user.target is additive_mask and len(user.args) == 1 and not user.kwargs:
             on, off, dtype, final = (0.0, None), (float("-inf"), None), torch.get_default_dtype(), None
         else:
+            continue
+        if dtype not in _lib.DTYPE_CODE:  # (a default type of 64 bits)
             continue
         with gm.graph.inserting_before(start):
             selected = gm.graph.call_function(select_mask, (start.args[0], on[0], off[0], dtype))

@@ -125,3 +125,75 @@ def test_conversions_that_move_the_mask_are_left_alone(convert, fused):
     got = gm(mask)
     assert taken == fused and got.device == want.device and got.dtype == want.dtype and got.shape == want.shape
     assert want.is_meta or torch.equal(got, want)
+
+
+# masks that are not contiguous: sliced out of a longer one, columns and rows; every other column; transposed
+LAYOUTS = {"columns": lambda m: m[:, :7], "rows": lambda m: m[1:3, 2:], "steps": lambda m: m[:, ::2], "transposed": lambda m: m.t(),
+           "expanded": lambda m: m[:, :1].expand(4, 5), "four": lambda m: m[:, None, None, :5]}
+
+
+def _check_selection_of_a_layout(layout, device, dtype):
+    from kernl_amd.optimizer.mask import select_mask
+
+    mask = LAYOUTS[layout](torch.tensor([[1, 0, 3, 0, 1, 1, 0, 1 << 33, 0]] * 3 + [[0] * 9], device=device))
+    assert not mask.is_contiguous()
+    want = torch.where(mask.to(torch.bool), *(torch.full((), v, dtype=dtype, device=device) for v in (0.0, -1e4)))
+    got = select_mask(mask, 0.0, -1e4, dtype)
+    assert got.dtype == dtype and torch.equal(got, want) and got.stride() == want.stride()
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_selection_of_masks_that_are_not_contiguous(layout, monkeypatch):
+    def host_tensor(*args, **kwargs):
+        raise AssertionError("a copy from the host, which stream capture refuses")
+
+    with monkeypatch.context() as patch:
+        patch.setattr("kernl_amd.optimizer.mask.torch.tensor", host_tensor)
+        from kernl_amd.optimizer.mask import select_mask
+
+        select_mask(torch.ones(4, 9, dtype=torch.long)[:, :7], 0.0, -1.0, torch.float16)
+    for dtype in (torch.float16, torch.float32, torch.float64):
+        _check_selection_of_a_layout(layout, "cpu", dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32, torch.float64], ids=str)
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_selection_of_masks_that_are_not_contiguous_on_the_gpu(layout, dtype):
+    _check_selection_of_a_layout(layout, "cuda", dtype)
+
+
+def test_selections_outside_the_kernels_types_are_left_alone():
+    mask = torch.tensor([[1, 0, 1]])
+    before = torch.get_default_dtype()
+    torch.set_default_dtype(torch.float64)
+    try:
+        gm, taken = _fused_selection(lambda m: torch.where(m.to(torch.bool), 0.0, -1e300), mask)
+        assert not taken and torch.equal(gm(mask), torch.tensor([[0.0, -1e300, 0.0]]))
+    finally:
+        torch.set_default_dtype(before)
+    gm, taken = _fused_selection(lambda m: torch.where(m.to(torch.bool).view(torch.int8) == 1, 0.0, -1.0), mask)
+    assert not taken and torch.equal(gm(mask), torch.tensor([[0.0, -1.0, 0.0]]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch, seq", [(1, 33), (3, 77)], ids=str)
+def test_encoder_with_a_mask_sliced_out_of_a_longer_one(batch, seq):
+    """What a loop over batches of a tokenizer with a fixed length hands over; captured, so nothing may synchronise."""
+    from transformers import BertConfig, BertModel
+
+    from kernl_amd.model_optimization import optimize_model
+
+    torch._dynamo.reset()
+    cfg = BertConfig(num_hidden_layers=1)
+    cfg._attn_implementation = "eager"
+    torch.manual_seed(0)
+    model = BertModel(cfg).eval().half().cuda()
+    ids = torch.randint(0, 30522, (batch, 128), device="cuda")
+    full = (torch.arange(128, device="cuda")[None, :] < torch.randint(seq // 2, seq + 1, (batch, 1), device="cuda")).long()
+    with torch.inference_mode():
+        optimize_model(model)
+        want = model(input_ids=ids[:, :seq].contiguous(), attention_mask=full[:, :seq].contiguous()).last_hidden_state.clone()
+        for _ in range(2):
+            got = model(input_ids=ids[:, :seq], attention_mask=full[:, :seq]).last_hidden_state
+            assert torch.equal(got, want)
