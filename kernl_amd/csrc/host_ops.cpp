@@ -6,8 +6,8 @@
 //
 // Two kinds of functions:
 //   *_fwd        what kernl_amd/_lib.py exposes under the same name: tensors in, one launch, no checks beyond the ABI's;
-//   op_*, plan_* the whole operator for plain inputs (strided GPU tensors of one device, no autocast, nothing that autograd
-//                records).  Everything else — and every error — is answered with None: the caller then takes the Python
+//   op_*, plan_* the whole operator for plain inputs (strided GPU tensors of one device, no autocast, nothing that autograd,
+//                a tracer or a transform records).  Everything else — and every error — is answered with None: the caller then takes the Python
 //                route, which casts, copies or raises as it always did.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -17,6 +17,7 @@
 #include <ATen/core/grad_mode.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -340,8 +341,19 @@ PyObject *layernorm_fwd(PyObject *const *a, Py_ssize_t n) {  // x2d w bias out2d
 
 // ---- whole operators
 
-// What an operator runs right here: plain tensors on one GPU, outside autocast, with nothing for autograd to record.
-bool plain_call() { return !at::autocast::is_autocast_enabled(at::kCUDA); }
+// What an operator runs right here: plain tensors on one GPU, outside autocast, with nothing for autograd to record — and
+// nothing for anyone else who watches the operators go by: a launch made here is seen by no tracer, dispatch mode or
+// functorch transform (vmap, jvp, grad), which the autograd functions of the Python route record or refuse.
+bool plain_call() {
+    static const c10::DispatchKeySet watchers({c10::DispatchKey::Tracer, c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot,
+                                               c10::DispatchKey::FuncTorchDynamicLayerFrontMode});
+    return !at::autocast::is_autocast_enabled(at::kCUDA) && !c10::impl::tls_local_dispatch_key_set().included_.has_any(watchers);
+}
+
+PyObject *takes_call(PyObject *const *, Py_ssize_t n) {  // whether plain tensors would be taken where this is called
+    count(n, 0);
+    return PyBool_FromLong(plain_call());
+}
 
 const at::Tensor *plain(PyObject *o, const c10::Device *device = nullptr) {
     if (!THPVariable_CheckExact(o)) return nullptr;
@@ -349,6 +361,7 @@ const at::Tensor *plain(PyObject *o, const c10::Device *device = nullptr) {
     if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage()) return nullptr;
     if (device != nullptr && t.device() != *device) return nullptr;
     if (at::GradMode::is_enabled() && t.requires_grad()) return nullptr;
+    if (t._fw_grad(0).defined()) return nullptr;  // a tangent (forward mode), with or without grad mode
     return &t;
 }
 
@@ -577,7 +590,7 @@ PyObject *copy_many(PyObject *const *a, Py_ssize_t n) {
     const at::Tensor *first = nullptr;
     for (Py_ssize_t i = 0; i < pairs; ++i) {
         PyObject *d = PyList_GET_ITEM(a[0], i), *s = PyList_GET_ITEM(a[1], i);
-        if (!THPVariable_Check(d) || !THPVariable_Check(s)) Py_RETURN_NONE;
+        if (!THPVariable_CheckExact(d) || !THPVariable_CheckExact(s)) Py_RETURN_NONE;
         const at::Tensor &D = THPVariable_Unpack(d), &S = THPVariable_Unpack(s);
         if (first == nullptr) first = &D;
         if (!D.is_cuda() || D.device() != first->device() || S.device() != D.device() || S.scalar_type() != D.scalar_type() || S.sizes() != D.sizes() ||
@@ -606,7 +619,7 @@ PyObject *set_error_type(PyObject *, PyObject *type) {
 PyMethodDef kMethods[] = {
     ENTRY(attention_fwd), ENTRY(attention_cached_fwd), ENTRY(attention_skinny_fwd), ENTRY(linear_fwd), ENTRY(linear_rms_fwd),
     ENTRY(linear_decode_fwd), ENTRY(linear_fewrow_fwd), ENTRY(layernorm_fwd), ENTRY(op_layer_norm), ENTRY(op_attention),
-    ENTRY(op_skinny_attention), ENTRY(op_linear), ENTRY(plan_few_rows), ENTRY(copy_many),
+    ENTRY(op_skinny_attention), ENTRY(op_linear), ENTRY(plan_few_rows), ENTRY(copy_many), ENTRY(takes_call),
     {"set_error_type", set_error_type, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

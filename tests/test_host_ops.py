@@ -106,3 +106,79 @@ def test_autocast_and_recorded_calls_take_the_python_route():
     assert layer_norm(x, w.requires_grad_(), None, 1e-5).requires_grad
     with torch.no_grad():
         assert not layer_norm(x, w, None, 1e-5).requires_grad
+
+
+def _operators():
+    """Every operator with a native route, as (name, function of its first tensor, that tensor)."""
+    from kernl_amd.implementations.attention import attention_forward
+    from kernl_amd.implementations.attention_skinny import skinny_attention_forward
+    from kernl_amd.implementations.layer_norm import add_layer_norm, layer_norm
+    from kernl_amd.implementations.linear_layer import linear_layer
+
+    x, w = torch.randn(4, 64, device="cuda").half(), torch.randn(64, 64, device="cuda").half()
+    q, k, v = torch.randn(3, 1, 2, 8, 64, device="cuda").half()
+    return [
+        ("layer_norm", lambda t: layer_norm(t, w[0], None, 1e-5), x),
+        ("add_layer_norm", lambda t: add_layer_norm(t, x, w[0], None, 1e-5), x),
+        ("linear_layer", lambda t: linear_layer(t, w, None), x),
+        ("linear_layer (weight)", lambda t: linear_layer(x, t, None), w),
+        ("attention_forward", lambda t: attention_forward(t, k, v, torch.empty_like(q), 0.125), q),
+        ("skinny_attention_forward", lambda t: skinny_attention_forward(t, k[:, :, :1], v[:, :, :1], torch.empty_like(k[:, :, :1]), 0.125), q[:, :, :1].contiguous()),
+    ]
+
+
+@pytest.mark.gpu
+def test_forward_mode_is_refused():
+    """The autograd functions have no jvp: a tangent is an error, not a result without it."""
+    import torch.autograd.forward_ad as fwAD
+
+    for name, op, x in _operators():
+        for grad in (False, True):
+            with fwAD.dual_level(), torch.set_grad_enabled(grad):
+                with pytest.raises(NotImplementedError):
+                    op(fwAD.make_dual(x, torch.ones_like(x)))
+                    pytest.fail(f"{name}: a tangent went lost")
+
+
+@pytest.mark.gpu
+def test_traced_calls_are_recorded():
+    """What torch.jit.trace keeps is the autograd function, not an allocation that nothing fills."""
+    from kernl_amd.implementations.layer_norm import layer_norm
+
+    x, w = torch.randn(4, 64, device="cuda").half(), torch.randn(64, device="cuda").half()
+    traced = torch.jit.trace(lambda t: layer_norm(t, w, None, 1e-5), x, check_trace=False)
+    assert "LayerNorm" in str(traced.graph) and "aten::empty" not in str(traced.graph)
+
+
+@pytest.mark.gpu
+def test_transforms_are_refused():
+    for name, op, x in _operators():
+        for transformed in (lambda t: torch.vmap(op)(t), lambda t: torch.func.jvp(op, (t,), (torch.ones_like(t),)),
+                            lambda t: torch.vmap(lambda i: op(x) + i)(torch.zeros(3, device="cuda"))):
+            with pytest.raises(RuntimeError):  # (NotImplementedError among them)
+                transformed(torch.stack((x, x)))
+                pytest.fail(f"{name}: carried out inside a transform")
+
+
+def test_calls_that_someone_watches_are_declined():
+    """Under a transform, a tracer or a dispatch mode the native route declines before it looks at the tensors, and an
+    operator goes to its autograd function."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    h, x = _lib.host(), torch.zeros(2, 8)
+    seen = []
+
+    def probe(t):
+        seen.append([h.takes_call(), torch._C._are_functorch_transforms_active()])
+        return t + 1
+
+    probe(x)
+    assert seen == [[True, False]]
+    torch.vmap(probe)(x)
+    torch.func.jvp(probe, (x,), (x,))
+    assert seen[1:] == [[False, True]] * 2
+    del seen[:]
+    torch.jit.trace(probe, x, check_trace=False)
+    with TorchDispatchMode():
+        seen.append([h.takes_call(), False])
+    assert seen == [[False, False]] * 2
