@@ -19,6 +19,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/kernl_hip.h"
@@ -118,14 +119,14 @@ PyObject *launched(const at::Tensor &on, const char *what, F &&launch) {
 
 template <PyObject *(*F)(PyObject *const *, Py_ssize_t)>
 PyObject *guarded(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    // (PyTorch's own translation: a failed allocation is torch.OutOfMemoryError, which callers catch to try less)
+    HANDLE_TH_ERRORS
     try {
         return F(args, n);
     } catch (const BadArgument &) {
         return nullptr;
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
     }
+    END_HANDLE_TH_ERRORS
 }
 
 // ---- the ABI's entry points on tensors

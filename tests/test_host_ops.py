@@ -182,3 +182,14 @@ def test_calls_that_someone_watches_are_declined():
     with TorchDispatchMode():
         seen.append([h.takes_call(), False])
     assert seen == [[False, False]] * 2
+
+
+@pytest.mark.gpu
+def test_a_failed_allocation_is_pytorchs_error():
+    """4 M x 128 K results are 1 TB: refused by the allocator before anything is launched."""
+    from kernl_amd.implementations.linear_layer import LinearLayer, linear_layer
+
+    x, w = torch.zeros(1 << 22, 8, dtype=torch.float16, device="cuda"), torch.zeros(1 << 17, 8, dtype=torch.float16, device="cuda")
+    for call in (linear_layer, lambda *a: LinearLayer.apply(*a, "", None)):
+        with pytest.raises(torch.OutOfMemoryError):
+            call(x, w, None)
