@@ -56,8 +56,10 @@ double number(PyObject *o) {
     return v;
 }
 
-int64_t integer(PyObject *o) {
-    const int64_t v = PyLong_AsLongLong(o);
+int64_t integer(PyObject *o) {  // int(o): a float is cut off, a 0-d tensor is read
+    PyObject *whole = PyLong_Check(o) ? (Py_INCREF(o), o) : PyNumber_Long(o);
+    const int64_t v = whole == nullptr ? -1 : PyLong_AsLongLong(whole);
+    Py_XDECREF(whole);
     if (v == -1 && PyErr_Occurred()) throw BadArgument();
     return v;
 }
@@ -435,7 +437,9 @@ PyObject *op_attention(PyObject *const *a, Py_ssize_t n) {  // q k v out mask sc
     const at::Tensor *q, *k, *v, *out, *mask;
     float clamp;
     if (!attention_arguments(a, &q, &k, &v, &out, &mask, &clamp)) Py_RETURN_NONE;
-    Py_XDECREF(run_attention(*q, *k, *v, *out, mask, (float)number(a[5]), truth(a[6]), integer(a[7]), clamp));
+    const bool causal = truth(a[6]);
+    const int64_t start = causal && truth(a[7]) ? integer(a[7]) : 0;  // (looked at where it is used: None is as good as 0)
+    Py_XDECREF(run_attention(*q, *k, *v, *out, mask, (float)number(a[5]), causal, start, clamp));
     Py_INCREF(a[3]);
     return a[3];
 }

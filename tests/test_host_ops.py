@@ -193,3 +193,27 @@ def test_a_failed_allocation_is_pytorchs_error():
     for call in (linear_layer, lambda *a: LinearLayer.apply(*a, "", None)):
         with pytest.raises(torch.OutOfMemoryError):
             call(x, w, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal, start, same_as", [(False, None, 0), (True, None, 0), (False, 5.0, 0), (True, 5.0, 5), (False, "x", 0)], ids=str)
+def test_start_position_is_read_where_it_is_used(causal, start, same_as):
+    from kernl_amd.implementations.attention import Attention, attention_forward
+
+    q, k, v = torch.randn(3, 1, 2, 9, 64, device="cuda").half()
+    out = [torch.empty_like(q) for _ in range(3)]
+    attention_forward(q, k, v, out[0], 0.125, causal, None, start)
+    Attention.apply(q, k, v, out[1], 0.125, causal, None, start)
+    attention_forward(q, k, v, out[2], 0.125, causal, None, same_as)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+@pytest.mark.gpu
+def test_sizes_of_a_projection_may_be_floats():
+    """int() is taken of them, as it always was."""
+    from kernl_amd.implementations.linear_layer import decode_linear_layer
+
+    x, w, g = torch.randn(3, 128, device="cuda").half(), torch.randn(256, 128, device="cuda").half(), torch.ones(128, device="cuda").half()
+    cos, sin = torch.randn(2, 1, 3, 64, device="cuda").half()
+    want = decode_linear_layer(x, w, None, g, 1e-5, None, cos, sin, 64, 128)
+    assert torch.equal(decode_linear_layer(x, w, None, g, 1e-5, None, cos, sin, 64.0, 128.0), want)
