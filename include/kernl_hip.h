@@ -484,17 +484,6 @@ int kernl_embedding_layernorm_fwd(const void *table0, const int64_t *ids0, int64
 /* The process-wide test and tuning hooks are not part of this interface: they are declared in kernl_hip_test.h. */
 
 /*
- * kernl_embedding_layernorm_fwd with one of the lookups going through a vector: the ids of table `slot` (0 .. 2) are
- * source[ids], source a contiguous vector of source_len int64 entries (token types read at the position ids).
- */
-int kernl_embedding_layernorm_via_fwd(const void *table0, const int64_t *ids0, int64_t ids0_batch_stride, int64_t ids0_seq_stride,
-                                      int64_t rows0, const void *table1, const int64_t *ids1, int64_t ids1_batch_stride,
-                                      int64_t ids1_seq_stride, int64_t rows1, const void *table2, const int64_t *ids2,
-                                      int64_t ids2_batch_stride, int64_t ids2_seq_stride, int64_t rows2, int slot,
-                                      const int64_t *source, int64_t source_len, const void *w, const void *bias, void *out,
-                                      int64_t batch, int64_t seq, int64_t N, float eps, int dtype, void *stream);
-
-/*
  * Up to 8 device-to-device copies (16-byte aligned, not overlapping) in one launch: a captured graph's inputs on their way into
  * its static buffers (the reference copies them one by one, src/kernl/optimizer/cuda_graph.py:103-138).
  */

@@ -47,7 +47,6 @@ EXPORTED_SYMBOLS = (
     "kernl_linear_norm_add_fwd",
     "kernl_linear_norm_apply_fwd",
     "kernl_embedding_layernorm_fwd",
-    "kernl_embedding_layernorm_via_fwd",
     "kernl_copy_many",
     "kernl_select_mask_fwd",
     "kernl_linear_decode_fwd",
@@ -163,10 +162,6 @@ def load() -> ctypes.CDLL:
     lib.kernl_embedding_layernorm_fwd.restype = ctypes.c_int
     lib.kernl_embedding_layernorm_fwd.argtypes = [_vp, _vp, _i64, _i64, _i64] * 3 + [_vp, _vp, _vp, _i64, _i64, _i64,
                                                                                       ctypes.c_float, ctypes.c_int, _vp]
-    lib.kernl_embedding_layernorm_via_fwd.restype = ctypes.c_int
-    lib.kernl_embedding_layernorm_via_fwd.argtypes = (
-        [_vp, _vp, _i64, _i64, _i64] * 3 + [ctypes.c_int, _vp, _i64] + [_vp, _vp, _vp, _i64, _i64, _i64, ctypes.c_float, ctypes.c_int, _vp]
-    )
     lib.kernl_copy_many.restype = ctypes.c_int
     lib.kernl_copy_many.argtypes = [ctypes.c_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _i64p, _vp]
     lib.kernl_select_mask_fwd.restype = ctypes.c_int
@@ -475,10 +470,9 @@ def linear_residual_fwd(x2d, weight, bias, residual2d, out2d) -> None:
     _check(st, "kernl_linear_residual_fwd")
 
 
-def embedding_layernorm_fwd(tables, ids, weight, bias, out, eps: float, via=None) -> None:
+def embedding_layernorm_fwd(tables, ids, weight, bias, out, eps: float) -> None:
     """out[b, s] = LayerNorm(sum of tables[i][ids[i][b, s]]) (rows added one after the other in the tables' dtype).
-    tables: 1 to 3 contiguous [rows, N] matrices; ids: int64 [batch, seq] views (stride 0 allowed); out [batch, seq, N].
-    via: None or (slot, vector): the ids of table `slot` are vector[ids[slot]]."""
+    tables: 1 to 3 contiguous [rows, N] matrices; ids: int64 [batch, seq] views (stride 0 allowed); out [batch, seq, N]."""
     _require_gpu(*tables, *ids, weight, bias, out)
     batch, seq, n = out.shape
     if not 1 <= len(tables) <= 3 or len(ids) != len(tables):
@@ -495,15 +489,8 @@ def embedding_layernorm_fwd(tables, ids, weight, bias, out, eps: float, via=None
             args += [None, None, 0, 0, 0]
     lib = load()
     with torch.cuda.device(out.device):
-        rest = (weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(), batch, seq, n, float(eps),
-                DTYPE_CODE[out.dtype], _stream(out))
-        if via is None:
-            st = lib.kernl_embedding_layernorm_fwd(*args, *rest)
-        else:
-            slot, source = via
-            if source.dtype != torch.int64 or source.dim() != 1 or not source.is_contiguous() or not source.is_cuda:
-                raise ValueError("the vector that ids go through is a contiguous int64 vector on the GPU")
-            st = lib.kernl_embedding_layernorm_via_fwd(*args, int(slot), source.data_ptr(), source.numel(), *rest)
+        st = lib.kernl_embedding_layernorm_fwd(*args, weight.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(),
+                                               batch, seq, n, float(eps), DTYPE_CODE[out.dtype], _stream(out))
     _check(st, "kernl_embedding_layernorm_fwd")
 
 

@@ -383,14 +383,10 @@ __global__ void __launch_bounds__(256) add_rms_stats_kernel(const T *__restrict_
 // Embedding lookups summed and normalised: out[m] = LayerNorm(round(round(t0[i0[m]] + t1[i1[m]]) + t2[i2[m]])) — the
 // rows are added in the tensors' dtype, one addition after the other, as the eager model adds them.  One wave per output
 // row, a lane keeps up to 4 chunks of 8 values (N <= 2048); an index outside its table is clamped into it.
-// A table's ids may go through a vector (token types read at the position ids): a gather of a few KB before this kernel would cost its
-// launch, 3.5 us of a captured encoder.
 struct EmbedTable {
     const void *table;   // [rows, N] contiguous, or null
     const int64_t *ids;  // entry (b, s) at b * ids_bs + s * ids_ss
     int64_t ids_bs, ids_ss, rows;
-    const int64_t *via;  // null, or the vector through which the ids go
-    int64_t via_len;
 };
 template <typename T>
 __global__ void __launch_bounds__(256) embedding_layernorm_kernel(EmbedTable t0, EmbedTable t1, EmbedTable t2,
@@ -402,7 +398,6 @@ __global__ void __launch_bounds__(256) embedding_layernorm_kernel(EmbedTable t0,
     const int bi = row / S, si = row % S;
     auto row_of = [&](const EmbedTable &t) __attribute__((always_inline)) -> const vec8 * {
         int64_t id = t.ids[bi * t.ids_bs + si * t.ids_ss];
-        if (t.via != nullptr) id = t.via[id < 0 ? 0 : (id >= t.via_len ? t.via_len - 1 : id)];
         id = id < 0 ? 0 : (id >= t.rows ? t.rows - 1 : id);
         return reinterpret_cast<const vec8 *>(static_cast<const T *>(t.table) + id * N);
     };
@@ -536,12 +531,12 @@ extern "C" int kernl_add_rms_stats_fwd(const void *a, const void *b, void *sum, 
     return check_launch("add_rms_stats");
 }
 
-static int embedding_layernorm_entry(const void *table0, const int64_t *ids0, int64_t ids0_batch_stride, int64_t ids0_seq_stride,
-                                     int64_t rows0, const void *table1, const int64_t *ids1, int64_t ids1_batch_stride,
-                                     int64_t ids1_seq_stride, int64_t rows1, const void *table2, const int64_t *ids2,
-                                     int64_t ids2_batch_stride, int64_t ids2_seq_stride, int64_t rows2, int slot, const int64_t *source,
-                                     int64_t source_len, const void *w, const void *bias, void *out, int64_t batch, int64_t seq,
-                                     int64_t N, float eps, int dtype, void *stream) {
+extern "C" int kernl_embedding_layernorm_fwd(const void *table0, const int64_t *ids0, int64_t ids0_batch_stride,
+                                             int64_t ids0_seq_stride, int64_t rows0, const void *table1, const int64_t *ids1,
+                                             int64_t ids1_batch_stride, int64_t ids1_seq_stride, int64_t rows1,
+                                             const void *table2, const int64_t *ids2, int64_t ids2_batch_stride,
+                                             int64_t ids2_seq_stride, int64_t rows2, const void *w, const void *bias, void *out,
+                                             int64_t batch, int64_t seq, int64_t N, float eps, int dtype, void *stream) {
     using namespace kernl;
     if (table0 == nullptr || ids0 == nullptr || w == nullptr || out == nullptr || (table1 != nullptr && ids1 == nullptr) ||
         (table2 != nullptr && ids2 == nullptr))
@@ -558,9 +553,9 @@ static int embedding_layernorm_entry(const void *table0, const int64_t *ids0, in
         return set_error(KERNL_ERR_UNSUPPORTED, "embedding + layernorm: N must be a multiple of 8 and at most 2048, tables, w, bias "
                          "and out 16-byte aligned and contiguous");
     if (batch == 0 || seq == 0) return KERNL_OK;
-    const EmbedTable t0 = {table0, ids0, ids0_batch_stride, ids0_seq_stride, rows0, slot == 0 ? source : nullptr, source_len};
-    const EmbedTable t1 = {table1, ids1, ids1_batch_stride, ids1_seq_stride, rows1, slot == 1 ? source : nullptr, source_len};
-    const EmbedTable t2 = {table2, ids2, ids2_batch_stride, ids2_seq_stride, rows2, slot == 2 ? source : nullptr, source_len};
+    const EmbedTable t0 = {table0, ids0, ids0_batch_stride, ids0_seq_stride, rows0};
+    const EmbedTable t1 = {table1, ids1, ids1_batch_stride, ids1_seq_stride, rows1};
+    const EmbedTable t2 = {table2, ids2, ids2_batch_stride, ids2_seq_stride, rows2};
     const int M = (int)(batch * seq);
     const dim3 grid((unsigned)((M + 3) / 4)), block(256);
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -571,29 +566,4 @@ static int embedding_layernorm_entry(const void *table0, const int64_t *ids0, in
         hipLaunchKernelGGL((embedding_layernorm_kernel<bf16>), grid, block, 0, st, t0, t1, t2, static_cast<const bf16 *>(w),
                            static_cast<const bf16 *>(bias), static_cast<bf16 *>(out), M, (int)seq, (int)N, eps);
     return check_launch("embedding + layernorm");
-}
-
-extern "C" int kernl_embedding_layernorm_fwd(const void *table0, const int64_t *ids0, int64_t ids0_batch_stride,
-                                             int64_t ids0_seq_stride, int64_t rows0, const void *table1, const int64_t *ids1,
-                                             int64_t ids1_batch_stride, int64_t ids1_seq_stride, int64_t rows1,
-                                             const void *table2, const int64_t *ids2, int64_t ids2_batch_stride,
-                                             int64_t ids2_seq_stride, int64_t rows2, const void *w, const void *bias, void *out,
-                                             int64_t batch, int64_t seq, int64_t N, float eps, int dtype, void *stream) {
-    return embedding_layernorm_entry(table0, ids0, ids0_batch_stride, ids0_seq_stride, rows0, table1, ids1, ids1_batch_stride,
-                                     ids1_seq_stride, rows1, table2, ids2, ids2_batch_stride, ids2_seq_stride, rows2, -1, nullptr, 0, w,
-                                     bias, out, batch, seq, N, eps, dtype, stream);
-}
-
-extern "C" int kernl_embedding_layernorm_via_fwd(const void *table0, const int64_t *ids0, int64_t ids0_batch_stride,
-                                                 int64_t ids0_seq_stride, int64_t rows0, const void *table1, const int64_t *ids1,
-                                                 int64_t ids1_batch_stride, int64_t ids1_seq_stride, int64_t rows1,
-                                                 const void *table2, const int64_t *ids2, int64_t ids2_batch_stride,
-                                                 int64_t ids2_seq_stride, int64_t rows2, int slot, const int64_t *source,
-                                                 int64_t source_len, const void *w, const void *bias, void *out, int64_t batch,
-                                                 int64_t seq, int64_t N, float eps, int dtype, void *stream) {
-    if (slot < 0 || slot > 2 || source == nullptr || source_len <= 0)
-        return kernl::set_error(KERNL_ERR_INVALID_ARG, "embedding + layernorm: the gathered slot is 0 .. 2 with a source of at least one entry");
-    return embedding_layernorm_entry(table0, ids0, ids0_batch_stride, ids0_seq_stride, rows0, table1, ids1, ids1_batch_stride,
-                                     ids1_seq_stride, rows1, table2, ids2, ids2_batch_stride, ids2_seq_stride, rows2, slot, source,
-                                     source_len, w, bias, out, batch, seq, N, eps, dtype, stream);
 }

@@ -112,10 +112,10 @@ def embedding_layer_norm_supported(tables, ids, weight, bias) -> bool:
     return bool(params_ok and (bias is None or (bias.dtype == t0.dtype and bias.is_contiguous() and bias.numel() == t0.shape[1])))
 
 
-def embedding_layer_norm(tables, ids, weight: torch.Tensor, bias: Optional[torch.Tensor], eps: float, via=None) -> torch.Tensor:
+def embedding_layer_norm(tables, ids, weight: torch.Tensor, bias: Optional[torch.Tensor], eps: float) -> torch.Tensor:
     """LayerNorm(tables[0][ids[0]] + tables[1][ids[1]] + tables[2][ids[2]]) in one launch: the embedding stage of an
     encoder (word, token-type and position embeddings; the rows are added in the tables' dtype, in that order, as the
-    eager model adds them).  `via` = (slot, vector): the ids of table `slot` are vector[ids[slot]].  The fp16 eps policy is
+    eager model adds them).  The fp16 eps policy is
     the LayerNorm operator's.  No counterpart in the reference, which leaves the lookups and additions to PyTorch in front
     of its LayerNorm kernel (implementations/layer_norm.py:279-335)."""
     assert embedding_layer_norm_supported(tables, ids, weight, bias)
@@ -124,5 +124,5 @@ def embedding_layer_norm(tables, ids, weight: torch.Tensor, bias: Optional[torch
     if t0.dtype == torch.float16:
         eps = max(eps, 1.6e-5)
     out = torch.empty((shape[0], shape[1], t0.shape[1]), device=t0.device, dtype=t0.dtype)
-    _lib.embedding_layernorm_fwd(list(tables), [i.expand(shape) for i in ids], weight, bias, out, eps, via)
+    _lib.embedding_layernorm_fwd(list(tables), [i.expand(shape) for i in ids], weight, bias, out, eps)
     return out

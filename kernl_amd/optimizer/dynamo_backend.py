@@ -14,7 +14,6 @@ from kernl_amd.optimizer.dropout import remove_dropout
 from kernl_amd.optimizer.kv_cache import drop_empty_cat_operands
 from kernl_amd.optimizer.layer_norm import (
     fuse_embeddings_into_layer_norm,
-    gather_ids_in_embeddings,
     replace_layer_norm,
     replace_layer_norm_fn,
     replace_layer_norm_rms,
@@ -65,7 +64,6 @@ def dynamo_backend_ofi(gm: torch.fx.GraphModule, assume_causal=False):
     replace_layer_norm_fn(gm)
     replace_layer_norm_rms(gm)
     fuse_embeddings_into_layer_norm(gm)
-    gather_ids_in_embeddings(gm)
     fuse_rms_norm_into_linears(gm)
     fuse_rotary_into_projections(gm)
     fuse_residual_into_linears(gm)

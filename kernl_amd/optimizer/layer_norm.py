@@ -68,59 +68,6 @@ def layer_norm_rms_wrapper(v: torch.Tensor, weight: torch.Tensor, eps: float):
     return layer_norm(v, weight, None, eps, None, use_rms_norm=True)
 
 
-class GatheredIds:
-    """`torch.gather(source, 1, index).expand(shape)` that the embedding kernel carries out itself."""
-
-    def __init__(self, source: torch.Tensor, index: torch.Tensor, shape):
-        self.source, self.shape = source, shape
-        self.vector = None
-        # one source row for every batch entry, read at [1, seq] or [batch, seq] positions
-        if source.dim() == 2 and (source.shape[0] == 1 or source.stride(0) == 0) and source.stride(1) == 1 and source.dtype == torch.int64:
-            self.vector = source[0]
-        self.raw_index = index
-        self.index = index.expand(shape)
-
-    def carried_out(self) -> torch.Tensor:
-        return torch.gather(self.source, 1, self.raw_index).expand(self.shape)
-
-
-def gathered_ids(source: torch.Tensor, index: torch.Tensor, shape):
-    return GatheredIds(source, index, shape)
-
-
-torch.fx.wrap("gathered_ids")
-
-
-def gather_ids_in_embeddings(gm: torch.fx.GraphModule):
-    """`gather(source, 1, index).expand(sizes)` that is read only as ids of an `embedding_layer_norm_wrapper` (transformers reads its
-    token-type buffer at the position ids that way) becomes a `gathered_ids` node: the embedding kernel looks the ids up itself.
-    Runs after `fuse_embeddings_into_layer_norm`."""
-    changed = False
-    for node in list(gm.graph.nodes):
-        if not (node.op == "call_function" and node.target is embedding_layer_norm_wrapper):
-            continue
-        for k in (0, 2, 4):
-            ids = node.args[k]
-            if not (isinstance(ids, torch.fx.Node) and ids.op == "call_method" and ids.target == "expand" and len(ids.users) == 1):
-                continue
-            g = ids.args[0]
-            if not (isinstance(g, torch.fx.Node) and g.op == "call_function" and g.target is torch.gather and len(g.users) == 1):
-                continue
-            bound = dict(zip(("input", "dim", "index"), g.args), **g.kwargs)
-            sizes = ids.args[1] if len(ids.args) == 2 and isinstance(ids.args[1], (tuple, list)) else ids.args[1:]
-            if set(bound) != {"input", "dim", "index"} or bound["dim"] != 1 or len(sizes) != 2 or not all(isinstance(s, int) and s > 0 for s in sizes):
-                continue
-            with gm.graph.inserting_before(ids):
-                new = gm.graph.call_function(gathered_ids, (bound["input"], bound["index"], tuple(sizes)))
-            ids.replace_all_uses_with(new)
-            gm.graph.erase_node(ids)
-            gm.graph.erase_node(g)
-            changed = True
-    if changed:
-        gm.graph.lint()
-        gm.recompile()
-
-
 def embedding_layer_norm_wrapper(ids0, table0, ids1, table1, ids2, table2, normalized_shape, weight, bias, eps: float):
     """layer_norm((embedding(ids0, table0) + embedding(ids1, table1)) + embedding(ids2, table2)) — the third pair may be
     None — as one launch where the kernel takes the operands (`embedding_layer_norm`), as the lookups, additions and the
@@ -128,19 +75,11 @@ def embedding_layer_norm_wrapper(ids0, table0, ids1, table1, ids2, table2, norma
     from kernl_amd.implementations.layer_norm import embedding_layer_norm, embedding_layer_norm_supported
 
     pairs = [(i, t) for i, t in ((ids0, table0), (ids1, table1), (ids2, table2)) if t is not None]
-    tables, ids, via = [t for _, t in pairs], [i for i, _ in pairs], None
-    gathered = [k for k, i in enumerate(ids) if isinstance(i, GatheredIds)]
-    if len(gathered) == 1 and ids[gathered[0]].vector is not None:
-        via = (gathered[0], ids[gathered[0]].vector)
-        ids = [i.index if isinstance(i, GatheredIds) else i for i in ids]
-    else:
-        ids = [i.carried_out() if isinstance(i, GatheredIds) else i for i in ids]
+    tables, ids = [t for _, t in pairs], [i for i, _ in pairs]
     if all(t.dtype == torch.float16 for t in tables):
         _half_params_once(tables[0], weight, bias)
     if len(normalized_shape) == 1 and not torch.is_autocast_enabled("cuda") and embedding_layer_norm_supported(tables, ids, weight, bias):
-        return embedding_layer_norm(tables, ids, weight, bias, eps, via)
-    if via is not None:
-        ids[via[0]] = via[1][ids[via[0]]]
+        return embedding_layer_norm(tables, ids, weight, bias, eps)
     total = torch.nn.functional.embedding(ids[0], tables[0])
     for i, t in zip(ids[1:-1], tables[1:-1]):
         total = total + torch.nn.functional.embedding(i, t)

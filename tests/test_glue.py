@@ -43,20 +43,28 @@ def test_mask_selection(shape, mask_dtype, dtype):
         assert torch.equal(select_mask(mask, 0.0, off, dtype), want)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("slot", [0, 1, 2])
-def test_embedding_ids_through_a_vector(slot):
-    from kernl_amd.implementations.layer_norm import embedding_layer_norm
+def test_token_types_gathered_at_the_position_ids_stay_gathered():
+    """A position id outside the token-type buffer is torch.gather's to refuse: the lookups that follow it must not replace it."""
+    from kernl_amd.optimizer.dynamo_backend import dynamo_backend_ofi
+    from kernl_amd.optimizer.layer_norm import embedding_layer_norm_wrapper
 
-    gen = torch.Generator().manual_seed(slot)
-    tables = [torch.randn(r, 96, generator=gen).half().cuda() for r in (50, 3, 70)]
-    ids = [torch.randint(0, t.shape[0], (2, 19), generator=gen).cuda() for t in tables]
-    vector = torch.randint(0, tables[slot].shape[0], (64,), generator=gen).cuda()
-    w = torch.randn(96, generator=gen).half().cuda()
-    index = torch.randint(0, 64, (1, 19), generator=gen).cuda()
-    through = list(ids)
-    ids[slot], through[slot] = vector[index].expand(2, 19), index
-    assert torch.equal(embedding_layer_norm(tables, through, w, None, 1e-5, via=(slot, vector)), embedding_layer_norm(tables, ids, w, None, 1e-5))
+    class Embeddings(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.words, self.types, self.places = (torch.nn.Parameter(torch.randn(n, 32)) for n in (50, 2, 16))
+            self.weight, self.bias = torch.nn.Parameter(torch.ones(32)), torch.nn.Parameter(torch.zeros(32))
+            self.register_buffer("type_ids", torch.zeros(1, 16, dtype=torch.long))
+
+        def forward(self, ids, position_ids):
+            types = torch.gather(self.type_ids.expand(1, -1), dim=1, index=position_ids).expand(3, 7)
+            lookup = torch.nn.functional.embedding
+            total = lookup(ids, self.words) + lookup(types, self.types) + lookup(position_ids, self.places)
+            return torch.nn.functional.layer_norm(total, (32,), self.weight, self.bias, 1e-5)
+
+    gm = torch.fx.symbolic_trace(Embeddings())
+    dynamo_backend_ofi(gm)
+    targets = [n.target for n in gm.graph.nodes if n.op == "call_function"]
+    assert embedding_layer_norm_wrapper in targets and torch.gather in targets
 
 
 def test_mask_selection_pass_leaves_other_readers_alone():
