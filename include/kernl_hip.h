@@ -275,27 +275,32 @@ int kernl_linear_residual_fwd(const void *x, const void *w, const void *bias, co
                               const int64_t residual_strides[2], int dtype, void *stream);
 
 /*
- * A LayerNorm between linear layers without a launch of its own, for small problems (a few hundred rows; widths that are a
- * multiple of 32, up to 1024).  The layer in front of the norm,
- *     kernl_linear_norm_add_fwd:    out = s = round(x @ w^T + bias + residual),
- *                                   out_stats[m][n / g] = (sum, sum of squared deviations from their mean) of s[m][n .. n + g - 1],
- *                                   g = kernl_linear_norm_group(M) columns (16 or 32),
+ * A LayerNorm between linear layers without a launch of its own, for 8 to 64 rows (widths that are a multiple of 32, up to 1024).
+ * The layer in front of the norm,
+ *     kernl_linear_norm_add_fwd:    out = s = x @ w^T + bias + residual, in fp32,
+ *                                   out_stats[m][n / 16] = (sum, sum of squared deviations from their mean) of s[m][n .. n + 15],
  * leaves the rows un-normalised; the layer behind,
- *     kernl_linear_norm_apply_fwd:  out = act(LN(x) @ w^T + bias) = act(rstd (x @ w_folded^T - mean colsum) + bias32),
- * with w_folded = w * gamma (columns), colsum[n] = sum_k w_folded[n][k], bias32 = bias + w @ beta, normalises its sums.  A
- * residual that is such a deferred norm itself (residual_stats given) is normalised on the fly: residual stands for
- * (residual - mean) * rstd * gamma + beta.  kernl_linear_norm_kind: 0 where the small-problem kernels do not take M x N x K.
+ *     kernl_linear_norm_apply_fwd:  out = act(round(LN(x)) @ w^T + bias), x such rows with their statistics,
+ * normalises them on their way into its products (LN(x) = (x - mean) * rstd * gamma + beta, rounded once to `dtype`).  A residual
+ * that is such a deferred norm itself (residual_stats given; then it is fp32 rows, otherwise rows of `dtype`) is normalised on
+ * the fly.  kernl_linear_norm_kind: 0 where these kernels do not take M x N x K.
  * The reference runs a LayerNorm kernel between its linear kernels (src/kernl/implementations/layer_norm.py:279-335).
  */
 int kernl_linear_norm_kind(int64_t M, int64_t N, int64_t K);
-int kernl_linear_norm_group(int64_t M);
 int kernl_linear_norm_add_fwd(const void *x, const void *w, const void *bias, const void *residual, const float *residual_stats,
-                              const void *gamma, const void *beta, float eps, void *out, float *out_stats, int64_t M, int64_t N,
+                              const void *gamma, const void *beta, float eps, float *out, float *out_stats, int64_t M, int64_t N,
                               int64_t K, int64_t x_row_stride, int64_t out_row_stride, int64_t residual_row_stride, int dtype,
                               void *stream);
-int kernl_linear_norm_apply_fwd(const void *x, const float *x_stats, float eps, const void *w_folded, const float *colsum,
-                                const float *bias32, void *out, int64_t M, int64_t N, int64_t K, int64_t x_row_stride,
+int kernl_linear_norm_apply_fwd(const float *x, const float *x_stats, const void *gamma, const void *beta, float eps, const void *w,
+                                const void *bias, void *out, int64_t M, int64_t N, int64_t K, int64_t x_row_stride,
                                 int64_t out_row_stride, int activation, int dtype, void *stream);
+
+/*
+ * LayerNorm of fp32 rows into a tensor of `dtype` (f16 / bf16, as w and bias): the rows of a deferred norm as the tensor they stand for.
+ * N a multiple of 4, at most 1024.
+ */
+int kernl_layernorm_rows32_fwd(const float *x, const void *w, const void *bias, void *out, int64_t M, int64_t N, int64_t x_row_stride,
+                               int64_t out_row_stride, float eps, int dtype, void *stream);
 
 /*
  * Whether kernl_linear_fwd runs M x N x K (16-bit, plain epilogue, x with unit feature stride) on one of its

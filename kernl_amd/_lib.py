@@ -43,9 +43,9 @@ EXPORTED_SYMBOLS = (
     "kernl_linear_wide_kind",
     "kernl_linear_mid_kind",
     "kernl_linear_norm_kind",
-    "kernl_linear_norm_group",
     "kernl_linear_norm_add_fwd",
     "kernl_linear_norm_apply_fwd",
+    "kernl_layernorm_rows32_fwd",
     "kernl_embedding_layernorm_fwd",
     "kernl_copy_many",
     "kernl_select_mask_fwd",
@@ -176,12 +176,12 @@ def load() -> ctypes.CDLL:
     lib.kernl_linear_mid_kind.argtypes = [_i64] * 3 + [ctypes.c_int]
     lib.kernl_linear_norm_kind.restype = ctypes.c_int
     lib.kernl_linear_norm_kind.argtypes = [_i64] * 3
-    lib.kernl_linear_norm_group.restype = ctypes.c_int
-    lib.kernl_linear_norm_group.argtypes = [_i64]
     lib.kernl_linear_norm_add_fwd.restype = ctypes.c_int
     lib.kernl_linear_norm_add_fwd.argtypes = [_vp] * 7 + [ctypes.c_float, _vp, _vp] + [_i64] * 6 + [ctypes.c_int, _vp]
     lib.kernl_linear_norm_apply_fwd.restype = ctypes.c_int
-    lib.kernl_linear_norm_apply_fwd.argtypes = [_vp, _vp, ctypes.c_float] + [_vp] * 4 + [_i64] * 5 + [ctypes.c_int, ctypes.c_int, _vp]
+    lib.kernl_linear_norm_apply_fwd.argtypes = [_vp] * 4 + [ctypes.c_float] + [_vp] * 3 + [_i64] * 5 + [ctypes.c_int, ctypes.c_int, _vp]
+    lib.kernl_layernorm_rows32_fwd.restype = ctypes.c_int
+    lib.kernl_layernorm_rows32_fwd.argtypes = [_vp] * 4 + [_i64] * 4 + [ctypes.c_float, ctypes.c_int, _vp]
     lib.kernl_linear_glu_fwd.restype = ctypes.c_int
     lib.kernl_linear_glu_fwd.argtypes = [_vp] * 4 + [_i64] * 3 + [_i64p] * 2 + [ctypes.c_int, ctypes.c_int, _vp]
     lib.kernl_layernorm_fwd.restype = ctypes.c_int
@@ -341,48 +341,67 @@ def linear_norm_kind(M: int, N: int, K: int) -> int:
     return int(load().kernl_linear_norm_kind(int(M), int(N), int(K)))
 
 
-def linear_norm_group(M: int) -> int:
-    """Columns per statistics pair of a deferred norm over M rows."""
-    return int(load().kernl_linear_norm_group(int(M)))
+NORM_GROUP = 16  # columns per statistics pair of a deferred norm
+
+
+def _norm_checks(x2d, weight, out2d, statistics, parameters, width: int) -> None:
+    """Layouts of the deferred-norm entry points: what their pointers are taken to mean."""
+    if any(t is not None and (t.dtype != torch.float32 or t.numel() != x2d.shape[0] * width // NORM_GROUP * 2 or not t.is_contiguous()) for t in statistics):
+        raise ValueError("statistics are contiguous fp32 [rows, columns / 16, 2]")
+    if any(p is not None and (p.dtype != weight.dtype or p.shape != (n,) or not p.is_contiguous()) for p, n in parameters):
+        raise ValueError("bias and norm parameters are contiguous vectors of the weight's type")
+    if x2d.stride(1) != 1 or out2d.stride(1) != 1 or not weight.is_contiguous() or x2d.shape[1] != weight.shape[1] or out2d.shape != (x2d.shape[0], weight.shape[0]):
+        raise ValueError("unit feature strides, a contiguous weight and matching sizes")
 
 
 def linear_norm_add_fwd(x2d, weight, bias, residual2d, residual_stats, gamma, beta, eps: float, out2d, out_stats) -> None:
-    """out = x @ w^T + bias + residual with the statistics of its rows; with `residual_stats` the residual is the
-    un-normalised rows of a deferred LayerNorm (gamma, beta, eps)."""
+    """out = x @ w^T + bias + residual in fp32 with the statistics of its rows; with `residual_stats` the residual is the fp32
+    rows of a deferred LayerNorm (gamma, beta, eps)."""
     _require_gpu(x2d, weight, bias, residual2d, residual_stats, gamma, beta, out2d, out_stats)
     M, K = x2d.shape
     N = weight.shape[0]
-    if any(t is not None and (t.dtype != torch.float32 or t.numel() != M * N // linear_norm_group(M) * 2 or not t.is_contiguous()) for t in (residual_stats, out_stats)):
-        raise ValueError("statistics are contiguous fp32 [rows, columns / linear_norm_group(rows), 2]")
-    if x2d.stride(1) != 1 or residual2d.stride(1) != 1 or out2d.stride(1) != 1 or not weight.is_contiguous():
-        raise ValueError("unit feature strides and a contiguous weight")
+    _norm_checks(x2d, weight, out2d, (residual_stats, out_stats), ((bias, N), (gamma, N), (beta, N)), N)
+    if out2d.dtype != torch.float32 or residual2d.dtype != (weight.dtype if residual_stats is None else torch.float32) or residual2d.shape != (M, N) \
+            or residual2d.stride(1) != 1 or x2d.dtype != weight.dtype:
+        raise ValueError("fp32 rows out, a residual of x's type (fp32 rows where it has statistics)")
     with torch.cuda.device(x2d.device):
         st = load().kernl_linear_norm_add_fwd(
             x2d.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), residual2d.data_ptr(),
             None if residual_stats is None else residual_stats.data_ptr(), None if gamma is None else gamma.data_ptr(),
             None if beta is None else beta.data_ptr(), float(eps), out2d.data_ptr(), out_stats.data_ptr(), M, N, K, x2d.stride(0),
-            out2d.stride(0), residual2d.stride(0), DTYPE_CODE[x2d.dtype], _stream(x2d),
+            out2d.stride(0), residual2d.stride(0), DTYPE_CODE[weight.dtype], _stream(x2d),
         )
     _check(st, "kernl_linear_norm_add_fwd")
 
 
-def linear_norm_apply_fwd(x2d, x_stats, eps: float, weight_folded, colsum, bias32, out2d, activation: int) -> None:
-    """out = act(LN(x) @ w^T + bias) of un-normalised rows x with their statistics and the folded parameters."""
-    _require_gpu(x2d, x_stats, weight_folded, colsum, bias32, out2d)
+def linear_norm_apply_fwd(x2d, x_stats, gamma, beta, eps: float, weight, bias, out2d, activation: int) -> None:
+    """out = act(LN(x) @ w^T + bias) of fp32 rows x with their statistics, LN(x) rounded to the weight's type."""
+    _require_gpu(x2d, x_stats, gamma, beta, weight, bias, out2d)
     M, K = x2d.shape
-    N = weight_folded.shape[0]
-    if x_stats.dtype != torch.float32 or x_stats.numel() != M * K // linear_norm_group(M) * 2 or not x_stats.is_contiguous():
-        raise ValueError("statistics are contiguous fp32 [rows, columns / linear_norm_group(rows), 2]")
-    if any(t.dtype != torch.float32 or t.numel() != N or not t.is_contiguous() for t in (colsum, bias32)):
-        raise ValueError("colsum and bias32 are contiguous fp32 vectors with one entry per column")
-    if x2d.stride(1) != 1 or out2d.stride(1) != 1 or not weight_folded.is_contiguous():
-        raise ValueError("unit feature strides and a contiguous weight")
+    N = weight.shape[0]
+    _norm_checks(x2d, weight, out2d, (x_stats,), ((bias, N), (gamma, K), (beta, K)), K)
+    if x2d.dtype != torch.float32 or out2d.dtype != weight.dtype:
+        raise ValueError("fp32 rows in, rows of the weight's type out")
     with torch.cuda.device(x2d.device):
         st = load().kernl_linear_norm_apply_fwd(
-            x2d.data_ptr(), x_stats.data_ptr(), float(eps), weight_folded.data_ptr(), colsum.data_ptr(), bias32.data_ptr(),
-            out2d.data_ptr(), M, N, K, x2d.stride(0), out2d.stride(0), int(activation), DTYPE_CODE[x2d.dtype], _stream(x2d),
+            x2d.data_ptr(), x_stats.data_ptr(), gamma.data_ptr(), None if beta is None else beta.data_ptr(), float(eps), weight.data_ptr(),
+            None if bias is None else bias.data_ptr(), out2d.data_ptr(), M, N, K, x2d.stride(0), out2d.stride(0), int(activation),
+            DTYPE_CODE[weight.dtype], _stream(x2d),
         )
     _check(st, "kernl_linear_norm_apply_fwd")
+
+
+def layernorm_rows32_fwd(x2d, weight, bias, out2d, eps: float) -> None:
+    """out = LN(x) of fp32 rows x in the weight's 16-bit type."""
+    _require_gpu(x2d, weight, bias, out2d)
+    M, N = x2d.shape
+    if x2d.dtype != torch.float32 or out2d.dtype != weight.dtype or out2d.shape != x2d.shape or x2d.stride(1) != 1 or out2d.stride(1) != 1 \
+            or any(p is not None and (p.dtype != weight.dtype or p.shape != (N,) or not p.is_contiguous()) for p in (weight, bias)):
+        raise ValueError("fp32 rows in, rows of the weight's type out, contiguous parameters")
+    with torch.cuda.device(x2d.device):
+        st = load().kernl_layernorm_rows32_fwd(x2d.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), out2d.data_ptr(), M, N,
+                                               x2d.stride(0), out2d.stride(0), float(eps), DTYPE_CODE[weight.dtype], _stream(x2d))
+    _check(st, "kernl_layernorm_rows32_fwd")
 
 
 def linear_w8_supported(x2d, weight8) -> bool:

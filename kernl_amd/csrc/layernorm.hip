@@ -7,6 +7,7 @@
 // RMS branch keeps mean = 0 and uses mean(x^2).  The variance is the exact two-pass form Σ(x-mean)²/N on the
 // register copy, which is at least as accurate as the reference's chunked Welford merge (:159-180).
 #include "common.h"
+#include "norm_fold.h"
 
 namespace kernl {
 
@@ -456,6 +457,43 @@ __global__ void __launch_bounds__(256) embedding_layernorm_kernel(EmbedTable t0,
     }
 }
 
+// LayerNorm of fp32 rows into a 16-bit tensor (the rows of a deferred norm, where they are needed as a tensor after all): one wave
+// per row, a lane keeps up to 4 chunks of 4 values (N <= 1024).  A few rows: bound by its launch and one trip to memory.
+template <typename T>
+__global__ void __launch_bounds__(256) layernorm_rows32_kernel(const float *__restrict__ x, const T *__restrict__ w, const T *__restrict__ b,
+                                                               T *__restrict__ out, int M, int N, int64_t x_rs, int64_t out_rs, float eps) {
+    const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (threadIdx.x >> 6), chunks = N / 4;
+    if (row >= M) return;
+    const f32x4 *xp = reinterpret_cast<const f32x4 *>(x + (int64_t)row * x_rs);
+    f32x4 v[4];
+    float sum = 0.0f, sq = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[i] = lane + 64 * i < chunks ? xp[lane + 64 * i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum += v[i][e];
+    }
+    const float mean = wave_sum(sum) / (float)N;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (lane + 64 * i < chunks)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sq = fmaf(v[i][e] - mean, v[i][e] - mean, sq);
+    const float rstd = rsqrtf(wave_sum(sq) / (float)N + eps);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int c = lane + 64 * i;
+        if (c >= chunks) continue;
+        const u32x2 wr = reinterpret_cast<const u32x2 *>(w)[c], br = b != nullptr ? reinterpret_cast<const u32x2 *>(b)[c] : u32x2{0, 0};
+        float g[4], be[4], y[4];
+        unpack4<T>(wr, g);
+        unpack4<T>(br, be);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = fmaf((v[i][e] - mean) * rstd, g[e], be[e]);
+        reinterpret_cast<u32x2 *>(out + (int64_t)row * out_rs)[c] = u32x2{pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
+    }
+}
+
 static int layernorm_entry(const void *x, const void *res, const void *w, const void *b, void *out,
                            float *mean, float *rstd, int64_t M, int64_t N, int64_t x_rs, int64_t x_cs,
                            int64_t res_rs, int64_t res_cs, int64_t out_rs, int64_t out_cs, float eps,
@@ -504,6 +542,28 @@ extern "C" int kernl_add_layernorm_fwd(const void *x, const void *residual, cons
     return kernl::layernorm_entry(x, residual, w, bias, out, mean, rstd, M, N, x_row_stride, x_col_stride,
                                   res_row_stride, res_col_stride, out_row_stride, out_col_stride, eps,
                                   is_rms, dtype, stream);
+}
+
+extern "C" int kernl_layernorm_rows32_fwd(const float *x, const void *w, const void *bias, void *out, int64_t M, int64_t N,
+                                          int64_t x_row_stride, int64_t out_row_stride, float eps, int dtype, void *stream) {
+    using namespace kernl;
+    if (x == nullptr || w == nullptr || out == nullptr) return set_error(KERNL_ERR_INVALID_ARG, "layernorm of fp32 rows: x, w and out must not be NULL");
+    if (M < 0 || N <= 0) return set_error(KERNL_ERR_INVALID_ARG, "layernorm of fp32 rows: bad sizes M=%lld N=%lld", (long long)M, (long long)N);
+    if (dtype != KERNL_F16 && dtype != KERNL_BF16)
+        return set_error(KERNL_ERR_UNSUPPORTED, "layernorm of fp32 rows: results are f16 or bf16, got dtype %d", dtype);
+    if (N % 4 != 0 || N > 1024 || M > INT32_MAX - 4 || !aligned16(x) || x_row_stride % 4 != 0 || !aligned16(w) || !aligned16(bias) ||
+        !aligned16(out) || out_row_stride % 4 != 0)
+        return set_error(KERNL_ERR_UNSUPPORTED, "layernorm of fp32 rows: N must be a multiple of 4 up to 1024, the arrays 16-byte aligned");
+    if (M == 0) return KERNL_OK;
+    const dim3 grid((unsigned)((M + 3) / 4)), block(256);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (dtype == KERNL_F16)
+        hipLaunchKernelGGL((layernorm_rows32_kernel<f16>), grid, block, 0, st, x, static_cast<const f16 *>(w), static_cast<const f16 *>(bias),
+                           static_cast<f16 *>(out), (int)M, (int)N, x_row_stride, out_row_stride, eps);
+    else
+        hipLaunchKernelGGL((layernorm_rows32_kernel<bf16>), grid, block, 0, st, x, static_cast<const bf16 *>(w), static_cast<const bf16 *>(bias),
+                           static_cast<bf16 *>(out), (int)M, (int)N, x_row_stride, out_row_stride, eps);
+    return check_launch("layernorm of fp32 rows");
 }
 
 extern "C" int kernl_add_rms_stats_fwd(const void *a, const void *b, void *sum, float *rstd, int64_t M, int64_t N,

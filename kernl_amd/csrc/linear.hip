@@ -6,25 +6,29 @@ namespace kernl {
 
 int g_linear_force_tile = 0;
 
+// Dealt k-tiles: time is what a workgroup pulls from memory, so the smallest tiles that are still one round (us, 32 x 32 -> 16 x 16
+// tiles): 17 x 768 x 3072 6.9 -> 5.6, 64 x 768 x 3072 7.8 -> 5.9, 64 x 768 x 768 4.5 -> 4.0, 64 x 1024 x 4096 8.6 -> 6.5; 16 x 32:
+// 96 x 768 x 3072 7.8 -> 6.7, 48 x 2304 x 768 5.0 -> 4.7.
+static void dealt_tile(int M, int N, int kind, int &rows, int &cols) {
+    auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    rows = kind == 12 || kind == 16 ? 16 : kind == 13 ? 32 : 64;
+    cols = kind == 16 ? 16 : 32;
+    if (kind != 12 && kind != 13) return;
+    if (tiles(16, 16) <= 256) rows = cols = 16;
+    else if (M <= 96 && tiles(16, 32) <= 256) rows = 16;
+}
+
 // Runs the kernel a value of small_problem_kind / mid_kind (or of the hook) names; 0: it does not take this epilogue.
-static int run_one_launch(const LinearArgs &a, int dtype, int kind, int mode, const NormFold &nf) {
-    if (kind == 11 || kind == 15 || kind >= 17) return run_mid(a, dtype, kind, mode, nf);
+static int run_one_launch(const LinearArgs &a, int dtype, int kind) {
+    if (kind == 11 || kind == 15 || kind >= 17) return run_mid(a, dtype, kind);
     if ((a.act & kGluBit) || a.row_scale != nullptr || a.residual != nullptr) return 0;
     if (kind == 10) {
-        run_small(a, dtype, mode, nf);
+        run_small(a, dtype);
         return 1;
     }
-    // Dealt k-tiles: time is what a workgroup pulls from memory, so the smallest tiles that are still one round (us, 32 x 32 -> 16 x 16
-    // tiles): 17 x 768 x 3072 6.9 -> 5.6, 64 x 768 x 3072 7.8 -> 5.9, 64 x 768 x 768 4.5 -> 4.0, 64 x 1024 x 4096 8.6 -> 6.5; 16 x 32:
-    // 96 x 768 x 3072 7.8 -> 6.7, 48 x 2304 x 768 5.0 -> 4.7.
-    auto tiles = [&](int bm, int bn) { return (int64_t)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
-    int rows = kind == 12 || kind == 16 ? 16 : kind == 13 ? 32 : 64, cols = kind == 16 ? 16 : 32;
-    if (kind == 12 || kind == 13) {
-        const bool narrow = mode != kNormAdd || nf.group == kNormGroupFew;  // (a tile row holds whole statistics groups)
-        if (narrow && tiles(16, 16) <= 256) rows = cols = 16;
-        else if (a.M <= 96 && tiles(16, 32) <= 256) rows = 16;
-    }
-    run_small_dealt(a, dtype, rows, cols, mode, nf);
+    int rows, cols;
+    dealt_tile(a.M, a.N, kind, rows, cols);
+    run_small_dealt(a, dtype, rows, cols, kNormNone, NormFold());
     return 1;
 }
 
@@ -42,7 +46,7 @@ static int linear_mfma_dispatch(const LinearArgs &a) {
     // one launch of small or middling tiles over the whole K (the hook forces any of them)
     if (pick == 0) pick = (a.act & kGluBit) ? 0 : small_problem_kind(a.M, a.N, a.K);
     if (pick == 0) pick = mid_kind(a.M, a.N, a.K, (a.act & kGluBit) != 0);
-    if (pick >= 10 && run_one_launch(a, kDtype, pick, kNormNone, NormFold())) return check_launch("linear (one launch over the whole K)");
+    if (pick >= 10 && run_one_launch(a, kDtype, pick)) return check_launch("linear (one launch over the whole K)");
     if (pick == 0 || pick >= 9) pick = pick_tile(a.M, a.N, a.K, (a.act & kGluBit) != 0);
     if (a.act & kGluBit) {
         if (pick == 5) run_wide(a, kDtype, 256);
@@ -256,7 +260,7 @@ extern "C" int kernl_linear_scaled_fwd(const void *x, const void *w, const void 
     // the wide kernels take per-row factors (5 / 6: 256-row tiles, 7 / 8: 128-row tiles; gated: 256 x 256 only), and the 8-wave tiles
     if (g_linear_force_tile == 0 && small_problem_kind(a.M, a.N, a.K) == 0)
         if (const int mid = mid_kind(a.M, a.N, a.K, gated != 0))
-            if (run_one_launch(a, dtype, mid, kNormNone, NormFold())) return check_launch("scaled linear (8-wave tiles)");
+            if (run_one_launch(a, dtype, mid)) return check_launch("scaled linear (8-wave tiles)");
     int pick = g_linear_force_tile >= 5 && g_linear_force_tile <= 8 ? g_linear_force_tile : pick_tile(a.M, a.N, a.K, gated != 0, true);
     if (gated) pick = 5;
     if (pick == 5) run_wide(a, dtype, 256);
@@ -299,7 +303,7 @@ extern "C" int kernl_linear_residual_fwd(const void *x, const void *w, const voi
     // the wide kernels add a residual (5 / 6: 256-row tiles, 7 / 8: 128-row tiles), and the 8-wave tiles
     if (g_linear_force_tile == 0 && small_problem_kind(a.M, a.N, a.K) == 0)
         if (const int mid = mid_kind(a.M, a.N, a.K, false))
-            if (run_one_launch(a, dtype, mid, kNormNone, NormFold())) return check_launch("linear + residual (8-wave tiles)");
+            if (run_one_launch(a, dtype, mid)) return check_launch("linear + residual (8-wave tiles)");
     const int pick = g_linear_force_tile >= 5 && g_linear_force_tile <= 8 ? g_linear_force_tile : pick_tile(a.M, a.N, a.K, false, true);
     if (pick == 5) run_wide(a, dtype, 256);
     else if (pick == 6) run_wide(a, dtype, 192);
@@ -308,89 +312,88 @@ extern "C" int kernl_linear_residual_fwd(const void *x, const void *w, const voi
     return check_launch("linear + residual");
 }
 
-// Both sides of a deferred LayerNorm run on the small-problem kernels or the 8-wave tiles whose waves own 32 columns.
+// Both sides of a deferred LayerNorm run on the dealt tiles (in front of it always on 16 x 16: 64 x 1024 are 256 of them).
 static int norm_kind(int64_t M, int64_t N, int64_t K) {
     using namespace kernl;
-    int pick = g_linear_force_tile >= 10 ? g_linear_force_tile : small_problem_kind(M, N, K);
-    if (M <= kNormFewRows) return pick == 12 || pick == 13 || pick == 16 ? pick : 0;  // (16-column groups: tiles that stage that many)
-    if (pick == 0) pick = mid_kind(M, N, K, false);
-    return pick <= 17 && pick != 16 ? pick : 0;
+    if (M > kNormMaxRows) return 0;
+    const int pick = small_problem_kind(M, N, K);
+    return pick == 12 || pick == 13 ? pick : 0;
 }
 
-// (128 x 64 tiles stage the statistics of up to 24 groups)
-static bool norm_groups_fit(int kind, int64_t groups) { return kind != 15 || groups <= 24; }
-
 extern "C" int kernl_linear_norm_kind(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0 || N % kernl::kNormGroup != 0 || K % 8 != 0 || M > INT32_MAX || N > INT32_MAX) return 0;
+    if (M <= 0 || N <= 0 || K <= 0 || N % 32 != 0 || K % 8 != 0 || N > INT32_MAX) return 0;
     return norm_kind(M, N, K);
 }
 
-extern "C" int kernl_linear_norm_group(int64_t M) { return kernl::norm_group_of(M); }
-
-static int norm_arguments_bad(const char *what, const void *x, const void *w, const void *out, int64_t M, int64_t N, int64_t K, int64_t x_rs,
-                              int64_t out_rs, int dtype) {
+// sizes and layouts of both entry points; x and out in elements of `x_bytes` / `out_bytes`
+static int norm_arguments_bad(const char *what, const void *x, int x_bytes, const void *w, const void *out, int out_bytes, int64_t M, int64_t N,
+                              int64_t K, int64_t x_rs, int64_t out_rs, int dtype) {
     using namespace kernl;
     if (x == nullptr || w == nullptr || out == nullptr) return set_error(KERNL_ERR_INVALID_ARG, "%s: x, w and out must not be NULL", what);
     if (M < 0 || N <= 0 || K <= 0)
         return set_error(KERNL_ERR_INVALID_ARG, "%s: bad sizes M=%lld N=%lld K=%lld", what, (long long)M, (long long)N, (long long)K);
     if (dtype != KERNL_F16 && dtype != KERNL_BF16) return set_error(KERNL_ERR_UNSUPPORTED, "%s: only f16 and bf16 are supported, got dtype %d", what, dtype);
-    if (!aligned16(x) || !aligned16(w) || x_rs % 8 != 0 || x_rs < K || x_rs >= (1 << 22) || K >= (1 << 22) || !aligned16(out) || out_rs % 8 != 0 || out_rs < N)
+    if (!aligned16(x) || !aligned16(w) || x_rs * x_bytes % 16 != 0 || x_rs < K || x_rs >= (1 << 22) || K >= (1 << 22) || !aligned16(out) ||
+        out_rs * out_bytes % 16 != 0 || out_rs < N)
         return set_error(KERNL_ERR_UNSUPPORTED, "%s: x, w and out need 16-byte aligned rows", what);
     if (M > 0 && kernl_linear_norm_kind(M, N, K) == 0)
-        return set_error(KERNL_ERR_UNSUPPORTED, "%s: M=%lld N=%lld K=%lld is not a small problem (kernl_linear_norm_kind)", what, (long long)M,
-                         (long long)N, (long long)K);
+        return set_error(KERNL_ERR_UNSUPPORTED, "%s: M=%lld N=%lld K=%lld is not a problem of few rows (kernl_linear_norm_kind)", what,
+                         (long long)M, (long long)N, (long long)K);
     return KERNL_OK;
 }
 
-extern "C" int kernl_linear_norm_apply_fwd(const void *x, const float *x_stats, float eps, const void *w_folded, const float *colsum,
-                                           const float *bias32, void *out, int64_t M, int64_t N, int64_t K, int64_t x_row_stride,
+static kernl::LinearArgs norm_linear_args(const void *x, const void *w, const void *bias, void *out, int64_t M, int64_t N, int64_t K, int64_t x_rs,
+                                          int64_t out_rs, int act, void *stream) {
+    kernl::LinearArgs a;
+    a.x = x; a.w = w; a.bias = bias; a.out = out; a.act_in = nullptr;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K;
+    a.x_rs = x_rs; a.x_cs = 1; a.out_rs = out_rs; a.out_cs = 1; a.ai_rs = a.ai_cs = 0;
+    a.act = act; a.st = static_cast<hipStream_t>(stream);
+    return a;
+}
+
+extern "C" int kernl_linear_norm_apply_fwd(const float *x, const float *x_stats, const void *gamma, const void *beta, float eps, const void *w,
+                                           const void *bias, void *out, int64_t M, int64_t N, int64_t K, int64_t x_row_stride,
                                            int64_t out_row_stride, int activation, int dtype, void *stream) {
     using namespace kernl;
-    if (x_stats == nullptr || colsum == nullptr || bias32 == nullptr || !aligned16(x_stats) || !aligned16(colsum) || !aligned16(bias32))
-        return set_error(KERNL_ERR_INVALID_ARG, "linear (deferred norm): x_stats, colsum and bias32 must be 16-byte aligned fp32 arrays");
+    if (x_stats == nullptr || gamma == nullptr || !aligned16(x_stats) || !aligned16(gamma) || !aligned16(beta))
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (deferred norm): x_stats and the norm's parameters must be 16-byte aligned arrays");
     if (activation < KERNL_ACT_NONE || activation > KERNL_ACT_SILU)
         return set_error(KERNL_ERR_INVALID_ARG, "linear (deferred norm): unknown activation %d", activation);
-    const int bad = norm_arguments_bad("linear (deferred norm)", x, w_folded, out, M, N, K, x_row_stride, out_row_stride, dtype);
+    const int bad = norm_arguments_bad("linear (deferred norm)", x, 4, w, out, 2, M, N, K, x_row_stride, out_row_stride, dtype);
     if (bad != KERNL_OK) return bad;
-    if (K % kNormGroup != 0 || K > kNormGroup * kNormMaxGroups)
+    if (K % 32 != 0 || K > kNormGroup * kNormMaxGroups)
         return set_error(KERNL_ERR_UNSUPPORTED, "linear (deferred norm): normalised width %lld is no multiple of 32 up to 1024", (long long)K);
     if (M == 0) return KERNL_OK;
-    LinearArgs a;
-    a.x = x; a.w = w_folded; a.bias = nullptr; a.out = out; a.act_in = nullptr;
-    a.M = (int)M; a.N = (int)N; a.K = (int)K;
-    a.x_rs = x_row_stride; a.x_cs = 1; a.out_rs = out_row_stride; a.out_cs = 1; a.ai_rs = a.ai_cs = 0;
-    a.act = activation; a.st = static_cast<hipStream_t>(stream);
+    const LinearArgs a = norm_linear_args(x, w, bias, out, M, N, K, x_row_stride, out_row_stride, activation, stream);
     NormFold nf;
-    nf.stats_of(M, K); nf.in_stats = x_stats; nf.eps = eps; nf.colsum = colsum; nf.bias32 = bias32;
-    const int kind = norm_kind(M, N, K);
-    run_one_launch(a, dtype, norm_groups_fit(kind, nf.in_groups) ? kind : 11, kNormApply, nf);
+    nf.stats_of(K); nf.in_stats = x_stats; nf.eps = eps; nf.gamma = gamma; nf.beta = beta;
+    int rows, cols;
+    dealt_tile(a.M, a.N, norm_kind(M, N, K), rows, cols);
+    run_norm_apply(a, dtype, rows, cols, nf);
     return check_launch("linear (deferred norm)");
 }
 
 extern "C" int kernl_linear_norm_add_fwd(const void *x, const void *w, const void *bias, const void *residual, const float *residual_stats,
-                                         const void *gamma, const void *beta, float eps, void *out, float *out_stats, int64_t M, int64_t N,
+                                         const void *gamma, const void *beta, float eps, float *out, float *out_stats, int64_t M, int64_t N,
                                          int64_t K, int64_t x_row_stride, int64_t out_row_stride, int64_t residual_row_stride, int dtype,
                                          void *stream) {
     using namespace kernl;
-    if (residual == nullptr || out_stats == nullptr || !aligned16(residual) || residual_row_stride % 8 != 0 || !aligned16(out_stats))
+    if (residual == nullptr || out_stats == nullptr || !aligned16(residual) || residual_row_stride * (residual_stats != nullptr ? 4 : 2) % 16 != 0 ||
+        !aligned16(out_stats))
         return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: residual needs 16-byte aligned rows, out_stats a 16-byte aligned array");
     if (residual_stats != nullptr && (gamma == nullptr || !aligned16(residual_stats) || !aligned16(gamma) || !aligned16(beta)))
         return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: a deferred residual comes with its statistics and aligned norm parameters");
-    const int bad = norm_arguments_bad("linear + addition + statistics", x, w, out, M, N, K, x_row_stride, out_row_stride, dtype);
+    const int bad = norm_arguments_bad("linear + addition + statistics", x, 2, w, out, 4, M, N, K, x_row_stride, out_row_stride, dtype);
     if (bad != KERNL_OK) return bad;
     if (N > kNormGroup * kNormMaxGroups)
         return set_error(KERNL_ERR_UNSUPPORTED, "linear + addition + statistics: width %lld exceeds 1024", (long long)N);
     if (M == 0) return KERNL_OK;
-    LinearArgs a;
-    a.x = x; a.w = w; a.bias = bias; a.out = out; a.act_in = nullptr;
-    a.M = (int)M; a.N = (int)N; a.K = (int)K;
-    a.x_rs = x_row_stride; a.x_cs = 1; a.out_rs = out_row_stride; a.out_cs = 1; a.ai_rs = a.ai_cs = 0;
-    a.act = KERNL_ACT_NONE; a.st = static_cast<hipStream_t>(stream);
+    const LinearArgs a = norm_linear_args(x, w, bias, out, M, N, K, x_row_stride, out_row_stride, KERNL_ACT_NONE, stream);
     NormFold nf;
-    nf.stats_of(M, N); nf.in_stats = residual_stats; nf.eps = eps;
+    nf.stats_of(N); nf.in_stats = residual_stats; nf.eps = eps;
     nf.residual = residual; nf.res_rs = residual_row_stride; nf.gamma = gamma; nf.beta = beta; nf.out_stats = out_stats;
-    const int kind = norm_kind(M, N, K);
-    run_one_launch(a, dtype, norm_groups_fit(kind, nf.in_groups) ? kind : 11, kNormAdd, nf);
+    run_small_dealt(a, dtype, 16, 16, kNormAdd, nf);
     return check_launch("linear + addition + statistics");
 }
 

@@ -32,11 +32,13 @@ void run_wide_w8(const LinearArgs &a);                               // fp8 e5m2
 void run_wide_half(const LinearArgs &a, int dtype, int cols);        // 128-row tiles
 void run_wide_half_w8(const LinearArgs &a);
 void run_half_split(const LinearArgs &a, const HalfSplitPlan &p, float *part, int dtype);
-struct NormFold;
-void run_small(const LinearArgs &a, int dtype, int mode, const NormFold &nf);  // mode: norm_fold.h; 32 x 64 tiles over the whole K (linear_small.hip)
+void run_small(const LinearArgs &a, int dtype);                      // 32 x 64 tiles over the whole K (linear_small.hip)
 // 8-wave tiles over the whole K (linear_mid.hip), by hook value 11, 15, 17 .. 21; 0: that tile does not take the epilogue asked for
-int run_mid(const LinearArgs &a, int dtype, int kind, int mode, const NormFold &nf);
-void run_small_dealt(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf);      // 16- to 64-row, 16- or 32-column tiles, k-tiles dealt to the waves
+int run_mid(const LinearArgs &a, int dtype, int kind);
+struct NormFold;
+// 16- to 64-row, 16- or 32-column tiles, k-tiles dealt to the waves; mode: norm_fold.h (kNormAdd: a.out is fp32)
+void run_small_dealt(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf);
+void run_norm_apply(const LinearArgs &a, int dtype, int rows, int cols, const NormFold &nf);  // a.x is fp32 rows to be normalised
 
 
 // ----------------------------------------------------------------------------------------------------

@@ -45,12 +45,12 @@ __device__ __forceinline__ int mid_weight_row(int row) {
     return 64 * (c >> 5) + (c & 31) + 32 * (j / (H > 0 ? H : 1));
 }
 
-template <typename T, typename Cfg, bool GATED, int MODE>
+template <typename T, typename Cfg, bool GATED>
 __global__ void __launch_bounds__(512, 2)
 linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
                   T *__restrict__ act_in, const float *__restrict__ row_scale, const T *__restrict__ residual, int M, int N, int K,
                   int64_t ldx, int64_t out_rs, int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int64_t res_rs, int64_t res_cs, int act,
-                  int tiles_m, MidGrid grid, NormFold nf) {
+                  int tiles_m, MidGrid grid) {
     typedef typename Vec8<T>::type vec8;
     constexpr int BM = Cfg::BM, BN = Cfg::BN, S = Cfg::S, NBM = Cfg::NBM, NBN = Cfg::NBN, STAGE = Cfg::STAGE, L = Cfg::L;
     constexpr int LX = Cfg::LX, LW = Cfg::LW, BK = Cfg::BK;
@@ -137,75 +137,16 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     const int out_n = GATED ? N / 2 : N;
     const int n_first = (GATED ? n0 / 2 : n0) + wave_n * (GATED ? Cfg::TN / 2 : Cfg::TN) + C * g;
     float bz[NBN][4];
-    f32x4 cs[MODE == kNormApply ? NBN : 1];
     const bool bias_vec = ((uintptr_t)bias & 7) == 0;
 #pragma unroll
-    for (int j = 0; j < NBN; ++j) {
-        const int n = n0 + mid_weight_row<GATED, Cfg::TN>(wave_n * Cfg::TN + 16 * j + 4 * g);
-        if (MODE == kNormApply) {
-            const bool in = n < N;  // (N is a multiple of 32 with a norm)
-            const f32x4 b32 = in ? *reinterpret_cast<const f32x4 *>(nf.bias32 + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            cs[j] = in ? *reinterpret_cast<const f32x4 *>(nf.colsum + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) bz[j][e] = b32[e];
-        } else {
-            load_bias4<T>(bias, n, N, bias_vec, bz[j]);
-        }
-    }
-    static_assert(MODE == kNormNone || (!GATED && Cfg::TN == kNormGroup), "with a norm a wave's columns are one statistics group");
-    const bool row_stats = MODE == kNormApply || (MODE == kNormAdd && nf.in_stats != nullptr);
-    words res[MODE == kNormAdd ? NBM : 1], gam = {}, bet = {};
-    if (MODE == kNormAdd) {
-#pragma unroll
-        for (int i = 0; i < NBM; ++i) {
-            const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
-            res[i] = m < M && n_first < N ? *reinterpret_cast<const words *>(static_cast<const T *>(nf.residual) + (int64_t)m * nf.res_rs + n_first) : words{};
-        }
-        if (row_stats && n_first < N) {
-            gam = *reinterpret_cast<const words *>(static_cast<const T *>(nf.gamma) + n_first);
-            if (nf.beta != nullptr) bet = *reinterpret_cast<const words *>(static_cast<const T *>(nf.beta) + n_first);
-        }
-    }
+    for (int j = 0; j < NBN; ++j)
+        load_bias4<T>(bias, n0 + mid_weight_row<GATED, Cfg::TN>(wave_n * Cfg::TN + 16 * j + 4 * g), N, bias_vec, bz[j]);
     auto wait_loads = [&](auto n_c) __attribute__((always_inline)) {
         constexpr int n = decltype(n_c)::value;
         __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
     };
-    // Row statistics: the pairs of the tile's rows lie in one piece of memory.  They travel to the last stage of the ring, in front of
-    // the tiles, are merged by 512 / BM threads a row while the first k-tiles are on their way, and leave (mean, 1 / std) in LDS.
-    __shared__ f32x2 row_norm[MODE != kNormNone ? BM : 1];
-    if (MODE != kNormNone && row_stats) {
-        const uint64_t addr = (uint64_t)(uintptr_t)(nf.in_stats + (int64_t)m0 * nf.in_groups * 2);
-        const int bytes = rows_x * nf.in_groups * 8;
-        const u32x4 rsrc = {(uint32_t)addr, (uint32_t)(addr >> 32) & 0xFFFFu, (uint32_t)bytes, 0x00020000u};
-        for (int piece = wave; piece * 1024 < bytes; piece += 8)
-            load1(rsrc, piece * 1024 + lane * 16, lds_base - wave * 1024 + (S - 1) * STAGE + piece * 1024, 0);
-    }
 #pragma unroll
-    for (int kt = 0; kt < S - 1; ++kt) request(kt, kt);
-    if (MODE != kNormNone && row_stats) {
-        wait_loads(IntC<(S - 1) * L>());
-        __syncthreads();
-        constexpr int LPR = 512 / BM;  // lanes of a row: 4 or 8
-        constexpr int PER = kNormMaxGroups / LPR;
-        const int row = tid / LPR, c = tid % LPR;
-        const f32x2 *pairs = reinterpret_cast<const f32x2 *>(smem + (S - 1) * STAGE) + row * nf.in_groups;
-        f32x2 v[PER];
-#pragma unroll
-        for (int i = 0; i < PER; ++i) v[i] = pairs[c + LPR * i < nf.in_groups ? c + LPR * i : 0];
-        const float pivot = pairs[0][0] * nf.inv_group;
-        NormMerge mg;
-#pragma unroll
-        for (int i = 0; i < PER; ++i)
-            if (c + LPR * i < nf.in_groups) mg.take(v[i], pivot, nf.inv_group);
-        auto lpr_sum = [](float x) __attribute__((always_inline)) { return LPR == 8 ? oct_sum(x) : quad_sum(x); };
-        mg.d = lpr_sum(mg.d);
-        mg.dd = lpr_sum(mg.dd);
-        mg.m2 = lpr_sum(mg.m2);
-        const f32x2 norm = mg.finish(pivot, nf);
-        if (c == 0) row_norm[row] = norm;
-        __syncthreads();  // the stage is free
-    }
-    request(S - 1, S - 1);
+    for (int kt = 0; kt < S; ++kt) request(kt, kt);
 
     vec8 xf[2][NBM], wf[2][NBN];
     auto read = [&](int st, int stage) __attribute__((always_inline)) {
@@ -244,69 +185,6 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     __builtin_amdgcn_s_waitcnt(0x0F70);
 
     // ---- epilogue
-    if (MODE != kNormNone) {
-        auto finish_norm = [&](auto act_c) __attribute__((always_inline)) {
-            constexpr int ACT = decltype(act_c)::value;
-            float gm[8], bt[8];
-            if (MODE == kNormAdd) {
-                unpack4<T>(u32x2{gam[0], gam[1]}, gm);
-                unpack4<T>(u32x2{gam[2 % (V / 2)], gam[3 % (V / 2)]}, gm + 4);
-                unpack4<T>(u32x2{bet[0], bet[1]}, bt);
-                unpack4<T>(u32x2{bet[2 % (V / 2)], bet[3 % (V / 2)]}, bt + 4);
-            }
-#pragma unroll
-            for (int i = 0; i < NBM; ++i) {
-                const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
-                float mean = 0.0f, rstd = 0.0f;
-                if (row_stats) {
-                    const f32x2 norm = row_norm[wave_m * Cfg::TM + 16 * i + r];
-                    mean = norm[0];
-                    rstd = norm[1];
-                }
-                float y[8], h[8] = {};
-                if (MODE == kNormAdd) {
-                    unpack4<T>(u32x2{res[i][0], res[i][1]}, h);
-                    unpack4<T>(u32x2{res[i][2 % (V / 2)], res[i][3 % (V / 2)]}, h + 4);
-                    if (row_stats)
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) h[e] = fmaf((h[e] - mean) * rstd, gm[e], bt[e]);
-                }
-                float sum = 0.0f, m2 = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float a = acc[i][(e >> 2) % NBN][e & 3];
-                    if (MODE == kNormApply) y[e] = apply_act16(fmaf(fmaf(-mean, cs[(e >> 2) % NBN][e & 3], a), rstd, bz[(e >> 2) % NBN][e & 3]), ACT);
-                    else y[e] = to_float(from_float<T>(a + bz[(e >> 2) % NBN][e & 3] + h[e]));
-                    sum += y[e];
-                }
-                const bool in = m < M && n_first < N;
-                if (in)
-                    *reinterpret_cast<u32x4 *>(out + (int64_t)m * out_rs + n_first) =
-                        u32x4{pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3]), pack2<T>(y[4], y[5]), pack2<T>(y[6], y[7])};
-                if (MODE == kNormAdd) {
-                    sum = halves32_sum(sum + __shfl_xor(sum, 16));
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) m2 = fmaf(y[e] - sum * (1.0f / kNormGroup), y[e] - sum * (1.0f / kNormGroup), m2);
-                    m2 = halves32_sum(m2 + __shfl_xor(m2, 16));
-                    if (g == 0 && in)
-                        *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / kNormGroup) + n_first / kNormGroup) * 2) = f32x2{sum, m2};
-                }
-            }
-        };
-        if (MODE == kNormAdd) {
-            finish_norm(IntC<KERNL_ACT_NONE>());
-            return;
-        }
-        switch (act) {
-            case KERNL_ACT_RELU: finish_norm(IntC<KERNL_ACT_RELU>()); break;
-            case KERNL_ACT_TANH: finish_norm(IntC<KERNL_ACT_TANH>()); break;
-            case KERNL_ACT_GELU_ERF: finish_norm(IntC<KERNL_ACT_GELU_ERF>()); break;
-            case KERNL_ACT_GELU_TANH: finish_norm(IntC<KERNL_ACT_GELU_TANH>()); break;
-            case KERNL_ACT_SILU: finish_norm(IntC<KERNL_ACT_SILU>()); break;
-            default: finish_norm(IntC<KERNL_ACT_NONE>()); break;
-        }
-        return;
-    }
     const bool out_vec = out_cs == 1 && (out_rs & (V - 1)) == 0 && ((uintptr_t)out & (2 * V - 1)) == 0;
     const bool ai_vec = act_in != nullptr && ai_cs == 1 && (ai_rs & (V - 1)) == 0 && ((uintptr_t)act_in & (2 * V - 1)) == 0;
     const bool res_vec = residual != nullptr && res_cs == 1 && (res_rs & (V - 1)) == 0 && ((uintptr_t)residual & (2 * V - 1)) == 0;
@@ -371,9 +249,9 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     }
 }
 
-template <typename T, typename Cfg, bool GATED, int MODE = kNormNone>
-static void launch_mid_cfg(const LinearArgs &a, const NormFold &nf = NormFold()) {
-    auto kern = linear_mid_kernel<T, Cfg, GATED, MODE>;
+template <typename T, typename Cfg, bool GATED>
+static void launch_mid_cfg(const LinearArgs &a) {
+    auto kern = linear_mid_kernel<T, Cfg, GATED>;
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);
@@ -395,7 +273,7 @@ static void launch_mid_cfg(const LinearArgs &a, const NormFold &nf = NormFold())
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(512), Cfg::LDS, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out), static_cast<T *>(a.act_in),
                        a.row_scale, static_cast<const T *>(a.residual), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs,
-                       a.res_rs, a.res_cs, a.act & (kGluBit - 1), tiles_m, grid, nf);
+                       a.res_rs, a.res_cs, a.act & (kGluBit - 1), tiles_m, grid);
 }
 
 // the tiles, by the kernl_linear_force_tile value that forces them
@@ -408,15 +286,7 @@ typedef MidTile<128, 256, 2, 4, 3> Mid128x256;  // 20
 typedef MidTile<256, 128, 4, 2, 3> Mid256x128;  // 21
 
 template <typename T, typename Cfg>
-static int launch_mid(const LinearArgs &a, int mode, const NormFold &nf) {
-    if (mode != kNormNone) {
-        if constexpr (Cfg::TN == kNormGroup) {
-            if (mode == kNormApply) launch_mid_cfg<T, Cfg, false, kNormApply>(a, nf);
-            else launch_mid_cfg<T, Cfg, false, kNormAdd>(a, nf);
-            return 1;
-        }
-        return 0;
-    }
+static int launch_mid(const LinearArgs &a) {
     if (a.act & kGluBit) {
         if constexpr (Cfg::NBN % 2 == 0) {
             launch_mid_cfg<T, Cfg, true>(a);
@@ -429,21 +299,19 @@ static int launch_mid(const LinearArgs &a, int mode, const NormFold &nf) {
 }
 
 template <typename T>
-static int run_mid_t(const LinearArgs &a, int kind, int mode, const NormFold &nf) {
+static int run_mid_t(const LinearArgs &a, int kind) {
     switch (kind) {
-        case 11: return launch_mid<T, Mid64x64>(a, mode, nf);
-        case 15: return launch_mid<T, Mid128x64>(a, mode, nf);
-        case 17: return launch_mid<T, Mid128x128>(a, mode, nf);
-        case 18: return launch_mid<T, Mid192x128>(a, mode, nf);
-        case 19: return launch_mid<T, Mid192x192>(a, mode, nf);
-        case 20: return launch_mid<T, Mid128x256>(a, mode, nf);
-        case 21: return launch_mid<T, Mid256x128>(a, mode, nf);
+        case 11: return launch_mid<T, Mid64x64>(a);
+        case 15: return launch_mid<T, Mid128x64>(a);
+        case 17: return launch_mid<T, Mid128x128>(a);
+        case 18: return launch_mid<T, Mid192x128>(a);
+        case 19: return launch_mid<T, Mid192x192>(a);
+        case 20: return launch_mid<T, Mid128x256>(a);
+        case 21: return launch_mid<T, Mid256x128>(a);
         default: return 0;
     }
 }
 
-int run_mid(const LinearArgs &a, int dtype, int kind, int mode, const NormFold &nf) {
-    return dtype == KERNL_F16 ? run_mid_t<f16>(a, kind, mode, nf) : run_mid_t<bf16>(a, kind, mode, nf);
-}
+int run_mid(const LinearArgs &a, int dtype, int kind) { return dtype == KERNL_F16 ? run_mid_t<f16>(a, kind) : run_mid_t<bf16>(a, kind); }
 
 }  // namespace kernl

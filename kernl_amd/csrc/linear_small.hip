@@ -3,12 +3,12 @@
 // split kernels pay for a second launch and for partial tiles larger than the output.
 //
 // Same operator as the other kernels (reference: `kernel_fma`, src/kernl/implementations/linear_layer.py:92-210 —
-// C = act(A @ W^T + bias), optional store of the pre-activation); what differs is the shape of the work.  A workgroup of
-// 4 waves (2 x 2) owns a 64 x 64 or 32 x 64 output tile over the WHOLE of K: one launch, no partial sums in memory,
-// 50 to 256 workgroups.  Such a tile is 4 or 8 MFMAs per wave and 64-wide k-tile — the loop is bound by how fast the
-// CU can pull its operand tiles (12 KB per k-tile) out of L2, i.e. by latency unless many k-tiles are in
-// flight: operand tiles travel HBM/L2 -> LDS directly (buffer loads with the LDS flag, every lane fetching the 16-byte
-// chunk that belongs at its LDS position under the XOR swizzle) through a ring of 8 stages, 7 k-tiles requested
+// C = act(A @ W^T + bias), optional store of the pre-activation); what differs is the shape of the work.  A workgroup
+// owns a small output tile — 32 x 64 here, 16 x 16 to 64 x 32 in the kernel below — over the WHOLE of K: one launch, no
+// partial sums in memory, 50 to 256 workgroups.  Such a tile is a few MFMAs per wave and 64-wide k-tile — the loop is
+// bound by how fast the CU can pull its operand tiles (12 KB per k-tile of 32 x 64) out of L2, i.e. by latency unless many
+// k-tiles are in flight: operand tiles travel HBM/L2 -> LDS directly (buffer loads with the LDS flag, every lane fetching the
+// 16-byte chunk that belongs at its LDS position under the XOR swizzle) through a ring of 8 stages, 7 k-tiles requested
 // ahead, one barrier per k-tile and waits by count.  A last k-tile that reaches beyond K has the chunks that
 // start there pointed out of range (zeros, in both operands).
 #include "linear_kernels.h"
@@ -16,9 +16,9 @@
 
 namespace kernl {
 
-// Row statistics on their way to the epilogue: the pairs of a row tile lie in one piece of memory and travel to LDS in
-// front of the first k-tile, `per_wave` KB-sized loads per wave (pieces past the end arrive as zeros or are not asked for).
-constexpr int norm_stats_bytes(int bm) { return bm * 8 * (bm <= 32 ? 2 * kNormMaxGroups : kNormMaxGroups); }
+// Row statistics of a deferred norm: the pairs of a row tile lie in one piece of memory and travel to LDS in front of
+// everything else, `per_wave` KB-sized loads per wave (pieces past the end arrive as zeros or are not asked for).
+constexpr int norm_stats_bytes(int bm) { return bm * 8 * kNormMaxGroups; }
 template <int BM, int WAVES>
 __device__ __forceinline__ void request_norm_stats(const NormFold &nf, int m0, int rows, uint32_t lds, int wave, int lane) {
     constexpr int PER_WAVE = norm_stats_bytes(BM) / 1024 / WAVES;
@@ -33,23 +33,49 @@ __device__ __forceinline__ void request_norm_stats(const NormFold &nf, int m0, i
                          :: "s"(lds + piece * 1024), "v"(piece * 1024 + lane * 16), "s"(rsrc) : "memory", "m0");
     }
 }
+// The staged pairs (at `staged`) merged by up to 16 threads a row: (mean, 1 / std) of row i of the tile to row_norm[i].
+template <int BM, int WAVES>
+__device__ __forceinline__ void merge_norm_stats(const NormFold &nf, const unsigned char *staged, f32x2 *row_norm, int tid) {
+    constexpr int SPAN = 64 * WAVES / BM < 16 ? 64 * WAVES / BM : 16, PER = kNormMaxGroups / SPAN;
+    static_assert(SPAN == 8 || SPAN == 16, "the lanes of a row are a DPP group");
+    const int row = tid / SPAN, c = tid % SPAN;
+    if (row >= BM) return;
+    const f32x2 *pairs = reinterpret_cast<const f32x2 *>(staged) + row * nf.in_groups;
+    const float pivot = pairs[0][0] * NormMerge::kInvGroup;
+    NormMerge mg;
+    auto merge = [&](int first, int last) __attribute__((always_inline)) {
+        f32x2 v[PER];  // (read together: one after the other each costs an LDS round trip)
+#pragma unroll
+        for (int q = first; q < last; ++q) v[q] = pairs[SPAN * q + c < nf.in_groups ? SPAN * q + c : 0];
+#pragma unroll
+        for (int q = first; q < last; ++q)
+            if (SPAN * q + c < nf.in_groups) mg.take(v[q], pivot);
+    };
+    merge(0, PER / 2);
+    if (SPAN * (PER / 2) < nf.in_groups) merge(PER / 2, PER);
+    auto span_sum = [](float x) __attribute__((always_inline)) { return SPAN == 16 ? row16_sum(x) : oct_sum(x); };
+    mg.d = span_sum(mg.d);
+    mg.dd = span_sum(mg.dd);
+    mg.m2 = span_sum(mg.m2);
+    if (c == 0) row_norm[row] = mg.finish(pivot, nf);
+}
 
 constexpr int kSmallBK = 64;  // measured against 128-wide k-tiles in 6 / 4 stages: 5-10 % faster
 // ring stages of the shared-tile kernel: 8 of them, or as many as fit 144 KB
 constexpr int small_stages(int bm, int bn) { return (bm + bn) * kSmallBK * 2 * 8 <= 144 * 1024 ? 8 : (144 * 1024) / ((bm + bn) * kSmallBK * 2); }
 
-template <typename T, int BM, int BN, int MODE>
+template <typename T, int BM, int BN>
 __global__ void __launch_bounds__(256, 1)
 linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
                     T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs, int64_t out_cs,
-                    int64_t ai_rs, int64_t ai_cs, int act, int tiles_m, NormFold nf) {
+                    int64_t ai_rs, int64_t ai_cs, int act, int tiles_m) {
     typedef typename Vec8<T>::type vec8;
     constexpr int BK = kSmallBK, RB = BK * 2, CPR = BK / 8, S = small_stages(BM, BN), KSTEPS = BK / 32;
     static_assert(RB == SmallTileMap::ROW_BYTES && CPR == SmallTileMap::CHUNKS_PER_ROW, "tile rows as the tile map lays them out");
     constexpr int X_BYTES = BM * RB, W_BYTES = BN * RB, STAGE = X_BYTES + W_BYTES;
     constexpr int LX = BM * CPR / 256, LW = BN * CPR / 256, L = LX + LW;  // 1 KB loads per wave... per thread and stage
     constexpr int NBM = BM / 32, NBN = BN / 32;                            // 16 x 16 blocks per wave: rows of x, rows of w
-    static_assert((BM == 32 || BM == 64) && (BN == 64 || BN == 128), "tile shapes");
+    static_assert(BM == 32 && BN == 64, "tile shape");
     static_assert(S >= 3 && (S - 2) * L <= 63, "ring depth; the wait count must be encodable");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -141,38 +167,12 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
     for (int i = 0; i < NBM; ++i)
 #pragma unroll
         for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
-    // what the epilogue needs of the lane's rows and columns, requested before anything else: fetched where it is used,
-    // every block of the epilogue would cost the wave a memory round trip of its own
+    // the bias, requested before anything else: fetched where it is used, every block of the epilogue would cost the wave a
+    // memory round trip of its own
     float bz[NBN][4];
-    f32x4 cs[MODE == kNormApply ? NBN : 1];
-    u32x2 res[MODE == kNormAdd ? NBM : 1][MODE == kNormAdd ? NBN : 1], gam[MODE == kNormAdd ? NBN : 1], bet[MODE == kNormAdd ? NBN : 1];
     const bool bias_vec = ((uintptr_t)bias & 7) == 0;
 #pragma unroll
-    for (int j = 0; j < NBN; ++j) {
-        const int n = n0 + wave_n * (BN / 2) + 16 * j + 4 * g;
-        if (MODE == kNormApply) {
-            const bool in = n < N;  // (N is a multiple of 32 with a norm)
-            const f32x4 b32 = in ? *reinterpret_cast<const f32x4 *>(nf.bias32 + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            cs[j] = in ? *reinterpret_cast<const f32x4 *>(nf.colsum + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) bz[j][e] = b32[e];
-        } else {
-            load_bias4<T>(bias, n, N, bias_vec, bz[j]);
-        }
-        if (MODE == kNormAdd) {
-#pragma unroll
-            for (int i = 0; i < NBM; ++i) {
-                const int m = m0 + wave_m * (BM / 2) + 16 * i + r;
-                res[i][j] = m < M && n < N ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + (int64_t)m * nf.res_rs + n) : u32x2{0, 0};
-            }
-            if (nf.in_stats != nullptr) {
-                gam[j] = n < N ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.gamma) + n) : u32x2{0, 0};
-                bet[j] = n < N && nf.beta != nullptr ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.beta) + n) : u32x2{0, 0};
-            }
-        }
-    }
-    const bool row_stats = MODE == kNormApply || (MODE == kNormAdd && nf.in_stats != nullptr);
-    if (MODE != kNormNone && row_stats) request_norm_stats<BM, 4>(nf, m0, rows_x, lds_base + S * STAGE, wave, lane);
+    for (int j = 0; j < NBN; ++j) load_bias4<T>(bias, n0 + wave_n * (BN / 2) + 16 * j + 4 * g, N, bias_vec, bz[j]);
 
 #pragma unroll
     for (int kt = 0; kt < S - 1; ++kt) request(kt, kt);
@@ -201,96 +201,6 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
         stage = stage == S - 1 ? 0 : stage + 1;
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the out-of-range requests of the last rounds are done with before the LDS goes away
-
-    if (MODE != kNormNone) {
-        // mean and 1 / std of the lane's rows: the four lanes of a row take a quarter of its statistics pairs each
-        float mean[NBM], rstd[NBM];
-        if (row_stats) {
-            const unsigned char *st = smem + S * STAGE;
-            const int groups = nf.in_groups;
-#pragma unroll
-            for (int i = 0; i < NBM; ++i) {
-                const f32x2 *row = reinterpret_cast<const f32x2 *>(st) + (wave_m * (BM / 2) + 16 * i + r) * groups;
-                const float pivot = row[0][0] * nf.inv_group;
-                NormMerge mg;
-                f32x2 pairs[kNormMaxGroups / 2];  // (read together: one after the other each costs an LDS round trip)
-#pragma unroll
-                for (int q = 0; q < kNormMaxGroups / 2; ++q) pairs[q] = row[4 * q + g < groups ? 4 * q + g : 0];
-#pragma unroll
-                for (int q = 0; q < kNormMaxGroups / 2; ++q)
-                    if (4 * q + g < groups) mg.take(pairs[q], pivot, nf.inv_group);
-                mg.d = halves32_sum(mg.d + __shfl_xor(mg.d, 16));
-                mg.dd = halves32_sum(mg.dd + __shfl_xor(mg.dd, 16));
-                mg.m2 = halves32_sum(mg.m2 + __shfl_xor(mg.m2, 16));
-                const f32x2 norm = mg.finish(pivot, nf);
-                mean[i] = norm[0];
-                rstd[i] = norm[1];
-            }
-        }
-        auto finish_norm = [&](auto act_c) __attribute__((always_inline)) {
-            constexpr int ACT = decltype(act_c)::value;
-#pragma unroll
-            for (int i = 0; i < NBM; ++i) {
-                const int m = m0 + wave_m * (BM / 2) + 16 * i + r;
-                float y[NBN][4];
-#pragma unroll
-                for (int j = 0; j < NBN; ++j) {
-                    const int n = n0 + wave_n * (BN / 2) + 16 * j + 4 * g;
-                    float h[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if (MODE == kNormAdd) {
-                        unpack4<T>(res[i][j], h);
-                        if (row_stats) {
-                            float gm[4], bt[4];
-                            unpack4<T>(gam[j], gm);
-                            unpack4<T>(bet[j], bt);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) h[e] = fmaf((h[e] - mean[i]) * rstd[i], gm[e], bt[e]);
-                        }
-                    }
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (MODE == kNormApply) y[j][e] = apply_act16(fmaf(fmaf(-mean[i], cs[j][e], acc[i][j][e]), rstd[i], bz[j][e]), ACT);
-                        else y[j][e] = to_float(from_float<T>(acc[i][j][e] + bz[j][e] + h[e]));
-                    }
-                    if (m < M && n < N)
-                        *reinterpret_cast<u32x2 *>(out + (int64_t)m * out_rs + n) = u32x2{pack2<T>(y[j][0], y[j][1]), pack2<T>(y[j][2], y[j][3])};
-                }
-                if (MODE == kNormAdd) {
-                    // statistics of the stored values: 32 columns are two blocks of the row's four lanes
-#pragma unroll
-                    for (int j = 0; j < NBN; j += 2) {
-                        float sum = 0.0f, m2 = 0.0f;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) sum += y[j][e] + y[j + 1][e];
-                        sum = halves32_sum(sum + __shfl_xor(sum, 16));
-                        const float mu = sum * (1.0f / kNormGroup);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float a = y[j][e] - mu, b = y[j + 1][e] - mu;
-                            m2 = fmaf(a, a, fmaf(b, b, m2));
-                        }
-                        m2 = halves32_sum(m2 + __shfl_xor(m2, 16));
-                        const int n = n0 + wave_n * (BN / 2) + 16 * j;
-                        if (g == 0 && m < M && n < N)
-                            *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / kNormGroup) + n / kNormGroup) * 2) = f32x2{sum, m2};
-                    }
-                }
-            }
-        };
-        if (MODE == kNormAdd) {
-            finish_norm(IntC<KERNL_ACT_NONE>());
-            return;
-        }
-        switch (act) {
-            case KERNL_ACT_RELU: finish_norm(IntC<KERNL_ACT_RELU>()); break;
-            case KERNL_ACT_TANH: finish_norm(IntC<KERNL_ACT_TANH>()); break;
-            case KERNL_ACT_GELU_ERF: finish_norm(IntC<KERNL_ACT_GELU_ERF>()); break;
-            case KERNL_ACT_GELU_TANH: finish_norm(IntC<KERNL_ACT_GELU_TANH>()); break;
-            case KERNL_ACT_SILU: finish_norm(IntC<KERNL_ACT_SILU>()); break;
-            default: finish_norm(IntC<KERNL_ACT_NONE>()); break;
-        }
-        return;
-    }
 
     // ---- epilogue: bias, optional pre-activation, activation, one rounding; 4 consecutive columns per lane and block
     const bool out_vec = out_cs == 1 && (out_rs & 3) == 0 && ((uintptr_t)out & 7) == 0;
@@ -440,36 +350,34 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
         for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
 
     // In the epilogue LPR = BN / 4 neighbouring lanes finish a row of the tile, 4 columns each: whole row pieces per store, and
-    // a row's columns meet in neighbouring lanes (statistics).  What a thread needs of its row and columns is requested before
-    // anything else.
+    // a statistics group is four neighbouring lanes.  What a thread needs of its row and columns is requested before anything else.
     constexpr int LPR = BN / 4, ROWS = 64 * WAVES / LPR, OWN = (BM + ROWS - 1) / ROWS;
     const int own_row = tid / LPR, own_c = tid % LPR, n_own = n0 + 4 * own_c;
-    auto lpr_sum = [](float v) __attribute__((always_inline)) { return LPR == 8 ? oct_sum(v) : quad_sum(v); };
     float bz[4];
-    f32x4 cs = {0.0f, 0.0f, 0.0f, 0.0f};
-    u32x2 res[OWN], gam = {0, 0}, bet = {0, 0};
-    if (MODE == kNormApply) {  // (N is a multiple of 32 with a norm: every column of the tile exists)
-        const f32x4 b32 = *reinterpret_cast<const f32x4 *>(nf.bias32 + n_own);
-        cs = *reinterpret_cast<const f32x4 *>(nf.colsum + n_own);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bz[e] = b32[e];
-    } else {
-        load_bias4<T>(bias, n_own, N, ((uintptr_t)bias & 7) == 0, bz);
-    }
-    const bool row_stats = MODE == kNormApply || (MODE == kNormAdd && nf.in_stats != nullptr);
-    if (MODE == kNormAdd) {
+    load_bias4<T>(bias, n_own, N, ((uintptr_t)bias & 7) == 0, bz);
+    const bool row_stats = MODE == kNormAdd && nf.in_stats != nullptr;  // the residual is fp32 rows whose norm is to be applied
+    u32x4 res[OWN];  // raw: four fp32 values, or four 16-bit ones in the first half
+    u32x2 gam = {0, 0}, bet = {0, 0};
+    if (MODE == kNormAdd) {  // (N is a multiple of 32: every column of the tile exists)
 #pragma unroll
         for (int t = 0; t < OWN; ++t) {
-            const int m = m0 + own_row + ROWS * t;
-            res[t] = own_row + ROWS * t < rows_x ? *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + (int64_t)m * nf.res_rs + n_own) : u32x2{0, 0};
+            res[t] = u32x4{0, 0, 0, 0};
+            if (own_row + ROWS * t >= rows_x) continue;
+            const int64_t at = (int64_t)(m0 + own_row + ROWS * t) * nf.res_rs + n_own;
+            if (row_stats) {
+                res[t] = *reinterpret_cast<const u32x4 *>(static_cast<const float *>(nf.residual) + at);
+            } else {
+                const u32x2 half = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + at);
+                res[t][0] = half[0];
+                res[t][1] = half[1];
+            }
         }
         if (row_stats) {
             gam = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.gamma) + n_own);
             if (nf.beta != nullptr) bet = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.beta) + n_own);
+            request_norm_stats<BM, WAVES>(nf, m0, rows_x, (uint32_t)(uintptr_t)(lds_void *)smem + WAVES * RING, wave, lane);
         }
     }
-    if (MODE != kNormNone && row_stats)
-        request_norm_stats<BM, WAVES>(nf, m0, rows_x, (uint32_t)(uintptr_t)(lds_void *)smem + WAVES * RING, wave, lane);
     const int mine = nk > wave ? (nk - wave + WAVES - 1) / WAVES : 0;  // k-tiles of this wave
 #pragma unroll
     for (int j = 0; j < S - 1; ++j) request(j, j);
@@ -500,32 +408,12 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     __builtin_amdgcn_s_waitcnt(0x0F70);  // the out-of-range requests of the last rounds are done with
     __syncthreads();                     // every ring is free: the partial tiles take their place
 
-    // row statistics (staged behind the rings) merged by up to 16 threads a row, beside the stores of the partial tiles
+    // row statistics (staged behind the rings), merged beside the stores of the partial tiles
     f32x2 *row_norm = reinterpret_cast<f32x2 *>(smem + WAVES * RING) - BM;  // (the end of the rings, which the partial tiles leave free)
     static_assert(WAVES * NBM * NBN * 1024 + BM * 8 <= WAVES * RING, "room behind the partial tiles");
-    if (MODE != kNormNone && row_stats) {
-        constexpr int SPAN = 64 * WAVES / BM < 16 ? 64 * WAVES / BM : 16, PER = norm_stats_bytes(BM) / BM / 8 / SPAN;
-        const int row = tid / SPAN, c = tid % SPAN;
-        if (row < BM) {
-            const f32x2 *pairs = reinterpret_cast<const f32x2 *>(smem + WAVES * RING) + row * nf.in_groups;
-            const float pivot = pairs[0][0] * nf.inv_group;
-            NormMerge mg;
-            auto merge = [&](int first, int last) __attribute__((always_inline)) {
-                f32x2 v[PER];  // (read together: one after the other each costs an LDS round trip)
-#pragma unroll
-                for (int q = first; q < last; ++q) v[q] = pairs[SPAN * q + c < nf.in_groups ? SPAN * q + c : 0];
-#pragma unroll
-                for (int q = first; q < last; ++q)
-                    if (SPAN * q + c < nf.in_groups) mg.take(v[q], pivot, nf.inv_group);
-            };
-            merge(0, PER / 2);
-            if (SPAN * (PER / 2) < nf.in_groups) merge(PER / 2, PER);
-            auto span_sum = [](float x) __attribute__((always_inline)) { return SPAN == 16 ? row16_sum(x) : SPAN == 8 ? oct_sum(x) : quad_sum(x); };
-            mg.d = span_sum(mg.d);
-            mg.dd = span_sum(mg.dd);
-            mg.m2 = span_sum(mg.m2);
-            if (c == 0) row_norm[row] = mg.finish(pivot, nf);
-        }
+    if constexpr (MODE == kNormAdd) {
+        static_assert(BM == 16 && BN == kNormGroup, "a row of the tile is one statistics group");
+        if (row_stats) merge_norm_stats<BM, WAVES>(nf, smem + WAVES * RING, row_norm, tid);
     }
     float *red = reinterpret_cast<float *>(smem);  // [wave][block][lane][4]
 #pragma unroll
@@ -549,43 +437,44 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
 #pragma unroll
         for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_acc *>(red + w * (NBM * NBN) * 256 + at);
         const int m = m0 + row, n = n_own;
-        float pre[4], y[4], mean = 0.0f, rstd = 0.0f;
-        if (MODE != kNormNone && row_stats) {
-            const f32x2 norm = row_norm[row];
-            mean = norm[0];
-            rstd = norm[1];
-        }
+        float pre[4], y[4];
         if (MODE == kNormAdd) {
-            float h[4], gm[4], bt[4];
-            unpack4<T>(res[t], h);
+            // fp32 rows and the statistics of what is stored
+            f32x4 h = __builtin_bit_cast(f32x4, res[t]);
             if (row_stats) {
+                const f32x2 norm = row_norm[row];
+                float gm[4], bt[4];
                 unpack4<T>(gam, gm);
                 unpack4<T>(bet, bt);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) h[e] = fmaf((h[e] - mean) * rstd, gm[e], bt[e]);
+                for (int e = 0; e < 4; ++e) h[e] = fmaf((h[e] - norm[0]) * norm[1], gm[e], bt[e]);
+            } else {
+                float h16[4];
+                unpack4<T>(u32x2{res[t][0], res[t][1]}, h16);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) h[e] = h16[e];
             }
             float total = 0.0f, m2 = 0.0f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                y[e] = to_float(from_float<T>(sum[e] + bz[e] + h[e]));
+                y[e] = sum[e] + bz[e] + h[e];
                 total += y[e];
             }
-            // statistics of the stored values: the row's lanes, or with 16-column groups in 32-column tiles half of them
-            const bool halves = LPR == 8 && nf.group == kNormGroupFew;
-            const int cols = halves ? kNormGroupFew : BN;
-            total = halves ? quad_sum(total) : lpr_sum(total);
-            const float mu = total / (float)cols;
+            total = quad_sum(total);
+            const float mu = total * NormMerge::kInvGroup;
 #pragma unroll
             for (int e = 0; e < 4; ++e) m2 = fmaf(y[e] - mu, y[e] - mu, m2);
-            m2 = halves ? quad_sum(m2) : lpr_sum(m2);
-            if (own_c % (cols / 4) == 0 && m < M)
-                *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / cols) + n_own / cols) * 2) = f32x2{total, m2};
-        } else {
+            m2 = quad_sum(m2);
+            if (m >= M) continue;
+            *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(out) + (int64_t)m * out_rs + n) = f32x4{y[0], y[1], y[2], y[3]};
+            if (own_c % 4 == 0)
+                *reinterpret_cast<f32x2 *>(nf.out_stats + ((int64_t)m * (N / kNormGroup) + n / kNormGroup) * 2) = f32x2{total, m2};
+            continue;
+        }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                pre[e] = MODE == kNormApply ? fmaf(fmaf(-mean, cs[e], sum[e]), rstd, bz[e]) : sum[e] + bz[e];
-                y[e] = apply_act16(pre[e], ACT);
-            }
+        for (int e = 0; e < 4; ++e) {
+            pre[e] = sum[e] + bz[e];
+            y[e] = apply_act16(pre[e], ACT);
         }
         if (m >= M || n >= N) continue;
         if (n + 4 <= N && out_vec) {
@@ -596,7 +485,7 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
             for (int e = 0; e < 4; ++e)
                 if (n + e < N) out[(int64_t)m * out_rs + (int64_t)(n + e) * out_cs] = from_float<T>(y[e]);
         }
-        if (MODE == kNormNone && act_in != nullptr) {
+        if (act_in != nullptr) {
             if (n + 4 <= N && ai_vec) {
                 const u32x2 p = {pack2<T>(pre[0], pre[1]), pack2<T>(pre[2], pre[3])};
                 *reinterpret_cast<u32x2 *>(act_in + (int64_t)m * ai_rs + n) = p;
@@ -612,6 +501,145 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
         finish(IntC<KERNL_ACT_NONE>());
         return;
     }
+    switch (act) {
+        case KERNL_ACT_RELU: finish(IntC<KERNL_ACT_RELU>()); break;
+        case KERNL_ACT_TANH: finish(IntC<KERNL_ACT_TANH>()); break;
+        case KERNL_ACT_GELU_ERF: finish(IntC<KERNL_ACT_GELU_ERF>()); break;
+        case KERNL_ACT_GELU_TANH: finish(IntC<KERNL_ACT_GELU_TANH>()); break;
+        case KERNL_ACT_SILU: finish(IntC<KERNL_ACT_SILU>()); break;
+        default: finish(IntC<KERNL_ACT_NONE>()); break;
+    }
+}
+
+// The layer BEHIND a deferred norm: out = act(LN(x) W^T + bias) for up to 64 fp32 rows of up to 1024 columns, LN(x) rounded once to
+// the 16-bit operand (norm_fold.h).  The tiles and the dealt k-tiles of the kernel above; but x does not go through LDS: a lane
+// fetches the 8 columns of its rows that its matrix-instruction operand wants, normalises and packs them in registers.  A wave has at
+// most four k-tiles, all of which — weight, x, gamma and beta — are requested before anything is waited for: one trip to memory.
+constexpr int kApplyTiles = 4;  // k-tiles of a wave, as many as 1024 columns are
+
+template <typename T, int BM, int BN>
+__global__ void __launch_bounds__(256, 1)
+linear_norm_apply_kernel(const float *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out, int M,
+                         int N, int K, int64_t ldx, int64_t out_rs, int act, int tiles_m, NormFold nf) {
+    typedef typename Vec8<T>::type vec8;
+    constexpr int WAVES = 4, BK = 64, W_BYTES = BN * BK * 2, LW = BN / 8, NBM = BM / 16, NBN = BN / 16;
+    constexpr int TILES = WAVES * kApplyTiles * W_BYTES;
+    static_assert(WAVES * NBM * NBN * 1024 <= TILES, "the partial tiles fit where the weight was");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // weight tiles, statistics
+    __shared__ f32x2 row_norm[BM];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int tile = tiles_m > 1 ? xcd_contiguous_index((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
+    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+    const int rows_x = min(BM, M - m0), rows_w = min(BN, N - n0), nk = (K + BK - 1) / BK;
+
+    // ---- everything this workgroup reads
+    typedef __attribute__((address_space(3))) void lds_void;
+    const uint32_t lds = (uint32_t)(uintptr_t)(lds_void *)smem;
+    request_norm_stats<BM, WAVES>(nf, m0, rows_x, lds + TILES, wave, lane);
+    const uint64_t waddr = (uint64_t)(uintptr_t)(W + (int64_t)n0 * K);
+    const u32x4 wrsrc = {(uint32_t)waddr, (uint32_t)(waddr >> 32) & 0xFFFFu, (uint32_t)((int64_t)rows_w * K * 2), 0x00020000u};
+#pragma unroll
+    for (int j = 0; j < kApplyTiles; ++j) {
+        const int kt = wave + WAVES * j;
+        if (kt >= nk) break;
+#pragma unroll
+        for (int i = 0; i < LW; ++i) {
+            // (rows past N, and the upper half of a last k-tile past K, lie outside the resource's range and arrive as zeros)
+            const int q = i * 64 + lane, row = SmallTileMap::load_row(q), k = kt * BK + SmallTileMap::load_chunk(q) * 8;
+            const uint32_t at = row < rows_w && k < K ? (uint32_t)((row * K + k) * 2) : 0x80000000u;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                         :: "s"(lds + (wave * kApplyTiles + j) * W_BYTES + i * 1024), "v"(at), "s"(wrsrc) : "memory", "m0");
+        }
+    }
+    constexpr int LPR = BN / 4, ROWS = 64 * WAVES / LPR;
+    static_assert(ROWS >= BM, "a thread finishes four columns of one row at most");
+    const int own_row = tid / LPR, own_c = tid % LPR, n_own = n0 + 4 * own_c;
+    float bz[4];
+    load_bias4<T>(bias, n_own, N, ((uintptr_t)bias & 7) == 0, bz);
+    f32x4 x[kApplyTiles][2][NBM][2];
+    vec8 gam[kApplyTiles][2], bet[kApplyTiles][2];
+#pragma unroll
+    for (int j = 0; j < kApplyTiles; ++j) {
+        const int kt = wave + WAVES * j;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            const int k = kt * BK + 32 * st;  // (K is a multiple of 32: a k-step is inside or outside as a whole)
+            if (k >= K) break;
+            gam[j][st] = *reinterpret_cast<const vec8 *>(static_cast<const T *>(nf.gamma) + k + 8 * g);
+            bet[j][st] = nf.beta != nullptr ? *reinterpret_cast<const vec8 *>(static_cast<const T *>(nf.beta) + k + 8 * g) : vec8{};
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) {
+                const f32x4 *p = reinterpret_cast<const f32x4 *>(X + (int64_t)min(m0 + 16 * i + r, M - 1) * ldx + k + 8 * g);
+                x[j][st][i][0] = p[0];
+                x[j][st][i][1] = p[1];
+            }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();  // the statistics have landed
+    merge_norm_stats<BM, WAVES>(nf, smem + TILES, row_norm, tid);
+    __syncthreads();
+
+    f32x4_acc acc[NBM][NBN];
+    float mean[NBM], rstd[NBM];
+#pragma unroll
+    for (int i = 0; i < NBM; ++i) {
+        const f32x2 norm = row_norm[16 * i + r];
+        mean[i] = norm[0];
+        rstd[i] = norm[1];
+#pragma unroll
+        for (int jj = 0; jj < NBN; ++jj) acc[i][jj] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int j = 0; j < kApplyTiles; ++j) {
+        const int kt = wave + WAVES * j;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            if (kt * BK + 32 * st >= K) break;
+            const unsigned char *sb = smem + (wave * kApplyTiles + j) * W_BYTES;
+            vec8 wf[NBN];
+#pragma unroll
+            for (int jj = 0; jj < NBN; ++jj) wf[jj] = *reinterpret_cast<const vec8 *>(sb + SmallTileMap::frag_offset(16 * jj + r, st, g));
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) {
+                u32x4 packed;
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    float y[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        y[e] = fmaf((x[j][st][i][p / 2][2 * (p % 2) + e] - mean[i]) * rstd[i], to_float(gam[j][st][2 * p + e]), to_float(bet[j][st][2 * p + e]));
+                    packed[p] = pack2<T>(y[0], y[1]);
+                }
+                const vec8 xf = __builtin_bit_cast(vec8, packed);
+#pragma unroll
+                for (int jj = 0; jj < NBN; ++jj) acc[i][jj] = mfma16(wf[jj], xf, acc[i][jj]);
+            }
+        }
+    }
+    __syncthreads();  // the weight tiles are done with: the partial tiles take their place
+    float *red = reinterpret_cast<float *>(smem);  // [wave][block][lane][4]
+#pragma unroll
+    for (int i = 0; i < NBM; ++i)
+#pragma unroll
+        for (int jj = 0; jj < NBN; ++jj)
+            *reinterpret_cast<f32x4_acc *>(red + ((wave * (NBM * NBN) + i * NBN + jj) * 64 + lane) * 4) = acc[i][jj];
+    __syncthreads();
+
+    if (own_row >= rows_x) return;
+    const int at = (((own_row >> 4) * NBN + (own_c >> 2)) * 64 + (own_c & 3) * 16 + (own_row & 15)) * 4;
+    f32x4_acc sum = *reinterpret_cast<const f32x4_acc *>(red + at);
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_acc *>(red + w * (NBM * NBN) * 256 + at);
+    auto finish = [&](auto act_c) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_c)::value;
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = apply_act16(sum[e] + bz[e], ACT);
+        // (N is a multiple of 32: every column of the tile exists)
+        *reinterpret_cast<u32x2 *>(out + (int64_t)(m0 + own_row) * out_rs + n_own) = u32x2{pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
+    };
     switch (act) {
         case KERNL_ACT_RELU: finish(IntC<KERNL_ACT_RELU>()); break;
         case KERNL_ACT_TANH: finish(IntC<KERNL_ACT_TANH>()); break;
@@ -641,9 +669,25 @@ static void launch_small_dealt_mode(const LinearArgs &a, const NormFold &nf) {
 
 template <typename T, int BM, int BN, int WAVES = 4>
 static void launch_small_dealt(const LinearArgs &a, int mode, const NormFold &nf) {
-    if (mode == kNormApply) launch_small_dealt_mode<T, BM, BN, WAVES, kNormApply>(a, nf);
-    else if (mode == kNormAdd) launch_small_dealt_mode<T, BM, BN, WAVES, kNormAdd>(a, nf);
-    else launch_small_dealt_mode<T, BM, BN, WAVES, kNormNone>(a, nf);
+    if constexpr (BM == 16 && BN == 16) {
+        if (mode == kNormAdd) return launch_small_dealt_mode<T, BM, BN, WAVES, kNormAdd>(a, nf);
+    }
+    launch_small_dealt_mode<T, BM, BN, WAVES, kNormNone>(a, nf);
+}
+
+template <typename T, int BM, int BN>
+static void launch_norm_apply(const LinearArgs &a, const NormFold &nf) {
+    auto kern = linear_norm_apply_kernel<T, BM, BN>;
+    constexpr int LDS_BYTES = 4 * kApplyTiles * BN * 128 + norm_stats_bytes(BM);
+    static bool attr_done = false;  // benign race: the attribute call is idempotent
+    if (!attr_done) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+        attr_done = true;
+    }
+    const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), LDS_BYTES, a.st, static_cast<const float *>(a.x),
+                       static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out), a.M, a.N, a.K, a.x_rs, a.out_rs,
+                       a.act, tiles_m, nf);
 }
 
 template <typename T>
@@ -656,16 +700,30 @@ static void run_small_dealt_t(const LinearArgs &a, int rows, int cols, int mode,
     else launch_small_dealt<T, 64, 32>(a, mode, nf);
 }
 
-// rows x cols of a tile: 16 x 16, 16 x 32, 32 x 32 or 64 x 32
+// rows x cols of a tile: 16 x 16 (the one in front of a norm), 16 x 32, 32 x 32 or 64 x 32
 void run_small_dealt(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf) {
     if (dtype == KERNL_F16) run_small_dealt_t<f16>(a, rows, cols, mode, nf);
     else run_small_dealt_t<bf16>(a, rows, cols, mode, nf);
 }
 
-template <typename T, int BM, int BN, int MODE>
-static void launch_small_mode(const LinearArgs &a, const NormFold &nf) {
-    auto kern = linear_small_kernel<T, BM, BN, MODE>;
-    constexpr int LDS_BYTES = small_stages(BM, BN) * (BM + BN) * kSmallBK * 2 + (MODE != kNormNone ? norm_stats_bytes(BM) : 0);
+template <typename T>
+static void run_norm_apply_t(const LinearArgs &a, int rows, int cols, const NormFold &nf) {
+    if (cols == 16) launch_norm_apply<T, 16, 16>(a, nf);
+    else if (rows == 16) launch_norm_apply<T, 16, 32>(a, nf);
+    else launch_norm_apply<T, 32, 32>(a, nf);
+}
+
+// the layer behind a deferred norm, in tiles of 16 x 16, 16 x 32 or 32 x 32
+void run_norm_apply(const LinearArgs &a, int dtype, int rows, int cols, const NormFold &nf) {
+    if (dtype == KERNL_F16) run_norm_apply_t<f16>(a, rows, cols, nf);
+    else run_norm_apply_t<bf16>(a, rows, cols, nf);
+}
+
+template <typename T>
+static void launch_small(const LinearArgs &a) {
+    constexpr int BM = 32, BN = 64;
+    auto kern = linear_small_kernel<T, BM, BN>;
+    constexpr int LDS_BYTES = small_stages(BM, BN) * (BM + BN) * kSmallBK * 2;
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
@@ -675,20 +733,13 @@ static void launch_small_mode(const LinearArgs &a, const NormFold &nf) {
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), LDS_BYTES, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out),
                        static_cast<T *>(a.act_in), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs, a.act,
-                       tiles_m, nf);
-}
-
-template <typename T, int BM, int BN>
-static void launch_small(const LinearArgs &a, int mode, const NormFold &nf) {
-    if (mode == kNormApply) launch_small_mode<T, BM, BN, kNormApply>(a, nf);
-    else if (mode == kNormAdd) launch_small_mode<T, BM, BN, kNormAdd>(a, nf);
-    else launch_small_mode<T, BM, BN, kNormNone>(a, nf);
+                       tiles_m);
 }
 
 // 32 x 64 tiles
-void run_small(const LinearArgs &a, int dtype, int mode, const NormFold &nf) {
-    if (dtype == KERNL_F16) launch_small<f16, 32, 64>(a, mode, nf);
-    else launch_small<bf16, 32, 64>(a, mode, nf);
+void run_small(const LinearArgs &a, int dtype) {
+    if (dtype == KERNL_F16) launch_small<f16>(a);
+    else launch_small<bf16>(a);
 }
 
 }  // namespace kernl

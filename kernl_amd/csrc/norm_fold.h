@@ -1,55 +1,52 @@
-// LayerNorm between two linear layers without a kernel of its own ("deferred" norm): the layer in front stores the
-// UN-normalised rows s = round(x W^T + b + residual) together with per-row statistics, the layer behind multiplies s by the
-// weight with gamma folded in and normalises its fp32 sums,
-//     LN(s) W^T + b  =  rstd (s (W gamma)^T - mean colsum) + (b + W beta),     colsum[n] = sum_k (W gamma)[n][k],
-// and where LN(s) itself is needed again — as the residual of the next addition — it is computed from s on the fly, in
-// fp32.  One rounding of s takes the place of the rounding of LN(s); no operand gains one.
+// LayerNorm between two linear layers without a kernel of its own ("deferred" norm), for up to 64 rows: the layer in front
+// stores the rows s = x W^T + b + residual in fp32, un-normalised, with statistics; the layer behind normalises them on
+// their way into its matrix instructions,
+//     LN(s) = (s - mean) rstd gamma + beta    in fp32, rounded once to the 16-bit operand,
+// which is what a LayerNorm kernel would have stored, and where LN(s) is needed again — as the residual of the next
+// addition — it is computed from s the same way and not rounded at all.  Against a linear kernel and an add + LayerNorm kernel two
+// roundings are gone (the projection's and the residual's) and none is new, whatever the rows' mean and the norm's parameters
+// are.  (An earlier form stored s in 16 bits and folded gamma into the weight: its error grew with mean / std of the rows.)
 //
-// Statistics of a row: for every 32 columns (16 up to 64 rows, whose tiles are that narrow) the pair (sum, sum of squared deviations from their mean) of the stored
-// 16-bit values, fp32, row-major [rows][groups].  Groups are merged around the first group's mean, so a mean far
-// from zero costs no accuracy.
+// More rows keep their LayerNorm kernel: a product in tiles of 64 rows and more is bound by its tile loads, and fp32 rows
+// double those of x.
+//
+// Statistics of a row: for every 16 columns the pair (sum, sum of squared deviations from their mean) of the fp32 values,
+// row-major [rows][groups].  Groups are merged around the first group's mean, so a mean far from zero costs no accuracy.
 #pragma once
 
 #include "common.h"
 
 namespace kernl {
 
-constexpr int kNormGroup = 32;       // columns per statistics pair ...
-constexpr int kNormGroupFew = 16;    // ... and of inputs of at most
-constexpr int kNormFewRows = 64;     // so many rows
-constexpr int kNormMaxGroups = 32;   // widths up to 1024
-static inline int norm_group_of(int64_t rows) { return rows <= kNormFewRows ? kNormGroupFew : kNormGroup; }
+constexpr int kNormGroup = 16;       // columns per statistics pair
+constexpr int kNormMaxRows = 64;     // rows that tiles of whole statistics groups are built for
+constexpr int kNormMaxGroups = 64;   // widths up to 1024
 
-// MODE of the kernels that take part
+// MODE of the kernels in front of a norm
 constexpr int kNormNone = 0;    // plain epilogue
-constexpr int kNormApply = 1;   // x is un-normalised: fold its norm into the epilogue
-constexpr int kNormAdd = 2;     // add a residual (itself normalised on the fly when it has statistics), store statistics
+constexpr int kNormAdd = 2;     // add a residual (itself normalised on the fly when it has statistics), store fp32 rows and statistics
 
 struct NormFold {
-    const float *in_stats = nullptr;   // kNormApply: of x; kNormAdd: of the residual, or null
+    const float *in_stats = nullptr;   // of the residual (kNormAdd; may be null) or of x (the layer behind)
     int in_groups = 0;                 // statistics pairs per row of in_stats
-    int group = kNormGroup;            // columns of a pair
-    float inv_group = 1.0f / kNormGroup, inv_groups = 1.0f;
+    float inv_groups = 1.0f;
     float eps = 0.0f;
-    const float *colsum = nullptr;     // kNormApply, [N]
-    const float *bias32 = nullptr;     // kNormApply, [N]
-    const void *residual = nullptr;    // kNormAdd, [M, N] 16-bit rows
+    const void *residual = nullptr;    // kNormAdd, [M, N]: fp32 rows with in_stats, 16-bit rows without
     int64_t res_rs = 0;
-    const void *gamma = nullptr, *beta = nullptr;  // kNormAdd with in_stats: of the residual's norm; beta may be null
-    void stats_of(int64_t rows, int64_t width) {  // in_stats describe `rows` rows of `width` columns
-        group = norm_group_of(rows);
-        in_groups = (int)(width / group);
-        inv_group = 1.0f / (float)group;
+    const void *gamma = nullptr, *beta = nullptr;  // with in_stats: of that norm; beta may be null
+    void stats_of(int64_t width) {     // in_stats describe rows of `width` columns
+        in_groups = (int)(width / kNormGroup);
         inv_groups = 1.0f / (float)in_groups;
     }
-    float *out_stats = nullptr;        // kNormAdd, [M, N / group] pairs
+    float *out_stats = nullptr;        // kNormAdd, [M, N / kNormGroup] pairs
 };
 
 // Running merge of a row's statistics pairs: deviations d of the groups' means from a pivot (any of them).
 struct NormMerge {
+    static constexpr float kInvGroup = 1.0f / kNormGroup;
     float d = 0.0f, dd = 0.0f, m2 = 0.0f;
-    __device__ __forceinline__ void take(const f32x2 pair, float pivot, float inv_group) {
-        const float e = fmaf(pair[0], inv_group, -pivot);
+    __device__ __forceinline__ void take(const f32x2 pair, float pivot) {
+        const float e = fmaf(pair[0], kInvGroup, -pivot);
         d += e;
         dd = fmaf(e, e, dd);
         m2 += pair[1];
@@ -57,7 +54,7 @@ struct NormMerge {
     // (mean, 1 / std) of the row
     __device__ __forceinline__ f32x2 finish(float pivot, const NormFold &nf) const {
         const float dm = d * nf.inv_groups;
-        const float var = fmaf(m2, nf.inv_groups * nf.inv_group, fmaxf(fmaf(-dm, dm, dd * nf.inv_groups), 0.0f));
+        const float var = fmaf(m2, nf.inv_groups * kInvGroup, fmaxf(fmaf(-dm, dm, dd * nf.inv_groups), 0.0f));
         return f32x2{pivot + dm, rsqrtf(var + nf.eps)};
     }
 };

@@ -9,7 +9,7 @@ from typing import Callable
 
 import torch
 
-from kernl_amd.implementations.deferred_norm import DeferredNorm, FoldedParams, deferrable, linear_add_deferred
+from kernl_amd.implementations.deferred_norm import DeferredNorm, deferrable, linear_add_deferred
 from kernl_amd.implementations.linear_layer import GLU_BLOCK, interleave_glu_rows, linear_glu_layer, linear_layer
 from kernl_amd.utils.extended_matcher import replace_pattern
 
@@ -22,16 +22,16 @@ torch.fx.wrap("linear_wrapper")
 
 
 def linear_wrapper_functional(v: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, activation=""):
-    if isinstance(v, DeferredNorm):
-        if weight.dtype == v.rows.dtype and v.takes_linear(weight.shape[0], activation):
-            return v.linear(_norm_folded_params(v, (weight,), (bias,)), activation)
-        v = v.normalised()
     # One-time, in-place down-cast of fp32 parameters so they are not converted on every call
     # (reference: optimizer/linear.py:33-36).  Only when the activations already are fp16 or autocast will make them so.
     if weight.dtype == torch.float32 and (v.dtype == torch.float16 or torch.is_autocast_enabled("cuda")):
         weight.data = weight.data.half()
     if bias is not None and bias.dtype == torch.float32 and (v.dtype == torch.float16 or torch.is_autocast_enabled("cuda")):
         bias.data = bias.data.half()
+    if isinstance(v, DeferredNorm):
+        if v.takes_linear(weight, bias, activation):
+            return v.linear(weight, bias, activation)
+        v = v.normalised()
     if not weight.is_contiguous():
         weight = weight.contiguous()
     return linear_layer(v, weight, bias, activation=activation)
@@ -259,10 +259,9 @@ def fused_linear_wrapper(v: torch.Tensor, weights, biases):
     long as the original parameters live unchanged, so capture and replays neither allocate nor copy.  No counterpart in the
     reference, which launches one Triton GEMM per projection."""
     if isinstance(v, DeferredNorm):
-        sizes = [w.shape[0] for w in weights]
-        if all(w.dtype == v.rows.dtype for w in weights) and v.takes_linear(sum(sizes), ""):
-            _concatenated_params(v.rows, weights, biases)  # (moves the parameters: before anything is keyed by where they are)
-            return tuple(torch.split(v.linear(_norm_folded_params(v, weights, biases)), sizes, dim=-1))
+        weight, bias, sizes = _concatenated_params(v, weights, biases)
+        if v.takes_linear(weight, bias, ""):
+            return tuple(torch.split(v.linear(weight, bias), sizes, dim=-1))
         v = v.normalised()
     weight, bias, sizes = _concatenated_params(v, weights, biases)
     out = linear_layer(v, weight, bias, activation="")
@@ -304,30 +303,6 @@ def _concatenated_params(v: torch.Tensor, weights, biases):
                     b.data = bias[row : row + n]
                 row += n
             _fused_params.put(originals, cached)  # keyed by the addresses the parameters now have inside the fused buffers
-    return cached
-
-
-def _norm_folded_params(norm: DeferredNorm, weights, biases) -> FoldedParams:
-    """Row-concatenated weights with the LayerNorm in front of them folded in (a copy, rewritten in place when a version
-    counter moves)."""
-    params = tuple(weights) + tuple(biases) + (norm.gamma, norm.beta)
-    cached = _fused_params.get(params)
-    if cached is None:
-        count = len(weights)
-
-        def build(originals):
-            ws, bs = originals[:count], originals[count : 2 * count]
-            bias = None
-            if any(b is not None for b in bs):
-                bias = torch.cat([torch.zeros_like(w[:, 0]) if b is None else b.detach() for w, b in zip(ws, bs)])
-            return FoldedParams.of(torch.cat([w.detach() for w in ws], dim=0), bias, originals[-2], originals[-1])
-
-        def rebuild(value, originals):
-            for old, new in zip(value, build(originals)):
-                old.copy_(new)
-
-        cached = build(params)
-        _fused_params.put(params, cached, rebuild)
     return cached
 
 
@@ -778,22 +753,23 @@ def rms_fused_linear_rope_wrapper(x: torch.Tensor, rms_weight, eps: float, weigh
 
 
 def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor, normalized_shape,
-                                  ln_weight, ln_bias, eps: float, defer: bool = False):
+                                  ln_weight, ln_bias, eps: float, behind=None):
     """layer_norm(residual + linear(v, weight, bias)): the attention-output and feed-forward-down projections of an
     encoder layer with the addition and LayerNorm behind them.  Where the projection runs the wide tile kernels the
     addition rides in their epilogue and the LayerNorm reads one tensor (16384 x 768, fp16: 15 us -> 11 us per norm);
     elsewhere the projection is followed by the fused add + LayerNorm kernel, as before.  No counterpart in the
     reference, whose graphs add in eager PyTorch in front of every LayerNorm.
 
-    `defer` (set by `defer_layer_norms` where every consumer can take it): small inputs leave the norm to the layers behind
-    it and return a `DeferredNorm`; `residual` may be one."""
+    `behind` (set by `defer_layer_norms` where every consumer can take it): the weights of the layers that read the result.
+    Few rows leave the norm to them and return a `DeferredNorm`, if all of them take it; `residual` may be one."""
     from kernl_amd.optimizer.layer_norm import _half_params_once, add_layer_norm_wrapper_functional, layer_norm_wrapper_functional
 
-    if (defer and isinstance(residual, torch.Tensor) or isinstance(residual, DeferredNorm)) and len(normalized_shape) == 1:
+    if (behind is not None and isinstance(residual, torch.Tensor) or isinstance(residual, DeferredNorm)) and len(normalized_shape) == 1:
         _half_params_once(v, weight, bias, ln_weight, ln_bias)
-        if deferrable(v, weight, bias, residual, ln_weight, ln_bias):
+        sizes = [(sum(w.shape[0] for w in weights), weights[0].shape[1]) for weights in behind or ()]
+        if deferrable(v, weight, bias, residual, ln_weight, ln_bias, sizes):
             norm = linear_add_deferred(v, weight, bias, residual, ln_weight, ln_bias, eps)
-            return norm if defer else norm.normalised()
+            return norm if behind is not None else norm.normalised()
     if isinstance(residual, DeferredNorm):
         residual = residual.normalised()
     if isinstance(residual, torch.Tensor):
@@ -875,21 +851,30 @@ def fuse_linears_into_add_layer_norms(gm: torch.fx.GraphModule):
 
 def defer_layer_norms(gm: torch.fx.GraphModule):
     """Marks the `linear_add_layer_norm_wrapper` calls whose result is read only as the input of linear layers and as the
-    residual of the next such call: those take the un-normalised rows of small inputs (`DeferredNorm`).  Runs last."""
+    residual of the next such call, with the weights of those layers: they take the un-normalised rows of small inputs
+    (`DeferredNorm`).  Runs last."""
 
-    def takes_deferred(user, node):
-        if user.op != "call_function" or sum(1 for inp in user.args if inp is node) != 1:
-            return False
-        if user.target in (linear_wrapper_functional, fused_linear_wrapper):
-            return user.args[0] is node and node not in user.kwargs.values()
-        return user.target is linear_add_layer_norm_wrapper and user.args[3] is node
+    def weights_of(user, node):
+        """The weights of a layer that takes a deferred norm from `node`, as one tuple; None for any other reader"""
+        if user.op != "call_function" or sum(1 for inp in user.args if inp is node) != 1 or node in user.kwargs.values():
+            return None
+        if user.target is linear_wrapper_functional and user.args[0] is node:
+            return (user.args[1],)
+        if user.target is fused_linear_wrapper and user.args[0] is node:
+            return tuple(user.args[1])
+        if user.target is linear_add_layer_norm_wrapper and user.args[3] is node:
+            return (user.args[1],)
+        return None
 
     changed = False
+    position = {node: i for i, node in enumerate(gm.graph.nodes)}
     for node in gm.graph.nodes:
         if node.op == "call_function" and node.target is linear_add_layer_norm_wrapper and len(node.args) == 8 and not node.kwargs:
-            if node.users and all(takes_deferred(u, node) for u in node.users):
-                node.kwargs = {"defer": True}
+            behind = tuple(weights_of(u, node) for u in node.users)
+            # (parameters come in front of the first call; a weight that is computed later cannot be looked at here)
+            if behind and None not in behind and all(position[w] < position[node] for weights in behind for w in weights):
                 changed = True
+                node.kwargs = {"behind": behind}
     if changed:
         gm.graph.lint()
         gm.recompile()
