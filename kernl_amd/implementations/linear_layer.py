@@ -266,11 +266,11 @@ def rms_linear_layer(
         and x_.shape[0] > FEW_ROW_MAX_ROWS
         and _lib.linear_scaled_supported(x_, folded_weight)
         and (bias is None or bias.dtype == x.dtype)
-        # only where the plain product would run the wide tile kernels anyway (not the small-tile or split-K forms)
+        # not where the row count is too small for the wide tile kernels to have one tile per CU.  (The 8-wave tiles that most of
+        # those products run on would take the row factors too; but weight * rms_weight is rounded to 16 bits, which a small
+        # norm weight makes coarser than the rounding of the normalised row, so the folded weight stays with the large prompts.)
         and not takes_small_problem_kernel(x_, folded_weight)
-        # (8-wave tiles take the row factors too: a large weight's product then saves the norm's launch and pass)
-        and (x_.shape[0] > SPLIT_K_MAX_ROWS or _lib.linear_splitk_workspace_bytes(x_, folded_weight) == 0
-             or (folded_weight.numel() >= 1 << 24 and takes_mid_kernel(x_, folded_weight, gated)))
+        and (x_.shape[0] > SPLIT_K_MAX_ROWS or _lib.linear_splitk_workspace_bytes(x_, folded_weight) == 0)
     ):
         if rstd is None:
             rstd = rms_stats(x_, eps, clamp=False)

@@ -943,3 +943,30 @@ def test_linear_fp8_weight_every_kernel(tile, close):
     finally:
         lib.kernl_linear_force_tile(0)
     close(out, linear_oracle(x, e5m2_decode_oracle(w8), b, "fast_gelu"), what=f"fp8 weight, kernel choice {tile}")
+
+
+@pytest.mark.parametrize("rows, out_features, gated", [(200, 4096, False), (130, 12288, False), (333, 4096, False), (150, 4096, True)], ids=str)
+def test_short_prompts_normalise_before_the_product(rows, out_features, gated, monkeypatch):
+    """Where split K used to take the product, a prompt's rows are normalised by the RMSNorm kernel and meet the weight as it is:
+    folding a small norm weight into an fp16 weight loses what the normalised row keeps (here 2^-12: the product of weights of 0.03
+    and 2^-12 is below the normal range)."""
+    from kernl_amd.implementations import linear_layer as ll
+
+    gen = torch.Generator().manual_seed(1)
+    k = 4096
+    x = torch.randn((rows, k), generator=gen).half().cuda()
+    g = torch.full((k,), 2.0 ** -12).half().cuda()
+    w = (torch.randn((out_features, k), generator=gen) * 0.03).half().cuda()
+    if _lib.linear_splitk_workspace_bytes(x, w) == 0:
+        pytest.skip("the wide tiles' problem")
+    calls = []
+    real = _lib.linear_scaled_fwd
+    monkeypatch.setattr(_lib, "linear_scaled_fwd", lambda *a, **kw: (calls.append(1), real(*a, **kw))[1])
+    folded = (w.float() * g.float()).half()
+    out = ll.rms_linear_layer(x, g, 1e-5, w, None, "silu" if gated else "", gated=gated, folded_weight=folded, unfolded=lambda: w)
+    assert not calls
+    if not gated:
+        xd = x.double()
+        ref = (xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1.6e-5) * g.double()) @ w.double().T
+        # the normalised row and the result rounded once each, a little more for results below the normal range
+        assert ((out.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -10
