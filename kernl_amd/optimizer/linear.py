@@ -9,6 +9,7 @@ from typing import Callable
 
 import torch
 
+from kernl_amd import _lib
 from kernl_amd.implementations.deferred_norm import DeferredNorm, deferrable, linear_add_deferred
 from kernl_amd.implementations.linear_layer import GLU_BLOCK, interleave_glu_rows, linear_glu_layer, linear_layer
 from kernl_amd.utils.extended_matcher import replace_pattern
@@ -752,6 +753,13 @@ def rms_fused_linear_rope_wrapper(x: torch.Tensor, rms_weight, eps: float, weigh
     return tuple(outs)
 
 
+def _epilogue_addition_pays_in_front_of_a_norm(v: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the projection runs the wide tile kernels (5 .. 8): the sum is rounded to 16 bits on its way to the LayerNorm, in
+    exchange for one tensor less to read (16384 x 768: 4 us).  The 8-wave tiles of fewer rows add in their epilogue too, but at
+    2048 x 768 the tensor is worth a microsecond, and the add + LayerNorm kernel adds in fp32."""
+    return 5 <= _lib.linear_wide_kind(v.numel() // v.shape[-1], weight.shape[0], weight.shape[1]) <= 8
+
+
 def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor, normalized_shape,
                                   ln_weight, ln_bias, eps: float, behind=None):
     """layer_norm(residual + linear(v, weight, bias)): the attention-output and feed-forward-down projections of an
@@ -772,7 +780,7 @@ def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, r
             return norm if behind is not None else norm.normalised()
     if isinstance(residual, DeferredNorm):
         residual = residual.normalised()
-    if isinstance(residual, torch.Tensor):
+    if isinstance(residual, torch.Tensor) and _epilogue_addition_pays_in_front_of_a_norm(v, weight):
         fused = _wide_residual_linear(v, weight, bias, residual)
         if fused is not None:
             return layer_norm_wrapper_functional(fused, normalized_shape, ln_weight, ln_bias, eps)

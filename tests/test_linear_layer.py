@@ -463,6 +463,24 @@ def test_projection_with_the_addition_and_layer_norm_behind_it(shape, dtype, clo
     close(other, ref, dtype, scale="magnitude", what=f"projection, then add + layernorm {shape}")
 
 
+@pytest.mark.parametrize("shape", [(1600, 768, 3072), (2048, 1024, 4096), (2700, 768, 768), (2100, 1024, 1024)], ids=str)
+def test_mid_sized_projections_are_not_rounded_between_addition_and_norm(shape, monkeypatch):
+    """The 8-wave tiles' sizes: the LayerNorm kernel adds in fp32, bit for bit the two operators one after the other."""
+    from kernl_amd.implementations.layer_norm import add_layer_norm
+    from kernl_amd.optimizer import linear as ol
+
+    rows, n, k = shape
+    gen = torch.Generator().manual_seed(3)
+    v, w = torch.randn((rows, k), generator=gen).half().cuda(), (torch.randn((n, k), generator=gen) * k ** -0.5).half().cuda()
+    res, g, be = (torch.randn(s, generator=gen).half().cuda() for s in ((rows, n), (n,), (n,)))
+    assert _lib.linear_mid_kind(rows, n, k) == _lib.linear_wide_kind(rows, n, k) >= 11
+    calls = []
+    real = _lib.linear_residual_fwd
+    monkeypatch.setattr(_lib, "linear_residual_fwd", lambda *a, **kw: (calls.append(1), real(*a, **kw))[1])
+    out = ol.linear_add_layer_norm_wrapper(v, w, None, res, (n,), g, be, 1e-5)
+    assert not calls and torch.equal(out, add_layer_norm(linear_layer(v, w, None), res, g, be, 1e-5))
+
+
 def test_residual_addition_with_row_statistics(close):
     """`add_rms_stats`: the sum is the fp16 / bf16 rounding of the fp32 sum (what `a + b` gives), the statistics are those
     of the ROUNDED sum; ragged row counts, 3-D inputs, non-contiguous operands."""
