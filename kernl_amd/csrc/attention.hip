@@ -1126,7 +1126,7 @@ static int attention_entry(const void *q, const void *k, const void *v, void *ou
     {
         const int64_t wgs = B * H * ((M + 63) / 64);
         const bool applies = mfma_ok && mask_mode != MASK_MATRIX && N <= kShortMaxKeys && wgs < (1ll << 31);
-        if (applies && (g_attention_variant == 6 || (g_attention_variant == 0 && attention_short_pays(wgs, (int)N, (int)D)))) {
+        if (applies && (g_attention_variant == 6 || (g_attention_variant == 0 && attention_short_pays(wgs, M, (int)N, (int)D, mask_mode == MASK_VECTOR)))) {
             run_attention_short(p, (int)D, dtype, mask_mode == MASK_VECTOR, causal, st);
             return check_launch("attention (mfma, short key sequences)");
         }

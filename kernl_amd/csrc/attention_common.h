@@ -68,8 +68,14 @@ static constexpr int kShortMaxKeys = 256;
 // Every wave reads all keys of its head from LDS, so with enough workgroups to fill the chip several times over the kernels
 // whose waves share 128-row tiles win: [64,12,128,64] 12.3 -> 12.3, [16,12,256,64] 8.5 -> 9.6 without a mask, [8,32,160,128] 15.0
 // -> 17.6.  The limits lie at the last grid of each size where it was ahead with and without a mask.
-static inline bool attention_short_pays(int64_t workgroups, int N, int D) {
-    if (N <= 64) return true;
+// Many query rows over few keys (cross-attention) stage keys and values once per 64 rows, where the other kernels do per 128.  Up to
+// 32 keys that is little (at worst [1,8,8192,128] over 16 keys 10.7 -> 11.0 without a mask, 12.0 -> 11.4 with one), and a mask costs
+// the others its classification ([16,16,8192,64] over 64 keys 150 -> 133); without one and beyond 32 keys they win from some grid on:
+// head size 128, 33 to 64 keys: 128 workgroups 5.8 -> 4.8, 192 5.9 -> 5.1, 512 7.1 -> 7.9, 1024 9.8 -> 11.5; head size 64: 16384
+// workgroups 59 -> 46, 32768 124 -> 133.  Up to 64 rows their 128-row tiles are half empty.
+static inline bool attention_short_pays(int64_t workgroups, int64_t M, int N, int D, bool masked) {
+    if (N <= 32 || (N <= 64 && (masked || M <= 64))) return true;
+    if (N <= 64) return workgroups <= (D == 64 ? 16384 : 384);
     if (D == 64) return workgroups <= (N <= 128 ? 1024 : N <= 192 ? 512 : 384);
     return workgroups <= (N <= 128 ? 384 : 256);
 }

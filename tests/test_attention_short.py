@@ -44,3 +44,22 @@ def test_short_key_sequences(m, n, kind, head, dtype, close):
     torch.cuda.synchronize()
     expected = attention_oracle(q, k, v, head ** -0.5, causal, mask, start_position=start)
     close(out, expected, dtype, what=f"{m}x{n} {kind} {head}")
+
+
+# (batch, heads, rows, keys, head size): many rows over few keys, on both sides of the lines of `attention_short_pays`
+CROSS = [(2, 3, 1000, 32, 128), (2, 3, 1000, 33, 64), (2, 3, 4096, 64, 128), (2, 3, 4160, 64, 128), (9, 16, 190, 40, 128), (7, 64, 64, 64, 128)]
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("b, h, m, n, head", CROSS, ids=str)
+def test_many_rows_over_few_keys(b, h, m, n, head, masked, close):
+    _lib.load().kernl_attention_set_variant(0)  # the kernel the rule takes
+    gen = torch.Generator().manual_seed(m + n)
+    q, (k, v) = torch.randn((b, h, m, head), generator=gen).half(), torch.randn((2, b, h, n, head), generator=gen).half()
+    mask = None
+    if masked:
+        mask = torch.zeros((b, n)).masked_fill_(torch.arange(n)[None, :] >= torch.randint(1, n + 1, (b, 1), generator=gen), float("-inf"))[:, None, None, :]
+    out = torch.full_like(q, float("nan"), device="cuda")
+    attention_forward(q.cuda(), k.cuda(), v.cuda(), out, head ** -0.5, False, None if mask is None else mask.cuda())
+    torch.cuda.synchronize()
+    close(out, attention_oracle(q, k, v, head ** -0.5, False, mask), what=f"{m} rows over {n} keys")
