@@ -356,8 +356,8 @@ extern "C" int kernl_linear_norm_apply_fwd(const float *x, const float *x_stats,
                                            const void *bias, void *out, int64_t M, int64_t N, int64_t K, int64_t x_row_stride,
                                            int64_t out_row_stride, int activation, int dtype, void *stream) {
     using namespace kernl;
-    if (x_stats == nullptr || gamma == nullptr || !aligned16(x_stats) || !aligned16(gamma) || !aligned16(beta))
-        return set_error(KERNL_ERR_INVALID_ARG, "linear (deferred norm): x_stats and the norm's parameters must be 16-byte aligned arrays");
+    if (x_stats == nullptr || gamma == nullptr || !aligned16(x_stats) || !aligned16(gamma) || !aligned16(beta) || !aligned16(bias))
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (deferred norm): x_stats, bias and the norm's parameters must be 16-byte aligned arrays");
     if (activation < KERNL_ACT_NONE || activation > KERNL_ACT_SILU)
         return set_error(KERNL_ERR_INVALID_ARG, "linear (deferred norm): unknown activation %d", activation);
     const int bad = norm_arguments_bad("linear (deferred norm)", x, 4, w, out, 2, M, N, K, x_row_stride, out_row_stride, dtype);
@@ -379,9 +379,9 @@ extern "C" int kernl_linear_norm_add_fwd(const void *x, const void *w, const voi
                                          int64_t K, int64_t x_row_stride, int64_t out_row_stride, int64_t residual_row_stride, int dtype,
                                          void *stream) {
     using namespace kernl;
-    if (residual == nullptr || out_stats == nullptr || !aligned16(residual) || residual_row_stride * (residual_stats != nullptr ? 4 : 2) % 16 != 0 ||
+    if (residual == nullptr || out_stats == nullptr || !aligned16(residual) || !aligned16(bias) || residual_row_stride * (residual_stats != nullptr ? 4 : 2) % 16 != 0 ||
         !aligned16(out_stats))
-        return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: residual needs 16-byte aligned rows, out_stats a 16-byte aligned array");
+        return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: residual needs 16-byte aligned rows, bias and out_stats 16-byte aligned arrays");
     if (residual_stats != nullptr && (gamma == nullptr || !aligned16(residual_stats) || !aligned16(gamma) || !aligned16(beta)))
         return set_error(KERNL_ERR_INVALID_ARG, "linear + addition + statistics: a deferred residual comes with its statistics and aligned norm parameters");
     const int bad = norm_arguments_bad("linear + addition + statistics", x, 2, w, out, 4, M, N, K, x_row_stride, out_row_stride, dtype);

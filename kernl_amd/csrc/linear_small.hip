@@ -33,7 +33,7 @@ __device__ __forceinline__ void request_norm_stats(const NormFold &nf, int m0, i
                          :: "s"(lds + piece * 1024), "v"(piece * 1024 + lane * 16), "s"(rsrc) : "memory", "m0");
     }
 }
-// The staged pairs (at `staged`) merged by up to 16 threads a row: (mean, 1 / std) of row i of the tile to row_norm[i].
+// The staged pairs (at `staged`) merged by 16 (8) threads a row: (mean, 1 / std) of row i of the tile to row_norm[i].
 template <int BM, int WAVES>
 __device__ __forceinline__ void merge_norm_stats(const NormFold &nf, const unsigned char *staged, f32x2 *row_norm, int tid) {
     constexpr int SPAN = 64 * WAVES / BM < 16 ? 64 * WAVES / BM : 16, PER = kNormMaxGroups / SPAN;
@@ -354,24 +354,18 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     constexpr int LPR = BN / 4, ROWS = 64 * WAVES / LPR, OWN = (BM + ROWS - 1) / ROWS;
     const int own_row = tid / LPR, own_c = tid % LPR, n_own = n0 + 4 * own_c;
     float bz[4];
-    load_bias4<T>(bias, n_own, N, ((uintptr_t)bias & 7) == 0, bz);
     const bool row_stats = MODE == kNormAdd && nf.in_stats != nullptr;  // the residual is fp32 rows whose norm is to be applied
-    u32x4 res[OWN];  // raw: four fp32 values, or four 16-bit ones in the first half
-    u32x2 gam = {0, 0}, bet = {0, 0};
-    if (MODE == kNormAdd) {  // (N is a multiple of 32: every column of the tile exists)
-#pragma unroll
-        for (int t = 0; t < OWN; ++t) {
-            res[t] = u32x4{0, 0, 0, 0};
-            if (own_row + ROWS * t >= rows_x) continue;
-            const int64_t at = (int64_t)(m0 + own_row + ROWS * t) * nf.res_rs + n_own;
-            if (row_stats) {
-                res[t] = *reinterpret_cast<const u32x4 *>(static_cast<const float *>(nf.residual) + at);
-            } else {
-                const u32x2 half = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + at);
-                res[t][0] = half[0];
-                res[t][1] = half[1];
-            }
-        }
+    f32x4 res32 = {0.0f, 0.0f, 0.0f, 0.0f};
+    u32x2 res16 = {0, 0}, gam = {0, 0}, bet = {0, 0}, bias16 = {0, 0};
+    if (MODE != kNormAdd) {
+        load_bias4<T>(bias, n_own, N, ((uintptr_t)bias & 7) == 0, bz);
+    } else {
+        // raw, and each in registers of its own: what is converted or moved here is waited for here.  (N is a multiple of 32:
+        // every column of the tile exists)
+        if (bias != nullptr) bias16 = *reinterpret_cast<const u32x2 *>(bias + n_own);
+        const int64_t at = (int64_t)(m0 + own_row) * nf.res_rs + n_own;
+        if (own_row < rows_x && row_stats) res32 = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(nf.residual) + at);
+        if (own_row < rows_x && !row_stats) res16 = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + at);
         if (row_stats) {
             gam = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.gamma) + n_own);
             if (nf.beta != nullptr) bet = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.beta) + n_own);
@@ -412,7 +406,7 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     f32x2 *row_norm = reinterpret_cast<f32x2 *>(smem + WAVES * RING) - BM;  // (the end of the rings, which the partial tiles leave free)
     static_assert(WAVES * NBM * NBN * 1024 + BM * 8 <= WAVES * RING, "room behind the partial tiles");
     if constexpr (MODE == kNormAdd) {
-        static_assert(BM == 16 && BN == kNormGroup, "a row of the tile is one statistics group");
+        static_assert(BM == 16 && BN == kNormGroup && OWN == 1, "a row of the tile is one statistics group, and a thread's");
         if (row_stats) merge_norm_stats<BM, WAVES>(nf, smem + WAVES * RING, row_norm, tid);
     }
     float *red = reinterpret_cast<float *>(smem);  // [wave][block][lane][4]
@@ -440,7 +434,8 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
         float pre[4], y[4];
         if (MODE == kNormAdd) {
             // fp32 rows and the statistics of what is stored
-            f32x4 h = __builtin_bit_cast(f32x4, res[t]);
+            f32x4 h = res32;
+            unpack4<T>(bias16, bz);
             if (row_stats) {
                 const f32x2 norm = row_norm[row];
                 float gm[4], bt[4];
@@ -450,7 +445,7 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
                 for (int e = 0; e < 4; ++e) h[e] = fmaf((h[e] - norm[0]) * norm[1], gm[e], bt[e]);
             } else {
                 float h16[4];
-                unpack4<T>(u32x2{res[t][0], res[t][1]}, h16);
+                unpack4<T>(res16, h16);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) h[e] = h16[e];
             }
@@ -512,73 +507,81 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
 }
 
 // The layer BEHIND a deferred norm: out = act(LN(x) W^T + bias) for up to 64 fp32 rows of up to 1024 columns, LN(x) rounded once to
-// the 16-bit operand (norm_fold.h).  The tiles and the dealt k-tiles of the kernel above; but x does not go through LDS: a lane
-// fetches the 8 columns of its rows that its matrix-instruction operand wants, normalises and packs them in registers.  A wave has at
-// most four k-tiles, all of which — weight, x, gamma and beta — are requested before anything is waited for: one trip to memory.
+// the 16-bit operand (norm_fold.h).  The tiles and the dealt k-tiles of the kernel above: a wave has at most four, and everything
+// the workgroup reads — weight, fp32 rows, statistics, gamma and beta — is on its way to LDS before anything is waited for: one
+// trip to memory.  A lane reads the 8 columns of its rows that its matrix-instruction operand wants, normalises and packs them in
+// registers.  (Fetched straight into registers such rows are 16 lines a load: 16 x 2304 x 768 5.6 us instead of 4.6, 16 x 3072 x 768
+// 6.0 instead of 4.9, under the profiler; the same product of rows that are normalised already 4.2 and 4.3, and the LayerNorm
+// kernel in front of it 2.7.)
 constexpr int kApplyTiles = 4;  // k-tiles of a wave, as many as 1024 columns are
+constexpr int kib(int bytes) { return (bytes + 1023) / 1024 * 1024; }
+// LDS: k-tiles of x and W of the four waves (the partial tiles take their place), statistics, gamma, beta
+constexpr int kApplyMaxLds = 160 * 1024 - 512;  // (the row factors are LDS too)
+static inline int apply_lds_bytes(int bm, int bn, int k) {
+    return 4 * (((k + 63) / 64 + 3) / 4) * (bm * 256 + bn * 128) + kib(bm * (k / kNormGroup) * 8) + 2 * 2 * k;
+}
 
 template <typename T, int BM, int BN>
 __global__ void __launch_bounds__(256, 1)
 linear_norm_apply_kernel(const float *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out, int M,
                          int N, int K, int64_t ldx, int64_t out_rs, int act, int tiles_m, NormFold nf) {
     typedef typename Vec8<T>::type vec8;
-    constexpr int WAVES = 4, BK = 64, W_BYTES = BN * BK * 2, LW = BN / 8, NBM = BM / 16, NBN = BN / 16;
-    constexpr int TILES = WAVES * kApplyTiles * W_BYTES;
-    static_assert(WAVES * NBM * NBN * 1024 <= TILES, "the partial tiles fit where the weight was");
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // weight tiles, statistics
+    constexpr int WAVES = 4, BK = 64, X_BYTES = BM * BK * 4, W_BYTES = BN * BK * 2, STAGE = X_BYTES + W_BYTES;
+    constexpr int LX = BM / 4, LW = BN / 8, NBM = BM / 16, NBN = BN / 16;
+    static_assert(NBM * NBN * 1024 <= STAGE, "the partial tiles fit where the first k-tiles were");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     __shared__ f32x2 row_norm[BM];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
     const int tile = tiles_m > 1 ? xcd_contiguous_index((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
     const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
-    const int rows_x = min(BM, M - m0), rows_w = min(BN, N - n0), nk = (K + BK - 1) / BK;
+    const int rows_x = min(BM, M - m0), rows_w = min(BN, N - n0), nk = (K + BK - 1) / BK, per_wave = (nk + WAVES - 1) / WAVES;
 
     // ---- everything this workgroup reads
     typedef __attribute__((address_space(3))) void lds_void;
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_void *)smem;
-    request_norm_stats<BM, WAVES>(nf, m0, rows_x, lds + TILES, wave, lane);
-    const uint64_t waddr = (uint64_t)(uintptr_t)(W + (int64_t)n0 * K);
-    const u32x4 wrsrc = {(uint32_t)waddr, (uint32_t)(waddr >> 32) & 0xFFFFu, (uint32_t)((int64_t)rows_w * K * 2), 0x00020000u};
+    auto load1 = [&](const u32x4 &rsrc, uint32_t off, uint32_t to) __attribute__((always_inline)) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" :: "s"(to), "v"(off), "s"(rsrc) : "memory", "m0");
+    };
+    auto resource = [](const void *p, int bytes) __attribute__((always_inline)) {
+        const uint64_t a = (uint64_t)(uintptr_t)p;
+        return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xFFFFu, (uint32_t)bytes, 0x00020000u};
+    };
+    constexpr uint32_t kOutOfRange = 0x80000000u;  // arrives as zeros: rows past M and N, the upper half of a last k-tile past K
+    const u32x4 wrsrc = resource(W + (int64_t)n0 * K, rows_w * K * 2);
+    const u32x4 xrsrc = resource(X + (int64_t)m0 * ldx, (int)(((rows_x - 1) * ldx + K) * 4));
+    const uint32_t my = lds + wave * per_wave * STAGE;
 #pragma unroll
     for (int j = 0; j < kApplyTiles; ++j) {
         const int kt = wave + WAVES * j;
         if (kt >= nk) break;
 #pragma unroll
         for (int i = 0; i < LW; ++i) {
-            // (rows past N, and the upper half of a last k-tile past K, lie outside the resource's range and arrive as zeros)
             const int q = i * 64 + lane, row = SmallTileMap::load_row(q), k = kt * BK + SmallTileMap::load_chunk(q) * 8;
-            const uint32_t at = row < rows_w && k < K ? (uint32_t)((row * K + k) * 2) : 0x80000000u;
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                         :: "s"(lds + (wave * kApplyTiles + j) * W_BYTES + i * 1024), "v"(at), "s"(wrsrc) : "memory", "m0");
+            load1(wrsrc, row < rows_w && k < K ? (uint32_t)((row * K + k) * 2) : kOutOfRange, my + j * STAGE + X_BYTES + i * 1024);
         }
+        // (a row's 16 pieces of 16 bytes are exchanged by its number: 16 rows read at one column meet every bank once)
+#pragma unroll
+        for (int i = 0; i < LX; ++i) {
+            const int row = 4 * i + (lane >> 4), k = kt * BK + ((lane ^ row) & 15) * 4;
+            load1(xrsrc, row < rows_x && k < K ? (uint32_t)((row * (int)ldx + k) * 4) : kOutOfRange, my + j * STAGE + i * 1024);
+        }
+    }
+    const int stats_at = WAVES * per_wave * STAGE, gamma_at = stats_at + kib(BM * nf.in_groups * 8), beta_at = gamma_at + 2 * K;
+    request_norm_stats<BM, WAVES>(nf, m0, rows_x, lds + stats_at, wave, lane);
+    const int param_at = (wave >> 1) * 1024;  // at most 2 KB of gamma and of beta: a wave each for a KB
+    if (param_at + lane * 16 < 2 * K) {
+        if ((wave & 1) == 0) load1(resource(nf.gamma, 2 * K), param_at + lane * 16, lds + gamma_at + param_at);
+        else load1(resource(nf.beta, nf.beta != nullptr ? 2 * K : 0), param_at + lane * 16, lds + beta_at + param_at);
     }
     constexpr int LPR = BN / 4, ROWS = 64 * WAVES / LPR;
     static_assert(ROWS >= BM, "a thread finishes four columns of one row at most");
-    const int own_row = tid / LPR, own_c = tid % LPR, n_own = n0 + 4 * own_c;
-    float bz[4];
-    load_bias4<T>(bias, n_own, N, ((uintptr_t)bias & 7) == 0, bz);
-    f32x4 x[kApplyTiles][2][NBM][2];
-    vec8 gam[kApplyTiles][2], bet[kApplyTiles][2];
-#pragma unroll
-    for (int j = 0; j < kApplyTiles; ++j) {
-        const int kt = wave + WAVES * j;
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-            const int k = kt * BK + 32 * st;  // (K is a multiple of 32: a k-step is inside or outside as a whole)
-            if (k >= K) break;
-            gam[j][st] = *reinterpret_cast<const vec8 *>(static_cast<const T *>(nf.gamma) + k + 8 * g);
-            bet[j][st] = nf.beta != nullptr ? *reinterpret_cast<const vec8 *>(static_cast<const T *>(nf.beta) + k + 8 * g) : vec8{};
-#pragma unroll
-            for (int i = 0; i < NBM; ++i) {
-                const f32x4 *p = reinterpret_cast<const f32x4 *>(X + (int64_t)min(m0 + 16 * i + r, M - 1) * ldx + k + 8 * g);
-                x[j][st][i][0] = p[0];
-                x[j][st][i][1] = p[1];
-            }
-        }
-    }
+    const int own_row = tid / LPR, own_c = tid % LPR, n_own = n0 + 4 * own_c;  // (N is a multiple of 32: every column of the tile exists)
+    // (converted where it is added: a conversion here would wait for everything above)
+    const u32x2 bias_raw = bias != nullptr ? *reinterpret_cast<const u32x2 *>(bias + n_own) : u32x2{0, 0};
     __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();  // the statistics have landed
-    merge_norm_stats<BM, WAVES>(nf, smem + TILES, row_norm, tid);
+    __syncthreads();
+    merge_norm_stats<BM, WAVES>(nf, smem + stats_at, row_norm, tid);
     __syncthreads();
 
     f32x4_acc acc[NBM][NBN];
@@ -596,20 +599,25 @@ linear_norm_apply_kernel(const float *__restrict__ X, const T *__restrict__ W, c
         const int kt = wave + WAVES * j;
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
-            if (kt * BK + 32 * st >= K) break;
-            const unsigned char *sb = smem + (wave * kApplyTiles + j) * W_BYTES;
+            const int k = kt * BK + 32 * st;  // (K is a multiple of 32: a k-step is inside or outside as a whole)
+            if (k >= K) break;
+            const unsigned char *xb = smem + (wave * per_wave + j) * STAGE, *wb = xb + X_BYTES;
             vec8 wf[NBN];
 #pragma unroll
-            for (int jj = 0; jj < NBN; ++jj) wf[jj] = *reinterpret_cast<const vec8 *>(sb + SmallTileMap::frag_offset(16 * jj + r, st, g));
+            for (int jj = 0; jj < NBN; ++jj) wf[jj] = *reinterpret_cast<const vec8 *>(wb + SmallTileMap::frag_offset(16 * jj + r, st, g));
+            const vec8 gam = *reinterpret_cast<const vec8 *>(smem + gamma_at + (k + 8 * g) * 2), bet = *reinterpret_cast<const vec8 *>(smem + beta_at + (k + 8 * g) * 2);
 #pragma unroll
             for (int i = 0; i < NBM; ++i) {
+                f32x4 x[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) x[h] = *reinterpret_cast<const f32x4 *>(xb + (16 * i + r) * 256 + (((8 * st + 2 * g + h) ^ r) & 15) * 16);
                 u32x4 packed;
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
                     float y[2];
 #pragma unroll
                     for (int e = 0; e < 2; ++e)
-                        y[e] = fmaf((x[j][st][i][p / 2][2 * (p % 2) + e] - mean[i]) * rstd[i], to_float(gam[j][st][2 * p + e]), to_float(bet[j][st][2 * p + e]));
+                        y[e] = fmaf((x[p / 2][2 * (p % 2) + e] - mean[i]) * rstd[i], to_float(gam[2 * p + e]), to_float(bet[2 * p + e]));
                     packed[p] = pack2<T>(y[0], y[1]);
                 }
                 const vec8 xf = __builtin_bit_cast(vec8, packed);
@@ -618,7 +626,7 @@ linear_norm_apply_kernel(const float *__restrict__ X, const T *__restrict__ W, c
             }
         }
     }
-    __syncthreads();  // the weight tiles are done with: the partial tiles take their place
+    __syncthreads();  // the k-tiles are done with
     float *red = reinterpret_cast<float *>(smem);  // [wave][block][lane][4]
 #pragma unroll
     for (int i = 0; i < NBM; ++i)
@@ -635,9 +643,9 @@ linear_norm_apply_kernel(const float *__restrict__ X, const T *__restrict__ W, c
     auto finish = [&](auto act_c) __attribute__((always_inline)) {
         constexpr int ACT = decltype(act_c)::value;
         float y[4];
+        unpack4<T>(bias_raw, y);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = apply_act16(sum[e] + bz[e], ACT);
-        // (N is a multiple of 32: every column of the tile exists)
+        for (int e = 0; e < 4; ++e) y[e] = apply_act16(sum[e] + y[e], ACT);
         *reinterpret_cast<u32x2 *>(out + (int64_t)(m0 + own_row) * out_rs + n_own) = u32x2{pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
     };
     switch (act) {
@@ -678,14 +686,13 @@ static void launch_small_dealt(const LinearArgs &a, int mode, const NormFold &nf
 template <typename T, int BM, int BN>
 static void launch_norm_apply(const LinearArgs &a, const NormFold &nf) {
     auto kern = linear_norm_apply_kernel<T, BM, BN>;
-    constexpr int LDS_BYTES = 4 * kApplyTiles * BN * 128 + norm_stats_bytes(BM);
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kApplyMaxLds);
         attr_done = true;
     }
     const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), LDS_BYTES, a.st, static_cast<const float *>(a.x),
+    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), apply_lds_bytes(BM, BN, a.K), a.st, static_cast<const float *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out), a.M, a.N, a.K, a.x_rs, a.out_rs,
                        a.act, tiles_m, nf);
 }
@@ -709,7 +716,7 @@ void run_small_dealt(const LinearArgs &a, int dtype, int rows, int cols, int mod
 template <typename T>
 static void run_norm_apply_t(const LinearArgs &a, int rows, int cols, const NormFold &nf) {
     if (cols == 16) launch_norm_apply<T, 16, 16>(a, nf);
-    else if (rows == 16) launch_norm_apply<T, 16, 32>(a, nf);
+    else if (rows == 16 || apply_lds_bytes(32, 32, a.K) > kApplyMaxLds) launch_norm_apply<T, 16, 32>(a, nf);
     else launch_norm_apply<T, 32, 32>(a, nf);
 }
 

@@ -65,6 +65,7 @@ __device__ __forceinline__ float quad_sum(float v) {
     v += dpp_mov<0x4E>(v);   // quad_perm [2,3,0,1]
     return v;
 }
+
 __device__ __forceinline__ float oct_sum(float v) {
     v = quad_sum(v);
     v += dpp_mov<0x141>(v);  // row_half_mirror
