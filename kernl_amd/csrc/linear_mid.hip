@@ -1,9 +1,9 @@
 // Linear layer for MIDDLING problems — 65 to some 3000 rows —, which give the big tile kernels less than a round of workgroups.
 //
-// What bounds such a launch: a CU's tile loads.  A CU takes 45 to 58 bytes per clock from L2 through its direct-to-LDS loads
-// whatever the depth of the ring (1024 x 4096 x 4096 with the matrix instructions and LDS reads taken out: 27 us with the weight
-// in the memory-side cache, 40 us from HBM; with the loads taken out: 28; whole: 42), so time is (BM + BN) x K x rounds, and
-// latency: barrier, LDS read and matrix instruction of a k-tile form a chain that four waves do not hide.  Hence
+// What bounds such a launch: a CU's tile loads, whatever the depth of the ring.  1024 x 4096 x 4096, 256 tiles of 128 x 128 that pull
+// 2.1 MB each: 42 us; with the matrix instructions and LDS reads taken out 27 us with the weight in the memory-side cache (78 GB/s
+// a CU) and 40 us from HBM (52 GB/s), with the loads taken out 28.  So time is (BM + BN) x K x rounds, and latency: barrier, LDS
+// read and matrix instruction of a k-tile form a chain that four waves do not hide.  Hence
 //   - tiles of 64 x 64 to 256 x 128, as large as still put a tile on (nearly) every CU;
 //   - eight waves, two per SIMD, and LDS fragments read one k-step ahead ACROSS the barrier (while k-step 1 of a k-tile is
 //     multiplied, k-step 0 of the next is read): 231 x 2304 x 768 in 64 x 64 tiles 7.6 -> 6.7 us against four waves that read, then
