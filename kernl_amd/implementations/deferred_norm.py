@@ -63,9 +63,9 @@ def _rows(t: torch.Tensor) -> Optional[torch.Tensor]:
     return t if t.stride(-1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 else None
 
 
-def deferrable(x: torch.Tensor, weight: torch.Tensor, bias, residual, gamma, beta, behind: Sequence[Tuple[int, int]]) -> bool:
-    """Whether layer_norm(linear(x, weight, bias) + residual, gamma, beta) can be left to the layers behind it, whose weights have
-    the sizes `behind`."""
+def deferrable(x: torch.Tensor, weight: torch.Tensor, bias, residual, gamma, beta, behind: Sequence[Tuple[torch.Tensor, ...]]) -> bool:
+    """Whether layer_norm(linear(x, weight, bias) + residual, gamma, beta) can be left to the layers behind it, whose weights are
+    `behind` (several for sibling projections, which run as one)."""
     n, k = weight.shape
     inner = residual.rows if isinstance(residual, DeferredNorm) else residual
     if not (x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and x.dim() >= 2 and x.numel() > 0 and gamma is not None):
@@ -75,8 +75,12 @@ def deferrable(x: torch.Tensor, weight: torch.Tensor, bias, residual, gamma, bet
     if inner.shape != (*x.shape[:-1], n) or gamma.shape != (n,) or n % 32 != 0 or n > MAX_WIDTH:
         return False
     rows = x.numel() // k
-    if not all(_takes(rows, a, b) for a, b in ((n, k), *behind)):
-        return False
+    for weights in ((weight,), *behind):
+        # (of siblings the rows are copied together, a single weight is read where and as it lies)
+        if len(weights) == 1 and not _plain(x.dtype, weights[0]) or any(w.dtype != x.dtype for w in weights):
+            return False
+        if not _takes(rows, sum(w.shape[0] for w in weights), weights[0].shape[1]):
+            return False
     return _rows(x) is not None and _rows(inner) is not None
 
 

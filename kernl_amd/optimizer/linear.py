@@ -773,9 +773,8 @@ def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, r
     from kernl_amd.optimizer.layer_norm import _half_params_once, add_layer_norm_wrapper_functional, layer_norm_wrapper_functional
 
     if (behind is not None and isinstance(residual, torch.Tensor) or isinstance(residual, DeferredNorm)) and len(normalized_shape) == 1:
-        _half_params_once(v, weight, bias, ln_weight, ln_bias)
-        sizes = [(sum(w.shape[0] for w in weights), weights[0].shape[1]) for weights in behind or ()]
-        if deferrable(v, weight, bias, residual, ln_weight, ln_bias, sizes):
+        _half_params_once(v, weight, bias, ln_weight, ln_bias, *(w for weights in behind or () for w in weights))
+        if deferrable(v, weight, bias, residual, ln_weight, ln_bias, behind or ()):
             norm = linear_add_deferred(v, weight, bias, residual, ln_weight, ln_bias, eps)
             return norm if behind is not None else norm.normalised()
     if isinstance(residual, DeferredNorm):

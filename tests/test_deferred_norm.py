@@ -193,6 +193,31 @@ def test_norms_whose_readers_do_not_take_them_are_carried_out(monkeypatch):
     assert list(calls.values()) == [0, 0, 0], calls
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("readers, deferred", [
+    ([["plain"]], True), ([["plain", "plain"], ["plain"]], True), ([["large"]], False), ([["large", "plain"]], False),
+    ([["plain"], ["transposed"]], False), ([["other type"]], False), ([["narrow"]], False),
+], ids=str)
+def test_a_norm_is_deferred_by_the_weights_that_read_it(readers, deferred):
+    from kernl_amd.implementations.deferred_norm import DeferredNorm
+    from kernl_amd.implementations.layer_norm import add_layer_norm
+    from kernl_amd.implementations.linear_layer import linear_layer
+    from kernl_amd.optimizer.linear import linear_add_layer_norm_wrapper
+
+    x, w, b, res, gamma, beta = _make(20, 768, 768, torch.float16, 1)
+    weights = {"plain": _make(1, 3072, 768, torch.float16, 2)[1], "large": torch.zeros(11008, 768, device="cuda").half(),
+               "transposed": torch.zeros(768, 768, device="cuda").half().t(), "other type": torch.zeros(768, 768, device="cuda").bfloat16(),
+               "narrow": torch.zeros(40, 768, device="cuda").half()}
+    behind = tuple(tuple(weights[name] for name in names) for names in readers)
+    out = linear_add_layer_norm_wrapper(x, w, b, res, (768,), gamma, beta, 1e-5, behind=behind)
+    assert isinstance(out, DeferredNorm) == deferred
+    want = add_layer_norm(linear_layer(x, w, b), res, gamma, beta, 1e-5)
+    if deferred:
+        assert (out.normalised() - want).abs().max() <= 2e-2  # (two roundings fewer)
+    else:
+        assert torch.equal(out, want)
+
+
 def test_only_norms_of_known_readers_are_marked():
     from kernl_amd.optimizer import linear
 
