@@ -33,7 +33,7 @@ void run_wide_half(const LinearArgs &a, int dtype, int cols);        // 128-row 
 void run_wide_half_w8(const LinearArgs &a);
 void run_half_split(const LinearArgs &a, const HalfSplitPlan &p, float *part, int dtype);
 void run_small(const LinearArgs &a, int dtype);                      // 32 x 64 tiles over the whole K (linear_small.hip)
-// 8-wave tiles over the whole K (linear_mid.hip), by hook value 11, 15, 17 .. 21; 0: that tile does not take the epilogue asked for
+// tiles with loading waves over the whole K (linear_mid.hip), by hook value 11, 15, 17 .. 22; 0: that tile does not take the epilogue asked for
 int run_mid(const LinearArgs &a, int dtype, int kind);
 struct NormFold;
 // 16- to 64-row, 16- or 32-column tiles, k-tiles dealt to the waves; mode: norm_fold.h (kNormAdd: a.out is fp32)
@@ -2068,15 +2068,44 @@ static int small_problem_kind(int64_t M, int64_t N, int64_t K) {
     return 0;
 }
 
-// Which 8-wave tile (linear_mid.hip) takes M x N x K beyond what small_problem_kind names, as its hook value, or 0 where another
-// kernel is faster.  `N`: rows of the weight (gated: twice the output columns).
-//  - short K: by tile counts, from a sweep of 65 .. 4096 rows over BERT's and wider weights (us, before -> with it): 768 x 3072 x 768
-//    12.9 -> 11.2, 1024 x 2304 x 768 12.1 -> 11.0, 1024 x 4096 x 1024 16.9 -> 15.5, 3072 x 768 x 768 12.0 -> 11.2.
-//  - long K: time = launch + k-tiles x rounds x the tile's measured time per k-tile (weights from HBM), or the weight's bytes at
-//    the HBM rate, against the same estimate for what would run otherwise: 1024 x 2048 x 2048 23.2 -> 15.3, 130 x 22016 x 4096 gated
-//    85 -> 53, 333 x 22016 x 4096 gated 88 -> 77, 160 x 12288 x 4096 44 -> 37, 768 x 4096 x 4096 50 -> 40, 768 x 4096 x 11008 126 -> 106,
-//    128 x 22016 x 4096 gated 64 -> 51 (few-row kernel), 1536 x 4096 x 11008 154 -> 139.  The kernels are within 5 % of the best tile
-//    of that sweep nearly everywhere.
+// Time of M x N x K on the tiles of linear_mid.hip, us: 2 (launch) + rounds x (ramp and epilogue + k-tiles x time of one).  Measured
+// per tile with the weight from the memory-side cache (up to 8 M elements) and from HBM, 65 .. 2048 rows, random data; the
+// estimates are within 10 % of the measurements.
+static double tile_round(int64_t tiles, double nk, double per_k) {  // a round in which every CU has a tile costs more than a sparse one
+    const int64_t rounds = (tiles + 255) / 256;
+    return nk * per_k * (0.74 + 0.26 * (double)tiles / (double)(256 * rounds));
+}
+struct MidChoice {
+    int tile = 0;  // hook value
+    double us = 1e30;
+};
+static MidChoice mid_tile_of(int64_t M, int64_t N, int64_t K, bool gated) {
+    struct Tile {
+        int kind, bm, bn;
+        double ramp, per_k_cached, per_k_hbm;
+    };
+    static constexpr Tile tiles[] = {{11, 64, 64, 1.8, 0.195, 0.26},  {15, 128, 64, 1.9, 0.27, 0.385},  {17, 128, 128, 2.9, 0.34, 0.53},
+                                     {22, 192, 96, 4.0, 0.36, 0.62},  {18, 192, 128, 4.2, 0.43, 0.67},  {19, 192, 192, 7.0, 0.60, 0.95},
+                                     {20, 128, 256, 4.6, 0.56, 0.86}, {21, 256, 128, 4.6, 0.555, 0.85}};
+    const bool cached = N * K <= ((int64_t)1 << 23);
+    const double nk = (double)((K + 63) / 64);
+    MidChoice best;
+    for (const Tile &t : tiles) {
+        if (gated && t.kind == 22) continue;
+        const int64_t n = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        double rounds = (double)((n + 255) / 256);
+        if (t.bn == 64 && n > 256) rounds *= 0.88;  // two workgroups share a CU
+        const double us = 2.0 + rounds * (t.ramp + tile_round(n, nk, cached ? t.per_k_cached : t.per_k_hbm));
+        if (us < best.us) best = MidChoice{t.kind, us};
+    }
+    return best;
+}
+
+// Whether M x N x K, beyond what small_problem_kind names, runs on the tiles of linear_mid.hip (or, 14, on 64 x 32 tiles with dealt
+// k-tiles), as a hook value; 0 where another kernel is faster.  `N`: rows of the weight (gated: twice the output columns).
+//  - short K: by tile counts, from a sweep of 65 .. 4096 rows over BERT's and wider weights.  15 and 17 stand for "short K" here: the
+//    tile itself is mid_tile_of's (768 x 3072 x 768: 128 x 128);
+//  - long K: by mid_tile_of against estimates for what would run otherwise.
 static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
     if (M <= 64 || N < 64 || K % 8 != 0 || K < 64 || M > 4096 || N > INT32_MAX / 64 || K >= (1 << 22) || (gated && N % 64 != 0)) return 0;
     auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -2089,27 +2118,13 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
     if (short_k || (M <= 128 && N * K < 12 * (1 << 20))) return 0;
     const double nk = (double)((K + 63) / 64), hbm = 4.0 + (double)(N * K) * 2.0 / 4.6e6;  // us at 4.6 TB/s
     auto cost = [&](int bm, int bn, double per_k) {
-        const int64_t t = tiles(bm, bn);
-        double rounds = (double)((t + 255) / 256);
-        if (bn == 64 && t > 256 && t <= 512) rounds = 1.6;  // two workgroups per CU
-        const double c = 3.5 + nk * per_k * rounds;
-        return c > hbm ? c : hbm;
+        const int64_t n = tiles(bm, bn);
+        return 3.5 + (double)((n + 255) / 256) * tile_round(n, nk, per_k);
     };
-    int best = 0;
-    double best_cost = 1e30;
-    auto offer = [&](int kind, double c) {
-        if (c < best_cost) { best_cost = c; best = kind; }
-    };
-    offer(11, cost(64, 64, 0.285));
-    offer(15, cost(128, 64, 0.45));
-    offer(17, cost(128, 128, 0.62));
-    offer(18, cost(192, 128, 0.83));
-    offer(19, cost(192, 192, 1.15));
-    offer(20, cost(128, 256, 0.98));
-    offer(21, cost(256, 128, 0.97));
-    double other = cost(256, 256, 1.38);
+    MidChoice best = mid_tile_of(M, N, K, gated);
+    double other = cost(256, 256, 1.55);
     if (!gated) {
-        const double c6 = cost(256, 192, 1.34), c7 = cost(128, 256, 0.90), c8 = cost(128, 192, 0.755);
+        const double c6 = cost(256, 192, 1.38), c7 = cost(128, 256, 0.90), c8 = cost(128, 192, 0.79);
         other = other < c6 ? other : c6;
         other = other < c7 ? other : c7;
         other = other < c8 ? other : c8;
@@ -2123,16 +2138,17 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
     if (M <= 128 && K % 64 == 0) {
         const double few = 10.0 + (double)(N * K) * 2.0 / 3.7e6;
         other = other < few ? other : few;
+        best.us = best.us > hbm ? best.us : hbm;
         // 64 x 32 tiles with dealt k-tiles, one round of them: 128 x 4096 x 4096 20.8 -> 17.3
         if (!gated && tiles(64, 32) <= 256) {
             const double c = 3.5 + nk * 0.2;
-            offer(14, c > hbm ? c : hbm);
+            if ((c > hbm ? c : hbm) < best.us) best = MidChoice{14, c > hbm ? c : hbm};
         }
     }
-    return best_cost < 0.97 * other ? best : 0;
+    return best.us < 0.97 * other ? best.tile : 0;
 }
 
-extern int g_linear_force_tile;  // test / tuning hook (defined in linear.hip): 0 = heuristic, 1 = 256x256, 2 = 256x192, 3 = 128x128, 4 = 256x128 k32, 5 = wide 256x256, 6 = wide 256x192, 7 = wide 128x256, 8 = wide 128x192, 10 = 32 x 64, 12 .. 14 and 16 = dealt k-tiles, 11, 15, 17 .. 21 = the 8-wave tiles of linear_mid.hip
+extern int g_linear_force_tile;  // test / tuning hook (defined in linear.hip): 0 = heuristic, 1 = 256x256, 2 = 256x192, 3 = 128x128, 4 = 256x128 k32, 5 = wide 256x256, 6 = wide 256x192, 7 = wide 128x256, 8 = wide 128x192, 10 = 32 x 64, 12 .. 14 and 16 = dealt k-tiles, 11, 15, 17 .. 22 = the tiles of linear_mid.hip
 
 template <typename T, bool GATED, int MB, int NR, bool W8, bool RMS = false, bool ROPE = false, bool XL = false>
 static void launch_skinny_blocks(const LinearArgs &a, const void *rms_w = nullptr, float eps = 0.0f,

@@ -1,30 +1,37 @@
 // Linear layer for MIDDLING problems — 65 to some 3000 rows —, which give the big tile kernels less than a round of workgroups.
 //
-// What bounds such a launch: a CU's tile loads, whatever the depth of the ring.  1024 x 4096 x 4096, 256 tiles of 128 x 128 that pull
-// 2.1 MB each: 42 us; with the matrix instructions and LDS reads taken out 27 us with the weight in the memory-side cache (78 GB/s
-// a CU) and 40 us from HBM (52 GB/s), with the loads taken out 28.  So time is (BM + BN) x K x rounds, and latency: barrier, LDS
-// read and matrix instruction of a k-tile form a chain that four waves do not hide.  Hence
-//   - tiles of 64 x 64 to 256 x 128, as large as still put a tile on (nearly) every CU;
-//   - eight waves, two per SIMD, and LDS fragments read one k-step ahead ACROSS the barrier (while k-step 1 of a k-tile is
-//     multiplied, k-step 0 of the next is read): 231 x 2304 x 768 in 64 x 64 tiles 7.6 -> 6.7 us against four waves that read, then
-//     multiply; sched_barrier keeps the compiler from moving the reads back behind the multiplications;
-//   - the small tiles in rings of 64 to 72 KB, so that two workgroups share a CU where there are more tiles than CUs (512 x 3072 x 768
-//     in 128 x 64 tiles 10.5 -> 8.4 us, 1024 x 3072 x 768 13.1 -> 12.0).
+// What bounds such a launch: the tile loads of a CU.  It keeps some 32 KB of loads in flight however deep the ring is, so that they
+// arrive at 32 KB per latency: 58 GB/s where the operands come from HBM, 110 from the memory-side cache, 140 from its L2 (a kernel
+// that only loads, 256 workgroups; ring depths of 64 and 128 KB and every cache policy the same).  Loads of a line by several CUs at
+// the same time wait the full latency each.  And where the waves that load also multiply, a full load path holds up their LDS reads
+// and matrix instructions: 1024 x 768 x 3072 in 64 x 64 tiles took 15.5 us, the same with the loads alone 11.6, without them 8.9.  Hence
+//   - waves that only load (four, behind the eight that multiply): what they wait for, nobody else waits for.  1024 x 768 x 3072
+//     15.5 -> 13.0 us, 1024 x 3072 x 768 11.3 -> 9.8 in 128 x 128 tiles, 231 x 2304 x 768 6.6 -> 5.9;
+//   - k-tiles dealt among the workgroups that share a weight tile: within a group of k-tiles each starts kDealt k-tiles behind the
+//     one before it and wraps around, so every line is fetched from HBM by one of them and found in the XCD's L2 by the others.
+//     1024 x 4096 x 4096 in 128 x 128 tiles (weights from HBM; before either: 41) 39.6 -> 34.3 us, 512 x 12288 x 4096 in 256 x 128
+//     tiles 54.7 -> 50.8, 333 x 22016 x 4096 in 192 x 192 tiles 66.5 -> 63.7.  Nothing to gain where the weight stays in the
+//     memory-side cache (1024 x 768 x 768 6.15 against 6.28);
+//   - tiles of 64 x 64 to 256 x 128, as large as still put a tile on (nearly) every CU: (BM + BN) x K bytes a tile;
+//   - LDS fragments read one k-step ahead ACROSS the barrier (while k-step 1 of a k-tile is multiplied, k-step 0 of the next is read);
+//     sched_barrier keeps the compiler from moving the reads back behind the multiplications;
+//   - the small tiles in rings of 64 to 72 KB, so that two workgroups share a CU where there are more tiles than CUs.
 // Weight rows are placed in LDS so that a lane's blocks are consecutive output columns: 16-byte stores.
 #include "linear_kernels.h"
 #include "norm_fold.h"
 
 namespace kernl {
 
-// tile shape, wave grid and ring depth of one build of the kernel
-template <int BM_, int BN_, int WM_, int WN_, int S_>
+// tile shape, grid of the eight multiplying waves, ring depth and number of loading waves (0: the multiplying waves load) of one build
+template <int BM_, int BN_, int WM_, int WN_, int S_, int NP_ = 4>
 struct MidTile {
-    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_;
-    static constexpr int BK = 64, RB = BK * 2;
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_, NP = NP_;
+    static constexpr int BK = 64, RB = BK * 2, WAVES = 8 + NP, LOADERS = NP > 0 ? NP : 8;
     static constexpr int TM = BM / WM, TN = BN / WN, NBM = TM / 16, NBN = TN / 16;
+    static constexpr bool X_AHEAD = TM * TN < 96 * 48;  // registers for two sets of x fragments
     static constexpr int X_BYTES = BM * RB, STAGE = (BM + BN) * RB, LDS = S * STAGE;
-    static constexpr int LX = BM / 64, LW = BN / 64, L = LX + LW;
-    static_assert(WM * WN == 8 && BM % 64 == 0 && BN % 64 == 0 && LDS <= 160 * 1024 && S >= 3 && (S - 1) * L <= 63, "tile shape");
+    static constexpr int LX = BM / (8 * LOADERS), LW = BN / (8 * LOADERS), L = LX + LW;  // 1 KB loads of a loading wave per k-tile
+    static_assert(WM * WN == 8 && LX * 8 * LOADERS == BM && LW * 8 * LOADERS == BN && LDS <= 160 * 1024 && S >= 3 && (S - 1) * L <= 63, "tile shape");
 };
 
 // How the tile grid is dealt to the 8 XCDs, each with an L2 of its own: as 2^xm_shift x 8 / 2^xm_shift blocks of per_m x per_n tiles,
@@ -32,7 +39,10 @@ struct MidTile {
 // the 55 that a run of 24 tiles per XCD, which spans all of x, asks for).  per_m = 0: runs of tiles, the row tile fastest.
 struct MidGrid {
     int xm_mask = 0, xm_shift = 0, per_m = 0, per_n = 0;
+    int k_group = 1;  // k-tiles are dealt in groups of `k_group` runs of kDealt k-tiles (below)
 };
+
+static constexpr int kDealt = 2;
 
 // which weight row of the tile LDS row `row` carries: the lane's blocks become consecutive output columns
 template <bool GATED, int TN>
@@ -46,7 +56,7 @@ __device__ __forceinline__ int mid_weight_row(int row) {
 }
 
 template <typename T, typename Cfg, bool GATED>
-__global__ void __launch_bounds__(512, 2)
+__global__ void __launch_bounds__(Cfg::WAVES * 64, Cfg::WAVES / 4)
 linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
                   T *__restrict__ act_in, const float *__restrict__ row_scale, const T *__restrict__ residual, int M, int N, int K,
                   int64_t ldx, int64_t out_rs, int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int64_t res_rs, int64_t res_cs, int act,
@@ -57,6 +67,8 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_m = wave % Cfg::WM, wave_n = wave / Cfg::WM;
+    const bool loads = Cfg::NP == 0 || wave >= 8;
+    const int loader = Cfg::NP == 0 ? wave : (wave & 7) % Cfg::LOADERS;
     const int r = lane & 15, g = lane >> 4;
     // workgroup b runs on XCD b % 8, which works on a block of the tile grid of its own (or on a contiguous run of tiles)
     int tile_m, tile_n;
@@ -71,6 +83,7 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
         tile_n = tile / tiles_m;
     }
     const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int k_first = tile_m % grid.k_group * kDealt;
 
     constexpr uint32_t kOutOfRange = 0x80000000u;
     const int rows_x = min(BM, M - m0), rows_w = min(BN, N - n0);
@@ -79,22 +92,22 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     const u32x4 xrsrc = {(uint32_t)xaddr, (uint32_t)(xaddr >> 32) & 0xFFFFu, (uint32_t)((((int64_t)rows_x - 1) * ldx + K) * 2), 0x00020000u};
     const u32x4 wrsrc = {(uint32_t)waddr, (uint32_t)(waddr >> 32) & 0xFFFFu, (uint32_t)((int64_t)rows_w * K * 2), 0x00020000u};
     const int nk = (K + BK - 1) / BK, k_last = K - (nk - 1) * BK;
-    // load i of a wave fills the 1 KB (8 rows) piece i * 8 + wave of the operand tile
+    // load i of a loading wave fills the 1 KB (8 rows) piece i * LOADERS + loader of the operand tile
     uint32_t xd[LX], wd[LW], tail_bits = 0;
 #pragma unroll
     for (int i = 0; i < LX; ++i) {
-        const int q = (i * 8 + wave) * 64 + lane, row = SmallTileMap::load_row(q), c = SmallTileMap::load_chunk(q);
+        const int q = (i * Cfg::LOADERS + loader) * 64 + lane, row = SmallTileMap::load_row(q), c = SmallTileMap::load_chunk(q);
         xd[i] = row < rows_x ? (uint32_t)(((int64_t)row * ldx + c * 8) * 2) : kOutOfRange;
         if (c * 8 < k_last) tail_bits |= 1u << i;
     }
 #pragma unroll
     for (int i = 0; i < LW; ++i) {
-        const int q = (i * 8 + wave) * 64 + lane, row = mid_weight_row<GATED, Cfg::TN>(SmallTileMap::load_row(q)), c = SmallTileMap::load_chunk(q);
+        const int q = (i * Cfg::LOADERS + loader) * 64 + lane, row = mid_weight_row<GATED, Cfg::TN>(SmallTileMap::load_row(q)), c = SmallTileMap::load_chunk(q);
         wd[i] = row < rows_w ? (uint32_t)(((int64_t)row * K + c * 8) * 2) : kOutOfRange;
         if (c * 8 < k_last) tail_bits |= 1u << (LX + i);
     }
     typedef __attribute__((address_space(3))) void lds_void;
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_void *)smem + wave * 1024;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_void *)smem + loader * 1024;
     auto load1 = [&](const u32x4 &rsrc, uint32_t off, uint32_t lds, int kbytes) __attribute__((always_inline)) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :: "s"(lds), "v"(off), "s"(rsrc), "s"(kbytes) : "memory", "m0");
@@ -106,22 +119,27 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
 #pragma unroll
         for (int i = 0; i < LW; ++i) wd[i] = ((keep >> (LX + i)) & 1u) != 0 ? wd[i] : kOutOfRange;
     };
+    // the order in which a workgroup walks its k-tiles: within every group of k_group * kDealt k-tiles it starts k_first behind the
+    // group's begin and wraps around
+    const int k_span = grid.k_group * kDealt, k_dealt = K / BK / k_span * k_span;
+    int k_at = k_first, k_base = 0;
     auto request = [&](int kt, int stage) __attribute__((always_inline)) {
         if (kt == nk - 1 || kt == nk) clip(kt == nk ? 0u : tail_bits);
         const uint32_t base = lds_base + (uint32_t)stage * STAGE;
-        const int kbytes = kt < nk ? kt * BK * 2 : 0;
+        const int kbytes = kt < nk ? (kt < k_dealt ? k_base + k_at : kt) * BK * 2 : 0;
+        k_at = k_at + 1 == k_span ? 0 : k_at + 1;
+        k_base = k_at == k_first ? k_base + k_span : k_base;
 #pragma unroll
-        for (int i = 0; i < LX; ++i) load1(xrsrc, xd[i], base + i * 8192, kbytes);
+        for (int i = 0; i < LX; ++i) load1(xrsrc, xd[i], base + i * Cfg::LOADERS * 1024, kbytes);
 #pragma unroll
-        for (int i = 0; i < LW; ++i) load1(wrsrc, wd[i], base + Cfg::X_BYTES + i * 8192, kbytes);
+        for (int i = 0; i < LW; ++i) load1(wrsrc, wd[i], base + Cfg::X_BYTES + i * Cfg::LOADERS * 1024, kbytes);
     };
-    int xoff[2][NBM], woff[2][NBN];
+    // (the blocks of a wave lie 16 rows apart, which leaves the swizzle as it is)
+    int xoff[2], woff[2];
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
-#pragma unroll
-        for (int i = 0; i < NBM; ++i) xoff[st][i] = SmallTileMap::frag_offset(wave_m * Cfg::TM + 16 * i + r, st, g);
-#pragma unroll
-        for (int j = 0; j < NBN; ++j) woff[st][j] = Cfg::X_BYTES + SmallTileMap::frag_offset(wave_n * Cfg::TN + 16 * j + r, st, g);
+        xoff[st] = SmallTileMap::frag_offset(wave_m * Cfg::TM + r, st, g);
+        woff[st] = Cfg::X_BYTES + SmallTileMap::frag_offset(wave_n * Cfg::TN + r, st, g);
     }
     f32x4_acc acc[NBM][NBN];
 #pragma unroll
@@ -136,49 +154,89 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     typedef uint32_t words __attribute__((ext_vector_type(V / 2)));
     const int out_n = GATED ? N / 2 : N;
     const int n_first = (GATED ? n0 / 2 : n0) + wave_n * (GATED ? Cfg::TN / 2 : Cfg::TN) + C * g;
-    float bz[NBN][4];
+    u32x2 bias_raw[NBN];  // 16-bit values until the epilogue: registers are short in the large tiles
     const bool bias_vec = ((uintptr_t)bias & 7) == 0;
 #pragma unroll
-    for (int j = 0; j < NBN; ++j)
-        load_bias4<T>(bias, n0 + mid_weight_row<GATED, Cfg::TN>(wave_n * Cfg::TN + 16 * j + 4 * g), N, bias_vec, bz[j]);
+    for (int j = 0; j < NBN; ++j) {
+        const int n = n0 + mid_weight_row<GATED, Cfg::TN>(wave_n * Cfg::TN + 16 * j + 4 * g);
+        if (bias != nullptr && bias_vec && n + 4 <= N) {
+            bias_raw[j] = *reinterpret_cast<const u32x2 *>(bias + n);
+            continue;
+        }
+        uint32_t b16[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b16[e] = bias != nullptr && n + e < N ? reinterpret_cast<const uint16_t *>(bias)[n + e] : 0;
+        bias_raw[j] = u32x2{b16[0] | b16[1] << 16, b16[2] | b16[3] << 16};
+    }
     auto wait_loads = [&](auto n_c) __attribute__((always_inline)) {
         constexpr int n = decltype(n_c)::value;
         __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
     };
+    if (loads)
 #pragma unroll
-    for (int kt = 0; kt < S; ++kt) request(kt, kt);
+        for (int kt = 0; kt < S; ++kt) request(kt, kt);
+    if constexpr (Cfg::NP > 0) {
+        if (loads) {
+            // a loading wave: its stalls on the load path hold up neither the LDS reads nor the matrix instructions of the others
+            wait_loads(IntC<(S - 1) * L>());
+            __syncthreads();
+            int stage = 0;
+            for (int kt = 0; kt < nk; ++kt) {
+                wait_loads(IntC<(S - 2) * L>());
+                __syncthreads();  // as below
+                request(kt + S, stage);
+                stage = stage == S - 1 ? 0 : stage + 1;
+            }
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            return;
+        }
+    }
 
-    vec8 xf[2][NBM], wf[2][NBN];
-    auto read = [&](int st, int stage) __attribute__((always_inline)) {
+    // Fragments are read one k-step ahead, across the barrier.  The large tiles have no registers for a second set of x fragments: theirs
+    // are overwritten one by one, each as soon as its row of blocks is done.
+    constexpr int XB = Cfg::X_AHEAD ? 2 : 1;
+    vec8 xf[XB][NBM], wf[2][NBN];
+    auto read = [&](int st, int stage, bool x_too) __attribute__((always_inline)) {
+        const unsigned char *sb = smem + stage * STAGE;
+        if (x_too)
+#pragma unroll
+            for (int i = 0; i < NBM; ++i) xf[st % XB][i] = *reinterpret_cast<const vec8 *>(sb + xoff[st] + i * 2048);
+#pragma unroll
+        for (int j = 0; j < NBN; ++j) wf[st][j] = *reinterpret_cast<const vec8 *>(sb + woff[st] + j * 2048);
+    };
+    // k-step st, and the x fragments of the next one (of `stage`) where they wait for registers
+    auto multiply = [&](int st, int stage) __attribute__((always_inline)) {
         const unsigned char *sb = smem + stage * STAGE;
 #pragma unroll
-        for (int i = 0; i < NBM; ++i) xf[st][i] = *reinterpret_cast<const vec8 *>(sb + xoff[st][i]);
+        for (int i = 0; i < NBM; ++i) {
 #pragma unroll
-        for (int j = 0; j < NBN; ++j) wf[st][j] = *reinterpret_cast<const vec8 *>(sb + woff[st][j]);
+            for (int j = 0; j < NBN; ++j) acc[i][j] = mfma16(wf[st][j], xf[st % XB][i], acc[i][j]);
+            if (XB == 1) {
+                xf[0][i] = *reinterpret_cast<const vec8 *>(sb + xoff[1 - st] + i * 2048);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
     };
-    auto multiply = [&](int st) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NBM; ++i)
-#pragma unroll
-            for (int j = 0; j < NBN; ++j) acc[i][j] = mfma16(wf[st][j], xf[st][i], acc[i][j]);
-    };
-    wait_loads(IntC<(S - 1) * L>());
+    if constexpr (Cfg::NP == 0) wait_loads(IntC<(S - 1) * L>());
     __syncthreads();
-    read(0, 0);
+    read(0, 0, true);
     int stage = 0;
     for (int kt = 0; kt < nk; ++kt) {
         const int next = stage == S - 1 ? 0 : stage + 1;
-        read(1, stage);
+        read(1, stage, XB == 2);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(0);
+        multiply(0, stage);
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        wait_loads(IntC<(S - 2) * L>());
+        if constexpr (Cfg::NP == 0) wait_loads(IntC<(S - 2) * L>());
         __syncthreads();  // k-tile kt + 1 has landed for everyone, and nobody reads k-tile kt any more
-        request(kt + S, stage);
-        read(0, next);
+        read(0, next, XB == 2);
+        if constexpr (Cfg::NP == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            request(kt + S, stage);
+        }
         __builtin_amdgcn_sched_barrier(0);
-        multiply(1);
+        multiply(1, next);
         __builtin_amdgcn_sched_barrier(0);
         stage = next;
     }
@@ -202,6 +260,9 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     };
     auto finish = [&](auto act_c) __attribute__((always_inline)) {
         constexpr int ACT = decltype(act_c)::value;
+        float bz[NBN][4];
+#pragma unroll
+        for (int j = 0; j < NBN; ++j) unpack4<T>(bias_raw[j], bz[j]);
 #pragma unroll
         for (int i = 0; i < NBM; ++i) {
             const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
@@ -270,44 +331,40 @@ static void launch_mid_cfg(const LinearArgs &a) {
         grid.xm_mask = xm - 1; grid.xm_shift = s; grid.per_m = pm; grid.per_n = pn;
         blocks = 8 * pm * pn;
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(512), Cfg::LDS, a.st, static_cast<const T *>(a.x),
+    // k-tiles are dealt where the weight comes from HBM: 8 M elements and more
+    if ((int64_t)a.N * a.K > ((int64_t)1 << 23)) grid.k_group = grid.per_m != 0 ? grid.per_m : tiles_m;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(Cfg::WAVES * 64), Cfg::LDS, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out), static_cast<T *>(a.act_in),
                        a.row_scale, static_cast<const T *>(a.residual), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs,
                        a.res_rs, a.res_cs, a.act & (kGluBit - 1), tiles_m, grid);
 }
 
-// the tiles, by the kernl_linear_force_tile value that forces them
+// the tiles, by the kernl_linear_force_tile value that forces them (and mid_tile_of names)
 typedef MidTile<64, 64, 4, 2, 4> Mid64x64;      // 11   64 KB: two workgroups per CU
 typedef MidTile<128, 64, 4, 2, 3> Mid128x64;    // 15   72 KB: two workgroups per CU
 typedef MidTile<128, 128, 2, 4, 4> Mid128x128;  // 17
 typedef MidTile<192, 128, 4, 2, 4> Mid192x128;  // 18
-typedef MidTile<192, 192, 4, 2, 3> Mid192x192;  // 19
+typedef MidTile<192, 192, 2, 4, 3> Mid192x192;  // 19   (six column blocks a wave spill without the gates' pairing,
+typedef MidTile<192, 192, 4, 2, 3> Mid192x192g; //       which needs them even in number)
 typedef MidTile<128, 256, 2, 4, 3> Mid128x256;  // 20
 typedef MidTile<256, 128, 4, 2, 3> Mid256x128;  // 21
-
-template <typename T, typename Cfg>
-static int launch_mid(const LinearArgs &a) {
-    if (a.act & kGluBit) {
-        if constexpr (Cfg::NBN % 2 == 0) {
-            launch_mid_cfg<T, Cfg, true>(a);
-            return 1;
-        }
-        return 0;
-    }
-    launch_mid_cfg<T, Cfg, false>(a);
-    return 1;
-}
+typedef MidTile<192, 96, 4, 2, 4> Mid192x96;    // 22   no gates: an odd number of column blocks
 
 template <typename T>
 static int run_mid_t(const LinearArgs &a, int kind) {
+    const bool gated = (a.act & kGluBit) != 0;
     switch (kind) {
-        case 11: return launch_mid<T, Mid64x64>(a);
-        case 15: return launch_mid<T, Mid128x64>(a);
-        case 17: return launch_mid<T, Mid128x128>(a);
-        case 18: return launch_mid<T, Mid192x128>(a);
-        case 19: return launch_mid<T, Mid192x192>(a);
-        case 20: return launch_mid<T, Mid128x256>(a);
-        case 21: return launch_mid<T, Mid256x128>(a);
+        case 11: gated ? launch_mid_cfg<T, Mid64x64, true>(a) : launch_mid_cfg<T, Mid64x64, false>(a); return 1;
+        case 15: gated ? launch_mid_cfg<T, Mid128x64, true>(a) : launch_mid_cfg<T, Mid128x64, false>(a); return 1;
+        case 17: gated ? launch_mid_cfg<T, Mid128x128, true>(a) : launch_mid_cfg<T, Mid128x128, false>(a); return 1;
+        case 18: gated ? launch_mid_cfg<T, Mid192x128, true>(a) : launch_mid_cfg<T, Mid192x128, false>(a); return 1;
+        case 19: gated ? launch_mid_cfg<T, Mid192x192g, true>(a) : launch_mid_cfg<T, Mid192x192, false>(a); return 1;
+        case 20: gated ? launch_mid_cfg<T, Mid128x256, true>(a) : launch_mid_cfg<T, Mid128x256, false>(a); return 1;
+        case 21: gated ? launch_mid_cfg<T, Mid256x128, true>(a) : launch_mid_cfg<T, Mid256x128, false>(a); return 1;
+        case 22:
+            if (gated) return 0;
+            launch_mid_cfg<T, Mid192x96, false>(a);
+            return 1;
         default: return 0;
     }
 }
