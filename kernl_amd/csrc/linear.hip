@@ -21,9 +21,9 @@ static void dealt_tile(int M, int N, int kind, int &rows, int &cols) {
 // Runs the kernel a value of small_problem_kind / mid_kind (or of the hook) names; 0: it does not take this epilogue.
 static int run_one_launch(const LinearArgs &a, int dtype, int kind) {
     if (kind == 11 || kind == 15 || kind >= 17) {
-        // (the hook's value as it is; otherwise the rules name the kernel and the estimate its tile)
-        const int tile = g_linear_force_tile != 0 ? kind : mid_tile_of(a.M, a.N, a.K, (a.act & kGluBit) != 0).tile;
-        return run_mid(a, dtype, tile);
+        // (the hook's value and what small_problem_kind names as they are; beyond them mid_kind names the kernel and the estimate its tile)
+        const bool as_named = g_linear_force_tile != 0 || (!(a.act & kGluBit) && small_problem_kind(a.M, a.N, a.K) != 0);
+        return run_mid(a, dtype, as_named ? kind : mid_tile_of(a.M, a.N, a.K, (a.act & kGluBit) != 0).tile);
     }
     if ((a.act & kGluBit) || a.row_scale != nullptr || a.residual != nullptr) return 0;
     if (kind == 10) {

@@ -30,6 +30,10 @@ struct HalfSplitPlan;
 void run_wide(const LinearArgs &a, int dtype, int cols);             // 256-row tiles; the gated epilogue when a.act says so
 void run_wide_w8(const LinearArgs &a);                               // fp8 e5m2 weights, fp16 activations
 void run_wide_half(const LinearArgs &a, int dtype, int cols);        // 128-row tiles
+// the same with dealt k-tiles (k_tiles_dealt): run_wide and run_wide_half hand over what run_wide_dealt_takes
+bool run_wide_dealt_takes(const LinearArgs &a);
+void run_wide_dealt(const LinearArgs &a, int dtype, int cols);
+void run_wide_half_dealt(const LinearArgs &a, int dtype, int cols);
 void run_wide_half_w8(const LinearArgs &a);
 void run_half_split(const LinearArgs &a, const HalfSplitPlan &p, float *part, int dtype);
 void run_small(const LinearArgs &a, int dtype);                      // 32 x 64 tiles over the whole K (linear_small.hip)
@@ -661,12 +665,21 @@ __device__ __forceinline__ void wide_epilogue(f32x4_acc (&acc)[NBM][NBN], int m_
                                                        ai_cs, out_vec_ok, ai_vec_ok, bf, rs, none);
 }
 
+// The order in which a workgroup walks the k-tiles of an output tile: within every group of four, k-tile kt ^ turn.  A line that
+// several CUs request from HBM at the same time costs each of them the full latency, and a CU keeps only some 32 KB of loads in
+// flight; with turns 0 .. 3 dealt along the rows and columns of the tile grid, each of the workgroups of an XCD that share
+// a weight (or x) tile is the first to ask for a quarter of its lines and finds the others in L2.  Measured in sustained replay with
+// weights from HBM: 2048 x 12288 x 4096 168.5 -> 160.5 us, 2048 x 4096 x 11008 163 -> 157, 1024 x 12288 x 4096 90 -> 84.5.  Where the
+// weight stays in the memory-side cache (8 M elements and less) there is nothing to gain (16384 x 2304 x 768 56.2 -> 59.6).
+__host__ __device__ static inline bool k_tiles_dealt(int64_t N, int64_t K) { return N * K > ((int64_t)1 << 23); }
+// (DEAL of the wide kernels: whole groups only, for the epilogues that products with large weights have; linear_wide_dealt.hip.)
+
 // W8: the weight is stored as one byte per element (fp8 e5m2, the upper byte of the fp16 encoding).  Its tile travels
 // HBM -> LDS as bytes (half the loads, 64-byte rows, chunks swizzled for 8-byte reads), a fragment is read as 8 bytes
 // and widened by four byte-permutes two read slots later, all in the shadow of the MFMAs; everything else is unchanged.
 // SCALED: the finished sums are multiplied by a factor per row of x (row_scale, fp32 [M]) before the bias is added.
 // RES: a residual matrix is added to the rounded results (plain epilogues only).
-template <typename T, int ACT, int NBN, bool W8 = false, bool SCALED = false, bool RES = false>
+template <typename T, int ACT, int NBN, bool W8 = false, bool SCALED = false, bool RES = false, bool DEAL = false>
 __global__ void __launch_bounds__(256, 1)
 linear_wide_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
                    T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs, int64_t out_cs,
@@ -833,7 +846,7 @@ linear_wide_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__
     if (!tile_origin(idx, m0, n0)) return;
 
     // the load side runs ahead of the multiply side: (load_idx, load_kt) is the next k-tile to request
-    int load_idx = idx, load_kt = 0;
+    int load_idx = idx, load_kt = 0, turn = DEAL ? (m0 / BM + n0 / BN) & 3 : 0;
     set_load_tile(true, m0, n0);
     if (tail_kt == 0) clip_tail();
     auto advance_load = [&]() __attribute__((always_inline)) {
@@ -843,14 +856,15 @@ linear_wide_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__
             int lm0 = 0, ln0 = 0;
             const bool more = tile_origin(load_idx, lm0, ln0);
             set_load_tile(more, lm0, ln0);
+            if constexpr (DEAL) turn = (lm0 / BM + ln0 / BN) & 3;
         }
         if (load_kt == tail_kt) clip_tail();
     };
 #pragma unroll
-    for (int l = 0; l < NL; ++l) tile_load(l, 0, load_kt * BK);
+    for (int l = 0; l < NL; ++l) tile_load(l, 0, (DEAL ? load_kt ^ turn : load_kt) * BK);
     advance_load();
 #pragma unroll
-    for (int l = 0; l < NL; ++l) tile_load(l, 1, load_kt * BK);
+    for (int l = 0; l < NL; ++l) tile_load(l, 1, (DEAL ? load_kt ^ turn : load_kt) * BK);
     advance_load();
     // vmcnt(NL): the first k-tile has landed, the second may still be in flight
     __builtin_amdgcn_s_waitcnt(0x0F70 | (NL & 15) | ((NL >> 4) << 14));
@@ -873,7 +887,7 @@ linear_wide_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__
     auto k_tile = [&](auto cur_c, bool landed, auto first_c) __attribute__((always_inline)) {
         constexpr int CUR = decltype(cur_c)::value;
         constexpr bool FIRST = decltype(first_c)::value;  // the first k-tile of an output tile: its first k-step starts the sums
-        const int k0 = load_kt * BK;
+        const int k0 = (DEAL ? load_kt ^ turn : load_kt) * BK;
 #pragma unroll
         for (int st = 0; st < KSTEPS; ++st) {
             const int sn = st ^ 1;                               // k-step whose fragments are fetched now
@@ -995,7 +1009,7 @@ __device__ __forceinline__ void half_tile_origin(int t, int tiles_m, int tiles_n
 // SPLIT: blockIdx.y selects one of `splits` ranges of k-tiles; the workgroup leaves its fp32 partial tile in `part`
 // (slot blockIdx.y * tiles + t; per wave and 16 x 16 block 64 lanes x 16 bytes: coalesced, and the same lane reads it
 // back in linear_wide_half_reduce_kernel, which adds the ranges in order and runs the epilogue).
-template <typename T, int ACT, int NBN, bool W8 = false, bool SPLIT = false, bool SCALED = false, bool RES = false>
+template <typename T, int ACT, int NBN, bool W8 = false, bool SPLIT = false, bool SCALED = false, bool RES = false, bool DEAL = false>
 __global__ void __launch_bounds__(256, 1)
 linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias,
                         T *__restrict__ out, T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs,
@@ -1123,9 +1137,10 @@ linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const 
         kb = (int)blockIdx.y * per_split;
         nk = min(per_split, nk - kb);   // the host keeps every range non-empty
     }
+    const int turn = DEAL ? (m0 / BM + n0 / BN) & 3 : 0;
 #pragma unroll
     for (int s3 = 0; s3 < 3; ++s3) {
-        const int k0 = (kb + min(s3, nk - 1)) * BK;
+        const int k0 = (kb + (DEAL ? min(s3, nk - 1) ^ turn : min(s3, nk - 1))) * BK;
         if (k0 == tail_k0) clip_tail();   // (clipping twice changes nothing)
 #pragma unroll
         for (int l = 0; l < NL; ++l) tile_load(l, s3, k0);
@@ -1171,7 +1186,7 @@ linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const 
     };
     auto k_tile = [&](auto cur_c, int kt) __attribute__((always_inline)) {
         constexpr int CUR = decltype(cur_c)::value, NXT = (CUR + 1) % 3;
-        const int k_next = (kb + min(kt + 3, nk - 1)) * BK;
+        const int k_next = (kb + (DEAL ? min(kt + 3, nk - 1) ^ turn : min(kt + 3, nk - 1))) * BK;
         if (k_next == tail_k0 && kt + 3 == nk - 1) clip_tail();   // once: later requests are for this k-tile again
 #pragma unroll
         for (int st = 0; st < KSTEPS; ++st) {
@@ -1817,9 +1832,9 @@ static void launch_mfma_glu(const LinearArgs &a) {
     }
 }
 
-template <typename T, int ACT, int NBN = 8, bool W8 = false, bool SCALED = false, bool RES = false>
+template <typename T, int ACT, int NBN = 8, bool W8 = false, bool SCALED = false, bool RES = false, bool DEAL = false>
 static void launch_wide_act(const LinearArgs &a) {
-    auto kern = linear_wide_kernel<T, ACT, NBN, W8, SCALED, RES>;
+    auto kern = linear_wide_kernel<T, ACT, NBN, W8, SCALED, RES, DEAL>;
     constexpr int LDS_BYTES = 2 * (256 + 256) * 128;  // two stages
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
@@ -1842,9 +1857,9 @@ static void launch_wide_act(const LinearArgs &a) {
                        a.ai_cs, tiles_m, tiles_n, out_vec_ok, ai_vec_ok, bias_vec_ok, a.row_scale, wide_residual_of<T, NBN>(a));
 }
 
-template <typename T, int ACT, int NBN, bool W8 = false, bool SCALED = false, bool RES = false>
+template <typename T, int ACT, int NBN, bool W8 = false, bool SCALED = false, bool RES = false, bool DEAL = false>
 static void launch_wide_half_act(const LinearArgs &a) {
-    auto kern = linear_wide_half_kernel<T, ACT, NBN, W8, false, SCALED, RES>;
+    auto kern = linear_wide_half_kernel<T, ACT, NBN, W8, false, SCALED, RES, DEAL>;
     constexpr int LDS_BYTES = 3 * 16384 + 3 * 32768;  // three stages
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
@@ -2122,9 +2137,9 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
         return 3.5 + (double)((n + 255) / 256) * tile_round(n, nk, per_k);
     };
     MidChoice best = mid_tile_of(M, N, K, gated);
-    double other = cost(256, 256, 1.55);
+    double other = cost(256, 256, 1.50);
     if (!gated) {
-        const double c6 = cost(256, 192, 1.38), c7 = cost(128, 256, 0.90), c8 = cost(128, 192, 0.79);
+        const double c6 = cost(256, 192, 1.30), c7 = cost(128, 256, 0.87), c8 = cost(128, 192, 0.79);
         other = other < c6 ? other : c6;
         other = other < c7 ? other : c7;
         other = other < c8 ? other : c8;

@@ -7,11 +7,9 @@
 // and matrix instructions: 1024 x 768 x 3072 in 64 x 64 tiles took 15.5 us, the same with the loads alone 11.6, without them 8.9.  Hence
 //   - waves that only load (four, behind the eight that multiply): what they wait for, nobody else waits for.  1024 x 768 x 3072
 //     15.5 -> 13.0 us, 1024 x 3072 x 768 11.3 -> 9.8 in 128 x 128 tiles, 231 x 2304 x 768 6.6 -> 5.9;
-//   - k-tiles dealt among the workgroups that share a weight tile: within a group of k-tiles each starts kDealt k-tiles behind the
-//     one before it and wraps around, so every line is fetched from HBM by one of them and found in the XCD's L2 by the others.
-//     1024 x 4096 x 4096 in 128 x 128 tiles (weights from HBM; before either: 41) 39.6 -> 34.3 us, 512 x 12288 x 4096 in 256 x 128
-//     tiles 54.7 -> 50.8, 333 x 22016 x 4096 in 192 x 192 tiles 66.5 -> 63.7.  Nothing to gain where the weight stays in the
-//     memory-side cache (1024 x 768 x 768 6.15 against 6.28);
+//   - k-tiles dealt among the workgroups that share a weight or x tile (k_turn_mask in linear_kernels.h): 1024 x 4096 x 4096 in 128 x 128
+//     tiles, weights from HBM, 39.6 -> 34.5 us, 512 x 12288 x 4096 in 256 x 128 tiles 54.7 -> 51, 333 x 22016 x 4096 in 192 x 192
+//     tiles 66.5 -> 63; from the memory-side cache 1024 x 768 x 3072 12.5 -> 12.1, 231 x 768 x 3072 11.9 -> 11.2;
 //   - tiles of 64 x 64 to 256 x 128, as large as still put a tile on (nearly) every CU: (BM + BN) x K bytes a tile;
 //   - LDS fragments read one k-step ahead ACROSS the barrier (while k-step 1 of a k-tile is multiplied, k-step 0 of the next is read);
 //     sched_barrier keeps the compiler from moving the reads back behind the multiplications;
@@ -39,10 +37,7 @@ struct MidTile {
 // the 55 that a run of 24 tiles per XCD, which spans all of x, asks for).  per_m = 0: runs of tiles, the row tile fastest.
 struct MidGrid {
     int xm_mask = 0, xm_shift = 0, per_m = 0, per_n = 0;
-    int k_group = 1;  // k-tiles are dealt in groups of `k_group` runs of kDealt k-tiles (below)
 };
-
-static constexpr int kDealt = 2;
 
 // which weight row of the tile LDS row `row` carries: the lane's blocks become consecutive output columns
 template <bool GATED, int TN>
@@ -83,7 +78,8 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
         tile_n = tile / tiles_m;
     }
     const int m0 = tile_m * BM, n0 = tile_n * BN;
-    const int k_first = tile_m % grid.k_group * kDealt;
+    // the order of the k-tiles, as in the wide kernels (linear_kernels.h) but for any K: whole groups of four are dealt
+    const int turn = (tile_m + tile_n) & 3, k_dealt = K / (4 * BK) * 4;
 
     constexpr uint32_t kOutOfRange = 0x80000000u;
     const int rows_x = min(BM, M - m0), rows_w = min(BN, N - n0);
@@ -119,16 +115,10 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
 #pragma unroll
         for (int i = 0; i < LW; ++i) wd[i] = ((keep >> (LX + i)) & 1u) != 0 ? wd[i] : kOutOfRange;
     };
-    // the order in which a workgroup walks its k-tiles: within every group of k_group * kDealt k-tiles it starts k_first behind the
-    // group's begin and wraps around
-    const int k_span = grid.k_group * kDealt, k_dealt = K / BK / k_span * k_span;
-    int k_at = k_first, k_base = 0;
     auto request = [&](int kt, int stage) __attribute__((always_inline)) {
         if (kt == nk - 1 || kt == nk) clip(kt == nk ? 0u : tail_bits);
         const uint32_t base = lds_base + (uint32_t)stage * STAGE;
-        const int kbytes = kt < nk ? (kt < k_dealt ? k_base + k_at : kt) * BK * 2 : 0;
-        k_at = k_at + 1 == k_span ? 0 : k_at + 1;
-        k_base = k_at == k_first ? k_base + k_span : k_base;
+        const int kbytes = kt < nk ? (kt < k_dealt ? kt ^ turn : kt) * BK * 2 : 0;
 #pragma unroll
         for (int i = 0; i < LX; ++i) load1(xrsrc, xd[i], base + i * Cfg::LOADERS * 1024, kbytes);
 #pragma unroll
@@ -331,8 +321,6 @@ static void launch_mid_cfg(const LinearArgs &a) {
         grid.xm_mask = xm - 1; grid.xm_shift = s; grid.per_m = pm; grid.per_n = pn;
         blocks = 8 * pm * pn;
     }
-    // k-tiles are dealt where the weight comes from HBM: 8 M elements and more
-    if ((int64_t)a.N * a.K > ((int64_t)1 << 23)) grid.k_group = grid.per_m != 0 ? grid.per_m : tiles_m;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(Cfg::WAVES * 64), Cfg::LDS, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out), static_cast<T *>(a.act_in),
                        a.row_scale, static_cast<const T *>(a.residual), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs,

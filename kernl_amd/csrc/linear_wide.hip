@@ -4,6 +4,7 @@
 namespace kernl {
 
 void run_wide(const LinearArgs &a, int dtype, int cols) {
+    if (run_wide_dealt_takes(a)) return run_wide_dealt(a, dtype, cols);
     if (cols == 192) {
         if (dtype == KERNL_F16) launch_wide192<f16>(a);
         else launch_wide192<bf16>(a);

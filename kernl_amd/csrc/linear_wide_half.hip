@@ -5,6 +5,7 @@
 namespace kernl {
 
 void run_wide_half(const LinearArgs &a, int dtype, int cols) {
+    if (run_wide_dealt_takes(a)) return run_wide_half_dealt(a, dtype, cols);
     if (cols == 192) {
         if (dtype == KERNL_F16) launch_wide_half<f16, 6>(a);
         else launch_wide_half<bf16, 6>(a);

@@ -57,3 +57,17 @@ def test_gates_with_dealt_k_tiles(force, close):
     _lib.linear_glu_fwd(x.cuda(), interleave_glu_rows(wg, wv).cuda(), None, out, _lib.ACT_SILU)
     torch.cuda.synchronize()
     close(out, glu_oracle(x, wg, None, wv, None, "silu"), scale="magnitude", what="gated")
+
+
+@pytest.mark.parametrize("tile", [5, 6, 7, 8])
+# whole groups of four k-tiles (dealt), an odd number of groups, and a K that leaves the order as it is
+@pytest.mark.parametrize("shape", [(600, 8300, 1024), (300, 4200, 2304), (1100, 4096, 2112)], ids=str)
+def test_dealt_k_tiles_of_the_wide_kernels(shape, tile, force, close):
+    M, N, K = shape
+    gen = torch.Generator().manual_seed(M + tile)
+    x, w = torch.randn((M, K), generator=gen).half(), (torch.randn((N, K), generator=gen) * K ** -0.5).half()
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    force(tile)
+    _lib.linear_fwd(x.cuda(), w.cuda(), None, out, None, _lib.ACT_NONE)
+    torch.cuda.synchronize()
+    close(out, linear_oracle(x, w, None, ""), what=f"tile {tile} {shape}")
