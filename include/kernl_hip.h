@@ -330,8 +330,8 @@ int kernl_linear_mid_kind(int64_t M, int64_t N, int64_t K, int gated);
 
 /*
  * kernl_linear_fwd for row counts between the two regimes (129 to a few hundred rows against a few thousand columns),
- * where the 128-row tiles of the tiled kernels are too few to occupy the chip: every output tile is computed by up to
- * four workgroups over disjoint ranges of K, and a second small launch adds their fp32 partial tiles in range order and
+ * where the tiles of the other kernels are too few to occupy the chip: every output tile is computed by up to
+ * eight workgroups over disjoint ranges of K, and a second small launch adds their fp32 sums in range order and
  * runs the epilogue (same semantics and arguments as kernl_linear_fwd, reference src/kernl/implementations/
  * linear_layer.py:92-210; the split over K is the `SPLIT_K` axis of the reference's configurations, which it leaves
  * at 1, linear_layer.py:47-67).
@@ -346,6 +346,20 @@ int kernl_linear_splitk_fwd(const void *x, const void *w, const void *bias, void
                             int64_t workspace_bytes, int64_t M, int64_t N, int64_t K, const int64_t x_strides[2],
                             const int64_t out_strides[2], const int64_t act_in_strides[2], int activation, int dtype,
                             void *stream);
+
+/*
+ * Split K for 65 to 4096 rows where it beats one pass over K, with the second launch finishing the rows.  `finish`: 0 bias and
+ * activation (kernl_linear_splitk_fwd takes it), 1 round(product + bias) + residual, 2 the same with rstd[m] = 1 / sqrt(mean(row^2) + eps)
+ * of the rounded row, 3 LayerNorm(product + bias + residual) * gamma + beta, added and normalised in fp32.
+ *   kernl_linear_split_workspace_bytes: 0 where splitting does not pay, else the bytes of a 16-byte aligned workspace (contents
+ *   irrelevant; calls that overlap in time need workspaces of their own).
+ *   f16 / bf16; x [M, K], residual and out [M, N] with unit feature strides and the given row strides, N a multiple of 4 up to 8192;
+ *   anything else returns KERNL_ERR_UNSUPPORTED.  No reference counterpart: its models add and normalise in kernels of their own.
+ */
+int64_t kernl_linear_split_workspace_bytes(int64_t M, int64_t N, int64_t K, int finish);
+int kernl_linear_split_fwd(const void *x, const void *w, const void *bias, const void *residual, const void *gamma, const void *beta,
+                           float eps, void *out, float *rstd, void *workspace, int64_t workspace_bytes, int64_t M, int64_t N, int64_t K,
+                           int64_t x_rs, int64_t res_rs, int64_t out_rs, int finish, int dtype, void *stream);
 
 /*
  * The linear layer for a FEW rows of x with many columns and a long K (batched decoding steps: 17 to 128 rows, where

@@ -52,6 +52,8 @@ EXPORTED_SYMBOLS = (
     "kernl_linear_decode_fwd",
     "kernl_linear_splitk_workspace_bytes",
     "kernl_linear_splitk_fwd",
+    "kernl_linear_split_workspace_bytes",
+    "kernl_linear_split_fwd",
     "kernl_linear_fewrow_workspace_bytes",
     "kernl_linear_fewrow_fwd",
     "kernl_linear_fewrow_w8_fwd",
@@ -140,6 +142,10 @@ def load() -> ctypes.CDLL:
     )
     lib.kernl_linear_splitk_workspace_bytes.restype = _i64
     lib.kernl_linear_splitk_workspace_bytes.argtypes = [_i64] * 3
+    lib.kernl_linear_split_workspace_bytes.restype = _i64
+    lib.kernl_linear_split_workspace_bytes.argtypes = [_i64] * 3 + [ctypes.c_int]
+    lib.kernl_linear_split_fwd.restype = ctypes.c_int
+    lib.kernl_linear_split_fwd.argtypes = [_vp] * 6 + [ctypes.c_float] + [_vp] * 3 + [_i64] * 7 + [ctypes.c_int, ctypes.c_int, _vp]
     lib.kernl_linear_splitk_fwd.restype = ctypes.c_int
     lib.kernl_linear_splitk_fwd.argtypes = [_vp] * 6 + [_i64] * 4 + [_i64p] * 3 + [ctypes.c_int, ctypes.c_int, _vp]
     lib.kernl_linear_fewrow_workspace_bytes.restype = _i64
@@ -585,6 +591,28 @@ def linear_splitk_fwd(x2d, weight, bias, out2d, act_in2d, activation: int, works
             None if act_in2d is None else _arr(act_in2d.stride()), int(activation), DTYPE_CODE[x2d.dtype], _stream(x2d),
         )
     _check(st, "kernl_linear_splitk_fwd")
+
+
+FINISH_PLAIN, FINISH_RESIDUAL, FINISH_RMS_STATS, FINISH_LAYER_NORM = range(4)
+
+
+def linear_split_workspace_bytes(M: int, N: int, K: int, finish: int = FINISH_PLAIN) -> int:
+    """Bytes of workspace where splitting K beats one pass over it (65 to 4096 rows); 0 where it does not."""
+    return int(load().kernl_linear_split_workspace_bytes(M, N, K, finish))
+
+
+def linear_split_fwd(x2d, weight, bias, residual2d, gamma, beta, eps: float, out2d, rstd, workspace, finish: int) -> None:
+    """`kernl_linear_split_fwd`: the product with K split, its rows finished (residual, row statistics or LayerNorm)."""
+    _require_gpu(x2d, weight, bias, residual2d, gamma, beta, out2d, rstd, workspace)
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    lib = load()
+    with torch.cuda.device(x2d.device):
+        st = lib.kernl_linear_split_fwd(
+            x2d.data_ptr(), weight.data_ptr(), ptr(bias), residual2d.data_ptr(), ptr(gamma), ptr(beta), float(eps), out2d.data_ptr(), ptr(rstd),
+            workspace.data_ptr(), workspace.numel() * workspace.element_size(), x2d.shape[0], out2d.shape[1], x2d.shape[1], x2d.stride(0),
+            residual2d.stride(0), out2d.stride(0), int(finish), DTYPE_CODE[x2d.dtype], _stream(x2d),
+        )
+    _check(st, "kernl_linear_split_fwd")
 
 
 def linear_fewrow_supported(x2d, weight) -> bool:

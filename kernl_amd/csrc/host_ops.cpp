@@ -510,6 +510,21 @@ PyObject *op_linear(PyObject *const *a, Py_ssize_t n) {
         Py_RETURN_NONE;
     const int act = (int)integer(a[3]);
     const bool vectors = r.vectors() && aligned16(*x) && aligned16(*w);
+    auto split = [&](int64_t need) {  // too few tiles to occupy the chip: ranges of K per tile, added by a second launch
+        const at::Tensor out = output_for(*x, N);
+        const int64_t os[2] = {N, 1};
+        const at::Tensor ws = at::empty({need}, x->options().dtype(at::kByte));
+        const int dt = dtype_code(*x);
+        Py_XDECREF(launched(*x, "kernl_linear_splitk_fwd", [&](void *stream) {
+            return kernl_linear_splitk_fwd(x->data_ptr(), w->data_ptr(), data(bias), out.data_ptr(), data(act_in), ws.data_ptr(), need, M, N, K,
+                                           r.strides, os, act_in == nullptr ? nullptr : act_in->strides().data(), act, dt, stream);
+        }));
+        return THPVariable_Wrap(out);
+    };
+    if (vectors && K % 64 == 0 && M > 64 && r.strides[0] < (1 << 22)) {
+        const int64_t need = kernl_linear_split_workspace_bytes(M, N, K, 0);
+        if (need > 0) return split(need);
+    }
     const bool small = vectors && ((truth(a[5]) && kernl_linear_small_kind(M, N, K) != 0) ||
                                    (M > 64 && r.strides[0] < (1 << 22) && kernl_linear_mid_kind(M, N, K, 0) != 0));
     const at::Tensor out = output_for(*x, N);
@@ -523,17 +538,7 @@ PyObject *op_linear(PyObject *const *a, Py_ssize_t n) {
         }
         if (M > kFewRowMax && M <= kSplitKMaxRows && r.strides[0] < (1 << 22) && K < (1 << 22)) {
             const int64_t need = kernl_linear_splitk_workspace_bytes(M, N, K);
-            if (need > 0) {
-                // too few 128-row tiles to occupy the chip: ranges of K per tile, added by a second launch
-                const at::Tensor ws = at::empty({need}, x->options().dtype(at::kByte));
-                const int dt = dtype_code(*x);
-                Py_XDECREF(launched(*x, "kernl_linear_splitk_fwd", [&](void *stream) {
-                    return kernl_linear_splitk_fwd(x->data_ptr(), w->data_ptr(), data(bias), out.data_ptr(), data(act_in), ws.data_ptr(),
-                                                   need, M, N, K, r.strides, os, act_in == nullptr ? nullptr : act_in->strides().data(),
-                                                   act, dt, stream);
-                }));
-                return THPVariable_Wrap(out);
-            }
+            if (need > 0) return split(need);
         }
     }
     Py_XDECREF(run_linear(*x, *w, bias, out, act_in, act, M, N, K, r.strides, os));

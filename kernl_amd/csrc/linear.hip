@@ -144,10 +144,24 @@ extern "C" int kernl_linear_fwd(const void *x, const void *w, const void *bias, 
     return set_error(KERNL_ERR_UNSUPPORTED, "linear: unknown dtype %d", dtype);
 }
 
+namespace kernl {
+static void run_split(const LinearArgs &a, int dtype, const SplitPlan &p, void *workspace, const SplitFinish &finish) {
+    MidSplit s;
+    s.splits = p.splits;
+    s.range_kt = p.range_kt;
+    s.part_rs = p.part_rs;
+    s.part = static_cast<float *>(workspace);
+    LinearArgs product = a;
+    product.bias = product.residual = nullptr;
+    run_mid_split(product, dtype, p.tile, s);
+    run_split_finish(a, dtype, s, finish);
+}
+}  // namespace kernl
+
 extern "C" int64_t kernl_linear_splitk_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     using namespace kernl;
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || M > INT32_MAX || N > INT32_MAX || K >= (1 << 22)) return 0;
-    return half_split_plan(M, N, K).bytes;
+    return half_split_takes(M, N, K) ? split_plan_of(M, N, K).bytes : 0;
 }
 
 extern "C" int kernl_linear_splitk_fwd(const void *x, const void *w, const void *bias, void *out, void *act_in,
@@ -170,11 +184,11 @@ extern "C" int kernl_linear_splitk_fwd(const void *x, const void *w, const void 
         x_strides[1] != 1 || x_strides[0] % 8 != 0 || !aligned16(x) || !aligned16(w))
         return set_error(KERNL_ERR_UNSUPPORTED, "linear (split K): K must be a multiple of 64, x needs unit feature stride "
                          "and 16-byte aligned rows, the weight a 16-byte aligned base");
-    const HalfSplitPlan p = half_split_plan(M, N, K);
-    if (p.splits < 2)
+    if (!half_split_takes(M, N, K) && split_plan_that_pays(M, N, K, kFinishPlain).tile == 0)
         return set_error(KERNL_ERR_UNSUPPORTED, "linear (split K): nothing to split for M=%lld N=%lld K=%lld "
                          "(kernl_linear_splitk_workspace_bytes returns 0): use kernl_linear_fwd", (long long)M, (long long)N,
                          (long long)K);
+    const SplitPlan p = split_plan_of(M, N, K);
     if (workspace == nullptr || workspace_bytes < p.bytes || !aligned16(workspace))
         return set_error(KERNL_ERR_INVALID_ARG, "linear (split K): the workspace must hold %lld bytes, 16-byte aligned",
                          (long long)p.bytes);
@@ -186,8 +200,61 @@ extern "C" int kernl_linear_splitk_fwd(const void *x, const void *w, const void 
     a.ai_rs = act_in ? act_in_strides[0] : 0; a.ai_cs = act_in ? act_in_strides[1] : 0;
     a.act = activation;
     a.st = static_cast<hipStream_t>(stream);
-    run_half_split(a, p, static_cast<float *>(workspace), dtype);
+    run_split(a, dtype, p, workspace, SplitFinish());
     return check_launch("linear (split K)");
+}
+
+extern "C" int64_t kernl_linear_split_workspace_bytes(int64_t M, int64_t N, int64_t K, int finish) {
+    using namespace kernl;
+    if (M <= 0 || N <= 0 || K <= 0 || M > INT32_MAX || finish < kFinishPlain || finish > kFinishLayerNorm) return 0;
+    const SplitPlan p = split_plan_that_pays(M, N, K, finish);
+    return p.tile != 0 ? p.bytes : 0;
+}
+
+extern "C" int kernl_linear_split_fwd(const void *x, const void *w, const void *bias, const void *residual, const void *gamma,
+                                      const void *beta, float eps, void *out, float *rstd, void *workspace, int64_t workspace_bytes,
+                                      int64_t M, int64_t N, int64_t K, int64_t x_rs, int64_t res_rs, int64_t out_rs, int finish, int dtype,
+                                      void *stream) {
+    using namespace kernl;
+    if (x == nullptr || w == nullptr || residual == nullptr || out == nullptr)
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (split K, rows finished): x, w, residual and out must not be NULL");
+    if (finish < kFinishResidual || finish > kFinishLayerNorm)
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (split K, rows finished): unknown finish %d", finish);
+    if ((finish == kFinishRmsStats && rstd == nullptr) || (finish == kFinishLayerNorm && gamma == nullptr))
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (split K, rows finished): row statistics need rstd, a LayerNorm gamma");
+    if (M <= 0 || N <= 0 || K <= 0 || workspace_bytes < 0)
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (split K, rows finished): bad sizes M=%lld N=%lld K=%lld", (long long)M, (long long)N,
+                         (long long)K);
+    if (dtype != KERNL_F16 && dtype != KERNL_BF16)
+        return set_error(KERNL_ERR_UNSUPPORTED, "linear (split K, rows finished): only f16 and bf16 are supported, got dtype %d", dtype);
+    auto aligned8 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; };
+    if (M > INT32_MAX || K >= (1 << 22) || x_rs >= (1 << 22) || K % 8 != 0 || x_rs % 8 != 0 || x_rs < K || !aligned16(x) || !aligned16(w) ||
+        res_rs % 4 != 0 || out_rs % 4 != 0 || !aligned8(bias) || !aligned8(residual) || !aligned8(gamma) || !aligned8(beta) || !aligned8(out))
+        return set_error(KERNL_ERR_UNSUPPORTED, "linear (split K, rows finished): K must be a multiple of 8, x and w 16-byte aligned with 16-byte "
+                         "aligned rows, everything else 8-byte aligned");
+    const SplitPlan p = split_plan_that_pays(M, N, K, finish);
+    if (p.tile == 0)
+        return set_error(KERNL_ERR_UNSUPPORTED, "linear (split K, rows finished): nothing to split for M=%lld N=%lld K=%lld "
+                         "(kernl_linear_split_workspace_bytes returns 0)", (long long)M, (long long)N, (long long)K);
+    if (workspace == nullptr || workspace_bytes < p.bytes || !aligned16(workspace))
+        return set_error(KERNL_ERR_INVALID_ARG, "linear (split K, rows finished): the workspace must hold %lld bytes, 16-byte aligned",
+                         (long long)p.bytes);
+    LinearArgs a;
+    a.x = x; a.w = w; a.bias = bias; a.out = out; a.act_in = nullptr;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K;
+    a.x_rs = x_rs; a.x_cs = 1;
+    a.out_rs = out_rs; a.out_cs = 1;
+    a.ai_rs = 0; a.ai_cs = 0;
+    a.act = KERNL_ACT_NONE;
+    a.st = static_cast<hipStream_t>(stream);
+    a.residual = residual;
+    a.res_rs = res_rs; a.res_cs = 1;
+    SplitFinish f;
+    f.kind = finish;
+    f.gamma = gamma; f.beta = beta; f.eps = eps;
+    f.rstd = rstd;
+    run_split(a, dtype, p, workspace, f);
+    return check_launch("linear (split K, rows finished)");
 }
 
 extern "C" int kernl_linear_glu_fwd(const void *x, const void *w, const void *bias, void *out, int64_t M, int64_t N,

@@ -26,7 +26,6 @@ namespace kernl {
 // units of their own (linear_wide.hip, linear_wide_half.hip) behind these functions, so that a build runs them in parallel.
 // dtype: KERNL_F16 / KERNL_BF16; cols: 256 or 192 output columns per tile.
 struct LinearArgs;
-struct HalfSplitPlan;
 void run_wide(const LinearArgs &a, int dtype, int cols);             // 256-row tiles; the gated epilogue when a.act says so
 void run_wide_w8(const LinearArgs &a);                               // fp8 e5m2 weights, fp16 activations
 void run_wide_half(const LinearArgs &a, int dtype, int cols);        // 128-row tiles
@@ -35,10 +34,28 @@ bool run_wide_dealt_takes(const LinearArgs &a);
 void run_wide_dealt(const LinearArgs &a, int dtype, int cols);
 void run_wide_half_dealt(const LinearArgs &a, int dtype, int cols);
 void run_wide_half_w8(const LinearArgs &a);
-void run_half_split(const LinearArgs &a, const HalfSplitPlan &p, float *part, int dtype);
 void run_small(const LinearArgs &a, int dtype);                      // 32 x 64 tiles over the whole K (linear_small.hip)
 // tiles with loading waves over the whole K (linear_mid.hip), by hook value 11, 15, 17 .. 22; 0: that tile does not take the epilogue asked for
 int run_mid(const LinearArgs &a, int dtype, int kind);
+// the same with K split over `splits` workgroups a tile, which leave fp32 sums [splits][M][part_rs] for run_split_finish
+struct MidSplit {
+    int splits = 1, range_kt = 0;
+    int64_t part_rs = 0;
+    float *part = nullptr;
+};
+void run_mid_split(const LinearArgs &a, int dtype, int tile, const MidSplit &split);
+// what becomes of the ranges' sums (linear_finish.hip)
+constexpr int kFinishPlain = 0;       // bias, activation
+constexpr int kFinishResidual = 1;    // bias, rounded, residual added, rounded
+constexpr int kFinishRmsStats = 2;    // the same, with 1 / sqrt(mean(sum^2) + eps) per row
+constexpr int kFinishLayerNorm = 3;   // bias and residual added in fp32, LayerNorm
+struct SplitFinish {
+    int kind = kFinishPlain;
+    const void *gamma = nullptr, *beta = nullptr;
+    float eps = 0.0f;
+    float *rstd = nullptr;
+};
+void run_split_finish(const LinearArgs &a, int dtype, const MidSplit &split, const SplitFinish &finish);
 struct NormFold;
 // 16- to 64-row, 16- or 32-column tiles, k-tiles dealt to the waves; mode: norm_fold.h (kNormAdd: a.out is fp32)
 void run_small_dealt(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf);
@@ -1006,17 +1023,12 @@ __device__ __forceinline__ void half_tile_origin(int t, int tiles_m, int tiles_n
     n0 = (in_group / gsize) * BN;
 }
 
-// SPLIT: blockIdx.y selects one of `splits` ranges of k-tiles; the workgroup leaves its fp32 partial tile in `part`
-// (slot blockIdx.y * tiles + t; per wave and 16 x 16 block 64 lanes x 16 bytes: coalesced, and the same lane reads it
-// back in linear_wide_half_reduce_kernel, which adds the ranges in order and runs the epilogue).
-template <typename T, int ACT, int NBN, bool W8 = false, bool SPLIT = false, bool SCALED = false, bool RES = false, bool DEAL = false>
+template <typename T, int ACT, int NBN, bool W8 = false, bool SCALED = false, bool RES = false, bool DEAL = false>
 __global__ void __launch_bounds__(256, 1)
 linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias,
                         T *__restrict__ out, T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs,
                         int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int tiles_m, int tiles_n, int out_vec_ok,
-                        int ai_vec_ok, int bias_vec_ok, float *__restrict__ part, int splits,
-                        const float *__restrict__ row_scale, const WideResidual residual) {
-    static_assert(!RES || !SPLIT, "the split form leaves its epilogue to the reduction launch");
+                        int ai_vec_ok, int bias_vec_ok, const float *__restrict__ row_scale, const WideResidual residual) {
     typedef typename Vec8<T>::type vec8;
     static_assert((ACT & kGluBit) == 0 && (NBN == 8 || NBN == 6), "plain epilogues, 256 or 192 columns");
     constexpr int NBM = 4, BM = 32 * NBM, BN = 32 * NBN, BK = 64, RB = BK * 2, CPR = BK / 8, KSTEPS = BK / 32;
@@ -1081,8 +1093,8 @@ linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const 
     };
     // K % 64 != 0: chunks of the last k-tile that start at or beyond K are pointed out of range and arrive as zeros,
     // in both operands (as in the wide kernel); bit l of `tail_bits`: load l of this lane stays inside
-    const int nk_all = (K + BK - 1) / BK;
-    const int k_last = K - (nk_all - 1) * BK;
+    const int nk = (K + BK - 1) / BK;
+    const int k_last = K - (nk - 1) * BK;
     uint32_t tail_bits = 0;
 #pragma unroll
     for (int i = 0; i < LOADS_X; ++i) {
@@ -1096,7 +1108,7 @@ linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const 
     }
     // clipped in place when the ragged k-tile is the next one to request: every request after it is for that k-tile
     // again.  A branch that K % 64 == 0 never takes; a select per load would cost every k-tile of every shape.
-    const int tail_k0 = (K % BK) != 0 ? (nk_all - 1) * BK : -1;
+    const int tail_k0 = (K % BK) != 0 ? (nk - 1) * BK : -1;
     auto clip_tail = [&]() __attribute__((always_inline)) {
         asm volatile("" ::: "memory");  // keeps this a branch: without it the compiler turns the block into selects
 #pragma unroll
@@ -1131,16 +1143,10 @@ linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const 
 
     // Every k-tile slot issues its NL loads, so that the counter waits stay exact up to the end; requests past the
     // last k-tile fetch that tile again (into a stage nobody reads any more) instead of running past the row ends.
-    int nk = nk_all, kb = 0;   // k-tiles of this workgroup: kb .. kb + nk - 1
-    if constexpr (SPLIT) {
-        const int per_split = (nk + splits - 1) / splits;
-        kb = (int)blockIdx.y * per_split;
-        nk = min(per_split, nk - kb);   // the host keeps every range non-empty
-    }
     const int turn = DEAL ? (m0 / BM + n0 / BN) & 3 : 0;
 #pragma unroll
     for (int s3 = 0; s3 < 3; ++s3) {
-        const int k0 = (kb + (DEAL ? min(s3, nk - 1) ^ turn : min(s3, nk - 1))) * BK;
+        const int k0 = (DEAL ? min(s3, nk - 1) ^ turn : min(s3, nk - 1)) * BK;
         if (k0 == tail_k0) clip_tail();   // (clipping twice changes nothing)
 #pragma unroll
         for (int l = 0; l < NL; ++l) tile_load(l, s3, k0);
@@ -1186,7 +1192,7 @@ linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const 
     };
     auto k_tile = [&](auto cur_c, int kt) __attribute__((always_inline)) {
         constexpr int CUR = decltype(cur_c)::value, NXT = (CUR + 1) % 3;
-        const int k_next = (kb + (DEAL ? min(kt + 3, nk - 1) ^ turn : min(kt + 3, nk - 1))) * BK;
+        const int k_next = (DEAL ? min(kt + 3, nk - 1) ^ turn : min(kt + 3, nk - 1)) * BK;
         if (k_next == tail_k0 && kt + 3 == nk - 1) clip_tail();   // once: later requests are for this k-tile again
 #pragma unroll
         for (int st = 0; st < KSTEPS; ++st) {
@@ -1246,15 +1252,6 @@ linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const 
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): no load may still be writing LDS when the workgroup ends
 
-    if constexpr (SPLIT) {
-        float4 *dst = reinterpret_cast<float4 *>(part) + ((((int64_t)blockIdx.y * total + t) * 4 + wave) * (NBM * NBN)) * 64 + lane;
-#pragma unroll
-        for (int i = 0; i < NBM; ++i)
-#pragma unroll
-            for (int j = 0; j < NBN; ++j)
-                dst[(i * NBN + j) * 64] = float4{acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-        return;
-    }
     const int n_wave = n0 + wave_n * (NBN * 16);
     uint32_t braw[NBN / 2];
     float bf[NBN];
@@ -1269,61 +1266,6 @@ linear_wide_half_kernel(const T *__restrict__ X, const T *__restrict__ W, const 
     KERNL_HALF_EPILOGUE(2);
     KERNL_HALF_EPILOGUE(3);
 #undef KERNL_HALF_EPILOGUE
-}
-
-// Second launch of the split form: workgroup (t, I) adds the k ranges' partial sums of 16-row block I of every wave of
-// tile t, in range order, and runs the epilogue the unsplit kernel runs (same wave and lane geometry).
-template <typename T, int ACT, int NBN>
-__global__ void __launch_bounds__(256)
-linear_wide_half_reduce_kernel(const float *__restrict__ part, const T *__restrict__ bias, T *__restrict__ out,
-                               T *__restrict__ act_in, int M, int N, int64_t out_rs, int64_t out_cs, int64_t ai_rs,
-                               int64_t ai_cs, int tiles_m, int tiles_n, int out_vec_ok, int ai_vec_ok, int bias_vec_ok,
-                               int splits) {
-    constexpr int NBM = 4, BM = 32 * NBM, BN = 32 * NBN;
-    const int t = (int)blockIdx.x, I = (int)blockIdx.y, total = tiles_m * tiles_n;
-    int m0, n0;
-    half_tile_origin(t, tiles_m, tiles_n, BM, BN, m0, n0);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wave_m = wave & 1, wave_n = wave >> 1;
-    const int l16 = lane & 15, g = lane >> 4;
-    f32x4_acc acc[NBM][NBN];
-#pragma unroll
-    for (int i = 0; i < NBM; ++i)
-#pragma unroll
-        for (int j = 0; j < NBN; ++j) acc[i][j] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
-    const float4 *src = reinterpret_cast<const float4 *>(part) + (((int64_t)t * 4 + wave) * (NBM * NBN) + I * NBN) * 64 + lane;
-    const int64_t split_stride = (int64_t)total * 4 * (NBM * NBN) * 64;
-    for (int sp = 0; sp < splits; ++sp) {
-        float4 v[NBN];
-#pragma unroll
-        for (int j = 0; j < NBN; ++j) v[j] = src[sp * split_stride + j * 64];
-#pragma unroll
-        for (int i = 0; i < NBM; ++i) {
-            if (i != I) continue;   // (the block index of the accumulators is a compile-time constant in the epilogue)
-#pragma unroll
-            for (int j = 0; j < NBN; ++j) {
-                acc[i][j][0] += v[j].x;
-                acc[i][j][1] += v[j].y;
-                acc[i][j][2] += v[j].z;
-                acc[i][j][3] += v[j].w;
-            }
-        }
-    }
-    const int n_wave = n0 + wave_n * (NBN * 16);
-    uint32_t braw[NBN / 2];
-    float bf[NBN];
-    wide_bias_fetch<T, false, NBN>(bias, n_wave, l16, N, bias_vec_ok, braw);
-    wide_bias_unpack<T, NBN>(braw, bf);
-    const float ones[4] = {1.0f, 1.0f, 1.0f, 1.0f};  // (the split form takes no per-row factors)
-#define KERNL_HALF_REDUCE_EPILOGUE(IB)                                                                                   \
-    if (I == IB)                                                                                                         \
-    wide_epilogue<T, ACT, IB, NBN, NBM>(acc, m0 + wave_m * (NBM * 16), n_wave, l16, g, out, act_in, M, N, out_rs, out_cs, \
-                                        ai_rs, ai_cs, out_vec_ok, ai_vec_ok, bf, ones)
-    KERNL_HALF_REDUCE_EPILOGUE(0);
-    KERNL_HALF_REDUCE_EPILOGUE(1);
-    KERNL_HALF_REDUCE_EPILOGUE(2);
-    KERNL_HALF_REDUCE_EPILOGUE(3);
-#undef KERNL_HALF_REDUCE_EPILOGUE
 }
 
 // ----------------------------------------------------------------------------------------------------
@@ -1859,7 +1801,7 @@ static void launch_wide_act(const LinearArgs &a) {
 
 template <typename T, int ACT, int NBN, bool W8 = false, bool SCALED = false, bool RES = false, bool DEAL = false>
 static void launch_wide_half_act(const LinearArgs &a) {
-    auto kern = linear_wide_half_kernel<T, ACT, NBN, W8, false, SCALED, RES, DEAL>;
+    auto kern = linear_wide_half_kernel<T, ACT, NBN, W8, SCALED, RES, DEAL>;
     constexpr int LDS_BYTES = 3 * 16384 + 3 * 32768;  // three stages
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
@@ -1876,69 +1818,15 @@ static void launch_wide_half_act(const LinearArgs &a) {
     const int bias_vec_ok = bias != nullptr && aligned16(bias);
     hipLaunchKernelGGL(kern, dim3(per_xcd * 8), dim3(256), LDS_BYTES, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), bias, out, act_in, a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs,
-                       a.ai_cs, tiles_m, tiles_n, out_vec_ok, ai_vec_ok, bias_vec_ok, static_cast<float *>(nullptr), 1, a.row_scale,
+                       a.ai_cs, tiles_m, tiles_n, out_vec_ok, ai_vec_ok, bias_vec_ok, a.row_scale,
                        wide_residual_of<T, NBN>(a));
 }
 
-// Split form of the 128 x 192 kernel for row counts that leave most CUs without a tile (129 to about 700 rows against
-// a few thousand columns): `splits` ranges of k-tiles per output tile, then the launch that adds them.
-struct HalfSplitPlan {
-    int tiles_m, tiles_n, splits;
-    int64_t bytes;
-};
-static HalfSplitPlan half_split_plan(int64_t M, int64_t N, int64_t K) {
-    HalfSplitPlan p;
-    p.tiles_m = (int)((M + 127) / 128);
-    p.tiles_n = (int)((N + 191) / 192);
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-    const int nk = (int)(K / 64);
-    int64_t splits = 256 / tiles;           // one round of workgroups
-    if (splits > nk / 16) splits = nk / 16; // ranges of at least 16 k-tiles: with K = 768 two ranges cost more (14 us) than one tile pass (11)
-    if (splits > 4) splits = 4;             // partial tiles cost HBM traffic: rows x columns x 8 bytes per range
-    if (splits < 1) splits = 1;
-    // ranges of ceil(nk / splits) k-tiles: drop ranges that would be empty
-    const int per = (nk + (int)splits - 1) / (int)splits;
-    p.splits = (nk + per - 1) / per;
-    p.bytes = p.splits > 1 ? (int64_t)p.splits * tiles * 128 * 192 * 4 : 0;
-    return p;
-}
-
-template <typename T, int ACT>
-static void launch_half_split_act(const LinearArgs &a, const HalfSplitPlan &p, float *part) {
-    constexpr int NBN = 6;
-    auto kern = linear_wide_half_kernel<T, KERNL_ACT_NONE, NBN, false, true>;
-    constexpr int LDS_BYTES = 3 * 16384 + 3 * 32768;
-    static bool attr_done = false;  // benign race: the attribute call is idempotent
-    if (!attr_done) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-        attr_done = true;
-    }
-    const int per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
-    const T *bias = static_cast<const T *>(a.bias);
-    T *out = static_cast<T *>(a.out);
-    T *act_in = static_cast<T *>(a.act_in);
-    const int out_vec_ok = a.out_cs == 1 && a.out_rs % 8 == 0 && aligned16(out);
-    const int ai_vec_ok = act_in != nullptr && a.ai_cs == 1 && a.ai_rs % 8 == 0 && aligned16(act_in);
-    const int bias_vec_ok = bias != nullptr && aligned16(bias);
-    hipLaunchKernelGGL(kern, dim3(per_xcd * 8, p.splits), dim3(256), LDS_BYTES, a.st, static_cast<const T *>(a.x),
-                       static_cast<const T *>(a.w), bias, out, act_in, a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs,
-                       a.ai_cs, p.tiles_m, p.tiles_n, out_vec_ok, ai_vec_ok, bias_vec_ok, part, p.splits, static_cast<const float *>(nullptr),
-                       WideResidual());
-    hipLaunchKernelGGL((linear_wide_half_reduce_kernel<T, ACT, NBN>), dim3(p.tiles_m * p.tiles_n, 4), dim3(256), 0, a.st,
-                       part, bias, out, act_in, a.M, a.N, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs, p.tiles_m, p.tiles_n,
-                       out_vec_ok, ai_vec_ok, bias_vec_ok, p.splits);
-}
-
-template <typename T>
-static void launch_half_split(const LinearArgs &a, const HalfSplitPlan &p, float *part) {
-    switch (a.act) {
-        case KERNL_ACT_RELU: launch_half_split_act<T, KERNL_ACT_RELU>(a, p, part); break;
-        case KERNL_ACT_TANH: launch_half_split_act<T, KERNL_ACT_TANH>(a, p, part); break;
-        case KERNL_ACT_GELU_ERF: launch_half_split_act<T, KERNL_ACT_GELU_ERF>(a, p, part); break;
-        case KERNL_ACT_GELU_TANH: launch_half_split_act<T, KERNL_ACT_GELU_TANH>(a, p, part); break;
-        case KERNL_ACT_SILU: launch_half_split_act<T, KERNL_ACT_SILU>(a, p, part); break;
-        default: launch_half_split_act<T, KERNL_ACT_NONE>(a, p, part); break;
-    }
+// Row counts that leave most CUs without a 128 x 192 tile (129 to about 700 rows against a few thousand columns) and a K long enough
+// for ranges of 16 k-tiles: what kernl_linear_splitk_fwd takes.
+static bool half_split_takes(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ((M + 127) / 128) * ((N + 191) / 192);
+    return K % 64 == 0 && 256 / tiles >= 2 && K / 64 / 16 >= 2;
 }
 
 template <typename T, int NBN>
@@ -2116,6 +2004,54 @@ static MidChoice mid_tile_of(int64_t M, int64_t N, int64_t K, bool gated) {
     return best;
 }
 
+// the same estimate for the wide kernels
+static double wide_us(int64_t M, int64_t N, int64_t K, bool gated) {
+    auto cost = [&](int bm, int bn, double per_k) {
+        const int64_t n = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        return 3.5 + (double)((n + 255) / 256) * tile_round(n, (double)((K + 63) / 64), per_k);
+    };
+    double us = cost(256, 256, 1.50);
+    if (!gated) us = std::min(std::min(us, cost(256, 192, 1.30)), std::min(cost(128, 256, 0.87), cost(128, 192, 0.79)));
+    return us;
+}
+
+// K split over several workgroups a tile, and the launch that adds their fp32 sums (linear_finish.hip): tile, ranges and the
+// estimated time of both launches.  A range costs rows x columns x 8 bytes of traffic and keeps at least four k-tiles.
+struct SplitPlan {
+    int tile = 0, splits = 1, range_kt = 0;
+    int64_t part_rs = 0, bytes = 0;
+    double us = 1e30;
+};
+static SplitPlan split_plan_of(int64_t M, int64_t N, int64_t K) {
+    struct Tile {
+        int kind, bm, bn;
+        double ramp, per_k_cached, per_k_hbm;
+    };
+    static constexpr Tile tiles[] = {{11, 64, 64, 1.8, 0.195, 0.26}, {15, 128, 64, 1.9, 0.27, 0.385}, {17, 128, 128, 2.9, 0.34, 0.53},
+                                     {22, 192, 96, 4.0, 0.36, 0.62}, {18, 192, 128, 4.2, 0.43, 0.67}};
+    const bool cached = N * K <= ((int64_t)1 << 23);
+    const int64_t nk = (K + 63) / 64;
+    SplitPlan best;
+    best.part_rs = (N + 7) / 8 * 8;
+    for (const Tile &t : tiles)
+        for (int want = 2; want <= 8; ++want) {
+            const int64_t range = (nk + want - 1) / want, splits = (nk + range - 1) / range;
+            const int64_t n = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * splits;
+            if (splits < 2 || range < 4) continue;
+            const double sums = (double)splits * (double)(M * best.part_rs) * 4.0;
+            const double round = t.ramp + tile_round(n, (double)range, cached ? t.per_k_cached : t.per_k_hbm);
+            const double us = 2.0 + (double)((n + 255) / 256) * round + sums / 6e6 + 3.5 + sums / 5e6;
+            if (us < best.us) {
+                best.tile = t.kind;
+                best.splits = (int)splits;
+                best.range_kt = (int)range;
+                best.us = us;
+            }
+        }
+    best.bytes = (int64_t)best.splits * M * best.part_rs * 4;
+    return best;
+}
+
 // Whether M x N x K, beyond what small_problem_kind names, runs on the tiles of linear_mid.hip (or, 14, on 64 x 32 tiles with dealt
 // k-tiles), as a hook value; 0 where another kernel is faster.  `N`: rows of the weight (gated: twice the output columns).
 //  - short K: by tile counts, from a sweep of 65 .. 4096 rows over BERT's and wider weights.  15 and 17 stand for "short K" here: the
@@ -2132,24 +2068,8 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
     }
     if (short_k || (M <= 128 && N * K < 12 * (1 << 20))) return 0;
     const double nk = (double)((K + 63) / 64), hbm = 4.0 + (double)(N * K) * 2.0 / 4.6e6;  // us at 4.6 TB/s
-    auto cost = [&](int bm, int bn, double per_k) {
-        const int64_t n = tiles(bm, bn);
-        return 3.5 + (double)((n + 255) / 256) * tile_round(n, nk, per_k);
-    };
     MidChoice best = mid_tile_of(M, N, K, gated);
-    double other = cost(256, 256, 1.50);
-    if (!gated) {
-        const double c6 = cost(256, 192, 1.30), c7 = cost(128, 256, 0.87), c8 = cost(128, 192, 0.79);
-        other = other < c6 ? other : c6;
-        other = other < c7 ? other : c7;
-        other = other < c8 ? other : c8;
-        if (M > 128 && K % 64 == 0) {
-            const HalfSplitPlan p = half_split_plan(M, N, K);
-            const double per = (double)(((int64_t)nk + p.splits - 1) / p.splits);
-            const double c = 6.5 + per * 0.755 + (double)p.splits * (double)(M * N) * 8.0 / 4e6;
-            if (p.splits > 1 && c < other) other = c;
-        }
-    }
+    double other = wide_us(M, N, K, gated);
     if (M <= 128 && K % 64 == 0) {
         const double few = 10.0 + (double)(N * K) * 2.0 / 3.7e6;
         other = other < few ? other : few;
@@ -2161,6 +2081,34 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
         }
     }
     return best.us < 0.97 * other ? best.tile : 0;
+}
+
+// What M x N x K takes without a split, us, where a launch of its own adds or normalises afterwards.  (small problems: 32 x 32 tiles
+// 231 x 768 x 3072 8.1, x 768 4.6, 64 x 32 tiles 500 x 768 x 3072 10.6, x 768 5.5, 16 x 32 tiles 66 x 768 x 3072 5.5)
+static double unsplit_us(int64_t M, int64_t N, int64_t K) {
+    const double nk = (double)((K + 63) / 64);
+    switch (small_problem_kind(M, N, K)) {
+        case 12: case 13: return 3.5 + nk * (M <= 96 ? 0.045 : 0.09);
+        case 14: return 3.8 + nk * 0.14;
+        case 10: return 3.6 + nk * 0.2;
+        case 0: break;
+        default: return mid_tile_of(M, N, K, false).us;
+    }
+    const int mid = mid_kind(M, N, K, false);
+    if (mid == 14) return 3.5 + nk * 0.2;
+    if (mid != 0) return mid_tile_of(M, N, K, false).us;
+    const double few = M <= 128 && K % 64 == 0 ? 10.0 + (double)(N * K) * 2.0 / 3.7e6 : 1e30;
+    return std::min(few, wide_us(M, N, K, false));
+}
+
+// The split plan of M x N x K where it beats what would run instead: the product and, but for kFinishPlain, the launch behind it
+// (add + LayerNorm 4.3 us; row statistics 4.8; the residual alone rides in most unsplit epilogues).  tile 0: it does not.
+static SplitPlan split_plan_that_pays(int64_t M, int64_t N, int64_t K, int finish) {
+    if (M <= 64 || M > 4096 || K % 8 != 0 || K < 512 || K >= (1 << 22) || N < 64 || N > INT32_MAX / 64) return SplitPlan();
+    if (finish == kFinishPlain ? M <= 128 : N % 4 != 0 || N > 8192) return SplitPlan();  // (plain products of few rows: the stream-K kernel)
+    const SplitPlan p = split_plan_of(M, N, K);
+    const double behind = finish == kFinishLayerNorm ? 4.3 : finish == kFinishRmsStats ? 4.8 : 0.0;
+    return p.bytes <= ((int64_t)64 << 20) && p.us < 0.95 * (unsplit_us(M, N, K) + behind) ? p : SplitPlan();
 }
 
 extern int g_linear_force_tile;  // test / tuning hook (defined in linear.hip): 0 = heuristic, 1 = 256x256, 2 = 256x192, 3 = 128x128, 4 = 256x128 k32, 5 = wide 256x256, 6 = wide 256x192, 7 = wide 128x256, 8 = wide 128x192, 10 = 32 x 64, 12 .. 14 and 16 = dealt k-tiles, 11, 15, 17 .. 22 = the tiles of linear_mid.hip

@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(Cfg::WAVES * 64, Cfg::WAVES / 4)
 linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
                   T *__restrict__ act_in, const float *__restrict__ row_scale, const T *__restrict__ residual, int M, int N, int K,
                   int64_t ldx, int64_t out_rs, int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int64_t res_rs, int64_t res_cs, int act,
-                  int tiles_m, MidGrid grid) {
+                  int tiles_m, MidGrid grid, float *__restrict__ part, int64_t part_rs, int range_kt) {
     typedef typename Vec8<T>::type vec8;
     constexpr int BM = Cfg::BM, BN = Cfg::BN, S = Cfg::S, NBM = Cfg::NBM, NBN = Cfg::NBN, STAGE = Cfg::STAGE, L = Cfg::L;
     constexpr int LX = Cfg::LX, LW = Cfg::LW, BK = Cfg::BK;
@@ -78,15 +78,24 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
         tile_n = tile / tiles_m;
     }
     const int m0 = tile_m * BM, n0 = tile_n * BN;
+    // K split (part given): this workgroup's range of range_kt k-tiles
+    const int64_t ldw = K;
+    if (part != nullptr) {
+        const int k_begin = (int)blockIdx.y * range_kt * BK;
+        X += k_begin;
+        W += k_begin;
+        K = min(range_kt * BK, K - k_begin);
+        part += (int64_t)blockIdx.y * M * part_rs;
+    }
     // the order of the k-tiles, as in the wide kernels (linear_kernels.h) but for any K: whole groups of four are dealt
     const int turn = (tile_m + tile_n) & 3, k_dealt = K / (4 * BK) * 4;
 
     constexpr uint32_t kOutOfRange = 0x80000000u;
     const int rows_x = min(BM, M - m0), rows_w = min(BN, N - n0);
     const uint64_t xaddr = (uint64_t)(uintptr_t)(X + (int64_t)m0 * ldx);
-    const uint64_t waddr = (uint64_t)(uintptr_t)(W + (int64_t)n0 * K);
+    const uint64_t waddr = (uint64_t)(uintptr_t)(W + (int64_t)n0 * ldw);
     const u32x4 xrsrc = {(uint32_t)xaddr, (uint32_t)(xaddr >> 32) & 0xFFFFu, (uint32_t)((((int64_t)rows_x - 1) * ldx + K) * 2), 0x00020000u};
-    const u32x4 wrsrc = {(uint32_t)waddr, (uint32_t)(waddr >> 32) & 0xFFFFu, (uint32_t)((int64_t)rows_w * K * 2), 0x00020000u};
+    const u32x4 wrsrc = {(uint32_t)waddr, (uint32_t)(waddr >> 32) & 0xFFFFu, (uint32_t)((((int64_t)rows_w - 1) * ldw + K) * 2), 0x00020000u};
     const int nk = (K + BK - 1) / BK, k_last = K - (nk - 1) * BK;
     // load i of a loading wave fills the 1 KB (8 rows) piece i * LOADERS + loader of the operand tile
     uint32_t xd[LX], wd[LW], tail_bits = 0;
@@ -99,7 +108,7 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
 #pragma unroll
     for (int i = 0; i < LW; ++i) {
         const int q = (i * Cfg::LOADERS + loader) * 64 + lane, row = mid_weight_row<GATED, Cfg::TN>(SmallTileMap::load_row(q)), c = SmallTileMap::load_chunk(q);
-        wd[i] = row < rows_w ? (uint32_t)(((int64_t)row * K + c * 8) * 2) : kOutOfRange;
+        wd[i] = row < rows_w ? (uint32_t)(((int64_t)row * ldw + c * 8) * 2) : kOutOfRange;
         if (c * 8 < k_last) tail_bits |= 1u << (LX + i);
     }
     typedef __attribute__((address_space(3))) void lds_void;
@@ -233,6 +242,20 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     __builtin_amdgcn_s_waitcnt(0x0F70);
 
     // ---- epilogue
+    if (part != nullptr) {  // fp32 sums of the range, row-major; columns N .. part_rs - 1 hold zeros (their weight rows do)
+#pragma unroll
+        for (int i = 0; i < NBM; ++i) {
+            const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
+            if (m >= M) continue;
+            float *p = part + (int64_t)m * part_rs;
+#pragma unroll
+            for (int j = 0; j < NBN; ++j) {
+                const int n = n0 + mid_weight_row<GATED, Cfg::TN>(wave_n * Cfg::TN + 16 * j + 4 * g);
+                if (n < part_rs) *reinterpret_cast<f32x4_acc *>(p + n) = acc[i][j];
+            }
+        }
+        return;
+    }
     const bool out_vec = out_cs == 1 && (out_rs & (V - 1)) == 0 && ((uintptr_t)out & (2 * V - 1)) == 0;
     const bool ai_vec = act_in != nullptr && ai_cs == 1 && (ai_rs & (V - 1)) == 0 && ((uintptr_t)act_in & (2 * V - 1)) == 0;
     const bool res_vec = residual != nullptr && res_cs == 1 && (res_rs & (V - 1)) == 0 && ((uintptr_t)residual & (2 * V - 1)) == 0;
@@ -301,7 +324,7 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
 }
 
 template <typename T, typename Cfg, bool GATED>
-static void launch_mid_cfg(const LinearArgs &a) {
+static void launch_mid_cfg(const LinearArgs &a, const MidSplit &split = MidSplit()) {
     auto kern = linear_mid_kernel<T, Cfg, GATED>;
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
@@ -312,19 +335,20 @@ static void launch_mid_cfg(const LinearArgs &a) {
     // the XCD blocks: as square in bytes as 8 blocks can be, where they take no more rounds than the tiles themselves
     MidGrid grid;
     int blocks = tiles_m * tiles_n;
+    const int64_t all = (int64_t)blocks * split.splits;
     int64_t least = INT64_MAX;
     for (int s = 0; s <= 3; ++s) {
         const int xm = 1 << s, xn = 8 >> s, pm = (tiles_m + xm - 1) / xm, pn = (tiles_n + xn - 1) / xn;
         const int64_t bytes = (int64_t)pm * Cfg::BM + (int64_t)pn * Cfg::BN;
-        if ((int64_t)pm * pn > (int64_t)(tiles_m * tiles_n + 255) / 256 * 32 || bytes >= least) continue;
+        if ((int64_t)pm * pn * split.splits > (all + 255) / 256 * 32 || bytes >= least) continue;
         least = bytes;
         grid.xm_mask = xm - 1; grid.xm_shift = s; grid.per_m = pm; grid.per_n = pn;
         blocks = 8 * pm * pn;
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(Cfg::WAVES * 64), Cfg::LDS, a.st, static_cast<const T *>(a.x),
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)split.splits), dim3(Cfg::WAVES * 64), Cfg::LDS, a.st, static_cast<const T *>(a.x),
                        static_cast<const T *>(a.w), static_cast<const T *>(a.bias), static_cast<T *>(a.out), static_cast<T *>(a.act_in),
                        a.row_scale, static_cast<const T *>(a.residual), a.M, a.N, a.K, a.x_rs, a.out_rs, a.out_cs, a.ai_rs, a.ai_cs,
-                       a.res_rs, a.res_cs, a.act & (kGluBit - 1), tiles_m, grid);
+                       a.res_rs, a.res_cs, a.act & (kGluBit - 1), tiles_m, grid, split.part, split.part_rs, split.range_kt);
 }
 
 // the tiles, by the kernl_linear_force_tile value that forces them (and mid_tile_of names)
@@ -358,5 +382,22 @@ static int run_mid_t(const LinearArgs &a, int kind) {
 }
 
 int run_mid(const LinearArgs &a, int dtype, int kind) { return dtype == KERNL_F16 ? run_mid_t<f16>(a, kind) : run_mid_t<bf16>(a, kind); }
+
+// ranges of K: no gates (the value of the gate is not linear in the sums), and tiles whose partial results pay
+template <typename T>
+static void run_mid_split_t(const LinearArgs &a, int tile, const MidSplit &split) {
+    switch (tile) {
+        case 11: launch_mid_cfg<T, Mid64x64, false>(a, split); break;
+        case 15: launch_mid_cfg<T, Mid128x64, false>(a, split); break;
+        case 18: launch_mid_cfg<T, Mid192x128, false>(a, split); break;
+        case 22: launch_mid_cfg<T, Mid192x96, false>(a, split); break;
+        default: launch_mid_cfg<T, Mid128x128, false>(a, split); break;
+    }
+}
+
+void run_mid_split(const LinearArgs &a, int dtype, int tile, const MidSplit &split) {
+    if (dtype == KERNL_F16) run_mid_split_t<f16>(a, tile, split);
+    else run_mid_split_t<bf16>(a, tile, split);
+}
 
 }  // namespace kernl

@@ -1,5 +1,4 @@
-// Launchers of the 128-row wide kernel and its split-over-K form (see linear_kernels.h): a translation unit of its own
-// for build time.
+// Launchers of the 128-row wide kernel (see linear_kernels.h): a translation unit of its own for build time.
 #include "linear_kernels.h"
 
 namespace kernl {
@@ -28,10 +27,5 @@ static void launch_wide_half_w8(const LinearArgs &a) {
 }
 
 void run_wide_half_w8(const LinearArgs &a) { launch_wide_half_w8(a); }
-
-void run_half_split(const LinearArgs &a, const HalfSplitPlan &p, float *part, int dtype) {
-    if (dtype == KERNL_F16) launch_half_split<f16>(a, p, part);
-    else launch_half_split<bf16>(a, p, part);
-}
 
 }  // namespace kernl

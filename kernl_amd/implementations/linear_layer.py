@@ -71,6 +71,18 @@ def takes_mid_kernel(x2d: torch.Tensor, weight: torch.Tensor, gated: bool = Fals
     )
 
 
+def split_pays_bytes(x2d: torch.Tensor, weight: torch.Tensor) -> int:
+    """Workspace of `kernl_linear_splitk_fwd` where K split over several workgroups a tile, with a second launch that adds the ranges, beats
+    whatever would run the product in one pass; 0 elsewhere."""
+    if not (
+        x2d.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x2d.dtype and x2d.shape[1] % 64 == 0
+        and x2d.stride(1) == 1 and x2d.stride(0) % 8 == 0 and x2d.stride(0) < (1 << 22) and x2d.data_ptr() % 16 == 0
+        and weight.data_ptr() % 16 == 0
+    ):
+        return 0
+    return _lib.linear_split_workspace_bytes(x2d.shape[0], weight.shape[0], x2d.shape[1])
+
+
 def takes_few_row_kernel(x2d: torch.Tensor, weight: torch.Tensor) -> bool:
     return few_row_rule(x2d.shape[0], weight.shape[0], weight.shape[1]) and _lib.linear_fewrow_supported(x2d, weight)
 
@@ -121,16 +133,16 @@ class LinearLayer(torch.autograd.Function):
         outputs = torch.empty((M, N), device=x.device, dtype=x.dtype)
         if act_inputs is not None:
             assert act_inputs.shape == (M, N) and act_inputs.dtype == x.dtype
-        small = takes_small_problem_kernel(x_, weight) or takes_mid_kernel(x_, weight)
-        split_bytes = 0
-        if not small and FEW_ROW_MAX_ROWS < M <= SPLIT_K_MAX_ROWS:
+        split_bytes = split_pays_bytes(x_, weight)
+        small = not split_bytes and (takes_small_problem_kernel(x_, weight) or takes_mid_kernel(x_, weight))
+        if not split_bytes and not small and FEW_ROW_MAX_ROWS < M <= SPLIT_K_MAX_ROWS:
             split_bytes = _lib.linear_splitk_workspace_bytes(x_, weight)
         if small:
             _lib.linear_fwd(x_, weight, bias, outputs, act_inputs, ACTIVATIONS.get(activation, _lib.ACT_NONE))
-        elif act_inputs is None and takes_few_row_kernel(x_, weight):
+        elif not split_bytes and act_inputs is None and takes_few_row_kernel(x_, weight):
             _lib.linear_fewrow_fwd(x_, weight, bias, None, outputs, ACTIVATIONS.get(activation, _lib.ACT_NONE))
         elif split_bytes:
-            # too few 128-row tiles to occupy the chip: ranges of K per tile, added by a second launch
+            # too few tiles to occupy the chip: ranges of K per tile, added by a second launch
             workspace = torch.empty(split_bytes, dtype=torch.uint8, device=x.device)
             _lib.linear_splitk_fwd(x_, weight, bias, outputs, act_inputs, ACTIVATIONS.get(activation, _lib.ACT_NONE), workspace)
         else:

@@ -11,7 +11,10 @@ import torch
 
 from kernl_amd import _lib
 from kernl_amd.implementations.deferred_norm import DeferredNorm, deferrable, linear_add_deferred
-from kernl_amd.implementations.linear_layer import GLU_BLOCK, interleave_glu_rows, linear_glu_layer, linear_layer
+from kernl_amd.implementations.linear_layer import GLU_BLOCK, interleave_glu_rows, linear_glu_layer, linear_layer, rms_eps
+from kernl_amd.implementations.split_linear import (
+    FINISH_LAYER_NORM, FINISH_RESIDUAL, FINISH_RMS_STATS, split_finish_bytes, split_finish_linear,
+)
 from kernl_amd.utils.extended_matcher import replace_pattern
 
 
@@ -655,6 +658,9 @@ def linear_residual_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, residua
         and not torch.is_autocast_enabled("cuda")
     ):
         return decode_linear_layer(v, weight, bias, residual=residual)
+    need = split_finish_bytes(v, weight, bias, residual, FINISH_RESIDUAL)
+    if need:
+        return split_finish_linear(need, v, weight, bias, residual, FINISH_RESIDUAL)
     fused = _wide_residual_linear(v, weight, bias, residual)
     if fused is not None:
         return fused
@@ -682,7 +688,7 @@ def linear_residual_stats_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, r
     row statistics 1 / sqrt(mean(sum^2) + eps) of the RMSNorm that follows — the projections behind that norm take them
     (`rstd=` of the `rms_*` wrappers) and never see a normalised tensor.  rstd is None where the statistics are not
     wanted (decoding steps, whose one-launch kernels normalise inside the product; dtypes the kernel does not take)."""
-    from kernl_amd.implementations.linear_layer import add_rms_stats, add_rms_stats_supported, rms_eps, rms_stats
+    from kernl_amd.implementations.linear_layer import add_rms_stats, add_rms_stats_supported, rms_stats
 
     from kernl_amd.implementations.linear_layer import FEW_ROW_MAX_ROWS
 
@@ -694,6 +700,10 @@ def linear_residual_stats_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, r
     )
     if not prompt:
         return linear_residual_wrapper(v, weight, bias, residual), None
+    need = split_finish_bytes(v, weight, bias, residual, FINISH_RMS_STATS)
+    if need:
+        # the launch that adds the ranges of K has the rows in hand: residual and statistics
+        return split_finish_linear(need, v, weight, bias, residual, FINISH_RMS_STATS, eps=rms_eps(residual.dtype, eps))
     fused = _wide_residual_linear(v, weight, bias, residual)
     if fused is not None:
         # the addition rode in the projection: one pass over the sum for its row statistics
@@ -779,6 +789,12 @@ def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, r
             return norm if behind is not None else norm.normalised()
     if isinstance(residual, DeferredNorm):
         residual = residual.normalised()
+    if isinstance(residual, torch.Tensor) and isinstance(v, torch.Tensor) and len(normalized_shape) == 1:
+        _half_params_once(v, weight, bias, ln_weight, ln_bias)
+        need = split_finish_bytes(v, weight, bias, residual, FINISH_LAYER_NORM, ln_weight, ln_bias)
+        if need:
+            # K split, and the launch that adds its ranges normalises the rows
+            return split_finish_linear(need, v, weight, bias, residual, FINISH_LAYER_NORM, ln_weight, ln_bias, rms_eps(v.dtype, eps))
     if isinstance(residual, torch.Tensor) and _epilogue_addition_pays_in_front_of_a_norm(v, weight):
         fused = _wide_residual_linear(v, weight, bias, residual)
         if fused is not None:
