@@ -86,8 +86,9 @@ __global__ void __launch_bounds__(256, WPE) attention_stream_kernel(const AttnPa
         qt = slot % p.nq_tiles;
         if (b >= p.B) return;
     } else {
-        const int bh = (slot / p.nq_tiles) * 8 + xcd;
-        qt = slot % p.nq_tiles;
+        const RankedItem item = CAUSAL ? ranked_item(slot, (p.B * p.H + 7) / 8, p.nq_tiles) : RankedItem{slot / p.nq_tiles, slot % p.nq_tiles};
+        const int bh = item.head * 8 + xcd;
+        qt = item.rank;
         if (bh >= p.B * p.H) return;
         b = bh / p.H;
         h = bh % p.H;
@@ -1145,6 +1146,12 @@ static int attention_entry(const void *q, const void *k, const void *v, void *ou
             else launch_stream_wsplit<bf16>(p, mask_mode, st);
             return check_launch("attention (mfma, key tiles split over waves)");
         }
+    }
+    // Causal grids that 64-row workgroups fill once (hook: variant 7 takes this form wherever it applies)
+    if (mfma_ok && causal && mask_mode == MASK_NONE && B * H * ((M + 63) / 64) < (1ll << 31) &&
+        (g_attention_variant == 7 || (g_attention_variant == 0 && attention_split_pays(B * H, M, N, start_position, (int)D)))) {
+        run_attention_split(p, (int)D, dtype, st);
+        return check_launch("attention (mfma, key tiles split in the workgroup)");
     }
     // the software-pipelined kernel takes long key sequences of what it covers (hook: variant 3 keeps everything on the
     // streaming kernel, variant 4 sends everything the pipelined kernel covers to it)

@@ -52,6 +52,28 @@ __device__ __forceinline__ float scale_mask(float mv, float clamp) {
 }
 
 
+// The place of item `at` among an XCD's `heads` heads of `tiles` query tiles each, causal: kRankHeads heads at a time, the longest tiles
+// of all of them first, so that what comes last, beside other workgroups or after them, is short: with the tiles of a head next to each
+// other, a grid of one to a few rounds ended with long tiles that had started late (us, [heads, rows, head size], pipelined kernel up to
+// [32,..] and streaming kernel from [64,..]: [32,1500,128] 45.7 -> 30.6, [32,2048,64] 30.8 -> 25.8, [64,1500,128] 63.7 -> 47.9,
+// [128,333,128] 17.9 -> 15.8, [128,900,64] 33.4 -> 28.1, [512,512,64] 42.8 -> 37.5).  Not all heads at once: 32 heads of 333 rows and head
+// size 128 outgrow the XCD's L2, 24.9 -> 29.1, where 16 at a time take 25.8 (and 26.3 before).
+static constexpr int kRankHeads = 16;
+struct RankedItem { int head, rank; };  // rank 0: the last query tile
+__device__ static inline RankedItem ranked_item(int at, int heads, int tiles) {
+    const int first = at / (kRankHeads * tiles) * kRankHeads, members = heads - first < kRankHeads ? heads - first : kRankHeads;
+    const int in = at - first * tiles;
+    return {first + in % members, in / members};
+}
+
+// How attention_short.hip and attention_split.hip place value rows in LDS: the row's 16-byte chunk c at c ^ value_flip(row).  A transposing
+// read takes 8 bytes from each of 8 rows at 4 places a quarter of a row apart; rows of head size 64 alternate between the halves of the
+// banks, so one bit of the row spreads the rest, rows of head size 128 need two (with one bit: 4 lanes to a bank instead of 2).
+template <int D>
+__host__ __device__ static inline int value_flip(int row) {
+    return D == 64 ? (row >> 1) & 1 : row & 3;
+}
+
 // Software-pipelined MFMA kernel (attention_pipe.hip).  Handles head sizes 64 and 128 with no mask or with a per-key
 // mask of at most kPipeMaxMaskKeys keys (non-causal), and causal attention without a mask; taken from kPipeMinKeys keys
 // on — head size 128 only for causal problems with few (batch, head) pairs — or whenever it applies, with `force`.
@@ -78,6 +100,20 @@ static inline bool attention_short_pays(int64_t workgroups, int64_t M, int N, in
     if (N <= 64) return workgroups <= (D == 64 ? 16384 : 384);
     if (D == 64) return workgroups <= (N <= 128 ? 1024 : N <= 192 ? 512 : 384);
     return workgroups <= (N <= 128 ? 384 : 256);
+}
+// Kernel whose waves split every key tile (attention_split.hip): causal, no mask; workgroups of 64 rows.
+void run_attention_split(const AttnParams &p, int D, int dtype, hipStream_t st);
+// Where it is the fastest: as long as its workgroups, one a CU, are one round.  Beyond that the last to start are the shortest (the longest
+// go first), and with many tiles a head these still fit in behind; with few, or where new rows over a cache make all of them long, they do
+// not (us, pipelined or streaming kernel -> this one, [heads, rows, head size]: [48,333,128] 288 workgroups 11.3 -> 13.3; [24,700,128] 264
+// 15.6 -> 14.0; [32,700,128] 352 16.8 -> 17.3; [16,1111,128] 288 20.7 -> 18.4; [24,1024,128] 384 20.3 -> 21.1; [12,2048,128] 384 33.7 ->
+// 30.9; 300 rows over 1024 keys, 64 heads, 320 workgroups 23.8 -> 31.6).  At head size 64 the pipelined kernel is level from some 512 keys
+// on and ahead later ([32,333,64] 8.0 -> 7.6, [32,512,64] 9.1 -> 9.0, [24,1000,64] 12.5 -> 14.6); up to kShortMaxKeys keys
+// attention_short.hip is ahead by a fifth.
+static inline bool attention_split_pays(int64_t heads, int64_t M, int64_t N, int64_t start, int D) {
+    if (N <= kShortMaxKeys || (D == 64 && N > 512)) return false;
+    const int64_t tiles = (M + 63) / 64, behind = tiles >= 11 && start * 4 <= M ? 4 * tiles : 0;
+    return heads * tiles <= 256 + (behind < 128 ? behind : 128);
 }
 void run_attention_short(const AttnParams &p, int D, int dtype, bool masked, bool causal, hipStream_t st);
 

@@ -224,7 +224,8 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attention_pipe_kernel(co
         }
     };
     auto request_item = [&](int idx) __attribute__((always_inline)) {
-        const int bh = 8 * (idx / p.nq_tiles) + xcd, qt = idx % p.nq_tiles;
+        const RankedItem at = CAUSAL ? ranked_item(idx, (bh_total - xcd + 7) / 8, p.nq_tiles) : RankedItem{idx / p.nq_tiles, idx % p.nq_tiles};
+        const int bh = 8 * at.head + xcd, qt = at.rank;
         req_b = bh / p.H;
         req_h = bh % p.H;
         req_q0 = (CAUSAL ? p.nq_tiles - 1 - qt : qt) * BM;
@@ -798,6 +799,28 @@ static void launch_pipe_t(const AttnParams &p, int mask_mode, bool causal, hipSt
 #undef KERNL_PIPE_LAUNCH
 }
 
+// Causal grids.  A tile costs here what it costs the streaming kernel with its CU full (head size 64; head size 128, one workgroup a CU:
+// 12 % more, both sit at the chip's power limit), but a workgroup alone on its CU is faster here, and the fixed lists pair long tiles with
+// short ones.  So grids up to `full` items, what the chip holds at once, belong here, up to twice that as long as the pairs come out even,
+// which many tiles a head see to; beyond that the hardware's own dispatch is the better balance.  Measured, us, streaming kernel / this one,
+// [heads, rows, head size] (items a multiple of full): [16,2048,128] (1.0) 37.7 / 33.6; [40,1024,128] (1.25) 26.0 / 23.1; [48,1024,128]
+// (1.5, 8 tiles a head) 27.5 / 27.7; [12,4096,128] (2.0) 83.6 / 72.9; [36,1600,128] (2.0, 13 tiles) 37.8 / 42.9; [32,2048,128] (2.0, 16
+// tiles) 48.4 / 45.3; [64,1024,128] (2.0, 8 tiles) 29.6 / 31.5; [48,1500,128] (2.3) 40.1 / 47.8; [64,1024,64] (1.0) 20.1 / 16.8;
+// [32,3000,64] (1.5) 52.2 / 47.1; [96,1024,64] (1.5, 8 tiles) 24.0 / 25.5; [64,2048,64] (2.0, 16 tiles) 42.9 / 45.8; [32,4096,64] (2.0, 32
+// tiles) 79.2 / 75.6; [24,6000,64] (2.2, 47 tiles) 118.0 / 114.6; [128,2048,64] (4.0) 82.7 / 85.3.  New rows over a cache are as long as
+// each other: no pairs to gain by at head size 128 (1024 rows, 4096 keys, 64 heads: 114.4 / 127.7; 32 heads, 1.0: 72.3 / 67.3), while at 64
+// this kernel is ahead at any grid (1024 over 4096, 64 heads, 1.0: 70.1 / 63.9; 2048 over 4096, 2.0: 120.6 / 104.9).
+// Below kPipeMinKeys keys only what the chip holds at once: [32,700,64] 12.2 / 10.3, [48,900,64] 16.5 / 13.6, [128,333,64] 10.8 / 10.3,
+// [128,320,64] 8.9 / 9.6, [80,800,64] (1.1) 17.0 / 18.8; [40,512,128] 14.8 / 14.3, [48,400,128] 12.7 / 12.8.
+static bool pipe_pays_causal(const AttnParams &p, int D) {
+    const int64_t tiles = (p.M + 127) / 128, full = D == 64 ? 512 : 256;
+    const int64_t items = (int64_t)((p.B * p.H + 7) / 8) * 8 * tiles;  // (the XCD with the most heads sets the pace)
+    if (p.N < kPipeMinKeys) return p.N >= (D == 64 ? 321 : 512) && items <= full;
+    if (4 * (int64_t)p.causal_off >= p.M) return D == 64 || items <= full;
+    return 4 * items <= 5 * full || (2 * items <= 3 * full && tiles >= 10) || (items <= 2 * full && tiles >= (D == 64 ? 24 : 16)) ||
+           (D == 64 ? tiles >= 40 && items <= 3 * full : tiles >= 64 && 4 * items <= 9 * full);
+}
+
 // true if the problem was launched here; false: not covered, the caller takes the streaming kernel
 bool launch_attention_pipe(const AttnParams &p, int D, int dtype, int mask_mode, bool causal, bool force, hipStream_t st) {
     if (D != 64 && D != 128) return false;
@@ -807,14 +830,9 @@ bool launch_attention_pipe(const AttnParams &p, int D, int dtype, int mask_mode,
     // From kPipeMinKeys keys on, and for SMALL grids (at most one 128-query item per CU) from 256 keys on: there the
     // streaming kernel has no other workgroup on the CU to fill a wave's dependent phases with, and this kernel's own
     // overlap is worth 10-16 % (head size 64, [1,64,512,64]: 10.6 -> 9.3 us, [1,32,512,768]: 13.0 -> 10.2; with 512 items 4 %,
-    // beyond that it ties or loses, as at BASELINE config 1).
-    const bool small_grid = D == 64 && !causal && p.N >= 256 && (int64_t)p.B * p.H * ((p.M + 127) / 128) <= 256;
-    if (!force && p.N < kPipeMinKeys && !small_grid) return false;
-    // Head size 128 runs one workgroup per CU here and is no faster per tile than the streaming kernel (both sit at the
-    // chip's power limit); what it wins is BALANCE when a causal problem has few (batch, head) pairs: a persistent
-    // workgroup pairs long and short query tiles, where the streaming kernel's grid is one round of unequal workgroups
-    // (measured, [1,32,2048,128] causal: 50 against 60 us; 64 pairs: +3..6 %; 128 pairs or 40: slower).
-    if (!force && D == 128 && !(causal && mask_mode == MASK_NONE && p.B * p.H <= 64 && (p.B * p.H) % 8 == 0)) return false;
+    // beyond that it ties or loses, as at [32,12,512,64]).
+    const bool small_grid = p.N >= 256 && (int64_t)p.B * p.H * ((p.M + 127) / 128) <= 256;
+    if (!force && !(causal ? pipe_pays_causal(p, D) : D == 64 && (p.N >= kPipeMinKeys || small_grid))) return false;
     if (D == 64) {
         if (dtype == KERNL_F16) launch_pipe_t<f16, 64>(p, mask_mode, causal, st);
         else launch_pipe_t<bf16, 64>(p, mask_mode, causal, st);

@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(256, 1) attention_short_kernel(const AttnParam
 #pragma unroll
         for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const vec8 *>(qrow + 32 * s + 8 * g);
     }
-    // LDS chunk q of 16 bytes holds chunk q % CPR of row q / CPR, swizzled: keys for whole-row fragment reads, values by one bit
+    // LDS chunk q of 16 bytes holds chunk q % CPR of row q / CPR, swizzled: keys for whole-row fragment reads, values by value_flip
     typedef __attribute__((address_space(3))) void lds_void;
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_void *)tiles;
     {
@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256, 1) attention_short_kernel(const AttnParam
         const u32x4 krsrc = {(uint32_t)ka, (uint32_t)(ka >> 32) & 0xFFFFu, (N - 1) * k_step + D * 2, 0x00020000u};
         const u32x4 vrsrc = {(uint32_t)va, (uint32_t)(va >> 32) & 0xFFFFu, (N - 1) * v_step + D * 2, 0x00020000u};
         const int row = wave * ROWS + lane / CPR, c = lane % CPR;
-        const uint32_t k_at = row * k_step, v_at = row * v_step + ((c ^ ((row >> 1) & 1)) * 16);
+        const uint32_t k_at = row * k_step, v_at = row * v_step + ((c ^ value_flip<D>(row)) * 16);
 #pragma unroll
         for (int i = 0; i < NB * 16 / (4 * ROWS); ++i)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(256, 1) attention_short_kernel(const AttnParam
 #pragma unroll
     for (int f = 0; f < FB; ++f) o[f] = f32x4_acc{0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t vbase = lds + TILE;
-    const int key = 4 * g + (r >> 2), flip = (key >> 1) & 1;  // (32- and 16-key steps leave the flip alone)
+    const int key = 4 * g + (r >> 2), flip = value_flip<D>(key);  // (32- and 16-key steps leave the flip alone)
 #pragma unroll
     for (int t = 0; t < NB / 2; ++t) {
         u32x2 lo[FB], hi[FB];
