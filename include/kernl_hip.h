@@ -192,6 +192,18 @@ int kernl_rope_fwd(const void *x, const void *cos, const void *sin, void *out, i
                    void *stream);
 
 /*
+ * Tables for kernl_rope_fwd:  cos[b,s,j] = cos[b,s,half + j] = cos(inv_freq[b,j] · positions[b,s]) · scale, sin likewise; the angle, the
+ * function and the scaling rounded to fp32, then once to dtype.
+ *
+ *   inv_freq         [B|.,half] of freq_dtype (f16 / bf16 / f32), freq_strides = {batch (0: one row for all), frequency}.
+ *   positions        [B|.,S], position_strides likewise: int64 when whole_positions != 0 (rounded to fp32), else f32.
+ *   cos, sin         [B,S,2·half] contiguous, f16, bf16 or f32 (dtype).
+ */
+int kernl_rope_tables(const void *inv_freq, const void *positions, void *cos, void *sin, int64_t B, int64_t S, int64_t half,
+                      const int64_t freq_strides[2], const int64_t position_strides[2], int freq_dtype, int whole_positions,
+                      float scale, int dtype, void *stream);
+
+/*
  * Fused linear layer:  out[M,N] = act(x[M,K] · w[N,K]ᵀ + bias[N]).
  * Replaces the `kernel_fma[grid](...)` launch of src/kernl/implementations/linear_layer.py:254-278
  * (kernel body :92-210).

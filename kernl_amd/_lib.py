@@ -34,6 +34,7 @@ EXPORTED_SYMBOLS = (
     "kernl_attention_skinny_static_init",
     "kernl_attention_skinny_static_fwd",
     "kernl_rope_fwd",
+    "kernl_rope_tables",
     "kernl_linear_fwd",
     "kernl_linear_small_kind",
     "kernl_linear_w8_fwd",
@@ -129,6 +130,8 @@ def load() -> ctypes.CDLL:
     lib.kernl_attention_skinny_static_fwd.argtypes = (
         [_vp] * 5 + [_i64] * 5 + [_i64p] * 6 + [ctypes.c_int, ctypes.c_float, ctypes.c_int, ctypes.c_float, ctypes.c_int, _vp]
     )
+    lib.kernl_rope_tables.restype = ctypes.c_int
+    lib.kernl_rope_tables.argtypes = [_vp] * 4 + [_i64] * 3 + [_i64p] * 2 + [ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_int, _vp]
     lib.kernl_rope_fwd.restype = ctypes.c_int
     lib.kernl_rope_fwd.argtypes = [_vp] * 4 + [_i64] * 4 + [_i64p] * 5 + [ctypes.c_int, ctypes.c_int, _vp]
     lib.kernl_linear_fwd.restype = ctypes.c_int
@@ -320,6 +323,21 @@ def rope_fwd(x, cos, sin, out) -> None:
             DTYPE_CODE[cos.dtype], DTYPE_CODE[x.dtype], _stream(x),
         )
     _check(st, "kernl_rope_fwd")
+
+
+def rope_tables(inv_freq, positions, cos, sin, scale: float) -> None:
+    """inv_freq [B|1,half,1], positions [B|1,1,S] (int64 or float32); cos, sin [B,S,2*half] contiguous, of the same dtype as each other."""
+    _require_gpu(inv_freq, positions, cos, sin)
+    B, S, D = cos.shape
+    lib = load()
+    fs = _arr((0 if inv_freq.shape[0] == 1 else inv_freq.stride(0), inv_freq.stride(1)))
+    ps = _arr((0 if positions.shape[0] == 1 else positions.stride(0), positions.stride(2)))
+    with torch.cuda.device(cos.device):
+        st = lib.kernl_rope_tables(
+            inv_freq.data_ptr(), positions.data_ptr(), cos.data_ptr(), sin.data_ptr(), B, S, D // 2, fs, ps,
+            DTYPE_CODE[inv_freq.dtype], int(positions.dtype == torch.int64), float(scale), DTYPE_CODE[cos.dtype], _stream(cos),
+        )
+    _check(st, "kernl_rope_tables")
 
 
 def linear_small_kind(M: int, N: int, K: int) -> int:

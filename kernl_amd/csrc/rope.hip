@@ -110,7 +110,69 @@ static void launch_rope(const RopeParams &p, bool vec, bool table_f32, hipStream
     else hipLaunchKernelGGL((rope_kernel<T, false, false>), grid, block, 0, st, p);
 }
 
+// The tables of a rotation, cos and sin of position * frequency, both halves of the features alike.  A decoder traces into nine kernels
+// for them (conversions, a product of inner size one, a concatenation, cosine, sine, two scalings, two roundings) that move at most a few
+// MB and are bound by their launches: 47 us at 333 positions of head size 128 and 47 at 2048.  Here a thread owns one (position, frequency):
+// one launch, 4.8 us at either size, about what any kernel takes between large ones.  The angle is rounded to fp32 as that product's is
+// and cosine and sine are the functions the tables were made with, so the tables are the same to the bit.
+struct RopeTableParams {
+    const void *inv, *pos;
+    void *cos, *sin;
+    int B, S, half;
+    int64_t is[2], ps[2];  // element strides {batch, frequency} and {batch, position}; 0 on broadcast batches
+    int inv_dtype, pos_whole;
+    float scale;
+};
+
+template <typename T>
+__global__ void __launch_bounds__(256) rope_tables_kernel(const RopeTableParams p) {
+    const int64_t total = (int64_t)p.B * p.S * p.half;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+        const int j = (int)(i % p.half);
+        const int64_t r = i / p.half;
+        const int s = (int)(r % p.S), b = (int)(r / p.S);
+        const int64_t at = b * p.ps[0] + s * p.ps[1];
+        const float pos = p.pos_whole ? (float)static_cast<const int64_t *>(p.pos)[at] : static_cast<const float *>(p.pos)[at];
+        const float angle = rope_table(p.inv, p.inv_dtype, b * p.is[0] + j * p.is[1]) * pos;
+        float fc = cosf(angle) * p.scale, fs = sinf(angle) * p.scale;
+        asm volatile("" : "+v"(fc), "+v"(fs));  // (the scaled value is rounded to fp32 before it is to T: no mixed-precision product)
+        const T c = from_float<T>(fc), d = from_float<T>(fs);
+        T *cr = static_cast<T *>(p.cos) + r * 2 * p.half + j, *sr = static_cast<T *>(p.sin) + r * 2 * p.half + j;
+        cr[0] = c;
+        cr[p.half] = c;
+        sr[0] = d;
+        sr[p.half] = d;
+    }
+}
+
 }  // namespace kernl
+
+extern "C" int kernl_rope_tables(const void *inv_freq, const void *positions, void *cos, void *sin, int64_t B, int64_t S, int64_t half,
+                                 const int64_t freq_strides[2], const int64_t position_strides[2], int freq_dtype, int whole_positions,
+                                 float scale, int dtype, void *stream) {
+    using namespace kernl;
+    if (inv_freq == nullptr || positions == nullptr || cos == nullptr || sin == nullptr || freq_strides == nullptr || position_strides == nullptr)
+        return set_error(KERNL_ERR_INVALID_ARG, "rope tables: pointers and stride arrays must not be NULL");
+    if (B < 0 || S < 0 || half <= 0)
+        return set_error(KERNL_ERR_INVALID_ARG, "rope tables: bad sizes B=%lld S=%lld half=%lld", (long long)B, (long long)S, (long long)half);
+    if ((dtype != KERNL_F16 && dtype != KERNL_BF16 && dtype != KERNL_F32) ||
+        (freq_dtype != KERNL_F16 && freq_dtype != KERNL_BF16 && freq_dtype != KERNL_F32))
+        return set_error(KERNL_ERR_UNSUPPORTED, "rope tables: unknown dtype %d or %d", dtype, freq_dtype);
+    if (B >= (1ll << 24) || S >= (1ll << 30) || half >= (1ll << 20) || B * S >= (1ll << 36))
+        return set_error(KERNL_ERR_UNSUPPORTED, "rope tables: sizes too large");
+    if (B == 0 || S == 0) return KERNL_OK;
+    RopeTableParams p;
+    p.inv = inv_freq; p.pos = positions; p.cos = cos; p.sin = sin;
+    p.B = (int)B; p.S = (int)S; p.half = (int)half;
+    for (int i = 0; i < 2; ++i) { p.is[i] = freq_strides[i]; p.ps[i] = position_strides[i]; }
+    p.inv_dtype = freq_dtype; p.pos_whole = whole_positions; p.scale = scale;
+    const dim3 grid((unsigned)std::min<int64_t>((B * S * half + 255) / 256, 16384)), block(256);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (dtype == KERNL_F16) hipLaunchKernelGGL((rope_tables_kernel<f16>), grid, block, 0, st, p);
+    else if (dtype == KERNL_BF16) hipLaunchKernelGGL((rope_tables_kernel<bf16>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((rope_tables_kernel<float>), grid, block, 0, st, p);
+    return check_launch("rope tables");
+}
 
 extern "C" int kernl_rope_fwd(const void *x, const void *cos, const void *sin, void *out, int64_t B, int64_t H,
                               int64_t S, int64_t D, const int64_t x_strides[4], const int64_t out_strides[4],

@@ -25,3 +25,21 @@ def rotary_forward(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> tor
     out = torch.empty_like(x)
     _lib.rope_fwd(x, cos, sin, out)
     return out
+
+
+def rotary_tables(inv_freq: torch.Tensor, positions: torch.Tensor, scale: float, dtype: torch.dtype):
+    """(cos, sin) [B,S,2*half] of `cat((a, a), -1)` with a = (inv_freq @ positions).transpose(1, 2), times scale, in dtype.
+    inv_freq [B|1,half,1] floating, positions [B|1,1,S]: float32, or int64 to be rounded to it."""
+    batch = max(inv_freq.shape[0], positions.shape[0])
+    taken = (inv_freq.is_cuda and inv_freq.device == positions.device and inv_freq.dim() == 3 and positions.dim() == 3
+             and inv_freq.shape[2] == 1 and positions.shape[1] == 1 and inv_freq.shape[0] in (1, batch) and positions.shape[0] in (1, batch)
+             and inv_freq.dtype in _lib.DTYPE_CODE and positions.dtype in (torch.int64, torch.float32) and dtype in _lib.DTYPE_CODE
+             and inv_freq.shape[1] > 0 and not torch.is_autocast_enabled("cuda"))
+    if not taken:
+        angles = (inv_freq.to(torch.float32) @ positions.to(torch.float32)).transpose(1, 2)
+        both = torch.cat((angles, angles), dim=-1)
+        return (both.cos() * scale).to(dtype), (both.sin() * scale).to(dtype)
+    cos = torch.empty((batch, positions.shape[2], 2 * inv_freq.shape[1]), dtype=dtype, device=inv_freq.device)
+    sin = torch.empty_like(cos)
+    _lib.rope_tables(inv_freq, positions, cos, sin, scale)
+    return cos, sin

@@ -12,12 +12,14 @@ import torch._dynamo as torchdynamo
 from kernl_amd import _lib
 from kernl_amd.optimizer.cuda_graph import cuda_graphs_wrapper, static_inputs_pool
 from kernl_amd.optimizer.dynamo_backend import dynamo_backend_ofi
+from kernl_amd.optimizer.rotary import fuse_rotary_tables
 
 
 # Module level so that several forwards of one model (encoder / decoder) share it
 # (reference: model_optimization.py:25-29).
 def _compiler(gm: torch.fx.GraphModule, example_inputs: List[torch.Tensor]):
     dynamo_backend_ofi(gm)
+    fuse_rotary_tables(gm)  # after the passes that recognise the tables by the nodes they end in
     return cuda_graphs_wrapper(gm, example_inputs)
 
 
