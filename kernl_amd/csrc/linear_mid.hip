@@ -20,16 +20,17 @@
 
 namespace kernl {
 
-// tile shape, grid of the eight multiplying waves, ring depth and number of loading waves (0: the multiplying waves load) of one build
-template <int BM_, int BN_, int WM_, int WN_, int S_, int NP_ = 4>
+// tile shape, grid of the eight multiplying waves and ring depth of one build
+template <int BM_, int BN_, int WM_, int WN_, int S_>
 struct MidTile {
-    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_, NP = NP_;
-    static constexpr int BK = 64, RB = BK * 2, WAVES = 8 + NP, LOADERS = NP > 0 ? NP : 8;
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_;
+    static constexpr int BK = 64, RB = BK * 2, LOADERS = 4, WAVES = 8 + LOADERS;
     static constexpr int TM = BM / WM, TN = BN / WN, NBM = TM / 16, NBN = TN / 16;
     static constexpr bool X_AHEAD = TM * TN < 96 * 48;  // registers for two sets of x fragments
+    static constexpr bool STAGED = TM * TN >= 64 * 32;  // 16-bit results leave through LDS (see the epilogue)
     static constexpr int X_BYTES = BM * RB, STAGE = (BM + BN) * RB, LDS = S * STAGE;
     static constexpr int LX = BM / (8 * LOADERS), LW = BN / (8 * LOADERS), L = LX + LW;  // 1 KB loads of a loading wave per k-tile
-    static_assert(WM * WN == 8 && LX * 8 * LOADERS == BM && LW * 8 * LOADERS == BN && LDS <= 160 * 1024 && S >= 3 && (S - 1) * L <= 63, "tile shape");
+    static_assert(WM * WN == 8 && LX * 8 * LOADERS == BM && LW * 8 * LOADERS == BN && LDS <= 160 * 1024 && (S == 3 || S == 4) && (S - 1) * L <= 63, "tile shape");
 };
 
 // How the tile grid is dealt to the 8 XCDs, each with an L2 of its own: as 2^xm_shift x 8 / 2^xm_shift blocks of per_m x per_n tiles,
@@ -62,8 +63,7 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_m = wave % Cfg::WM, wave_n = wave / Cfg::WM;
-    const bool loads = Cfg::NP == 0 || wave >= 8;
-    const int loader = Cfg::NP == 0 ? wave : (wave & 7) % Cfg::LOADERS;
+    const int loader = (wave & 7) % Cfg::LOADERS;
     const int r = lane & 15, g = lane >> 4;
     // workgroup b runs on XCD b % 8, which works on a block of the tile grid of its own (or on a contiguous run of tiles)
     int tile_m, tile_n;
@@ -125,9 +125,9 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
         for (int i = 0; i < LW; ++i) wd[i] = ((keep >> (LX + i)) & 1u) != 0 ? wd[i] : kOutOfRange;
     };
     auto request = [&](int kt, int stage) __attribute__((always_inline)) {
-        if (kt == nk - 1 || kt == nk) clip(kt == nk ? 0u : tail_bits);
+        if (kt == nk - 1) clip(tail_bits);
         const uint32_t base = lds_base + (uint32_t)stage * STAGE;
-        const int kbytes = kt < nk ? (kt < k_dealt ? kt ^ turn : kt) * BK * 2 : 0;
+        const int kbytes = (kt < k_dealt ? kt ^ turn : kt) * BK * 2;
 #pragma unroll
         for (int i = 0; i < LX; ++i) load1(xrsrc, xd[i], base + i * Cfg::LOADERS * 1024, kbytes);
 #pragma unroll
@@ -152,7 +152,6 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
     constexpr int V = C % 8 == 0 ? 8 : 4;         // columns per access
     typedef uint32_t words __attribute__((ext_vector_type(V / 2)));
     const int out_n = GATED ? N / 2 : N;
-    const int n_first = (GATED ? n0 / 2 : n0) + wave_n * (GATED ? Cfg::TN / 2 : Cfg::TN) + C * g;
     u32x2 bias_raw[NBN];  // 16-bit values until the epilogue: registers are short in the large tiles
     const bool bias_vec = ((uintptr_t)bias & 7) == 0;
 #pragma unroll
@@ -171,24 +170,31 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
         constexpr int n = decltype(n_c)::value;
         __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
     };
-    if (loads)
+    if (wave >= 8) {
+        // a loading wave: its stalls on the load path hold up neither the LDS reads nor the matrix instructions of the others.  Nothing
+        // is requested beyond the last k-tile, so that after its barrier LDS is free for the epilogue without another one.
+        auto landed = [&](int kt) __attribute__((always_inline)) {  // k-tile kt; at most S - 1 have been requested behind it
+            const int behind = min(kt + S, nk) - 1 - kt;
+            if (behind >= S - 1) wait_loads(IntC<(S - 1) * L>());
+            else if (behind == S - 2) wait_loads(IntC<(S - 2) * L>());
+            else if (S > 3 && behind == S - 3) wait_loads(IntC<(S - 3) * L>());
+            else wait_loads(IntC<0>());
+        };
 #pragma unroll
-        for (int kt = 0; kt < S; ++kt) request(kt, kt);
-    if constexpr (Cfg::NP > 0) {
-        if (loads) {
-            // a loading wave: its stalls on the load path hold up neither the LDS reads nor the matrix instructions of the others
-            wait_loads(IntC<(S - 1) * L>());
-            __syncthreads();
-            int stage = 0;
-            for (int kt = 0; kt < nk; ++kt) {
-                wait_loads(IntC<(S - 2) * L>());
-                __syncthreads();  // as below
-                request(kt + S, stage);
-                stage = stage == S - 1 ? 0 : stage + 1;
-            }
-            __builtin_amdgcn_s_waitcnt(0x0F70);
-            return;
+        for (int kt = 0; kt < S; ++kt)
+            if (kt < nk) request(kt, kt);
+        landed(0);
+        __syncthreads();
+        int stage = 0;
+        for (int kt = 0; kt < nk; ++kt) {
+            // (before this iteration's request: one k-tile fewer behind the next one)
+            if (kt + S < nk) wait_loads(IntC<(S - 2) * L>());
+            else if (kt + 1 < nk) landed(kt + 1);
+            __syncthreads();  // as below
+            if (kt + S < nk) request(kt + S, stage);
+            stage = stage == S - 1 ? 0 : stage + 1;
         }
+        return;
     }
 
     // Fragments are read one k-step ahead, across the barrier.  The large tiles have no registers for a second set of x fragments: theirs
@@ -216,7 +222,6 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
             }
         }
     };
-    if constexpr (Cfg::NP == 0) wait_loads(IntC<(S - 1) * L>());
     __syncthreads();
     read(0, 0, true);
     int stage = 0;
@@ -227,100 +232,169 @@ linear_mid_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__r
         multiply(0, stage);
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if constexpr (Cfg::NP == 0) wait_loads(IntC<(S - 2) * L>());
         __syncthreads();  // k-tile kt + 1 has landed for everyone, and nobody reads k-tile kt any more
         read(0, next, XB == 2);
-        if constexpr (Cfg::NP == 0) {
-            __builtin_amdgcn_sched_barrier(0);
-            request(kt + S, stage);
-        }
         __builtin_amdgcn_sched_barrier(0);
         multiply(1, next);
         __builtin_amdgcn_sched_barrier(0);
         stage = next;
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);
+    // (past the last barrier nothing lands in LDS any more and nobody reads a fragment that counts)
 
-    // ---- epilogue
+    // ---- epilogue.  A lane holds 4 to 24 consecutive columns of one row: stored from there, every 8 or 16 bytes are an access to a line
+    // of their own, one a clock.  So a wave's results go through LDS (a region of its own, rows 16 bytes further apart than they are long)
+    // and leave as whole rows of its block: the fp32 sums of a range of K always (333 x 4096 x 11008 in 192 x 128 tiles and four ranges,
+    // 48 -> 44 us; 333 x 4096 x 4096 in 128 x 128 and two 22.8 -> 21.7), 16-bit results of the larger tiles (384 x 19200 x 64 in 192 x 192
+    // 11.9 -> 9.7 us, 384 x 9600 x 64 in 192 x 96 8.1 -> 7.3, 333 x 32000 x 4096 in 192 x 128 101 -> 99).  The two smallest gain nothing
+    // and would wait for LDS (231 x 2304 x 768 in 64 x 64 6.1 -> 6.2); they stage only what no vector store takes.
+    constexpr int TNO = GATED ? Cfg::TN / 2 : Cfg::TN;  // output columns of a wave
+    auto settle = [&]() __attribute__((always_inline)) {  // the wave's own LDS accesses, in order for the compiler too
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    };
+    const int mw = m0 + wave_m * Cfg::TM;
     if (part != nullptr) {  // fp32 sums of the range, row-major; columns N .. part_rs - 1 hold zeros (their weight rows do)
+        constexpr int PITCH = Cfg::TN * 4 + 16, CH = Cfg::TN / 4;
+        static_assert(8 * 16 * PITCH <= Cfg::LDS, "a row block of every wave");
+        unsigned char *mine = smem + wave * (16 * PITCH);
+        const int nw = n0 + wave_n * Cfg::TN;
 #pragma unroll
         for (int i = 0; i < NBM; ++i) {
-            const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
-            if (m >= M) continue;
-            float *p = part + (int64_t)m * part_rs;
 #pragma unroll
-            for (int j = 0; j < NBN; ++j) {
-                const int n = n0 + mid_weight_row<GATED, Cfg::TN>(wave_n * Cfg::TN + 16 * j + 4 * g);
-                if (n < part_rs) *reinterpret_cast<f32x4_acc *>(p + n) = acc[i][j];
+            for (int j = 0; j < NBN; ++j) *reinterpret_cast<f32x4_acc *>(mine + r * PITCH + (C * g + 4 * j) * 4) = acc[i][j];
+            settle();
+#pragma unroll
+            for (int it = 0; it < 16 * CH / 64; ++it) {
+                const int at = it * 64 + lane, row = at / CH, c = at % CH, m = mw + 16 * i + row, n = nw + 4 * c;
+                const f32x4_acc v = *reinterpret_cast<const f32x4_acc *>(mine + row * PITCH + c * 16);
+                if (m < M && n < part_rs) *reinterpret_cast<f32x4_acc *>(part + (int64_t)m * part_rs + n) = v;
             }
+            settle();
         }
         return;
     }
-    const bool out_vec = out_cs == 1 && (out_rs & (V - 1)) == 0 && ((uintptr_t)out & (2 * V - 1)) == 0;
-    const bool ai_vec = act_in != nullptr && ai_cs == 1 && (ai_rs & (V - 1)) == 0 && ((uintptr_t)act_in & (2 * V - 1)) == 0;
-    const bool res_vec = residual != nullptr && res_cs == 1 && (res_rs & (V - 1)) == 0 && ((uintptr_t)residual & (2 * V - 1)) == 0;
-    auto store = [&](T *p, int64_t cs, bool vec, int n, const float *y) __attribute__((always_inline)) {
-        if (vec && n + V <= out_n) {
-            words w;
+    constexpr int PITCH = TNO * 2 + 16, CH = TNO / 8, ITER = (Cfg::TM * CH + 63) / 64;
+    static_assert(8 * Cfg::TM * PITCH <= Cfg::LDS, "the results of every wave");
+    unsigned char *const mine = smem + wave * (Cfg::TM * PITCH);
+    const int nw = (GATED ? n0 / 2 : n0) + wave_n * TNO;
+    if (mw >= M || nw >= out_n) return;
+    // the staged results to dst, + res rounded a second time as the sum of two 16-bit tensors is
+    auto emit = [&](T *dst, int64_t rs, int64_t cs, const T *res) __attribute__((always_inline)) {
+        settle();
+        const bool rows16 = cs == 1 && (rs & 7) == 0 && ((uintptr_t)dst & 15) == 0 &&
+                            (res == nullptr || (res_cs == 1 && (res_rs & 7) == 0 && ((uintptr_t)res & 15) == 0));
+        if (rows16 && (nw + TNO <= out_n || (out_n & 7) == 0)) {
+            vec8 rv[ITER];
+            if (res != nullptr) {
 #pragma unroll
-            for (int e = 0; e < V / 2; ++e) w[e] = pack2<T>(y[2 * e], y[2 * e + 1]);
-            *reinterpret_cast<words *>(p) = w;
+                for (int it = 0; it < ITER; ++it) {
+                    const int at = it * 64 + lane, row = at / CH, c = at % CH;
+                    rv[it] = *reinterpret_cast<const vec8 *>(res + (int64_t)min(mw + row, M - 1) * res_rs + min(nw + 8 * c, out_n - 8));
+                }
+            }
+#pragma unroll
+            for (int it = 0; it < ITER; ++it) {
+                const int at = it * 64 + lane, row = at / CH, c = at % CH;
+                if ((Cfg::TM * CH % 64 != 0 && row >= Cfg::TM) || mw + row >= M || nw + 8 * c >= out_n) continue;
+                vec8 v = *reinterpret_cast<const vec8 *>(mine + row * PITCH + c * 16);
+                if (res != nullptr)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = from_float<T>(to_float(v[e]) + to_float(rv[it][e]));
+                *reinterpret_cast<vec8 *>(dst + (int64_t)(mw + row) * rs + nw + 8 * c) = v;
+            }
         } else {
-#pragma unroll
-            for (int e = 0; e < V; ++e)
-                if (n + e < out_n) p[e * cs] = from_float<T>(y[e]);
-        }
-    };
-    auto finish = [&](auto act_c) __attribute__((always_inline)) {
-        constexpr int ACT = decltype(act_c)::value;
-        float bz[NBN][4];
-#pragma unroll
-        for (int j = 0; j < NBN; ++j) unpack4<T>(bias_raw[j], bz[j]);
-#pragma unroll
-        for (int i = 0; i < NBM; ++i) {
-            const int m = m0 + wave_m * Cfg::TM + 16 * i + r;
-            if (m >= M) continue;
-            const float scale = row_scale != nullptr ? row_scale[m] : 1.0f;
-            float y[C], v[C];
-#pragma unroll
-            for (int j = 0; j < (GATED ? NBN / 2 : NBN); ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float a = fmaf(acc[i][j][e], scale, bz[j][e]);
-                    if (GATED) {
-                        constexpr int H = GATED ? NBN / 2 : 0;
-                        y[4 * j + e] = apply_act16(a, ACT) * fmaf(acc[i][(j + H) % NBN][e], scale, bz[(j + H) % NBN][e]);
-                    } else {
-                        v[4 * j + e] = a;
-                        y[4 * j + e] = apply_act16(a, ACT);
-                    }
-                }
-#pragma unroll
-            for (int c = 0; c < C; c += V) {
-                const int n = n_first + c;
-                if (residual != nullptr) {
-                    const T *rp = residual + (int64_t)m * res_rs + (int64_t)n * res_cs;
-                    T rv[V];
-                    if (res_vec && n + V <= out_n) *reinterpret_cast<words *>(rv) = *reinterpret_cast<const words *>(rp);
-                    else
-#pragma unroll
-                        for (int e = 0; e < V; ++e) rv[e] = n + e < out_n ? rp[e * res_cs] : from_float<T>(0.0f);
-#pragma unroll
-                    for (int e = 0; e < V; ++e) y[c + e] = to_float(from_float<T>(y[c + e])) + to_float(rv[e]);
-                }
-                store(out + (int64_t)m * out_rs + (int64_t)n * out_cs, out_cs, out_vec, n, y + c);
-                if (!GATED && act_in != nullptr) store(act_in + (int64_t)m * ai_rs + (int64_t)n * ai_cs, ai_cs, ai_vec, n, v + c);
+#pragma unroll 1
+            for (int at = lane; at < Cfg::TM * TNO; at += 64) {
+                const int row = at / TNO, c = at % TNO, m = mw + row, n = nw + c;
+                if (m >= M || n >= out_n) continue;
+                T v = *reinterpret_cast<const T *>(mine + row * PITCH + c * 2);
+                if (res != nullptr) v = from_float<T>(to_float(v) + to_float(res[(int64_t)m * res_rs + (int64_t)n * res_cs]));
+                dst[(int64_t)m * rs + (int64_t)n * cs] = v;
             }
         }
+        settle();
     };
-    switch (act) {
-        case KERNL_ACT_RELU: finish(IntC<KERNL_ACT_RELU>()); break;
-        case KERNL_ACT_TANH: finish(IntC<KERNL_ACT_TANH>()); break;
-        case KERNL_ACT_GELU_ERF: finish(IntC<KERNL_ACT_GELU_ERF>()); break;
-        case KERNL_ACT_GELU_TANH: finish(IntC<KERNL_ACT_GELU_TANH>()); break;
-        case KERNL_ACT_SILU: finish(IntC<KERNL_ACT_SILU>()); break;
-        default: finish(IntC<KERNL_ACT_NONE>()); break;
+    float bz[NBN][4], scale[NBM];
+#pragma unroll
+    for (int j = 0; j < NBN; ++j) unpack4<T>(bias_raw[j], bz[j]);
+#pragma unroll
+    for (int i = 0; i < NBM; ++i) scale[i] = row_scale != nullptr ? row_scale[min(mw + 16 * i + r, M - 1)] : 1.0f;
+    auto results = [&](auto act_c, int i, float (&y)[C]) __attribute__((always_inline)) {  // of the lane's row of row block i
+        constexpr int ACT = decltype(act_c)::value;
+#pragma unroll
+        for (int j = 0; j < (GATED ? NBN / 2 : NBN); ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                y[4 * j + e] = apply_act16(fmaf(acc[i][j][e], scale[i], bz[j][e]), ACT);
+                if (GATED) {
+                    constexpr int H = GATED ? NBN / 2 : 0;
+                    y[4 * j + e] *= fmaf(acc[i][(j + H) % NBN][e], scale[i], bz[(j + H) % NBN][e]);
+                }
+                asm("" : "+v"(y[4 * j + e]));  // rounded to fp32 before it is to T, in every form alike: no mixed-precision product
+            }
+    };
+    auto packed = [&](const float *y) __attribute__((always_inline)) -> words {
+        words w;
+#pragma unroll
+        for (int e = 0; e < V / 2; ++e) w[e] = pack2<T>(y[2 * e], y[2 * e + 1]);
+        return w;
+    };
+    auto stage_as = [&](auto act_c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NBM; ++i) {
+            float y[C];
+            results(act_c, i, y);
+#pragma unroll
+            for (int c = 0; c < C; c += V) *reinterpret_cast<words *>(mine + (16 * i + r) * PITCH + (C * g + c) * 2) = packed(y + c);
+        }
+    };
+    auto with_act = [&](auto then) __attribute__((always_inline)) {
+        switch (act) {
+            case KERNL_ACT_RELU: then(IntC<KERNL_ACT_RELU>()); break;
+            case KERNL_ACT_TANH: then(IntC<KERNL_ACT_TANH>()); break;
+            case KERNL_ACT_GELU_ERF: then(IntC<KERNL_ACT_GELU_ERF>()); break;
+            case KERNL_ACT_GELU_TANH: then(IntC<KERNL_ACT_GELU_TANH>()); break;
+            case KERNL_ACT_SILU: then(IntC<KERNL_ACT_SILU>()); break;
+            default: then(IntC<KERNL_ACT_NONE>()); break;
+        }
+    };
+    if constexpr (!Cfg::STAGED) {
+        auto whole = [&](const void *p, int64_t rs, int64_t cs) __attribute__((always_inline)) { return p == nullptr || (cs == 1 && (rs & (V - 1)) == 0 && ((uintptr_t)p & (2 * V - 1)) == 0); };
+        if (nw + TNO <= out_n && whole(out, out_rs, out_cs) && whole(act_in, ai_rs, ai_cs) && whole(residual, res_rs, res_cs)) {
+            with_act([&](auto act_c) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NBM; ++i) {
+                    const int m = mw + 16 * i + r;
+                    if (m >= M) continue;
+                    const int64_t n = nw + C * g;
+                    float y[C];
+                    if (!GATED && act_in != nullptr) {
+                        results(IntC<KERNL_ACT_NONE>(), i, y);
+#pragma unroll
+                        for (int c = 0; c < C; c += V) *reinterpret_cast<words *>(act_in + m * ai_rs + n + c) = packed(y + c);
+                    }
+                    results(act_c, i, y);
+                    if (residual != nullptr)
+#pragma unroll
+                        for (int c = 0; c < C; c += V) {
+                            T rv[V];
+                            *reinterpret_cast<words *>(rv) = *reinterpret_cast<const words *>(residual + m * res_rs + n + c);
+#pragma unroll
+                            for (int e = 0; e < V; ++e) y[c + e] = to_float(from_float<T>(y[c + e])) + to_float(rv[e]);
+                        }
+#pragma unroll
+                    for (int c = 0; c < C; c += V) *reinterpret_cast<words *>(out + m * out_rs + n + c) = packed(y + c);
+                }
+            });
+            return;
+        }
     }
+    if (!GATED && act_in != nullptr) {
+        stage_as(IntC<KERNL_ACT_NONE>());
+        emit(act_in, ai_rs, ai_cs, nullptr);
+    }
+    with_act(stage_as);
+    emit(out, out_rs, out_cs, residual);
 }
 
 template <typename T, typename Cfg, bool GATED>

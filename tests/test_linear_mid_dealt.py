@@ -71,3 +71,27 @@ def test_dealt_k_tiles_of_the_wide_kernels(shape, tile, force, close):
     _lib.linear_fwd(x.cuda(), w.cuda(), None, out, None, _lib.ACT_NONE)
     torch.cuda.synchronize()
     close(out, linear_oracle(x, w, None, ""), what=f"tile {tile} {shape}")
+
+
+@pytest.mark.parametrize("tile", [11, 15, 17, 18, 19, 20, 21, 22])
+@pytest.mark.parametrize("K", [8, 64, 128, 192, 200, 256, 264, 320])  # fewer k-tiles than the ring is deep, as many, one and two more
+@pytest.mark.parametrize("layout", ["rows", "odd rows", "columns"])   # whole vectors; row strides that no vector has; column-major
+def test_short_rings_and_the_epilogues_forms(layout, K, tile, force, close):
+    M, N = 200, 208
+    gen = torch.Generator().manual_seed(K + tile)
+    x, w = torch.randn((M, K), generator=gen).half(), (torch.randn((N, K), generator=gen) * K ** -0.5).half()
+    b = torch.randn((N,), generator=gen).half()
+
+    def tensor():
+        if layout == "columns":
+            return torch.full((N, M), float("nan"), dtype=torch.float16, device="cuda").t()
+        return torch.full((M, N + (3 if layout == "odd rows" else 8)), float("nan"), dtype=torch.float16, device="cuda")[:, :N]
+
+    out, saved, plain = tensor(), tensor(), tensor()
+    force(tile)
+    _lib.linear_fwd(x.cuda(), w.cuda(), b.cuda(), out, saved, _lib.ACT_SILU)
+    _lib.linear_fwd(x.cuda(), w.cuda(), b.cuda(), plain, None, _lib.ACT_NONE)
+    torch.cuda.synchronize()
+    close(out, linear_oracle(x, w, b, "silu"), scale="magnitude", what=f"tile {tile}")
+    close(saved, linear_oracle(x, w, b, ""), what=f"tile {tile} pre-activation")
+    assert torch.equal(saved, plain)
