@@ -325,7 +325,7 @@ int kernl_layernorm_rows32_fwd(const float *x, const void *w, const void *bias, 
 int kernl_linear_small_kind(int64_t M, int64_t N, int64_t K);
 
 /*
- * Whether kernl_linear_fwd runs M x N x K (16-bit, plain epilogue) on one of its wide or 8-wave tile kernels, and which: 0 = no,
+ * Whether kernl_linear_fwd runs M x N x K (16-bit, plain epilogue) on one of its wide kernels or middling tiles, and which: 0 = no,
  * otherwise the kernl_linear_force_tile value of the kernel.  kernl_linear_residual_fwd and
  * kernl_linear_scaled_fwd exist on those kernels only and run them whatever the shape: a caller asks here first and
  * keeps the separate addition (or normalisation) where another kernel is the faster one.  No counterpart in the
@@ -335,7 +335,7 @@ int kernl_linear_wide_kind(int64_t M, int64_t N, int64_t K);
 
 /*
  * Whether kernl_linear_fwd (gated: kernl_linear_glu_fwd, N = rows of the interleaved weight) runs M x N x K, more than 64 rows and
- * no small problem, on one of its 8-wave tiles over the whole K, and which (the kernl_linear_force_tile value).  A caller that
+ * no small problem, on one of its middling tiles (65 to some 3000 rows) over the whole K, and which (the kernl_linear_force_tile value).  A caller that
  * would otherwise route such a shape to the stream-K or split-K entry points should call kernl_linear_fwd instead.
  */
 int kernl_linear_mid_kind(int64_t M, int64_t N, int64_t K, int gated);

@@ -346,7 +346,7 @@ def linear_small_kind(M: int, N: int, K: int) -> int:
 
 
 def linear_mid_kind(M: int, N: int, K: int, gated: bool = False) -> int:
-    """Non-zero when `kernl_linear_fwd` (`kernl_linear_glu_fwd`) runs the problem on one of its 8-wave tiles: such shapes are not
+    """Non-zero when `kernl_linear_fwd` (`kernl_linear_glu_fwd`) runs the problem on one of its middling tiles: such shapes are not
     handed to the stream-K or split-K entry points."""
     return int(load().kernl_linear_mid_kind(int(M), int(N), int(K), int(bool(gated))))
 

@@ -328,10 +328,10 @@ extern "C" int kernl_linear_scaled_fwd(const void *x, const void *w, const void 
     a.act = gated ? (kGluBit | activation) : activation;
     a.st = static_cast<hipStream_t>(stream);
     a.row_scale = row_scale;
-    // the wide kernels take per-row factors (5 / 6: 256-row tiles, 7 / 8: 128-row tiles; gated: 256 x 256 only), and the 8-wave tiles
+    // the wide kernels take per-row factors (5 / 6: 256-row tiles, 7 / 8: 128-row tiles; gated: 256 x 256 only), and the middling tiles
     if (g_linear_force_tile == 0 && small_problem_kind(a.M, a.N, a.K) == 0)
         if (const int mid = mid_kind(a.M, a.N, a.K, gated != 0))
-            if (run_one_launch(a, dtype, mid)) return check_launch("scaled linear (8-wave tiles)");
+            if (run_one_launch(a, dtype, mid)) return check_launch("scaled linear (middling tiles)");
     int pick = g_linear_force_tile >= 5 && g_linear_force_tile <= 8 ? g_linear_force_tile : pick_tile(a.M, a.N, a.K, gated != 0, true);
     if (gated) pick = 5;
     if (pick == 5) run_wide(a, dtype, 256);
@@ -371,10 +371,10 @@ extern "C" int kernl_linear_residual_fwd(const void *x, const void *w, const voi
     a.st = static_cast<hipStream_t>(stream);
     a.residual = residual;
     a.res_rs = residual_strides[0]; a.res_cs = residual_strides[1];
-    // the wide kernels add a residual (5 / 6: 256-row tiles, 7 / 8: 128-row tiles), and the 8-wave tiles
+    // the wide kernels add a residual (5 / 6: 256-row tiles, 7 / 8: 128-row tiles), and the middling tiles
     if (g_linear_force_tile == 0 && small_problem_kind(a.M, a.N, a.K) == 0)
         if (const int mid = mid_kind(a.M, a.N, a.K, false))
-            if (run_one_launch(a, dtype, mid)) return check_launch("linear + residual (8-wave tiles)");
+            if (run_one_launch(a, dtype, mid)) return check_launch("linear + residual (middling tiles)");
     const int pick = g_linear_force_tile >= 5 && g_linear_force_tile <= 8 ? g_linear_force_tile : pick_tile(a.M, a.N, a.K, false, true);
     if (pick == 5) run_wide(a, dtype, 256);
     else if (pick == 6) run_wide(a, dtype, 192);

@@ -62,7 +62,7 @@ def takes_small_problem_kernel(x2d: torch.Tensor, weight: torch.Tensor) -> bool:
 
 
 def takes_mid_kernel(x2d: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
-    """Whether the product runs on one of the 8-wave tiles over the whole K (65 to some 3000 rows): faster there than the
+    """Whether the product runs on one of the middling tiles over the whole K (65 to some 3000 rows): faster there than the
     stream-K and split-K kernels the shape would otherwise qualify for."""
     return (
         x2d.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x2d.dtype
@@ -278,7 +278,7 @@ def rms_linear_layer(
         and x_.shape[0] > FEW_ROW_MAX_ROWS
         and _lib.linear_scaled_supported(x_, folded_weight)
         and (bias is None or bias.dtype == x.dtype)
-        # not where the row count is too small for the wide tile kernels to have one tile per CU.  (The 8-wave tiles that most of
+        # not where the row count is too small for the wide tile kernels to have one tile per CU.  (The middling tiles that most of
         # those products run on would take the row factors too; but weight * rms_weight is rounded to 16 bits, which a small
         # norm weight makes coarser than the rounding of the normalised row, so the folded weight stays with the large prompts.)
         and not takes_small_problem_kernel(x_, folded_weight)

@@ -765,7 +765,7 @@ def rms_fused_linear_rope_wrapper(x: torch.Tensor, rms_weight, eps: float, weigh
 
 def _epilogue_addition_pays_in_front_of_a_norm(v: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether the projection runs the wide tile kernels (5 .. 8): the sum is rounded to 16 bits on its way to the LayerNorm, in
-    exchange for one tensor less to read (16384 x 768: 4 us).  The 8-wave tiles of fewer rows add in their epilogue too, but at
+    exchange for one tensor less to read (16384 x 768: 4 us).  The middling tiles of fewer rows add in their epilogue too, but at
     2048 x 768 the tensor is worth a microsecond, and the add + LayerNorm kernel adds in fp32."""
     return 5 <= _lib.linear_wide_kind(v.numel() // v.shape[-1], weight.shape[0], weight.shape[1]) <= 8
 
