@@ -782,14 +782,16 @@ def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, r
     Few rows leave the norm to them and return a `DeferredNorm`, if all of them take it; `residual` may be one."""
     from kernl_amd.optimizer.layer_norm import _half_params_once, add_layer_norm_wrapper_functional, layer_norm_wrapper_functional
 
-    if (behind is not None and isinstance(residual, torch.Tensor) or isinstance(residual, DeferredNorm)) and len(normalized_shape) == 1:
+    # parameters follow the sum's type: a residual kept in fp32 keeps them (and the layers behind) in fp32
+    alike = isinstance(residual, (torch.Tensor, DeferredNorm)) and residual.dtype == v.dtype and len(normalized_shape) == 1
+    if alike and (behind is not None or isinstance(residual, DeferredNorm)):
         _half_params_once(v, weight, bias, ln_weight, ln_bias, *(w for weights in behind or () for w in weights))
         if deferrable(v, weight, bias, residual, ln_weight, ln_bias, behind or ()):
             norm = linear_add_deferred(v, weight, bias, residual, ln_weight, ln_bias, eps)
             return norm if behind is not None else norm.normalised()
     if isinstance(residual, DeferredNorm):
         residual = residual.normalised()
-    if isinstance(residual, torch.Tensor) and isinstance(v, torch.Tensor) and len(normalized_shape) == 1:
+    if alike and isinstance(v, torch.Tensor):
         _half_params_once(v, weight, bias, ln_weight, ln_bias)
         need = split_finish_bytes(v, weight, bias, residual, FINISH_LAYER_NORM, ln_weight, ln_bias)
         if need:
