@@ -311,7 +311,7 @@ static void launch_skinny_part1(const SkinnyParams &p, hipStream_t st) {
     // keys and values beyond the 256 MB of the memory-side cache (head size 64 and 128): read once and not kept, [24,32,1,3001,128] bf16
     // 197 -> 172 us (6.0 -> 6.9 TB/s); storage that fits the cache is read from it at 7.5 TB/s and 5.7 with these loads
     if constexpr (!KV8)
-        if (p.M == 1 && (int64_t)p.B * p.H * p.N * p.D * 4 > ((int64_t)256 << 20) && (p.D == 64 || p.D == 128)) {
+        if (p.M == 1 && (p.D == 64 || p.D == 128) && skinny_streams_keys(p.B, p.H, p.N, p.D, p.ks, p.vs)) {
             if (p.D == 64) hipLaunchKernelGGL((attention_skinny_part1<T, 8, KV8, KPI, true>), grid, dim3(256), 0, st, p);
             else hipLaunchKernelGGL((attention_skinny_part1<T, 16, KV8, KPI, true>), grid, dim3(256), 0, st, p);
             return;

@@ -3,6 +3,8 @@
 // the same functions lane by lane on the CPU.  Nothing in here may depend on HIP types.
 #pragma once
 
+#include <stdint.h>
+
 #if defined(__HIPCC__)
 #define KERNL_HD __host__ __device__ __forceinline__
 #else
@@ -128,6 +130,17 @@ struct FewRowStageMap {
     }
     static KERNL_HD int frag_offset(int mb, int r, int g, int s) { return swz_offset<128>(16 * mb + r, 2 * g + s); }
 };
+
+// ----------------------------------------------------------------------------------------------------
+// Single-query attention (attention_skinny.hip): whether keys and values, [B,H,N,D] of 16-bit values with element strides ks and vs, are read
+// past the 256 MB memory-side cache.  Only where every key row is read once: a batch or head dimension of stride 0 is one storage read by
+// several workgroups, which the caches serve, whatever its size (32 query heads over one key head, head size 128: 24 x 3000 keys 65 us, past
+// the cache 130; 64 x 12000 keys, 393 MB of storage, 820 and 1570).
+// ----------------------------------------------------------------------------------------------------
+KERNL_HD bool skinny_streams_keys(int64_t B, int64_t H, int64_t N, int64_t D, const int64_t *ks, const int64_t *vs) {
+    const bool shared = (B > 1 && (ks[0] == 0 || vs[0] == 0)) || (H > 1 && (ks[1] == 0 || vs[1] == 0)) || ks[2] == 0 || vs[2] == 0;
+    return !shared && B * H * N * D * 4 > ((int64_t)256 << 20);
+}
 
 // ----------------------------------------------------------------------------------------------------
 // Small-problem linear kernels (linear_small.hip): an operand tile of a k-tile is ROWS rows of 128 bytes (64 k-values)

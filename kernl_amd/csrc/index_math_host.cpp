@@ -86,6 +86,11 @@ int kernl_idx_wide_weight_row(int layout, int row) {
     return -1;
 }
 
+// strides {batch, head, key}, in elements
+int kernl_idx_skinny_streams(int64_t B, int64_t H, int64_t N, int64_t D, const int64_t *ks, const int64_t *vs) {
+    return skinny_streams_keys(B, H, N, D, ks, vs) ? 1 : 0;
+}
+
 int kernl_idx_xcd_contiguous(int b, int n) { return xcd_contiguous_index(b, n); }
 
 // which: 0 load_row(q=a), 1 load_chunk(q=a), 2 frag_offset(row=a, kstep=b, g=c)

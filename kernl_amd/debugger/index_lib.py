@@ -28,6 +28,8 @@ class IndexLib:
             fn = getattr(cdll, name)
             fn.restype = ctypes.c_int
             fn.argtypes = [ctypes.c_int] * n
+        cdll.kernl_idx_skinny_streams.restype = ctypes.c_int
+        cdll.kernl_idx_skinny_streams.argtypes = [ctypes.c_int64] * 4 + [ctypes.POINTER(ctypes.c_int64)] * 2
 
     def rowperm16(self, i: int) -> int:
         return self._c.kernl_idx_rowperm16(i)
@@ -49,6 +51,11 @@ class IndexLib:
 
     def xcd_contiguous(self, b: int, n: int) -> int:
         return self._checked(self._c.kernl_idx_xcd_contiguous(b, n))
+
+    def skinny_streams(self, shape, key_strides, value_strides) -> bool:
+        """shape [B,H,N,D] and element strides of keys and values."""
+        ks, vs = ((ctypes.c_int64 * 3)(*s[:3]) for s in (key_strides, value_strides))
+        return bool(self._c.kernl_idx_skinny_streams(*shape, ks, vs))
 
     def small_tile(self, what: str, a: int, b: int = 0, c: int = 0) -> int:
         return self._checked(self._c.kernl_idx_small_tile(self.SMALL[what], a, b, c))
