@@ -58,9 +58,24 @@ def _plain(dtype: torch.dtype, *params: Optional[torch.Tensor]) -> bool:
     return all(p is None or (p.dtype == dtype and p.is_contiguous() and p.data_ptr() % 16 == 0) for p in params)
 
 
-def _rows(t: torch.Tensor) -> Optional[torch.Tensor]:
-    t = t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
-    return t if t.stride(-1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 else None
+def rows_of(t: torch.Tensor) -> torch.Tensor:
+    """t as [rows, features]; a copy where its strides have no such view."""
+    return t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
+
+
+def row_stride(t: torch.Tensor) -> Optional[int]:
+    """The row stride of `rows_of(t)`, found without making it; None unless its features are contiguous and its 16-bit rows 16-byte aligned."""
+    features, row, step = t.shape[-1], 0, None
+    for size, stride in zip(reversed(t.shape[:-1]), reversed(t.stride()[:-1])):
+        if size == 1:
+            continue
+        if step is None:
+            row, step = stride, stride * size
+        elif stride == step:
+            step *= size
+        else:  # no view: the rows of the copy lie one behind the other
+            return features if features % 8 == 0 else None
+    return row if t.stride(-1) == 1 and row % 8 == 0 and t.data_ptr() % 16 == 0 else None
 
 
 def deferrable(x: torch.Tensor, weight: torch.Tensor, bias, residual, gamma, beta, behind: Sequence[Tuple[torch.Tensor, ...]]) -> bool:
@@ -81,7 +96,7 @@ def deferrable(x: torch.Tensor, weight: torch.Tensor, bias, residual, gamma, bet
             return False
         if not _takes(rows, sum(w.shape[0] for w in weights), weights[0].shape[1]):
             return False
-    return _rows(x) is not None and _rows(inner) is not None
+    return row_stride(x) is not None and row_stride(inner) is not None
 
 
 def linear_add_deferred(x: torch.Tensor, weight: torch.Tensor, bias, residual, gamma, beta, eps: float) -> DeferredNorm:
@@ -90,8 +105,8 @@ def linear_add_deferred(x: torch.Tensor, weight: torch.Tensor, bias, residual, g
     out = torch.empty((*x.shape[:-1], n), device=x.device, dtype=torch.float32)
     stats = torch.empty((x.numel() // x.shape[-1], n // _lib.NORM_GROUP, 2), device=x.device, dtype=torch.float32)
     if isinstance(residual, DeferredNorm):
-        args = (_rows(residual.rows), residual.stats, residual.gamma, residual.beta, residual.kernel_eps)
+        args = (rows_of(residual.rows), residual.stats, residual.gamma, residual.beta, residual.kernel_eps)
     else:
-        args = (_rows(residual), None, None, None, 0.0)
-    _lib.linear_norm_add_fwd(_rows(x), weight, bias, *args, out.view(-1, n), stats)
+        args = (rows_of(residual), None, None, None, 0.0)
+    _lib.linear_norm_add_fwd(rows_of(x), weight, bias, *args, out.view(-1, n), stats)
     return DeferredNorm(out, stats, gamma, beta, eps)

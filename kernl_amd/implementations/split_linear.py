@@ -1,19 +1,13 @@
 """Linear layers with K split over several workgroups a tile, whose second launch finishes the rows: the residual, the row statistics of
 the RMSNorm behind it, or the whole add + LayerNorm (`kernl_linear_split_fwd`).  No counterpart in the reference, whose models add and
 normalise in kernels of their own behind its linear kernel (implementations/linear_layer.py:213-292)."""
-from typing import Optional
-
 import torch
 from torch.autograd import forward_ad
 
 from kernl_amd import _lib
+from kernl_amd.implementations.deferred_norm import row_stride, rows_of
 
 FINISH_RESIDUAL, FINISH_RMS_STATS, FINISH_LAYER_NORM = _lib.FINISH_RESIDUAL, _lib.FINISH_RMS_STATS, _lib.FINISH_LAYER_NORM
-
-
-def _rows(t: torch.Tensor) -> Optional[torch.Tensor]:
-    t = t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
-    return t if t.stride(-1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 else None
 
 
 def split_finish_bytes(x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor, finish: int, gamma=None, beta=None) -> int:
@@ -34,8 +28,8 @@ def split_finish_bytes(x: torch.Tensor, weight: torch.Tensor, bias, residual: to
         return 0
     if torch.is_grad_enabled() and any(t.requires_grad for t in (x, residual, *params)):
         return 0
-    x_ = _rows(x)
-    return need if x_ is not None and x_.stride(0) >= k and x_.stride(0) < (1 << 22) and _rows(residual) is not None else 0
+    stride = row_stride(x)
+    return need if stride is not None and k <= stride < (1 << 22) and row_stride(residual) is not None else 0
 
 
 def split_finish_linear(need: int, x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor, finish: int, gamma=None, beta=None,
@@ -46,5 +40,5 @@ def split_finish_linear(need: int, x: torch.Tensor, weight: torch.Tensor, bias, 
     rows = x.numel() // x.shape[-1]
     rstd = torch.empty((rows,), device=x.device, dtype=torch.float32) if finish == FINISH_RMS_STATS else None
     workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
-    _lib.linear_split_fwd(_rows(x), weight, bias, _rows(residual), gamma, beta, eps, out.view(rows, -1), rstd, workspace, finish)
+    _lib.linear_split_fwd(rows_of(x), weight, bias, rows_of(residual), gamma, beta, eps, out.view(rows, -1), rstd, workspace, finish)
     return (out, rstd) if finish == FINISH_RMS_STATS else out
