@@ -2069,6 +2069,14 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
     if (short_k || (M <= 128 && N * K < 12 * (1 << 20))) return 0;
     const double nk = (double)((K + 63) / 64), hbm = 4.0 + (double)(N * K) * 2.0 / 4.6e6;  // us at 4.6 TB/s
     MidChoice best = mid_tile_of(M, N, K, gated);
+    // Two regions where the tiles fall behind their estimate, which holds from some 130 to 3000 rows (us, these tiles / what runs instead):
+    //  - a weight of whole 192-column tiles from the memory-side cache under more than 3000 rows: x comes from there too, and the 256 x 192
+    //    kernel has no edge to pay for (3204 x 3072 x 2560 73 / 66, 3999 x 3072 x 2048 60 / 52, 4082 x 2304 x 2560 59 / 51; with an edge it
+    //    loses, 3810 x 2560 x 2048 49 / 60);
+    //  - one or two row tiles over a long K: most of a tile's loads are x again (108 x 12288 x 11008 93 / 82, 89 x 11008 x 11008 85 / 73, gates of
+    //    128 x 5120 x 11008 92 / 71; at K = 8192 they are level, 91 x 11008 x 8192 61 / 59).
+    if (!gated && M > 3000 && N % 192 == 0 && N * K <= ((int64_t)1 << 23)) best.us *= 1.35;
+    if (M <= 128 && K > 8192) best.us *= 1.3;
     double other = wide_us(M, N, K, gated);
     if (M <= 128 && K % 64 == 0) {
         const double few = 10.0 + (double)(N * K) * 2.0 / 3.7e6;
