@@ -65,7 +65,7 @@ def rows_of(t: torch.Tensor) -> torch.Tensor:
 
 def row_stride(t: torch.Tensor) -> Optional[int]:
     """The row stride of `rows_of(t)`, found without making it; None unless its features are contiguous and its 16-bit rows 16-byte aligned."""
-    features, row, step = t.shape[-1], 0, None
+    features, row, step = t.shape[-1], None, None
     for size, stride in zip(reversed(t.shape[:-1]), reversed(t.stride()[:-1])):
         if size == 1:
             continue
@@ -75,6 +75,10 @@ def row_stride(t: torch.Tensor) -> Optional[int]:
             step *= size
         else:  # no view: the rows of the copy lie one behind the other
             return features if features % 8 == 0 else None
+    if t.dim() == 2:  # as it lies, also with one row
+        row = t.stride(0)
+    elif row is None:  # one row: the view's rows lie one behind the other
+        row = features
     return row if t.stride(-1) == 1 and row % 8 == 0 and t.data_ptr() % 16 == 0 else None
 
 
