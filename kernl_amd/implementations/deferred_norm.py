@@ -100,7 +100,8 @@ def deferrable(x: torch.Tensor, weight: torch.Tensor, bias, residual, gamma, bet
             return False
         if not _takes(rows, sum(w.shape[0] for w in weights), weights[0].shape[1]):
             return False
-    return row_stride(x) is not None and row_stride(inner) is not None
+    stride = row_stride(x)  # (rows that lie over each other, as expanded ones do, are left to the other kernels)
+    return stride is not None and k <= stride < (1 << 22) and row_stride(inner) is not None
 
 
 def linear_add_deferred(x: torch.Tensor, weight: torch.Tensor, bias, residual, gamma, beta, eps: float) -> DeferredNorm:

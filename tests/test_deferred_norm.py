@@ -238,3 +238,22 @@ def test_only_norms_of_known_readers_are_marked():
         norms = [n for n in gm.graph.nodes if n.target is linear.linear_add_layer_norm_wrapper]
         names = [[[w.name for w in weights] for weights in n.kwargs.get("behind", ())] for n in norms]
         assert names == ([[], []] if leak else [[["w", "w2"], ["w"]], []])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["expanded", "one odd row"])
+def test_rows_the_kernel_does_not_take_are_left_to_the_others(form):
+    from kernl_amd.implementations.deferred_norm import DeferredNorm
+    from kernl_amd.implementations.layer_norm import add_layer_norm
+    from kernl_amd.implementations.linear_layer import linear_layer
+    from kernl_amd.optimizer.linear import linear_add_layer_norm_wrapper
+
+    x, w, b, res, gamma, beta = _make(20, 768, 768, torch.float16, 1)
+    if form == "expanded":
+        x = x[:1].expand(20, 768)
+    else:
+        x, res = torch.nn.functional.pad(x[:1], (0, 4))[:, :768], res[:1]
+    behind = ((_make(1, 3072, 768, torch.float16, 2)[1],),)
+    out = linear_add_layer_norm_wrapper(x, w, b, res, (768,), gamma, beta, 1e-5, behind=behind)
+    assert not isinstance(out, DeferredNorm)
+    assert torch.equal(out, add_layer_norm(linear_layer(x, w, b), res, gamma, beta, 1e-5))
