@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(256, WPE) attention_stream_kernel(const AttnPa
         qt = slot % p.nq_tiles;
         if (b >= p.B) return;
     } else {
-        const RankedItem item = CAUSAL ? ranked_item(slot, (p.B * p.H + 7) / 8, p.nq_tiles) : RankedItem{slot / p.nq_tiles, slot % p.nq_tiles};
+        const RankedItem item = CAUSAL ? ranked_item(slot, (p.B * p.H + 7) / 8, p.nq_tiles, p.rank_group) : RankedItem{slot / p.nq_tiles, slot % p.nq_tiles};
         const int bh = item.head * 8 + xcd;
         qt = item.rank;
         if (bh >= p.B * p.H) return;
@@ -1089,6 +1089,7 @@ static int attention_entry(const void *q, const void *k, const void *v, void *ou
     p.mask_fast = 0;
     p.xcd_by_batch = 0;
     p.causal_off = is_causal != 0 ? (int)start_position : 0;
+    p.rank_group = rank_group_of((B * H + 7) / 8, M, N, p.causal_off, D);
     if (mask_mode == MASK_MATRIX && (mask_dtype == KERNL_F32 || mask_dtype == dtype)) {
         const int64_t es = mask_dtype == KERNL_F32 ? 4 : 2;
         p.mask_fast = mask_strides[3] == 1 && p.ms[0] % 4 == 0 && p.ms[1] % 4 == 0 && p.ms[2] % 4 == 0 && p.ms[2] > 0 &&

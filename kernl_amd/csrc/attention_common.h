@@ -36,6 +36,7 @@ struct AttnParams {
     int mask_fast;  // matrix mask rows: 1 = readable as aligned 4-element vectors through 32-bit offsets,
                     // 2 = 16-byte chunks of a row are aligned too (they can be staged through LDS)
     int xcd_by_batch;  // workgroups of one batch entry (all heads) share an XCD instead of those of one head
+    int rank_group;  // causal: heads whose tiles are ranked together (ranked_item)
     int causal_off;  // causal: query row m sees keys 0 .. m + causal_off (0: top-left aligned)
 };
 
@@ -51,20 +52,6 @@ __device__ __forceinline__ float scale_mask(float mv, float clamp) {
     return fmaxf(mv * kLog2eA, kClampFloor);
 }
 
-
-// The place of item `at` among an XCD's `heads` heads of `tiles` query tiles each, causal: kRankHeads heads at a time, the longest tiles
-// of all of them first, so that what comes last, beside other workgroups or after them, is short: with the tiles of a head next to each
-// other, a grid of one to a few rounds ended with long tiles that had started late (us, [heads, rows, head size], pipelined kernel up to
-// [32,..] and streaming kernel from [64,..]: [32,1500,128] 45.7 -> 30.6, [32,2048,64] 30.8 -> 25.8, [64,1500,128] 63.7 -> 47.9,
-// [128,333,128] 17.9 -> 15.8, [128,900,64] 33.4 -> 28.1, [512,512,64] 42.8 -> 37.5).  Not all heads at once: 32 heads of 333 rows and head
-// size 128 outgrow the XCD's L2, 24.9 -> 29.1, where 16 at a time take 25.8 (and 26.3 before).
-static constexpr int kRankHeads = 16;
-struct RankedItem { int head, rank; };  // rank 0: the last query tile
-__device__ static inline RankedItem ranked_item(int at, int heads, int tiles) {
-    const int first = at / (kRankHeads * tiles) * kRankHeads, members = heads - first < kRankHeads ? heads - first : kRankHeads;
-    const int in = at - first * tiles;
-    return {first + in % members, in / members};
-}
 
 // How attention_short.hip and attention_split.hip place value rows in LDS: the row's 16-byte chunk c at c ^ value_flip(row).  A transposing
 // read takes 8 bytes from each of 8 rows at 4 places a quarter of a row apart; rows of head size 64 alternate between the halves of the

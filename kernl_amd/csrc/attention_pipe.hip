@@ -104,9 +104,10 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attention_pipe_kernel(co
 
     // ---- the work of this workgroup.  The grid is persistent: 8 W workgroups, W per XCD (workgroup ids are dealt
     // round-robin to the XCDs by hardware).  XCD x owns the (batch, head) pairs bh = x, x + 8, ...; its items are
-    // (pair, query tile) with the query tiles of a pair next to each other, so that the workgroups working on one
-    // pair at the same time share its K and V through that XCD's L2.  Workgroup j of the XCD takes item j of every
-    // round of W items, in alternating direction (the long and the short query tiles of causal attention pair up).
+    // (pair, query tile), without causality with the query tiles of a pair next to each other, so that the workgroups working
+    // on one pair at the same time share its K and V through that XCD's L2; with it as ranked_item orders them, the longest tiles of
+    // a group of pairs first.  Workgroup j of the XCD takes item j of every round of W items, in alternating direction (the long
+    // and the short query tiles of causal attention pair up).
     const int xcd = blockIdx.x & 7, wg_j = blockIdx.x >> 3, wg_w = gridDim.x >> 3;
     const int bh_total = p.B * p.H;
     const int n_items = (xcd < bh_total) ? ((bh_total - xcd + 7) / 8) * p.nq_tiles : 0;
@@ -224,7 +225,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attention_pipe_kernel(co
         }
     };
     auto request_item = [&](int idx) __attribute__((always_inline)) {
-        const RankedItem at = CAUSAL ? ranked_item(idx, (bh_total - xcd + 7) / 8, p.nq_tiles) : RankedItem{idx / p.nq_tiles, idx % p.nq_tiles};
+        const RankedItem at = CAUSAL ? ranked_item(idx, (bh_total - xcd + 7) / 8, p.nq_tiles, p.rank_group) : RankedItem{idx / p.nq_tiles, idx % p.nq_tiles};
         const int bh = 8 * at.head + xcd, qt = at.rank;
         req_b = bh / p.H;
         req_h = bh % p.H;
@@ -811,11 +812,11 @@ static void launch_pipe_t(const AttnParams &p, int mask_mode, bool causal, hipSt
 // each other: no pairs to gain by at head size 128 (1024 rows, 4096 keys, 64 heads: 114.4 / 127.7; 32 heads, 1.0: 72.3 / 67.3), while at 64
 // this kernel is ahead at any grid (1024 over 4096, 64 heads, 1.0: 70.1 / 63.9; 2048 over 4096, 2.0: 120.6 / 104.9).
 // Below kPipeMinKeys keys only what the chip holds at once: [32,700,64] 12.2 / 10.3, [48,900,64] 16.5 / 13.6, [128,333,64] 10.8 / 10.3,
-// [128,320,64] 8.9 / 9.6, [80,800,64] (1.1) 17.0 / 18.8; [40,512,128] 14.8 / 14.3, [48,400,128] 12.7 / 12.8.
+// [128,320,64] 8.9 / 9.6, [80,800,64] (1.1) 17.0 / 18.8; of one-tile heads half as many, 120 rows over 404 keys, 366 heads: 16.2 / 19.2; [40,512,128] 14.8 / 14.3, [48,400,128] 12.7 / 12.8.
 static bool pipe_pays_causal(const AttnParams &p, int D) {
     const int64_t tiles = (p.M + 127) / 128, full = D == 64 ? 512 : 256;
     const int64_t items = (int64_t)((p.B * p.H + 7) / 8) * 8 * tiles;  // (the XCD with the most heads sets the pace)
-    if (p.N < kPipeMinKeys) return p.N >= (D == 64 ? 321 : 512) && items <= full;
+    if (p.N < kPipeMinKeys) return p.N >= (D == 64 ? 321 : 512) && items * (D == 64 && tiles == 1 ? 2 : 1) <= full;
     if (4 * (int64_t)p.causal_off >= p.M) return D == 64 || items <= full;
     return 4 * items <= 5 * full || (2 * items <= 3 * full && tiles >= 10) || (items <= 2 * full && tiles >= (D == 64 ? 24 : 16)) ||
            (D == 64 ? tiles >= 40 && items <= 3 * full : tiles >= 64 && 4 * items <= 9 * full);

@@ -132,6 +132,35 @@ struct FewRowStageMap {
 };
 
 // ----------------------------------------------------------------------------------------------------
+// Causal attention (attention.hip, attention_pipe.hip): the order of an XCD's items.
+// The place of item `at` among an XCD's `heads` heads of `tiles` query tiles each, causal: `group` heads at a time, the longest tiles
+// of all of them first, so that what comes last, beside other workgroups or after them, is short: with the tiles of a head next to each
+// other, a grid of one to a few rounds ended with long tiles that had started late (us, [heads, rows, head size], pipelined kernel up to
+// [32,..] and streaming kernel from [64,..]: [32,1500,128] 45.7 -> 30.6, [32,2048,64] 30.8 -> 25.8, [64,1500,128] 63.7 -> 47.9,
+// [128,333,128] 17.9 -> 15.8, [128,900,64] 33.4 -> 28.1, [512,512,64] 42.8 -> 37.5).
+struct RankedItem { int head, rank; };  // rank 0: the last query tile
+KERNL_HD RankedItem ranked_item(uint32_t at, uint32_t heads, uint32_t tiles, uint32_t group) {
+    if (tiles == 1) return {(int)at, 0};
+    const uint32_t whole = at / (group * tiles), first = whole * group, members = heads - first < group ? heads - first : group;
+    const uint32_t in = at - whole * group * tiles, rank = in / members;
+    return {(int)(first + in - rank * members), (int)rank};
+}
+// Heads of a group: 16 of head size 64, 8 of head size 128 (400 random causal problems: two rounds and more take 3 to 9 % less than with one
+// head at a time, with 32 up to 9 % more); new rows over a cache are long all of them, there is less to gain than an XCD's L2 can lose
+// (300 problems: 16 heads 2 to 6 % more than one at a time from 1.5 MB of keys and values a head on, this rule level or ahead).  Groups are
+// alike: a last one of a single head starts its longest tile when everything else ends ([132,1071,128], 17 heads an XCD: 16 + 1 76.9 us,
+// one at a time 69.7).
+KERNL_HD int rank_group_of(int64_t heads, int64_t M, int64_t N, int64_t start, int64_t D) {
+    int64_t most = D == 64 ? 16 : 8;
+    if (2 * start >= M) {
+        most = ((int64_t)6 << 20) / (N * D * 4);
+        most = most < 1 ? 1 : most > 8 ? 8 : most;
+    }
+    const int64_t groups = (heads + most - 1) / most;
+    return (int)((heads + groups - 1) / groups);
+}
+
+// ----------------------------------------------------------------------------------------------------
 // Single-query attention (attention_skinny.hip): whether keys and values, [B,H,N,D] of 16-bit values with element strides ks and vs, are read
 // past the 256 MB memory-side cache.  Only where every key row is read once: a batch or head dimension of stride 0 is one storage read by
 // several workgroups, which the caches serve, whatever its size (32 query heads over one key head, head size 128: 24 x 3000 keys 65 us, past

@@ -91,6 +91,10 @@ int kernl_idx_skinny_streams(int64_t B, int64_t H, int64_t N, int64_t D, const i
     return skinny_streams_keys(B, H, N, D, ks, vs) ? 1 : 0;
 }
 
+int kernl_idx_ranked_head(int at, int heads, int tiles, int group) { return ranked_item(at, heads, tiles, group).head; }
+int kernl_idx_ranked_rank(int at, int heads, int tiles, int group) { return ranked_item(at, heads, tiles, group).rank; }
+int kernl_idx_rank_group(int heads, int M, int N, int start, int D) { return rank_group_of(heads, M, N, start, D); }
+
 int kernl_idx_xcd_contiguous(int b, int n) { return xcd_contiguous_index(b, n); }
 
 // which: 0 load_row(q=a), 1 load_chunk(q=a), 2 frag_offset(row=a, kstep=b, g=c)

@@ -24,7 +24,8 @@ class IndexLib:
         self._c = cdll
         for name, n in (("kernl_idx_rowperm16", 1), ("kernl_idx_swz_offset", 3), ("kernl_idx_attention", 5),
                         ("kernl_idx_mask", 5), ("kernl_idx_wide_weight_row", 2), ("kernl_idx_fewrow", 7),
-                        ("kernl_idx_small_tile", 4), ("kernl_idx_xcd_contiguous", 2)):
+                        ("kernl_idx_small_tile", 4), ("kernl_idx_xcd_contiguous", 2),
+                        ("kernl_idx_ranked_head", 4), ("kernl_idx_ranked_rank", 4), ("kernl_idx_rank_group", 5)):
             fn = getattr(cdll, name)
             fn.restype = ctypes.c_int
             fn.argtypes = [ctypes.c_int] * n
@@ -51,6 +52,13 @@ class IndexLib:
 
     def xcd_contiguous(self, b: int, n: int) -> int:
         return self._checked(self._c.kernl_idx_xcd_contiguous(b, n))
+
+    def ranked_item(self, at: int, heads: int, tiles: int, group: int):
+        """(head, rank) of an XCD's item; rank 0 is a head's last query tile."""
+        return self._c.kernl_idx_ranked_head(at, heads, tiles, group), self._c.kernl_idx_ranked_rank(at, heads, tiles, group)
+
+    def rank_group(self, heads: int, rows: int, keys: int, start: int, head_size: int) -> int:
+        return self._c.kernl_idx_rank_group(heads, rows, keys, start, head_size)
 
     def skinny_streams(self, shape, key_strides, value_strides) -> bool:
         """shape [B,H,N,D] and element strides of keys and values."""
