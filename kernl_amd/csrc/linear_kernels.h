@@ -1971,34 +1971,52 @@ static int small_problem_kind(int64_t M, int64_t N, int64_t K) {
     return 0;
 }
 
-// Time of M x N x K on the tiles of linear_mid.hip, us: 2 (launch) + rounds x (ramp and epilogue + k-tiles x time of one).  Measured
-// per tile with the weight from the memory-side cache (up to 8 M elements) and from HBM, 65 .. 2048 rows, random data; the
-// estimates are within 10 % of the measurements.
-static double tile_round(int64_t tiles, double nk, double per_k) {  // a round in which every CU has a tile costs more than a sparse one
-    const int64_t rounds = (tiles + 255) / 256;
-    return nk * per_k * (0.74 + 0.26 * (double)tiles / (double)(256 * rounds));
+// Time of M x N x K on the tiles of linear_mid.hip and on the wide kernels, us: launch + rounds x (ramp and epilogue + k-tiles x time of
+// one).  A k-tile costs the more the more CUs have a tile: 0.74 + 0.26 x the full part of a round, within 10 % where the weight comes from
+// HBM or K is short.  With the weight from the memory-side cache (up to 8 M elements) and K from 1536, by a fit of 467 products of 140 to
+// 4096 rows, within 3 to 6 %: these had been timed in half-empty rounds and at up to 2048 rows, and full ones take 15 to 30 % more than
+// that gave (3958 x 4096 x 1536 in 256 x 128 tiles 57 us where the 256 x 256 kernel takes 44, 1777 x 3072 x 2048 in 192 x 128 27.1 where
+// the 128 x 192 kernel takes 25.0).
+struct CachedTime {
+    double ramp, per_k, per_k_full, edge;  // edge: a last column tile that is not whole (the wide kernels' epilogue)
+};
+struct TileTime {
+    int kind, bm, bn;  // hook value, rows, columns
+    double ramp, per_k_short, per_k_hbm;
+    CachedTime cached;
+};
+static constexpr TileTime kMidTiles[] = {
+    {11, 64, 64, 1.8, 0.195, 0.26, {0.52, 0.141, 0.092, 0.0}},  {15, 128, 64, 1.9, 0.27, 0.385, {0.81, 0.213, 0.140, 0.0}},
+    {17, 128, 128, 2.9, 0.34, 0.53, {3.28, 0.214, 0.249, 0.0}}, {22, 192, 96, 4.0, 0.36, 0.62, {4.02, 0.234, 0.275, 0.0}},
+    {18, 192, 128, 4.2, 0.43, 0.67, {4.67, 0.300, 0.327, 0.0}}, {19, 192, 192, 7.0, 0.60, 0.95, {5.95, 0.455, 0.430, 0.0}},
+    {20, 128, 256, 4.6, 0.56, 0.86, {5.45, 0.467, 0.334, 0.0}}, {21, 256, 128, 4.6, 0.555, 0.85, {5.25, 0.469, 0.317, 0.0}}};
+static constexpr int kSplitTiles = 5;  // the first of them also take ranges of K
+static constexpr TileTime kWideTiles[] = {{5, 256, 256, 0.0, 1.50, 1.50, {5.96, 0.876, 0.493, 3.1}},
+                                          {6, 256, 192, 0.0, 1.30, 1.30, {4.84, 0.765, 0.293, 6.4}},
+                                          {7, 128, 256, 0.0, 0.87, 0.87, {4.76, 0.543, 0.242, 0.0}},
+                                          {8, 128, 192, 0.0, 0.79, 0.79, {3.80, 0.406, 0.176, 2.2}}};
+static bool weight_cached(int64_t N, int64_t K) { return N * K <= ((int64_t)1 << 23); }
+static int64_t tiles_of(const TileTime &t, int64_t M, int64_t N) { return ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn); }
+static double full_part(int64_t tiles) { return (double)tiles / (double)(256 * ((tiles + 255) / 256)); }
+static double one_pass_us(const TileTime &t, int64_t M, int64_t N, int64_t K) {
+    const int64_t n = tiles_of(t, M, N);
+    const double rounds = (double)((n + 255) / 256) * (t.bn == 64 && n > 256 ? 0.88 : 1.0);  // (64 columns: two workgroups share a CU)
+    const double nk = (double)((K + 63) / 64);
+    if (weight_cached(N, K) && K >= 1536) {
+        const CachedTime &c = t.cached;
+        return 2.0 + rounds * (c.ramp + nk * (c.per_k + c.per_k_full * full_part(n)) + (N % t.bn != 0 ? c.edge : 0.0));
+    }
+    return (t.ramp > 0.0 ? 2.0 : 3.5) + rounds * (t.ramp + nk * (weight_cached(N, K) ? t.per_k_short : t.per_k_hbm) * (0.74 + 0.26 * full_part(n)));
 }
 struct MidChoice {
     int tile = 0;  // hook value
     double us = 1e30;
 };
 static MidChoice mid_tile_of(int64_t M, int64_t N, int64_t K, bool gated) {
-    struct Tile {
-        int kind, bm, bn;
-        double ramp, per_k_cached, per_k_hbm;
-    };
-    static constexpr Tile tiles[] = {{11, 64, 64, 1.8, 0.195, 0.26},  {15, 128, 64, 1.9, 0.27, 0.385},  {17, 128, 128, 2.9, 0.34, 0.53},
-                                     {22, 192, 96, 4.0, 0.36, 0.62},  {18, 192, 128, 4.2, 0.43, 0.67},  {19, 192, 192, 7.0, 0.60, 0.95},
-                                     {20, 128, 256, 4.6, 0.56, 0.86}, {21, 256, 128, 4.6, 0.555, 0.85}};
-    const bool cached = N * K <= ((int64_t)1 << 23);
-    const double nk = (double)((K + 63) / 64);
     MidChoice best;
-    for (const Tile &t : tiles) {
+    for (const TileTime &t : kMidTiles) {
         if (gated && t.kind == 22) continue;
-        const int64_t n = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-        double rounds = (double)((n + 255) / 256);
-        if (t.bn == 64 && n > 256) rounds *= 0.88;  // two workgroups share a CU
-        const double us = 2.0 + rounds * (t.ramp + tile_round(n, nk, cached ? t.per_k_cached : t.per_k_hbm));
+        const double us = one_pass_us(t, M, N, K);
         if (us < best.us) best = MidChoice{t.kind, us};
     }
     return best;
@@ -2006,12 +2024,9 @@ static MidChoice mid_tile_of(int64_t M, int64_t N, int64_t K, bool gated) {
 
 // the same estimate for the wide kernels
 static double wide_us(int64_t M, int64_t N, int64_t K, bool gated) {
-    auto cost = [&](int bm, int bn, double per_k) {
-        const int64_t n = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        return 3.5 + (double)((n + 255) / 256) * tile_round(n, (double)((K + 63) / 64), per_k);
-    };
-    double us = cost(256, 256, 1.50);
-    if (!gated) us = std::min(std::min(us, cost(256, 192, 1.30)), std::min(cost(128, 256, 0.87), cost(128, 192, 0.79)));
+    double us = 1e30;
+    for (const TileTime &t : kWideTiles)
+        if (!gated || t.kind == 5) us = std::min(us, one_pass_us(t, M, N, K));
     return us;
 }
 
@@ -2023,23 +2038,20 @@ struct SplitPlan {
     double us = 1e30;
 };
 static SplitPlan split_plan_of(int64_t M, int64_t N, int64_t K) {
-    struct Tile {
-        int kind, bm, bn;
-        double ramp, per_k_cached, per_k_hbm;
-    };
-    static constexpr Tile tiles[] = {{11, 64, 64, 1.8, 0.195, 0.26}, {15, 128, 64, 1.9, 0.27, 0.385}, {17, 128, 128, 2.9, 0.34, 0.53},
-                                     {22, 192, 96, 4.0, 0.36, 0.62}, {18, 192, 128, 4.2, 0.43, 0.67}};
-    const bool cached = N * K <= ((int64_t)1 << 23);
+    const bool cached = weight_cached(N, K);
     const int64_t nk = (K + 63) / 64;
     SplitPlan best;
     best.part_rs = (N + 7) / 8 * 8;
-    for (const Tile &t : tiles)
+    for (int i = 0; i < kSplitTiles; ++i)
         for (int want = 2; want <= 8; ++want) {
+            const TileTime &t = kMidTiles[i];
             const int64_t range = (nk + want - 1) / want, splits = (nk + range - 1) / range;
-            const int64_t n = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * splits;
+            const int64_t n = tiles_of(t, M, N) * splits;
             if (splits < 2 || range < 4) continue;
             const double sums = (double)splits * (double)(M * best.part_rs) * 4.0;
-            const double round = t.ramp + tile_round(n, (double)range, cached ? t.per_k_cached : t.per_k_hbm);
+            // (64-column tiles: a range takes less than the same k-tiles of a whole pass)
+            const double per_k = cached ? (t.bn == 64 ? 0.82 : 1.0) * (t.cached.per_k + t.cached.per_k_full * full_part(n)) : t.per_k_hbm * (0.74 + 0.26 * full_part(n));
+            const double round = t.ramp + (double)range * per_k;
             const double us = 2.0 + (double)((n + 255) / 256) * round + sums / 6e6 + 3.5 + sums / 5e6;
             if (us < best.us) {
                 best.tile = t.kind;
@@ -2069,13 +2081,9 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
     if (short_k || (M <= 128 && N * K < 12 * (1 << 20))) return 0;
     const double nk = (double)((K + 63) / 64), hbm = 4.0 + (double)(N * K) * 2.0 / 4.6e6;  // us at 4.6 TB/s
     MidChoice best = mid_tile_of(M, N, K, gated);
-    // Two regions where the tiles fall behind their estimate, which holds from some 130 to 3000 rows (us, these tiles / what runs instead):
-    //  - a weight of whole 192-column tiles from the memory-side cache under more than 3000 rows: x comes from there too, and the 256 x 192
-    //    kernel has no edge to pay for (3204 x 3072 x 2560 73 / 66, 3999 x 3072 x 2048 60 / 52, 4082 x 2304 x 2560 59 / 51; with an edge it
-    //    loses, 3810 x 2560 x 2048 49 / 60);
-    //  - one or two row tiles over a long K: most of a tile's loads are x again (108 x 12288 x 11008 93 / 82, 89 x 11008 x 11008 85 / 73, gates of
-    //    128 x 5120 x 11008 92 / 71; at K = 8192 they are level, 91 x 11008 x 8192 61 / 59).
-    if (!gated && M > 3000 && N % 192 == 0 && N * K <= ((int64_t)1 << 23)) best.us *= 1.35;
+    // One or two row tiles over a long K: most of a tile's loads are x again and the tiles fall behind their estimate (us, these tiles / what
+    // runs instead: 108 x 12288 x 11008 93 / 82, 89 x 11008 x 11008 85 / 73, gates of 128 x 5120 x 11008 92 / 71; at K = 8192 they are
+    // level, 91 x 11008 x 8192 61 / 59).
     if (M <= 128 && K > 8192) best.us *= 1.3;
     double other = wide_us(M, N, K, gated);
     if (M <= 128 && K % 64 == 0) {
@@ -2088,16 +2096,18 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
             if ((c > hbm ? c : hbm) < best.us) best = MidChoice{14, c > hbm ? c : hbm};
         }
     }
-    return best.us < 0.97 * other ? best.tile : 0;
+    return best.us < (weight_cached(N, K) ? 1.0 : 0.97) * other ? best.tile : 0;
 }
 
 // What M x N x K takes without a split, us, where a launch of its own adds or normalises afterwards.  (small problems: 32 x 32 tiles
-// 231 x 768 x 3072 8.1, x 768 4.6, 64 x 32 tiles 500 x 768 x 3072 10.6, x 768 5.5, 16 x 32 tiles 66 x 768 x 3072 5.5)
+// 231 x 768 x 3072 8.1, x 768 4.6, 16 x 32 tiles 66 x 768 x 3072 5.5; 64 x 32 tiles by a fit of 101 products with the launch behind them,
+// within 4 %: taken for 3.8 + 0.14 a k-tile, wide products of few rows were split for nothing, 207 x 2048 x 3072 and statistics 12.9 -> 14.1,
+// 67 x 4096 x 2048 and LayerNorm 11.7 -> 12.6)
 static double unsplit_us(int64_t M, int64_t N, int64_t K) {
     const double nk = (double)((K + 63) / 64);
     switch (small_problem_kind(M, N, K)) {
         case 12: case 13: return 3.5 + nk * (M <= 96 ? 0.045 : 0.09);
-        case 14: return 3.8 + nk * 0.14;
+        case 14: return 1.9 + nk * 0.125 + (double)(M * N) * 4e-6;
         case 10: return 3.6 + nk * 0.2;
         case 0: break;
         default: return mid_tile_of(M, N, K, false).us;
@@ -2110,12 +2120,12 @@ static double unsplit_us(int64_t M, int64_t N, int64_t K) {
 }
 
 // The split plan of M x N x K where it beats what would run instead: the product and, but for kFinishPlain, the launch behind it
-// (add + LayerNorm 4.3 us; row statistics 4.8; the residual alone rides in most unsplit epilogues).  tile 0: it does not.
+// (add + LayerNorm 4.3 us; row statistics 4.1; the residual alone rides in most unsplit epilogues).  tile 0: it does not.
 static SplitPlan split_plan_that_pays(int64_t M, int64_t N, int64_t K, int finish) {
     if (M <= 64 || M > 4096 || K % 8 != 0 || K < 512 || K >= (1 << 22) || N < 64 || N > INT32_MAX / 64) return SplitPlan();
     if (finish == kFinishPlain ? M <= 128 : N % 4 != 0 || N > 8192) return SplitPlan();  // (plain products of few rows: the stream-K kernel)
     const SplitPlan p = split_plan_of(M, N, K);
-    const double behind = finish == kFinishLayerNorm ? 4.3 : finish == kFinishRmsStats ? 4.8 : 0.0;
+    const double behind = finish == kFinishLayerNorm ? 4.3 : finish == kFinishRmsStats ? 4.1 : 0.0;
     return p.bytes <= ((int64_t)64 << 20) && p.us < 0.95 * (unsplit_us(M, N, K) + behind) ? p : SplitPlan();
 }
 
