@@ -510,36 +510,29 @@ PyObject *op_linear(PyObject *const *a, Py_ssize_t n) {
         Py_RETURN_NONE;
     const int act = (int)integer(a[3]);
     const bool vectors = r.vectors() && aligned16(*x) && aligned16(*w);
-    auto split = [&](int64_t need) {  // too few tiles to occupy the chip: ranges of K per tile, added by a second launch
-        const at::Tensor out = output_for(*x, N);
-        const int64_t os[2] = {N, 1};
-        const at::Tensor ws = at::empty({need}, x->options().dtype(at::kByte));
-        const int dt = dtype_code(*x);
-        Py_XDECREF(launched(*x, "kernl_linear_splitk_fwd", [&](void *stream) {
-            return kernl_linear_splitk_fwd(x->data_ptr(), w->data_ptr(), data(bias), out.data_ptr(), data(act_in), ws.data_ptr(), need, M, N, K,
-                                           r.strides, os, act_in == nullptr ? nullptr : act_in->strides().data(), act, dt, stream);
-        }));
-        return THPVariable_Wrap(out);
-    };
     if (vectors && K % 64 == 0 && M > 64 && r.strides[0] < (1 << 22)) {
         const int64_t need = kernl_linear_split_workspace_bytes(M, N, K, 0);
-        if (need > 0) return split(need);
+        if (need > 0) {  // too few tiles to occupy the chip: ranges of K per tile, added by a second launch
+            const at::Tensor out = output_for(*x, N);
+            const int64_t os[2] = {N, 1};
+            const at::Tensor ws = at::empty({need}, x->options().dtype(at::kByte));
+            const int dt = dtype_code(*x);
+            Py_XDECREF(launched(*x, "kernl_linear_splitk_fwd", [&](void *stream) {
+                return kernl_linear_splitk_fwd(x->data_ptr(), w->data_ptr(), data(bias), out.data_ptr(), data(act_in), ws.data_ptr(), need, M, N, K,
+                                               r.strides, os, act_in == nullptr ? nullptr : act_in->strides().data(), act, dt, stream);
+            }));
+            return THPVariable_Wrap(out);
+        }
     }
     const bool small = vectors && ((truth(a[5]) && kernl_linear_small_kind(M, N, K) != 0) ||
                                    (M > 64 && r.strides[0] < (1 << 22) && kernl_linear_mid_kind(M, N, K, 0) != 0));
     const at::Tensor out = output_for(*x, N);
     const int64_t os[2] = {N, 1};
-    if (!small && vectors && K % 64 == 0) {
-        if (act_in == nullptr && few_row_rule(M, N, K)) {
-            PyObject *x2d = x->dim() == 2 ? (Py_INCREF(a[0]), a[0]) : THPVariable_Wrap(rows_view(*x, r));
-            PyObject *y = THPVariable_Wrap(out);
-            PyObject *y2d = out.dim() == 2 ? (Py_INCREF(y), y) : THPVariable_Wrap(out.view({M, N}));
-            return Py_BuildValue("(NNN)", x2d, y2d, y);
-        }
-        if (M > kFewRowMax && M <= kSplitKMaxRows && r.strides[0] < (1 << 22) && K < (1 << 22)) {
-            const int64_t need = kernl_linear_splitk_workspace_bytes(M, N, K);
-            if (need > 0) return split(need);
-        }
+    if (!small && vectors && K % 64 == 0 && act_in == nullptr && few_row_rule(M, N, K)) {
+        PyObject *x2d = x->dim() == 2 ? (Py_INCREF(a[0]), a[0]) : THPVariable_Wrap(rows_view(*x, r));
+        PyObject *y = THPVariable_Wrap(out);
+        PyObject *y2d = out.dim() == 2 ? (Py_INCREF(y), y) : THPVariable_Wrap(out.view({M, N}));
+        return Py_BuildValue("(NNN)", x2d, y2d, y);
     }
     Py_XDECREF(run_linear(*x, *w, bias, out, act_in, act, M, N, K, r.strides, os));
     return THPVariable_Wrap(out);

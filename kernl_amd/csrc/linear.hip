@@ -161,7 +161,7 @@ static void run_split(const LinearArgs &a, int dtype, const SplitPlan &p, void *
 extern "C" int64_t kernl_linear_splitk_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     using namespace kernl;
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || M > INT32_MAX || N > INT32_MAX || K >= (1 << 22)) return 0;
-    return half_split_takes(M, N, K) ? split_plan_of(M, N, K).bytes : 0;
+    return few_tiles_long_k(M, N, K) ? split_plan_of(M, N, K).bytes : 0;
 }
 
 extern "C" int kernl_linear_splitk_fwd(const void *x, const void *w, const void *bias, void *out, void *act_in,
@@ -184,11 +184,11 @@ extern "C" int kernl_linear_splitk_fwd(const void *x, const void *w, const void 
         x_strides[1] != 1 || x_strides[0] % 8 != 0 || !aligned16(x) || !aligned16(w))
         return set_error(KERNL_ERR_UNSUPPORTED, "linear (split K): K must be a multiple of 64, x needs unit feature stride "
                          "and 16-byte aligned rows, the weight a 16-byte aligned base");
-    if (!half_split_takes(M, N, K) && split_plan_that_pays(M, N, K, kFinishPlain).tile == 0)
+    const SplitPlan p = few_tiles_long_k(M, N, K) ? split_plan_of(M, N, K) : split_plan_that_pays(M, N, K, kFinishPlain);
+    if (p.tile == 0)
         return set_error(KERNL_ERR_UNSUPPORTED, "linear (split K): nothing to split for M=%lld N=%lld K=%lld "
                          "(kernl_linear_splitk_workspace_bytes returns 0): use kernl_linear_fwd", (long long)M, (long long)N,
                          (long long)K);
-    const SplitPlan p = split_plan_of(M, N, K);
     if (workspace == nullptr || workspace_bytes < p.bytes || !aligned16(workspace))
         return set_error(KERNL_ERR_INVALID_ARG, "linear (split K): the workspace must hold %lld bytes, 16-byte aligned",
                          (long long)p.bytes);

@@ -1822,11 +1822,11 @@ static void launch_wide_half_act(const LinearArgs &a) {
                        wide_residual_of<T, NBN>(a));
 }
 
-// Row counts that leave most CUs without a 128 x 192 tile (129 to about 700 rows against a few thousand columns) and a K long enough
-// for ranges of 16 k-tiles: what kernl_linear_splitk_fwd takes.
-static bool half_split_takes(int64_t M, int64_t N, int64_t K) {
+// At most 128 tiles of 128 x 192 (129 to about 700 rows against a few thousand columns) over a K of 2048 or more: what
+// kernl_linear_splitk_fwd takes beside the shapes whose split pays.
+static bool few_tiles_long_k(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + 127) / 128) * ((N + 191) / 192);
-    return K % 64 == 0 && 256 / tiles >= 2 && K / 64 / 16 >= 2;
+    return tiles <= 128 && K % 64 == 0 && K >= 2048;
 }
 
 template <typename T, int NBN>

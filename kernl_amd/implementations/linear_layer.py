@@ -27,7 +27,7 @@ ONE_BYTE_WEIGHT_DTYPES = (torch.int8, torch.uint8, torch.float8_e5m2)
 
 FEW_ROW_MIN_ROWS = 17          # up to 16 rows the kernel that gives a workgroup 16 columns and all of K is as fast or faster
 FEW_ROW_MAX_ROWS = 128         # what `kernl_linear_fewrow_fwd` takes
-SPLIT_K_MAX_ROWS = 2048        # beyond that the tiled kernels always have tiles enough; the library decides below it
+SPLIT_K_MAX_ROWS = 2048        # beyond that the tiled kernels always have tiles enough
 FEW_ROW_MIN_WEIGHT = 1 << 22   # elements: below that (2048 x 2048) launch latency decides and one launch beats two ...
 
 
@@ -43,6 +43,12 @@ def few_row_rule(rows: int, n: int, k: int) -> bool:
     if not FEW_ROW_MIN_ROWS <= rows <= FEW_ROW_MAX_ROWS or k < 256 or k % 64 != 0:
         return False
     return n * k >= FEW_ROW_MIN_WEIGHT or (k >= FEW_ROW_LONG_K and rows > 32)
+
+
+def few_tiles_long_k(rows: int, n: int, k: int) -> bool:
+    """At most 128 tiles of 128 x 192, the wide kernels' smallest, over a K of 2048 or more: no problem of the wide kernels, whose
+    epilogues take a row factor or a residual.  Such a product gets its rows normalised, and its residual, by launches of their own."""
+    return rows <= SPLIT_K_MAX_ROWS and -(-rows // 128) * -(-n // 192) <= 128 and k % 64 == 0 and k >= 2048
 
 
 SMALL_PROBLEM_KERNELS = True   # tuning hook: False keeps such shapes on the stream-K / split-K / tile kernels
@@ -135,16 +141,12 @@ class LinearLayer(torch.autograd.Function):
             assert act_inputs.shape == (M, N) and act_inputs.dtype == x.dtype
         split_bytes = split_pays_bytes(x_, weight)
         small = not split_bytes and (takes_small_problem_kernel(x_, weight) or takes_mid_kernel(x_, weight))
-        if not split_bytes and not small and FEW_ROW_MAX_ROWS < M <= SPLIT_K_MAX_ROWS:
-            split_bytes = _lib.linear_splitk_workspace_bytes(x_, weight)
-        if small:
-            _lib.linear_fwd(x_, weight, bias, outputs, act_inputs, ACTIVATIONS.get(activation, _lib.ACT_NONE))
-        elif not split_bytes and act_inputs is None and takes_few_row_kernel(x_, weight):
-            _lib.linear_fewrow_fwd(x_, weight, bias, None, outputs, ACTIVATIONS.get(activation, _lib.ACT_NONE))
-        elif split_bytes:
+        if split_bytes:
             # too few tiles to occupy the chip: ranges of K per tile, added by a second launch
             workspace = torch.empty(split_bytes, dtype=torch.uint8, device=x.device)
             _lib.linear_splitk_fwd(x_, weight, bias, outputs, act_inputs, ACTIVATIONS.get(activation, _lib.ACT_NONE), workspace)
+        elif not small and act_inputs is None and takes_few_row_kernel(x_, weight):
+            _lib.linear_fewrow_fwd(x_, weight, bias, None, outputs, ACTIVATIONS.get(activation, _lib.ACT_NONE))
         else:
             _lib.linear_fwd(x_, weight, bias, outputs, act_inputs, ACTIVATIONS.get(activation, _lib.ACT_NONE))
         return outputs if x.ndim == 2 else outputs.reshape(*x.shape[:-1], N)
@@ -282,7 +284,7 @@ def rms_linear_layer(
         # those products run on would take the row factors too; but weight * rms_weight is rounded to 16 bits, which a small
         # norm weight makes coarser than the rounding of the normalised row, so the folded weight stays with the large prompts.)
         and not takes_small_problem_kernel(x_, folded_weight)
-        and (x_.shape[0] > SPLIT_K_MAX_ROWS or _lib.linear_splitk_workspace_bytes(x_, folded_weight) == 0)
+        and not few_tiles_long_k(x_.shape[0], *folded_weight.shape)
     ):
         if rstd is None:
             rstd = rms_stats(x_, eps, clamp=False)
@@ -361,7 +363,7 @@ def residual_linear_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optio
     x_ = x if x.ndim == 2 else x.reshape(-1, x.shape[-1])
     if not _lib.linear_scaled_supported(x_, weight):
         return False
-    if rows <= SPLIT_K_MAX_ROWS and not takes_mid_kernel(x_, weight) and _lib.linear_splitk_workspace_bytes(x_, weight) != 0:
+    if few_tiles_long_k(rows, *weight.shape) and not takes_mid_kernel(x_, weight):
         return False
     return _lib.linear_wide_kind(rows, weight.shape[0], weight.shape[1]) != 0
 
