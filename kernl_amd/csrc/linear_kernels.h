@@ -2101,8 +2101,7 @@ static int mid_kind(int64_t M, int64_t N, int64_t K, bool gated) {
 
 // What M x N x K takes without a split, us, where a launch of its own adds or normalises afterwards.  (small problems: 32 x 32 tiles
 // 231 x 768 x 3072 8.1, x 768 4.6, 16 x 32 tiles 66 x 768 x 3072 5.5; 64 x 32 tiles by a fit of 101 products with the launch behind them,
-// within 4 %: taken for 3.8 + 0.14 a k-tile, wide products of few rows were split for nothing, 207 x 2048 x 3072 and statistics 12.9 -> 14.1,
-// 67 x 4096 x 2048 and LayerNorm 11.7 -> 12.6)
+// within 4 %: taken for 3.8 + 0.14 a k-tile, wide products of few rows were split for nothing, 67 x 4096 x 2048 and LayerNorm 11.7 -> 12.6)
 static double unsplit_us(int64_t M, int64_t N, int64_t K) {
     const double nk = (double)((K + 63) / 64);
     switch (small_problem_kind(M, N, K)) {
@@ -2120,12 +2119,12 @@ static double unsplit_us(int64_t M, int64_t N, int64_t K) {
 }
 
 // The split plan of M x N x K where it beats what would run instead: the product and, but for kFinishPlain, the launch behind it
-// (add + LayerNorm 4.3 us; row statistics 4.1; the residual alone rides in most unsplit epilogues).  tile 0: it does not.
+// (add + LayerNorm 4.3 us; row statistics 4.1, and 0.8 a million elements; the residual alone rides in most unsplit epilogues).  tile 0: it does not.
 static SplitPlan split_plan_that_pays(int64_t M, int64_t N, int64_t K, int finish) {
     if (M <= 64 || M > 4096 || K % 8 != 0 || K < 512 || K >= (1 << 22) || N < 64 || N > INT32_MAX / 64) return SplitPlan();
     if (finish == kFinishPlain ? M <= 128 : N % 4 != 0 || N > 8192) return SplitPlan();  // (plain products of few rows: the stream-K kernel)
     const SplitPlan p = split_plan_of(M, N, K);
-    const double behind = finish == kFinishLayerNorm ? 4.3 : finish == kFinishRmsStats ? 4.1 : 0.0;
+    const double behind = finish == kFinishLayerNorm ? 4.3 : finish == kFinishRmsStats ? 4.1 + (double)(M * N) * 0.8e-6 : 0.0;
     return p.bytes <= ((int64_t)64 << 20) && p.us < 0.95 * (unsplit_us(M, N, K) + behind) ? p : SplitPlan();
 }
 
