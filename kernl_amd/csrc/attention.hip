@@ -1089,7 +1089,7 @@ static int attention_entry(const void *q, const void *k, const void *v, void *ou
     p.mask_fast = 0;
     p.xcd_by_batch = 0;
     p.causal_off = is_causal != 0 ? (int)start_position : 0;
-    p.rank_group = rank_group_of((B * H + 7) / 8, M, N, p.causal_off, D);
+    p.rank_group = (int16_t)rank_group_of((B * H + 7) / 8, M, N, p.causal_off, D);
     if (mask_mode == MASK_MATRIX && (mask_dtype == KERNL_F32 || mask_dtype == dtype)) {
         const int64_t es = mask_dtype == KERNL_F32 ? 4 : 2;
         p.mask_fast = mask_strides[3] == 1 && p.ms[0] % 4 == 0 && p.ms[1] % 4 == 0 && p.ms[2] % 4 == 0 && p.ms[2] > 0 &&
