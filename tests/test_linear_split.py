@@ -15,21 +15,24 @@ def _case(M, N, K, dtype, seed=0):
     return x, w, (0.3 * torch.randn((N,), generator=gen)).to(dtype), torch.randn((M, N), generator=gen).to(dtype), gen
 
 
-# one wave a row (768, 1024 columns and one that is neither), a workgroup a row (up to 4096, up to 8192), ragged rows, a K that ends inside
-# a k-tile, ranges of unequal length
-SHAPES = [(231, 768, 3072), (500, 772, 3080), (130, 1024, 4096), (333, 4096, 4096), (200, 4100, 11008), (140, 8192, 4104)]
+# a workgroup a row of up to 1024 columns (231, 500, 130 rows), of up to 4096, of up to 8192; a wave a row beyond 1024 rows of up to 768 and of
+# up to 1024 columns; ragged rows, a K that ends inside a k-tile, ranges of unequal length; two to eight ranges, on each of the tiles
+SHAPES = [(231, 768, 3072), (500, 772, 3080), (130, 1024, 4096), (333, 4096, 4096), (200, 4100, 11008), (140, 8192, 4104),
+          (100, 768, 3072), (150, 4096, 11008), (1500, 768, 4096), (1400, 1024, 4096), (3000, 768, 8192), (2000, 512, 8192)]
+# where the residual alone pays for a split: long K
+RESIDUAL_SHAPES = [(100, 4096, 11008), (150, 4096, 11008), (200, 4100, 11008), (700, 1024, 11008), (1500, 1024, 8192), (2000, 512, 8192), (2079, 1024, 11008)]
+FINISHES = ([(_lib.FINISH_RESIDUAL, shape) for shape in RESIDUAL_SHAPES] + [(_lib.FINISH_RMS_STATS, shape) for shape in SHAPES]
+            + [(_lib.FINISH_LAYER_NORM, shape) for shape in SHAPES])
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
-@pytest.mark.parametrize("shape", SHAPES, ids=str)
-@pytest.mark.parametrize("finish", [_lib.FINISH_RESIDUAL, _lib.FINISH_RMS_STATS, _lib.FINISH_LAYER_NORM], ids=["residual", "stats", "norm"])
-def test_finished_rows(shape, finish, dtype, close):
+@pytest.mark.parametrize("finish, shape", FINISHES, ids=lambda v: ("residual", "stats", "norm")[v - 1] if isinstance(v, int) else "x".join(map(str, v)))
+def test_finished_rows(finish, shape, dtype, close):
     M, N, K = shape
     x, w, b, res, gen = _case(M, N, K, dtype, M)
     gamma, beta = (1 + 0.1 * torch.randn((N,), generator=gen)).to(dtype), (0.1 * torch.randn((N,), generator=gen)).to(dtype)
     need = _lib.linear_split_workspace_bytes(M, N, K, finish)
-    if need == 0:
-        pytest.skip("one pass over K is faster")
+    assert need > 0, "the shape lists are meant for the split form"
     out = torch.full((M, N + 4), float("nan"), dtype=dtype, device="cuda")[:, :N]
     rstd = torch.full((M,), float("nan"), device="cuda")
     ws = torch.full((need // 4,), float("nan"), device="cuda")
@@ -43,6 +46,20 @@ def test_finished_rows(shape, finish, dtype, close):
     if finish == _lib.FINISH_RMS_STATS:
         ref = torch.rsqrt(out.float().square().mean(-1) + 1.6e-5)
         assert (rstd - ref).abs().max().item() <= 1e-5 * ref.max().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [(140, 12288, 4096), (150, 4096, 11008)], ids=str)  # 192 x 96 and 192 x 128 tiles, two and eight ranges
+def test_plain_sums(shape, dtype, close):
+    M, N, K = shape
+    x, w, b, _, _ = _case(M, N, K, dtype, M)
+    need = _lib.linear_split_workspace_bytes(M, N, K)
+    assert need > 0
+    out, saved = torch.full((2, M, N), float("nan"), dtype=dtype, device="cuda")
+    _lib.linear_splitk_fwd(x.cuda(), w.cuda(), b.cuda(), out, saved, _lib.ACT_SILU, torch.full((need // 4,), float("nan"), device="cuda"))
+    torch.cuda.synchronize()
+    close(out, linear_oracle(x, w, b, "silu"), dtype, scale="magnitude", what=f"{shape}")
+    close(saved, linear_oracle(x, w, b, ""), dtype, what=f"{shape} pre-activation")
 
 
 def test_the_operands_it_leaves_to_other_routes():
