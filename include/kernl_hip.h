@@ -347,8 +347,9 @@ int kernl_linear_mid_kind(int64_t M, int64_t N, int64_t K, int gated);
  * runs the epilogue (same semantics and arguments as kernl_linear_fwd, reference src/kernl/implementations/
  * linear_layer.py:92-210; the split over K is the `SPLIT_K` axis of the reference's configurations, which it leaves
  * at 1, linear_layer.py:47-67).
- *   kernl_linear_splitk_workspace_bytes(M, N, K) returns 0 when splitting does not pay (enough tiles, or a short K):
- *   call kernl_linear_fwd then.  Otherwise pass a 16-byte aligned workspace of at least that many bytes (contents
+ *   Takes what kernl_linear_split_workspace_bytes(M, N, K, 0) below says pays (pass a workspace of that size), and anything of
+ *   at most 128 tiles of 128 x 192 over a K of 2048 or more: kernl_linear_splitk_workspace_bytes(M, N, K), 0 for the others.
+ *   Pass a 16-byte aligned workspace of at least that many bytes (contents
  *   irrelevant before and after the call; calls that overlap in time need workspaces of their own).
  *   f16 / bf16, K % 64 == 0, x with unit feature stride and 16-byte aligned rows; anything else returns
  *   KERNL_ERR_UNSUPPORTED.
@@ -363,9 +364,9 @@ int kernl_linear_splitk_fwd(const void *x, const void *w, const void *bias, void
  * Split K for 65 to 4096 rows where it beats one pass over K, with the second launch finishing the rows.  `finish`: 0 bias and
  * activation (kernl_linear_splitk_fwd takes it), 1 round(product + bias) + residual, 2 the same with rstd[m] = 1 / sqrt(mean(row^2) + eps)
  * of the rounded row, 3 LayerNorm(product + bias + residual) * gamma + beta, added and normalised in fp32.
- *   kernl_linear_split_workspace_bytes: 0 where splitting does not pay, else the bytes of a 16-byte aligned workspace (contents
+ *   kernl_linear_split_workspace_bytes: 0 where splitting does not pay (call kernl_linear_fwd for finish 0), else the bytes of a 16-byte aligned workspace (contents
  *   irrelevant; calls that overlap in time need workspaces of their own).
- *   f16 / bf16; x [M, K], residual and out [M, N] with unit feature strides and the given row strides, N a multiple of 4 up to 8192;
+ *   f16 / bf16, K % 8 == 0; x [M, K], residual and out [M, N] with unit feature strides and the given row strides, N a multiple of 4 up to 8192;
  *   anything else returns KERNL_ERR_UNSUPPORTED.  No reference counterpart: its models add and normalise in kernels of their own.
  */
 int64_t kernl_linear_split_workspace_bytes(int64_t M, int64_t N, int64_t K, int finish);

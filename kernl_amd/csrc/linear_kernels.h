@@ -688,6 +688,8 @@ __device__ __forceinline__ void wide_epilogue(f32x4_acc (&acc)[NBM][NBN], int m_
 // a weight (or x) tile is the first to ask for a quarter of its lines and finds the others in L2.  Measured in sustained replay with
 // weights from HBM: 2048 x 12288 x 4096 168.5 -> 160.5 us, 2048 x 4096 x 11008 163 -> 157, 1024 x 12288 x 4096 90 -> 84.5.  Where the
 // weight stays in the memory-side cache (8 M elements and less) there is nothing to gain (16384 x 2304 x 768 56.2 -> 59.6).
+// With it the order of a row's fp32 sums depends on the row tile: the same row at another place of x may round to the neighbouring 16-bit
+// value.  The same call gives the same bits.
 __host__ __device__ static inline bool k_tiles_dealt(int64_t N, int64_t K) { return N * K > ((int64_t)1 << 23); }
 // (DEAL of the wide kernels: whole groups only, for the epilogues that products with large weights have; linear_wide_dealt.hip.)
 

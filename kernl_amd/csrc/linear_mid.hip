@@ -7,7 +7,7 @@
 // and matrix instructions: 1024 x 768 x 3072 in 64 x 64 tiles took 15.5 us, the same with the loads alone 11.6, without them 8.9.  Hence
 //   - waves that only load (four, behind the eight that multiply): what they wait for, nobody else waits for.  1024 x 768 x 3072
 //     15.5 -> 13.0 us, 1024 x 3072 x 768 11.3 -> 9.8 in 128 x 128 tiles, 231 x 2304 x 768 6.6 -> 5.9;
-//   - k-tiles dealt among the workgroups that share a weight or x tile (k_turn_mask in linear_kernels.h): 1024 x 4096 x 4096 in 128 x 128
+//   - k-tiles dealt among the workgroups that share a weight or x tile (`turn`; see k_tiles_dealt in linear_kernels.h): 1024 x 4096 x 4096 in 128 x 128
 //     tiles, weights from HBM, 39.6 -> 34.5 us, 512 x 12288 x 4096 in 256 x 128 tiles 54.7 -> 51, 333 x 22016 x 4096 in 192 x 192
 //     tiles 66.5 -> 63; from the memory-side cache 1024 x 768 x 3072 12.5 -> 12.1, 231 x 768 x 3072 11.9 -> 11.2;
 //   - tiles of 64 x 64 to 256 x 128, as large as still put a tile on (nearly) every CU: (BM + BN) x K bytes a tile;
