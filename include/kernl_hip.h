@@ -375,6 +375,24 @@ int kernl_linear_split_fwd(const void *x, const void *w, const void *bias, const
                            int64_t x_rs, int64_t res_rs, int64_t out_rs, int finish, int dtype, void *stream);
 
 /*
+ * out = LayerNorm(x w^T + bias + residual) * gamma + beta in ONE launch for more than 64 rows, added and normalised in fp32: the workgroups that
+ * share a row exchange its statistics through `region` (csrc/norm_exchange.h).
+ *   kernl_linear_exchange_bytes: bytes of a region; 0 where other routes are faster.
+ *   region, next_region: two regions of region_bytes each (a multiple of 8, at least that many), 8-byte aligned.  `region` must be all zeros; the
+ *   launch leaves zeros in next_region, so that a chain of launches on one stream takes two of them by turns and only the first is
+ *   cleared by the caller.  Launches that may overlap in time need pairs of their own.
+ *   sums: M x N floats, 16-byte aligned, contents irrelevant (written only by workgroups that stop waiting).
+ *   patience: how often a workgroup looks for the others' statistics before it leaves its rows to them; < 0 for the default.  Any value gives the
+ *   same result, and no wait is without an end.
+ *   f16 / bf16, K % 8 == 0; x [M, K], residual and out [M, N] with unit feature strides and the given row strides (x and out rows 16-byte
+ *   aligned, the rest 8); anything else returns KERNL_ERR_UNSUPPORTED.  No reference counterpart.
+ */
+int64_t kernl_linear_exchange_bytes(int64_t M, int64_t N, int64_t K);
+int kernl_linear_add_norm_fwd(const void *x, const void *w, const void *bias, const void *residual, const void *gamma, const void *beta, float eps,
+                              void *out, float *sums, void *region, void *next_region, int64_t region_bytes, int patience, int64_t M, int64_t N,
+                              int64_t K, int64_t x_rs, int64_t res_rs, int64_t out_rs, int dtype, void *stream);
+
+/*
  * The linear layer for a FEW rows of x with many columns and a long K (batched decoding steps: 17 to 128 rows, where
  * kernl_linear_fwd's weight-streaming kernel re-reads x once per 16 to 64 output columns and its tile kernels leave
  * most of their rows empty), with everything a decoder layer puts around its projections:

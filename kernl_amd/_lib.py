@@ -55,6 +55,8 @@ EXPORTED_SYMBOLS = (
     "kernl_linear_splitk_fwd",
     "kernl_linear_split_workspace_bytes",
     "kernl_linear_split_fwd",
+    "kernl_linear_exchange_bytes",
+    "kernl_linear_add_norm_fwd",
     "kernl_linear_fewrow_workspace_bytes",
     "kernl_linear_fewrow_fwd",
     "kernl_linear_fewrow_w8_fwd",
@@ -149,6 +151,10 @@ def load() -> ctypes.CDLL:
     lib.kernl_linear_split_workspace_bytes.argtypes = [_i64] * 3 + [ctypes.c_int]
     lib.kernl_linear_split_fwd.restype = ctypes.c_int
     lib.kernl_linear_split_fwd.argtypes = [_vp] * 6 + [ctypes.c_float] + [_vp] * 3 + [_i64] * 7 + [ctypes.c_int, ctypes.c_int, _vp]
+    lib.kernl_linear_exchange_bytes.restype = _i64
+    lib.kernl_linear_exchange_bytes.argtypes = [_i64] * 3
+    lib.kernl_linear_add_norm_fwd.restype = ctypes.c_int
+    lib.kernl_linear_add_norm_fwd.argtypes = [_vp] * 6 + [ctypes.c_float] + [_vp] * 4 + [_i64, ctypes.c_int] + [_i64] * 6 + [ctypes.c_int, _vp]
     lib.kernl_linear_splitk_fwd.restype = ctypes.c_int
     lib.kernl_linear_splitk_fwd.argtypes = [_vp] * 6 + [_i64] * 4 + [_i64p] * 3 + [ctypes.c_int, ctypes.c_int, _vp]
     lib.kernl_linear_fewrow_workspace_bytes.restype = _i64
@@ -631,6 +637,25 @@ def linear_split_fwd(x2d, weight, bias, residual2d, gamma, beta, eps: float, out
             residual2d.stride(0), out2d.stride(0), int(finish), DTYPE_CODE[x2d.dtype], _stream(x2d),
         )
     _check(st, "kernl_linear_split_fwd")
+
+
+def linear_exchange_bytes(M: int, N: int, K: int) -> int:
+    """Bytes of a region of `linear_add_norm_fwd`; 0 where other routes are faster."""
+    return int(load().kernl_linear_exchange_bytes(M, N, K))
+
+
+def linear_add_norm_fwd(x2d, weight, bias, residual2d, gamma, beta, eps: float, out2d, sums, region, next_region, patience: int = -1) -> None:
+    """`kernl_linear_add_norm_fwd`: product, addition and LayerNorm in one launch; `region` is all zeros, `next_region` is left so."""
+    _require_gpu(x2d, weight, bias, residual2d, gamma, beta, out2d, sums, region, next_region)
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    lib = load()
+    with torch.cuda.device(x2d.device):
+        st = lib.kernl_linear_add_norm_fwd(
+            x2d.data_ptr(), weight.data_ptr(), ptr(bias), residual2d.data_ptr(), gamma.data_ptr(), ptr(beta), float(eps), out2d.data_ptr(),
+            sums.data_ptr(), region.data_ptr(), next_region.data_ptr(), min(region.numel(), next_region.numel()) * 8, int(patience), x2d.shape[0],
+            out2d.shape[1], x2d.shape[1], x2d.stride(0), residual2d.stride(0), out2d.stride(0), DTYPE_CODE[x2d.dtype], _stream(x2d),
+        )
+    _check(st, "kernl_linear_add_norm_fwd")
 
 
 def linear_fewrow_supported(x2d, weight) -> bool:

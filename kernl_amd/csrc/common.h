@@ -235,6 +235,14 @@ __device__ __forceinline__ float halves32_sum(float v) {
     return lo + hi;
 }
 
+// sum over the four lanes that share lane % 16, to each of them (v_permlane16_swap exchanges the odd rows of 16 lanes of its first operand
+// with the even ones of its second)
+__device__ __forceinline__ float rows4_sum(float v) {
+    const uint32_t bits = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+    return halves32_sum(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+
 // ----------------------------------------------------------------------------------------------------
 // host side
 // ----------------------------------------------------------------------------------------------------

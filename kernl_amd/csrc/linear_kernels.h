@@ -37,6 +37,10 @@ void run_wide_half_w8(const LinearArgs &a);
 void run_small(const LinearArgs &a, int dtype);                      // 32 x 64 tiles over the whole K (linear_small.hip)
 // tiles with loading waves over the whole K (linear_mid.hip), by hook value 11, 15, 17 .. 22; 0: that tile does not take the epilogue asked for
 int run_mid(const LinearArgs &a, int dtype, int kind);
+// linear + residual + LayerNorm in one launch (norm_exchange.h): tiles of linear_mid.h by hook value, and dealt k-tiles of `rows` x 32
+struct NormExchange;
+void run_mid_norm(const LinearArgs &a, int dtype, int kind, const NormExchange &norm);
+void run_small_dealt_norm(const LinearArgs &a, int dtype, int rows, const NormExchange &norm);
 // the same with K split over `splits` workgroups a tile, which leave fp32 sums [splits][M][part_rs] for run_split_finish
 struct MidSplit {
     int splits = 1, range_kt = 0;

@@ -12,7 +12,7 @@
 // ahead, one barrier per k-tile and waits by count.  A last k-tile that reaches beyond K has the chunks that
 // start there pointed out of range (zeros, in both operands).
 #include "linear_kernels.h"
-#include "norm_fold.h"
+#include "norm_exchange.h"
 
 namespace kernl {
 
@@ -260,11 +260,14 @@ linear_small_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *_
 // a wave's ring: 32 KB, 36 KB for the 12 KB stages of 64 x 32 tiles (three of them)
 constexpr int small_ring_bytes(int bm, int bn, int waves) { return waves == 8 ? 16 * 1024 : (bm + bn) == 96 ? 36 * 1024 : 32 * 1024; }
 
+template <int MODE>
+using NormOf = typename std::conditional<MODE == kNormExchange, NormExchange, NormFold>::type;
+
 template <typename T, int BM, int BN, int WAVES, int MODE>
 __global__ void __launch_bounds__(64 * WAVES, 1)
 linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias,
                           T *__restrict__ out, T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs,
-                          int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int act, int tiles_m, NormFold nf) {
+                          int64_t out_cs, int64_t ai_rs, int64_t ai_cs, int act, int tiles_m, NormOf<MODE> nf) {
     typedef typename Vec8<T>::type vec8;
     constexpr int BK = 64, RB = BK * 2, CPR = BK / 8;
     static_assert(RB == SmallTileMap::ROW_BYTES && CPR == SmallTileMap::CHUNKS_PER_ROW, "tile rows as the tile map lays them out");
@@ -282,6 +285,7 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     // row tile nothing is shared, and workgroups that run side by side had better read neighbouring weight rows
     const int tile = tiles_m > 1 ? xcd_contiguous_index((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
     const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+    if constexpr (MODE == kNormExchange) exchange_clear(nf, tid, 64 * WAVES);
 
     constexpr uint32_t kOutOfRange = 0x80000000u;
     const int rows_x = min(BM, M - m0), rows_w = min(BN, N - n0);
@@ -356,8 +360,15 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
     float bz[4];
     const bool row_stats = MODE == kNormAdd && nf.in_stats != nullptr;  // the residual is fp32 rows whose norm is to be applied
     f32x4 res32 = {0.0f, 0.0f, 0.0f, 0.0f};
-    u32x2 res16 = {0, 0}, gam = {0, 0}, bet = {0, 0}, bias16 = {0, 0};
-    if (MODE != kNormAdd) {
+    u32x2 res16 = {0, 0}, gam = {0, 0}, bet = {0, 0}, bias16 = {0, 0}, res_own[MODE == kNormExchange ? OWN : 1];
+    if constexpr (MODE == kNormExchange) {
+        if (bias != nullptr) bias16 = *reinterpret_cast<const u32x2 *>(bias + n_own);
+#pragma unroll
+        for (int t = 0; t < OWN; ++t)
+            res_own[t] = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.residual) + (int64_t)(m0 + min(own_row + ROWS * t, rows_x - 1)) * nf.res_rs + n_own);
+        gam = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.gamma) + n_own);
+        if (nf.beta != nullptr) bet = *reinterpret_cast<const u32x2 *>(static_cast<const T *>(nf.beta) + n_own);
+    } else if (MODE != kNormAdd) {
         load_bias4<T>(bias, n_own, N, ((uintptr_t)bias & 7) == 0, bz);
     } else {
         // raw, and each in registers of its own: what is converted or moved here is waited for here.  (N is a multiple of 32:
@@ -409,6 +420,10 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
         static_assert(BM == 16 && BN == kNormGroup && OWN == 1, "a row of the tile is one statistics group, and a thread's");
         if (row_stats) merge_norm_stats<BM, WAVES>(nf, smem + WAVES * RING, row_norm, tid);
     }
+    // what the workgroup of a norm has to agree on, in front of the rows' factors
+    uint32_t *const failed = reinterpret_cast<uint32_t *>(row_norm) - 4;
+    static_assert(WAVES * NBM * NBN * 1024 + BM * 8 + 16 <= WAVES * RING, "room behind the partial tiles");
+    if (MODE == kNormExchange && tid == 0) *failed = 0;
     float *red = reinterpret_cast<float *>(smem);  // [wave][block][lane][4]
 #pragma unroll
     for (int i = 0; i < NBM; ++i)
@@ -416,6 +431,88 @@ linear_small_dealt_kernel(const T *__restrict__ X, const T *__restrict__ W, cons
         for (int j = 0; j < NBN; ++j)
             *reinterpret_cast<f32x4_acc *>(red + ((wave * (NBM * NBN) + i * NBN + j) * 64 + lane) * 4) = acc[i][j];
     __syncthreads();
+
+    if constexpr (MODE == kNormExchange) {
+        // sums + residual, the exchange (the lanes that own a row look for its words), the normalised row pieces
+        static_assert(LPR == 8, "the lanes of a row are those that look for its words");
+        const int tile_m = tile % tiles_m, tile_n = tile / tiles_m;
+        const RowExchange<BM, BN, LPR> exchange(nf, tile_m, tiles_m, N / BN);
+        const bool mine_too = BM >= ROWS || own_row < BM;  // (16-row tiles: whole waves have none)
+        float y[OWN][4], bias_own[4];
+        unpack4<T>(bias16, bias_own);
+        if (mine_too) {
+#pragma unroll
+            for (int t = 0; t < OWN; ++t) {
+                const int row = own_row + ROWS * t, at = (((row >> 4) * NBN + (own_c >> 2)) * 64 + (own_c & 3) * 16 + (row & 15)) * 4;
+                f32x4_acc sum = *reinterpret_cast<const f32x4_acc *>(red + at);
+#pragma unroll
+                for (int w = 1; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4_acc *>(red + w * (NBM * NBN) * 256 + at);
+                float h[4], total = 0.0f, m2 = 0.0f;
+                unpack4<T>(res_own[t], h);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    y[t][e] = sum[e] + bias_own[e] + h[e];
+                    total += y[t][e];
+                }
+                const float mean = oct_sum(total) * (1.0f / BN);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m2 = fmaf(y[t][e] - mean, y[t][e] - mean, m2);
+                m2 = oct_sum(m2);
+                if (own_c == 0) exchange.publish(tile_n, row, mean, m2);
+            }
+        }
+        f32x2 factors[OWN];
+        auto look = [&](int patience) __attribute__((always_inline)) {
+            bool there = true;
+            if (mine_too)
+#pragma unroll
+                for (int t = 0; t < OWN; ++t) {
+                    there = exchange.look(own_row + ROWS * t, own_c, patience, nf.inv_n, nf.eps, factors[t]) && there;
+                    if (there && own_c == 0) row_norm[own_row + ROWS * t] = factors[t];
+                }
+            return there;
+        };
+        if (!look(nf.patience) && lane == 0) *failed = 1;
+        published_words_landed();
+        __syncthreads();
+        if (*failed != 0) {
+            // out of patience: the sums to memory, a note, and a last look
+            if (mine_too)
+#pragma unroll
+                for (int t = 0; t < OWN; ++t)
+                    if (own_row + ROWS * t < rows_x)
+#pragma unroll
+                        for (int e = 0; e < 4; e += 2)
+                            store_agent(reinterpret_cast<uint64_t *>(nf.sums + (int64_t)(m0 + own_row + ROWS * t) * N + n_own + e),
+                                        (uint64_t)__builtin_bit_cast(uint32_t, y[t][e + 1]) << 32 | __builtin_bit_cast(uint32_t, y[t][e]));
+            published_words_landed();
+            __syncthreads();
+            if (tid == 0) {
+                exchange.note_leaving(tile_n);
+                *failed = 0;
+            }
+            __syncthreads();
+            if (!look(0) && lane == 0) *failed = 1;
+            __syncthreads();
+            if (*failed != 0) return;
+        }
+        uint64_t left = 0;
+        if (wave == 0) left = load_agent(exchange.notes);
+        float ga[4], be[4];
+        unpack4<T>(gam, ga);
+        unpack4<T>(bet, be);
+        if (mine_too)
+#pragma unroll
+            for (int t = 0; t < OWN; ++t) {
+                if (own_row + ROWS * t >= rows_x) continue;
+                float z[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) z[e] = exchange_normalised(y[t][e], factors[t], ga[e], be[e]);
+                *reinterpret_cast<u32x2 *>(out + (int64_t)(m0 + own_row + ROWS * t) * out_rs + n_own) = u32x2{pack2<T>(z[0], z[1]), pack2<T>(z[2], z[3])};
+            }
+        if (left != 0) exchange_finish_others<T, BM, BN>(nf, left, row_norm, out, out_rs, m0, M, N, lane, 64);
+        return;
+    }
 
     const bool out_vec = out_cs == 1 && (out_rs & 3) == 0 && ((uintptr_t)out & 7) == 0;
     const bool ai_vec = act_in != nullptr && ai_cs == 1 && (ai_rs & 3) == 0 && ((uintptr_t)act_in & 7) == 0;
@@ -659,9 +756,9 @@ linear_norm_apply_kernel(const float *__restrict__ X, const T *__restrict__ W, c
 }
 
 template <typename T, int BM, int BN, int WAVES, int MODE>
-static void launch_small_dealt_mode(const LinearArgs &a, const NormFold &nf) {
+static void launch_small_dealt_mode(const LinearArgs &a, const NormOf<MODE> &nf) {
     auto kern = linear_small_dealt_kernel<T, BM, BN, WAVES, MODE>;
-    constexpr int LDS_BYTES = WAVES * small_ring_bytes(BM, BN, WAVES) + (MODE != kNormNone ? norm_stats_bytes(BM) : 0);
+    constexpr int LDS_BYTES = WAVES * small_ring_bytes(BM, BN, WAVES) + (MODE == kNormAdd ? norm_stats_bytes(BM) : 0);
     static_assert(LDS_BYTES <= 160 * 1024, "one workgroup per CU");
     static bool attr_done = false;  // benign race: the attribute call is idempotent
     if (!attr_done) {
@@ -711,6 +808,19 @@ static void run_small_dealt_t(const LinearArgs &a, int rows, int cols, int mode,
 void run_small_dealt(const LinearArgs &a, int dtype, int rows, int cols, int mode, const NormFold &nf) {
     if (dtype == KERNL_F16) run_small_dealt_t<f16>(a, rows, cols, mode, nf);
     else run_small_dealt_t<bf16>(a, rows, cols, mode, nf);
+}
+
+// 32 columns and 16, 32 or 64 rows a tile, the rows normalised behind an exchange
+template <typename T>
+static void run_small_dealt_norm_t(const LinearArgs &a, int rows, const NormExchange &nx) {
+    if (rows == 16) launch_small_dealt_mode<T, 16, 32, 4, kNormExchange>(a, nx);
+    else if (rows == 32) launch_small_dealt_mode<T, 32, 32, 4, kNormExchange>(a, nx);
+    else launch_small_dealt_mode<T, 64, 32, 4, kNormExchange>(a, nx);
+}
+
+void run_small_dealt_norm(const LinearArgs &a, int dtype, int rows, const NormExchange &nx) {
+    if (dtype == KERNL_F16) run_small_dealt_norm_t<f16>(a, rows, nx);
+    else run_small_dealt_norm_t<bf16>(a, rows, nx);
 }
 
 template <typename T>

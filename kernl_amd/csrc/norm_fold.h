@@ -24,6 +24,7 @@ constexpr int kNormMaxGroups = 64;   // widths up to 1024
 
 // MODE of the kernels in front of a norm
 constexpr int kNormNone = 0;    // plain epilogue
+constexpr int kNormExchange = 1;  // add a 16-bit residual and normalise, the statistics exchanged with the other column tiles (norm_exchange.h)
 constexpr int kNormAdd = 2;     // add a residual (itself normalised on the fly when it has statistics), store fp32 rows and statistics
 
 struct NormFold {

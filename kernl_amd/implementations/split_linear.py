@@ -13,6 +13,12 @@ FINISH_RESIDUAL, FINISH_RMS_STATS, FINISH_LAYER_NORM = _lib.FINISH_RESIDUAL, _li
 def split_finish_bytes(x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor, finish: int, gamma=None, beta=None) -> int:
     """Bytes of workspace for `split_finish_linear` on these operands; 0 where another route is faster or they are not plain 16-bit GPU
     tensors with nothing to record about them."""
+    return finishing_bytes(lambda m, n, k: _lib.linear_split_workspace_bytes(m, n, k, finish), x, weight, bias, residual, finish, gamma, beta)
+
+
+def finishing_bytes(bytes_of, x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor, finish: int, gamma=None, beta=None) -> int:
+    """What `bytes_of(rows, out features, in features)` says if the operands are plain 16-bit GPU tensors with nothing to record about
+    them, of the layouts that the finishing kernels take; else 0."""
     n, k = weight.shape
     if not (isinstance(residual, torch.Tensor) and x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and x.dim() >= 2 and x.numel() > 0):
         return 0
@@ -23,7 +29,7 @@ def split_finish_bytes(x: torch.Tensor, weight: torch.Tensor, bias, residual: to
         return 0
     if any(p.shape != (n,) for p in (bias, gamma, beta) if p is not None) or (finish == FINISH_LAYER_NORM and gamma is None):
         return 0
-    need = _lib.linear_split_workspace_bytes(x.numel() // k, n, k, finish)
+    need = bytes_of(x.numel() // k, n, k)
     if need == 0 or not _lib.host().takes_call() or forward_ad._current_level >= 0:
         return 0
     if torch.is_grad_enabled() and any(t.requires_grad for t in (x, residual, *params)):

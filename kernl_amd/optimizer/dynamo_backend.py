@@ -26,6 +26,7 @@ from kernl_amd.optimizer.linear import (
     fuse_rms_stats_into_residual_adds,
     fuse_rotary_into_projections,
     replace_all_linear,
+    share_exchange_regions,
 )
 from kernl_amd.optimizer.mask import (
     constant_causal_masks_to_flag,
@@ -70,4 +71,5 @@ def dynamo_backend_ofi(gm: torch.fx.GraphModule, assume_causal=False):
     fuse_linears_into_add_layer_norms(gm)
     fuse_rms_stats_into_residual_adds(gm)
     defer_layer_norms(gm)
+    share_exchange_regions(gm)
     return gm

@@ -11,6 +11,7 @@ import torch
 
 from kernl_amd import _lib
 from kernl_amd.implementations.deferred_norm import DeferredNorm, deferrable, linear_add_deferred
+from kernl_amd.implementations.exchanged_norm import ExchangeRegions, exchange_bytes, linear_add_norm
 from kernl_amd.implementations.linear_layer import GLU_BLOCK, interleave_glu_rows, linear_glu_layer, linear_layer, rms_eps
 from kernl_amd.implementations.split_linear import (
     FINISH_LAYER_NORM, FINISH_RESIDUAL, FINISH_RMS_STATS, split_finish_bytes, split_finish_linear,
@@ -771,7 +772,7 @@ def _epilogue_addition_pays_in_front_of_a_norm(v: torch.Tensor, weight: torch.Te
 
 
 def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor, normalized_shape,
-                                  ln_weight, ln_bias, eps: float, behind=None):
+                                  ln_weight, ln_bias, eps: float, behind=None, regions=None):
     """layer_norm(residual + linear(v, weight, bias)): the attention-output and feed-forward-down projections of an
     encoder layer with the addition and LayerNorm behind them.  Where the projection runs the wide tile kernels the
     addition rides in their epilogue and the LayerNorm reads one tensor (16384 x 768, fp16: 15 us -> 11 us per norm);
@@ -779,7 +780,10 @@ def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, r
     reference, whose graphs add in eager PyTorch in front of every LayerNorm.
 
     `behind` (set by `defer_layer_norms` where every consumer can take it): the weights of the layers that read the result.
-    Few rows leave the norm to them and return a `DeferredNorm`, if all of them take it; `residual` may be one."""
+    Few rows leave the norm to them and return a `DeferredNorm`, if all of them take it; `residual` may be one.
+
+    `regions` (set by `share_exchange_regions`): where more rows are normalised by the product itself, the memory through which its
+    workgroups exchange their statistics."""
     from kernl_amd.optimizer.layer_norm import _half_params_once, add_layer_norm_wrapper_functional, layer_norm_wrapper_functional
 
     # parameters follow the sum's type: a residual kept in fp32 keeps them (and the layers behind) in fp32
@@ -793,6 +797,9 @@ def linear_add_layer_norm_wrapper(v: torch.Tensor, weight: torch.Tensor, bias, r
         residual = residual.normalised()
     if alike and isinstance(v, torch.Tensor):
         _half_params_once(v, weight, bias, ln_weight, ln_bias)
+        need = exchange_bytes(v, weight, bias, residual, ln_weight, ln_bias) if regions is not None else 0
+        if need:
+            return linear_add_norm(need, regions, v, weight, bias, residual, ln_weight, ln_bias, rms_eps(v.dtype, eps))
         need = split_finish_bytes(v, weight, bias, residual, FINISH_LAYER_NORM, ln_weight, ln_bias)
         if need:
             # K split, and the launch that adds its ranges normalises the rows
@@ -903,6 +910,20 @@ def defer_layer_norms(gm: torch.fx.GraphModule):
     if changed:
         gm.graph.lint()
         gm.recompile()
+
+
+def share_exchange_regions(gm: torch.fx.GraphModule):
+    """Gives the `linear_add_layer_norm_wrapper` calls of a graph the pair of regions that their launches take by turns.  Runs behind
+    `defer_layer_norms`."""
+    norms = [node for node in gm.graph.nodes if node.op == "call_function" and node.target is linear_add_layer_norm_wrapper]
+    if not norms:
+        return
+    with gm.graph.inserting_before(norms[0]):
+        regions = gm.graph.call_function(ExchangeRegions, ())
+    for node in norms:
+        node.kwargs = {**node.kwargs, "regions": regions}
+    gm.graph.lint()
+    gm.recompile()
 
 
 def fuse_rms_stats_into_residual_adds(gm: torch.fx.GraphModule):
