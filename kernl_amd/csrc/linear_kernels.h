@@ -40,6 +40,7 @@ int run_mid(const LinearArgs &a, int dtype, int kind);
 // linear + residual + LayerNorm in one launch (norm_exchange.h): tiles of linear_mid.h by hook value, and dealt k-tiles of `rows` x 32
 struct NormExchange;
 void run_mid_norm(const LinearArgs &a, int dtype, int kind, const NormExchange &norm);
+void run_wide_norm(const LinearArgs &a, int dtype, int cols, const NormExchange &norm);
 void run_small_dealt_norm(const LinearArgs &a, int dtype, int rows, const NormExchange &norm);
 // the same with K split over `splits` workgroups a tile, which leave fp32 sums [splits][M][part_rs] for run_split_finish
 struct MidSplit {
@@ -702,13 +703,19 @@ __host__ __device__ static inline bool k_tiles_dealt(int64_t N, int64_t K) { ret
 // and widened by four byte-permutes two read slots later, all in the shadow of the MFMAs; everything else is unchanged.
 // SCALED: the finished sums are multiplied by a factor per row of x (row_scale, fp32 [M]) before the bias is added.
 // RES: a residual matrix is added to the rounded results (plain epilogues only).
-template <typename T, int ACT, int NBN, bool W8 = false, bool SCALED = false, bool RES = false, bool DEAL = false>
+// Epi: NormExchange where the rows are added to a residual and normalised (linear_wide_norm.h; one tile a workgroup).
+struct NormExchange;
+template <typename T, int NBN>
+__device__ __forceinline__ void wide_norm_rows(const NormExchange &norm, f32x4_acc (&acc)[8][NBN], const float (&bf)[NBN], unsigned char *lds,
+                                               T *__restrict__ out, int64_t out_rs, int M, int N, int tiles_m, int m0, int n0, int tid);
+template <typename T, int ACT, int NBN, bool W8 = false, bool SCALED = false, bool RES = false, bool DEAL = false, typename Epi = WideResidual>
 __global__ void __launch_bounds__(256, 1)
 linear_wide_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__restrict__ bias, T *__restrict__ out,
                    T *__restrict__ act_in, int M, int N, int K, int64_t ldx, int64_t out_rs, int64_t out_cs,
                    int64_t ai_rs, int64_t ai_cs, int tiles_m, int tiles_n, int out_vec_ok, int ai_vec_ok,
-                   int bias_vec_ok, const float *__restrict__ row_scale, const WideResidual residual) {
+                   int bias_vec_ok, const float *__restrict__ row_scale, const Epi residual) {
     typedef typename Vec8<T>::type vec8;
+    constexpr bool NORM = std::is_same<Epi, NormExchange>::value;
     constexpr bool GATED = (ACT & kGluBit) != 0;
     static_assert(NBN == 8 || (NBN == 6 && !GATED), "256 or 192 columns per tile; gated epilogues need 256");
     constexpr int BM = 256, BN = 32 * NBN, BK = 64, RB = BK * 2, CPR = BK / 8, NB = 8, KSTEPS = BK / 32;
@@ -748,6 +755,7 @@ linear_wide_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_m = wave & 1, wave_n = wave >> 1;
     const int l16 = lane & 15, g = lane >> 4;
+    if constexpr (NORM) exchange_clear(residual, tid, 256);
 
     // ---- tile loads: load i of a wave fills the 1 KB of 16-byte chunks [256 i + 64 wave, +64) of an operand tile;
     // every lane fetches the chunk that belongs at its LDS position under the swizzle.  Rows beyond M / N lie outside
@@ -988,6 +996,10 @@ linear_wide_kernel(const T *__restrict__ X, const T *__restrict__ W, const T *__
         landed = true;
         float bf[NBN];
         wide_bias_unpack<T, NBN>(braw, bf);
+        if constexpr (NORM) {
+            wide_norm_rows<T, NBN>(residual, acc, bf, smem + 2 * (X_BYTES + W_BYTES), out, out_rs, M, N, tiles_m, m0, n0, tid);
+            return;
+        }
         // one call per 16-row block: each stays small enough for the compiler to unroll completely, so the
         // accumulators are only ever indexed by constants and never leave the register file
 #define KERNL_WIDE_EPILOGUE(I)                                                                                         \

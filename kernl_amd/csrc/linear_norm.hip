@@ -4,13 +4,14 @@
 
 namespace kernl {
 
-// The tiles it runs on, smallest first, by the hook's values (12 .. 14 dealt k-tiles, the others tiles of linear_mid.h), and the threads
-// that hold a tile's results.
+// The tiles it runs on, smallest first, by the hook's values (12 .. 14 dealt k-tiles, 5 and 6 the wide kernel, the others tiles of linear_mid.h),
+// and the threads that hold a tile's results.
 struct NormTile {
     int kind, bm, bn, threads;
 };
 static constexpr NormTile kNormTiles[] = {{12, 16, 32, 128}, {13, 32, 32, 256}, {14, 64, 32, 512}, {11, 64, 64, 512}, {15, 128, 64, 512},
-                                          {17, 128, 128, 512}, {18, 192, 128, 512}, {20, 128, 256, 512}, {21, 256, 128, 512}, {19, 192, 192, 512}};
+                                          {17, 128, 128, 512}, {18, 192, 128, 512}, {20, 128, 256, 512}, {21, 256, 128, 512}, {19, 192, 192, 512},
+                                          {6, 256, 192, 256}, {5, 256, 256, 256}};
 
 // The smallest tile of which one round covers the rows: all workgroups of a row have to run at the same time, and smaller tiles
 // are faster as long as they do.  us, this launch / what ran before it (product and add + LayerNorm, or K split with the LayerNorm in its second
@@ -22,7 +23,10 @@ static constexpr NormTile kNormTiles[] = {{12, 16, 32, 128}, {13, 32, 32, 256}, 
 //   2048     9.4 / 11.1    19.9 / 21.6    11.4 / 12.8    10.7 / 13.0
 //   4096    12.1 / 17.7    26.2 / 29.1    16.0 / 22.0    16.4 / 18.4
 //   8192    19.2 / 22.5    42.8 / 44.1    25.7 / 30.1    23.4 / 30.1
-//  12288    26.0 / 30.2    56.1 / 63.4    (two rounds)   31.3 / 35.7
+//  12288    26.0 / 30.2    56.1 / 63.4    39.2 / 47.9    31.3 / 35.7
+//  14000    29.5 / 33.2    65.0 / 69.9                                   (from here on, and 1024 columns beyond 8192 rows, the wide kernel: 256 x 192
+//  16384    30.8 / 36.4    69.6 / 74.4    42.2 / 57.8                     tiles, or 256 x 256; 16384 x 1024 x 4096 108.9 / 123.9)
+//  20000    35.9 / 49.4    84.0 / 102.9   (two rounds)   (24000) 55.3 / 68.9
 // Left to the others: weights that come from HBM (not measured); a K beyond 2048 where 32-row tiles no longer do and 64 x 64 leave the chip half
 // empty, which is where K split wins (512 x 768 x 3072 12.0 / 11.2, 600 rows 12.6 / 11.8, 682 12.8 / 13.3; 682 x 1024 x 4096 16.8 / 16.6, 800
 // rows 17.2 / 17.9).
@@ -92,6 +96,7 @@ extern "C" int kernl_linear_add_norm_fwd(const void *x, const void *w, const voi
     nx.inv_n = 1.0f / (float)N;
     const NormTile *t = norm_tile(M, N, K);
     if (t->kind >= 12 && t->kind <= 14) run_small_dealt_norm(a, dtype, t->bm, nx);
+    else if (t->kind == 5 || t->kind == 6) run_wide_norm(a, dtype, t->bn, nx);
     else run_mid_norm(a, dtype, t->kind, nx);
     return check_launch("linear + add + LayerNorm");
 }

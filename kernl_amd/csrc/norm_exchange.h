@@ -22,7 +22,7 @@
 namespace kernl {
 
 constexpr int kExchangePer = 4;              // words a lane can hold
-constexpr int exchange_lanes(int bm, int threads) { return threads / bm >= 8 ? 8 : threads / bm >= 4 ? 4 : 2; }  // lanes that look for a row's words
+constexpr int exchange_lanes(int bm, int threads) { return threads / bm >= 8 ? 8 : threads / bm >= 4 ? 4 : threads / bm >= 2 ? 2 : 1; }  // lanes that look for a row's words
 constexpr int kExchangePatience = 1 << 9;    // looks, at about a microsecond each
 
 struct NormExchange : NormFold {             // residual, res_rs, gamma, beta and eps of the norm behind the product
@@ -51,7 +51,7 @@ __device__ __forceinline__ void exchange_clear(const NormExchange &nx, int tid, 
 // The exchange of one workgroup of a row tile of BM rows, `tiles` column tiles of BN columns.  T neighbouring lanes look for the words of a row.
 template <int BM, int BN, int T>
 struct RowExchange {
-    static_assert(T == 2 || T == 4 || T == 8, "lanes a row");
+    static_assert(T == 1 || T == 2 || T == 4 || T == 8, "lanes a row");
     static constexpr int PER = kExchangePer;  // up to 32 column tiles: a note bit each
     uint64_t *notes, *words;
     int tiles;
@@ -85,7 +85,7 @@ struct RowExchange {
             __builtin_amdgcn_s_sleep(1);
         }
         auto lanes_sum = [](float v) __attribute__((always_inline)) {
-            v += dpp_mov<0xB1>(v);
+            if (T >= 2) v += dpp_mov<0xB1>(v);
             if (T >= 4) v += dpp_mov<0x4E>(v);
             if (T >= 8) v += dpp_mov<0x141>(v);
             return v;

@@ -12,7 +12,9 @@ DTYPES = pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=[
 # tile's columns and 24 of them
 SHAPES = [(65, 768, 768), (170, 768, 3072), (171, 768, 776), (341, 768, 768), (128, 1024, 4096), (600, 512, 2048), (342, 768, 768), (1365, 768, 768),
           (682, 768, 3072), (1366, 768, 768), (2730, 768, 768), (2731, 768, 776), (5461, 768, 768), (5462, 768, 768), (8192, 768, 768),
-          (8193, 768, 768), (10922, 768, 768), (10923, 768, 768), (12288, 768, 768), (16384, 384, 768), (300, 128, 64)]
+          (8193, 768, 768), (10922, 768, 768), (10923, 768, 768), (12288, 768, 768), (16384, 384, 768), (300, 128, 64),
+          # the wide kernel: 256 x 192 tiles, then 256 x 256
+          (12289, 768, 136), (16384, 768, 64), (16385, 768, 200), (21760, 768, 64), (8193, 1024, 136), (16384, 1024, 64), (32768, 512, 64)]
 
 
 def _operands(M, N, K, dtype):
