@@ -1994,7 +1994,7 @@ static int small_problem_kind(int64_t M, int64_t N, int64_t K) {
 // HBM or K is short.  With the weight from the memory-side cache (up to 8 M elements) and K from 1536, by a fit of 467 products of 140 to
 // 4096 rows, within 3 to 6 %: these had been timed in half-empty rounds and at up to 2048 rows, and full ones take 15 to 30 % more than
 // that gave (3958 x 4096 x 1536 in 256 x 128 tiles 57 us where the 256 x 256 kernel takes 44, 1777 x 3072 x 2048 in 192 x 128 27.1 where
-// the 128 x 192 kernel takes 25.0).
+// the 128 x 192 kernel takes 25.0).  64 x 64, 128 x 256 and 256 x 128 scaled by what they have gained since (linear_mid.h, `multiply`): 3 to 8 %.
 struct CachedTime {
     double ramp, per_k, per_k_full, edge;  // edge: a last column tile that is not whole (the wide kernels' epilogue)
 };
@@ -2004,10 +2004,10 @@ struct TileTime {
     CachedTime cached;
 };
 static constexpr TileTime kMidTiles[] = {
-    {11, 64, 64, 1.8, 0.195, 0.26, {0.52, 0.141, 0.092, 0.0}},  {15, 128, 64, 1.9, 0.27, 0.385, {0.81, 0.213, 0.140, 0.0}},
+    {11, 64, 64, 1.8, 0.175, 0.25, {0.52, 0.136, 0.090, 0.0}},  {15, 128, 64, 1.9, 0.27, 0.385, {0.81, 0.213, 0.140, 0.0}},
     {17, 128, 128, 2.9, 0.34, 0.53, {3.28, 0.214, 0.249, 0.0}}, {22, 192, 96, 4.0, 0.36, 0.62, {4.02, 0.234, 0.275, 0.0}},
     {18, 192, 128, 4.2, 0.43, 0.67, {4.67, 0.300, 0.327, 0.0}}, {19, 192, 192, 7.0, 0.60, 0.95, {5.95, 0.455, 0.430, 0.0}},
-    {20, 128, 256, 4.6, 0.56, 0.86, {5.45, 0.467, 0.334, 0.0}}, {21, 256, 128, 4.6, 0.555, 0.85, {5.25, 0.469, 0.317, 0.0}}};
+    {20, 128, 256, 4.6, 0.53, 0.86, {5.45, 0.432, 0.309, 0.0}}, {21, 256, 128, 4.6, 0.515, 0.85, {5.25, 0.434, 0.293, 0.0}}};
 static constexpr int kSplitTiles = 5;  // the first of them also take ranges of K
 static constexpr TileTime kWideTiles[] = {{5, 256, 256, 0.0, 1.50, 1.50, {5.96, 0.876, 0.493, 3.1}},
                                           {6, 256, 192, 0.0, 1.30, 1.30, {4.84, 0.765, 0.293, 6.4}},

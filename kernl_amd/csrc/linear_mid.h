@@ -6,17 +6,18 @@
 
 namespace kernl {
 
-// tile shape, grid of the eight multiplying waves and ring depth of one build
+// tile shape, grid of the multiplying waves (eight or four) and ring depth of one build
 template <int BM_, int BN_, int WM_, int WN_, int S_>
 struct MidTile {
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_;
-    static constexpr int BK = 64, RB = BK * 2, LOADERS = 4, WAVES = 8 + LOADERS;
+    static constexpr int BK = 64, RB = BK * 2, LOADERS = 4, MULS = WM * WN, WAVES = MULS + LOADERS;
     static constexpr int TM = BM / WM, TN = BN / WN, NBM = TM / 16, NBN = TN / 16;
     static constexpr bool X_AHEAD = TM * TN < 96 * 48;  // registers for two sets of x fragments
+    static constexpr bool SPREAD = MULS == 4 || TM * TN >= 64 * 64;  // fragment reads between the matrix instructions (see multiply)
     static constexpr bool STAGED = TM * TN >= 64 * 32;  // 16-bit results leave through LDS (see the epilogue)
     static constexpr int X_BYTES = BM * RB, STAGE = (BM + BN) * RB, LDS = S * STAGE;
     static constexpr int LX = BM / (8 * LOADERS), LW = BN / (8 * LOADERS), L = LX + LW;  // 1 KB loads of a loading wave per k-tile
-    static_assert(WM * WN == 8 && LX * 8 * LOADERS == BM && LW * 8 * LOADERS == BN && LDS <= 160 * 1024 && (S == 3 || S == 4) && (S - 1) * L <= 63, "tile shape");
+    static_assert((MULS == 8 || MULS == 4) && LX * 8 * LOADERS == BM && LW * 8 * LOADERS == BN && LDS <= 160 * 1024 && (S == 3 || S == 4) && (S - 1) * L <= 63, "tile shape");
 };
 
 // How the tile grid is dealt to the 8 XCDs, each with an L2 of its own: as 2^xm_shift x 8 / 2^xm_shift blocks of per_m x per_n tiles,
@@ -57,10 +58,10 @@ __device__ __forceinline__ void linear_mid_norm_rows(const NormExchange &norm, f
                                                      u32x2 (&res)[Cfg::NBM][Cfg::NBN], unsigned char *smem, T *out, int64_t out_rs, int M, int N, int tiles_m, int tile_m,
                                                      int tile_n, int tid) {
     typedef typename Vec8<T>::type vec8;
-    constexpr int BM = Cfg::BM, BN = Cfg::BN, TM = Cfg::TM, TN = Cfg::TN, NBM = Cfg::NBM, NBN = Cfg::NBN, C = 4 * NBN, LANES = exchange_lanes(BM, 512);
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, TM = Cfg::TM, TN = Cfg::TN, NBM = Cfg::NBM, NBN = Cfg::NBN, C = 4 * NBN, LANES = exchange_lanes(BM, Cfg::MULS * 64);
     constexpr int PITCH = TN * 2 + 16, CH = TN / 8, ITER = (TM * CH + 63) / 64;
     // LDS: the waves' results, the statistics of the waves' columns, the rows' factors, and what the workgroup has to agree on
-    constexpr int STATS = 8 * TM * PITCH, FACTORS = STATS + Cfg::WN * BM * 8, VERDICT = FACTORS + BM * 8;
+    constexpr int STATS = Cfg::MULS * TM * PITCH, FACTORS = STATS + Cfg::WN * BM * 8, VERDICT = FACTORS + BM * 8;
     static_assert(VERDICT + 16 <= Cfg::LDS, "all of it in the ring");
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wave_m = wave % Cfg::WM, wave_n = wave / Cfg::WM, r = lane & 15, g = lane >> 4;
     const int m0 = tile_m * BM, mw = m0 + wave_m * TM, nl = tile_n * BN + wave_n * TN + C * g;  // the wave's first row, the lane's first column
@@ -187,10 +188,10 @@ __device__ __forceinline__ void linear_mid_tile(const T *__restrict__ X, const T
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_m = wave % Cfg::WM, wave_n = wave / Cfg::WM;
-    const int loader = (wave & 7) % Cfg::LOADERS;
+    const int loader = wave % Cfg::LOADERS;
     const int r = lane & 15, g = lane >> 4;
     if constexpr (NORM)
-        if (wave < 8) exchange_clear(norm, tid, 512);
+        if (wave < Cfg::MULS) exchange_clear(norm, tid, Cfg::MULS * 64);
     // workgroup b runs on XCD b % 8, which works on a block of the tile grid of its own (or on a contiguous run of tiles)
     int tile_m, tile_n;
     if (grid.per_m != 0) {
@@ -294,13 +295,13 @@ __device__ __forceinline__ void linear_mid_tile(const T *__restrict__ X, const T
     }
     u32x2 res_raw[NORM ? NBM : 1][NORM ? NBN : 1];
     if constexpr (NORM && mid_residual_ahead<Cfg>()) {
-        if (wave < 8) mid_residual<T, Cfg>(norm, res_raw, m0, n0, M, wave, lane);
+        if (wave < Cfg::MULS) mid_residual<T, Cfg>(norm, res_raw, m0, n0, M, wave, lane);
     }
     auto wait_loads = [&](auto n_c) __attribute__((always_inline)) {
         constexpr int n = decltype(n_c)::value;
         __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
     };
-    if (wave >= 8) {
+    if (wave >= Cfg::MULS) {
         // a loading wave: its stalls on the load path hold up neither the LDS reads nor the matrix instructions of the others.  Nothing
         // is requested beyond the last k-tile, so that after its barrier LDS is free for the epilogue without another one.
         auto landed = [&](int kt) __attribute__((always_inline)) {  // k-tile kt; at most S - 1 have been requested behind it
@@ -331,42 +332,49 @@ __device__ __forceinline__ void linear_mid_tile(const T *__restrict__ X, const T
     // are overwritten one by one, each as soon as its row of blocks is done.
     constexpr int XB = Cfg::X_AHEAD ? 2 : 1;
     vec8 xf[XB][NBM], wf[2][NBN];
-    auto read = [&](int st, int stage, bool x_too) __attribute__((always_inline)) {
-        const unsigned char *sb = smem + stage * STAGE;
-        if (x_too)
-#pragma unroll
-            for (int i = 0; i < NBM; ++i) xf[st % XB][i] = *reinterpret_cast<const vec8 *>(sb + xoff[st] + i * 2048);
-#pragma unroll
-        for (int j = 0; j < NBN; ++j) wf[st][j] = *reinterpret_cast<const vec8 *>(sb + woff[st] + j * 2048);
-    };
-    // k-step st, and the x fragments of the next one (of `stage`) where they wait for registers
+    auto read_x = [&](int st, const unsigned char *sb, int i) __attribute__((always_inline)) { xf[st % XB][i] = *reinterpret_cast<const vec8 *>(sb + xoff[st] + i * 2048); };
+    auto read_w = [&](int st, const unsigned char *sb, int j) __attribute__((always_inline)) { wf[st][j] = *reinterpret_cast<const vec8 *>(sb + woff[st] + j * 2048); };
+    // k-step st, and the fragments of the next one (of `stage`).  With eight waves and registers for both sets the reads go first: while one wave of a
+    // SIMD requests, the other multiplies.  A SIMD's only multiplying wave, and waves of many blocks, request one behind every matrix
+    // instruction, and x fragments that wait for registers behind the last one that needs the old: 128 x 256 and 256 x 128 tiles of
+    // 4096 x 768 x 3072 34.8 -> 32.8 and 34.5 -> 32.0 us, of 1024 x 4096 x 4096 44.0 -> 41.8 and 44.2 -> 42.2.  (All others this way: 192 x 96 tiles of
+    // 2048 x 768 x 3072 22.2 -> 22.8, 128 x 128 the same.)
     auto multiply = [&](int st, int stage) __attribute__((always_inline)) {
         const unsigned char *sb = smem + stage * STAGE;
+        constexpr int READS = NBN + (XB == 2 ? NBM : 0), EACH = Cfg::SPREAD ? (READS + NBM * NBN - 1) / (NBM * NBN) : READS;
+        auto read = [&](int q) __attribute__((always_inline)) {
+            if (q < NBN) read_w(1 - st, sb, q);
+            else read_x(1 - st, sb, q - NBN);
+        };
+        if (!Cfg::SPREAD) {
 #pragma unroll
-        for (int i = 0; i < NBM; ++i) {
-#pragma unroll
-            for (int j = 0; j < NBN; ++j) acc[i][j] = mfma16(wf[st][j], xf[st % XB][i], acc[i][j]);
-            if (XB == 1) {
-                xf[0][i] = *reinterpret_cast<const vec8 *>(sb + xoff[1 - st] + i * 2048);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            for (int q = 0; q < READS; ++q) read(q);
+            __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int m = 0; m < NBM * NBN; ++m) {
+            const int i = m / NBN, j = m % NBN;
+            acc[i][j] = mfma16(wf[st][j], xf[st % XB][i], acc[i][j]);
+            if (!Cfg::SPREAD) continue;
+#pragma unroll
+            for (int q = m * EACH; q < (m + 1) * EACH && q < READS; ++q) read(q);
+            if (XB == 1 && j == NBN - 1) read_x(1 - st, sb, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
     __syncthreads();
-    read(0, 0, true);
+#pragma unroll
+    for (int i = 0; i < NBM; ++i) read_x(0, smem, i);
+#pragma unroll
+    for (int j = 0; j < NBN; ++j) read_w(0, smem, j);
     int stage = 0;
     for (int kt = 0; kt < nk; ++kt) {
         const int next = stage == S - 1 ? 0 : stage + 1;
-        read(1, stage, XB == 2);
-        __builtin_amdgcn_sched_barrier(0);
         multiply(0, stage);
-        __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __syncthreads();  // k-tile kt + 1 has landed for everyone, and nobody reads k-tile kt any more
-        read(0, next, XB == 2);
-        __builtin_amdgcn_sched_barrier(0);
         multiply(1, next);
-        __builtin_amdgcn_sched_barrier(0);
         stage = next;
     }
     // (past the last barrier nothing lands in LDS any more and nobody reads a fragment that counts)
@@ -385,7 +393,7 @@ __device__ __forceinline__ void linear_mid_tile(const T *__restrict__ X, const T
     const int mw = m0 + wave_m * Cfg::TM;
     if (part != nullptr) {  // fp32 sums of the range, row-major; columns N .. part_rs - 1 hold zeros (their weight rows do)
         constexpr int PITCH = Cfg::TN * 4 + 16, CH = Cfg::TN / 4;
-        static_assert(8 * 16 * PITCH <= Cfg::LDS, "a row block of every wave");
+        static_assert(Cfg::MULS * 16 * PITCH <= Cfg::LDS, "a row block of every wave");
         unsigned char *mine = smem + wave * (16 * PITCH);
         const int nw = n0 + wave_n * Cfg::TN;
 #pragma unroll
@@ -408,7 +416,7 @@ __device__ __forceinline__ void linear_mid_tile(const T *__restrict__ X, const T
         return;
     }
     constexpr int PITCH = TNO * 2 + 16, CH = TNO / 8, ITER = (Cfg::TM * CH + 63) / 64;
-    static_assert(8 * Cfg::TM * PITCH <= Cfg::LDS, "the results of every wave");
+    static_assert(Cfg::MULS * Cfg::TM * PITCH <= Cfg::LDS, "the results of every wave");
     unsigned char *const mine = smem + wave * (Cfg::TM * PITCH);
     const int nw = (GATED ? n0 / 2 : n0) + wave_n * TNO;
     if (mw >= M || nw >= out_n) return;
@@ -549,7 +557,7 @@ static int mid_grid(int tiles_m, int tiles_n, int splits, MidGrid &grid) {
 }
 
 // the tiles, by the kernl_linear_force_tile value that forces them (and mid_tile_of names)
-typedef MidTile<64, 64, 4, 2, 4> Mid64x64;      // 11   64 KB: two workgroups per CU
+typedef MidTile<64, 64, 2, 2, 4> Mid64x64;      // 11   64 KB: two workgroups per CU
 typedef MidTile<128, 64, 4, 2, 3> Mid128x64;    // 15   72 KB: two workgroups per CU
 typedef MidTile<128, 128, 2, 4, 4> Mid128x128;  // 17
 typedef MidTile<192, 128, 4, 2, 4> Mid192x128;  // 18

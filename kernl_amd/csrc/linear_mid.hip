@@ -5,7 +5,7 @@
 // that only loads, 256 workgroups; ring depths of 64 and 128 KB and every cache policy the same).  Loads of a line by several CUs at
 // the same time wait the full latency each.  And where the waves that load also multiply, a full load path holds up their LDS reads
 // and matrix instructions: 1024 x 768 x 3072 in 64 x 64 tiles took 15.5 us, the same with the loads alone 11.6, without them 8.9.  Hence
-//   - waves that only load (four, behind the eight that multiply): what they wait for, nobody else waits for.  1024 x 768 x 3072
+//   - waves that only load (four, behind those that multiply): what they wait for, nobody else waits for.  1024 x 768 x 3072
 //     15.5 -> 13.0 us, 1024 x 3072 x 768 11.3 -> 9.8 in 128 x 128 tiles, 231 x 2304 x 768 6.6 -> 5.9;
 //   - k-tiles dealt among the workgroups that share a weight or x tile (`turn`; see k_tiles_dealt in linear_kernels.h): 1024 x 4096 x 4096 in 128 x 128
 //     tiles, weights from HBM, 39.6 -> 34.5 us, 512 x 12288 x 4096 in 256 x 128 tiles 54.7 -> 51, 333 x 22016 x 4096 in 192 x 192
@@ -13,6 +13,8 @@
 //   - tiles of 64 x 64 to 256 x 128, as large as still put a tile on (nearly) every CU: (BM + BN) x K bytes a tile;
 //   - LDS fragments read one k-step ahead ACROSS the barrier (while k-step 1 of a k-tile is multiplied, k-step 0 of the next is read);
 //     sched_barrier keeps the compiler from moving the reads back behind the multiplications;
+//   - four multiplying waves of 32 x 32 in the 64 x 64 tile, two thirds of the LDS reads that eight of 16 x 32 need: 1024 x 768 x 3072 11.7 -> 10.9 us, 4096 x
+//     768 x 3072 34.0 -> 32.3, 231 x 2304 x 768 5.7 -> 5.4.  (Larger tiles in four waves: 128 x 64 within 2 %, 128 x 128 9.1 -> 9.9 at K = 768.)
 //   - the small tiles in rings of 64 to 72 KB, so that two workgroups share a CU where there are more tiles than CUs.
 // Weight rows are placed in LDS so that a lane's blocks are consecutive output columns: 16-byte stores.
 #include "linear_mid.h"

@@ -9,7 +9,7 @@ namespace kernl {
 struct NormTile {
     int kind, bm, bn, threads;
 };
-static constexpr NormTile kNormTiles[] = {{12, 16, 32, 128}, {13, 32, 32, 256}, {14, 64, 32, 512}, {11, 64, 64, 512}, {15, 128, 64, 512},
+static constexpr NormTile kNormTiles[] = {{12, 16, 32, 128}, {13, 32, 32, 256}, {14, 64, 32, 512}, {11, 64, 64, 256}, {15, 128, 64, 512},
                                           {17, 128, 128, 512}, {18, 192, 128, 512}, {20, 128, 256, 512}, {21, 256, 128, 512}, {19, 192, 192, 512},
                                           {6, 256, 192, 256}, {5, 256, 256, 256}};
 
@@ -33,12 +33,16 @@ static constexpr NormTile kNormTiles[] = {{12, 16, 32, 128}, {13, 32, 32, 256}, 
 static const NormTile *norm_tile(int64_t M, int64_t N, int64_t K) {
     for (const NormTile &t : kNormTiles) {
         const int64_t tiles_n = N / t.bn, tiles = (M + t.bm - 1) / t.bm * tiles_n;
-        if (N % t.bn != 0 || tiles_n > exchange_lanes(t.bm, t.threads) * kExchangePer) continue;
+        if (N % t.bn != 0 || tiles_n > exchange_most(exchange_lanes(t.bm, t.threads))) continue;
         if (g_linear_force_tile != 0) {
             if (t.kind == g_linear_force_tile) return &t;
             continue;
         }
         if (tiles > 256) continue;
+        // (the larger ones over more than 1024 columns, 600 x 2048 x 2048 16.8 against 16.2 and 800 x 1536 x 1536 15.5 against 13.3, and 128 x 64 tiles over a
+        // long K that leave a third of the chip empty, 1365 x 768 x 3072 20.7 against 19.8, 1365 x 1024 x 4096 27.2 against 26.3, are slower)
+        if (N > 1024 && t.bm * t.bn > 64 * 64) return nullptr;
+        if (t.kind == 15 && K > 2048 && tiles < (K <= 3072 ? 160 : 208)) return nullptr;
         // 64 x 32 tiles with dealt k-tiles: 682 x 512 x 2048 8.7 against 10.1 in 64 x 64, 1024 rows (a full round) 10.6 against 10.1, 682 x 768 x 768 7.6
         // against 7.5
         if (t.kind == 14 && (K < 1536 || K > 2048 || tiles > 208)) continue;

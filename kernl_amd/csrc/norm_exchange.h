@@ -21,8 +21,8 @@
 
 namespace kernl {
 
-constexpr int kExchangePer = 4;              // words a lane can hold
 constexpr int exchange_lanes(int bm, int threads) { return threads / bm >= 8 ? 8 : threads / bm >= 4 ? 4 : threads / bm >= 2 ? 2 : 1; }  // lanes that look for a row's words
+constexpr int exchange_most(int lanes) { return lanes < 4 ? 4 * lanes : 32; }  // column tiles whose words they can hold
 constexpr int kExchangePatience = 1 << 9;    // looks, at about a microsecond each
 
 struct NormExchange : NormFold {             // residual, res_rs, gamma, beta and eps of the norm behind the product
@@ -52,7 +52,7 @@ __device__ __forceinline__ void exchange_clear(const NormExchange &nx, int tid, 
 template <int BM, int BN, int T>
 struct RowExchange {
     static_assert(T == 1 || T == 2 || T == 4 || T == 8, "lanes a row");
-    static constexpr int PER = kExchangePer;  // up to 32 column tiles: a note bit each
+    static constexpr int PER = exchange_most(T) / T;  // up to 32 column tiles: a note bit each
     uint64_t *notes, *words;
     int tiles;
     __device__ __forceinline__ RowExchange(const NormExchange &nx, int tile_m, int tiles_m, int tiles_n)
