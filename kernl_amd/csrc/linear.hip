@@ -1,5 +1,6 @@
 // Fused linear layer: dispatch and C entry points (kernels and launchers: linear_kernels.h).
 #include "linear_kernels.h"
+#include "linear_stream.h"
 #include "norm_fold.h"
 
 namespace kernl {
@@ -43,7 +44,8 @@ static int linear_mfma_dispatch(const LinearArgs &a) {
     // few rows of x: stream the weight once with every CU (9 forces this kernel where it applies)
     const bool small_first = pick == 0 && !(a.act & kGluBit) && small_problem_kind(a.M, a.N, a.K) != 0;
     if ((pick == 0 || pick == 9) && !small_first && a.M <= 64 && a.K % 64 == 0) {
-        if (a.act & kGluBit) launch_skinny<T, true>(a);
+        if (stream_takes(a)) launch_stream<T>(a, nullptr, 0.0f, a.extra != nullptr ? *a.extra : SkinnyExtra{});
+        else if (a.act & kGluBit) launch_skinny<T, true>(a);
         else launch_skinny<T, false>(a);
         return check_launch("linear (skinny)");
     }
@@ -550,6 +552,12 @@ extern "C" int kernl_linear_rms_fwd(const void *x, const void *rms_weight, float
     a.ai_rs = 0; a.ai_cs = 0;
     a.act = activation;
     a.st = static_cast<hipStream_t>(stream);
+    if (gated) a.act |= kGluBit;
+    if (stream_takes(a)) {
+        if (dtype == KERNL_F16) launch_stream<f16>(a, rms_weight, eps, SkinnyExtra{});
+        else launch_stream<bf16>(a, rms_weight, eps, SkinnyExtra{});
+        return check_launch("rms linear (stream)");
+    }
     if (dtype == KERNL_F16) {
         if (gated) launch_skinny_rms<f16, true>(a, rms_weight, eps);
         else launch_skinny_rms<f16, false>(a, rms_weight, eps);
@@ -619,6 +627,11 @@ extern "C" int kernl_linear_decode_fwd(const void *x, const void *rms_weight, fl
     a.ai_rs = 0; a.ai_cs = 0;
     a.act = KERNL_ACT_NONE;
     a.st = static_cast<hipStream_t>(stream);
+    if (stream_takes(a)) {
+        if (dtype == KERNL_F16) launch_stream<f16>(a, rms_weight, eps, ex);
+        else launch_stream<bf16>(a, rms_weight, eps, ex);
+        return check_launch("decode linear (stream)");
+    }
     if (dtype == KERNL_F16) launch_skinny_decode<f16>(a, rms_weight, eps, ex);
     else launch_skinny_decode<bf16>(a, rms_weight, eps, ex);
     return check_launch("decode linear (skinny)");
