@@ -460,9 +460,11 @@ PyObject *op_skinny_attention(PyObject *const *a, Py_ssize_t n) {  // q k v out 
 
 // Rows that stream a weight on the stream-K kernel: `few_row_rule` of implementations/linear_layer.py (which says what was
 // measured) with what `kernl_linear_fewrow_fwd` takes.
-constexpr int64_t kFewRowMin = 17, kFewRowMax = 128, kFewRowMinWeight = 1 << 22, kFewRowLongK = 1536, kSplitKMaxRows = 2048;
+constexpr int64_t kFewRowMin = 17, kFewRowMax = 128, kFewRowMinWeight = 1 << 22, kFewRowLongK = 1536, kSplitKMaxRows = 2048, kFewRowLargeWeight = 24 << 20;
 
-bool few_row_rule(int64_t rows, int64_t n, int64_t k) {
+bool few_row_rule(int64_t rows, int64_t n, int64_t k, bool normed) {
+    if (rows > 4 && rows < kFewRowMin && k % 64 == 0 && k >= 256)
+        return n * k >= kFewRowLargeWeight && (normed ? rows >= 8 || k <= 8192 : rows >= 12 && k >= 5120);
     if (rows < kFewRowMin || rows > kFewRowMax || k < 256 || k % 64 != 0) return false;
     return n * k >= kFewRowMinWeight || (k >= kFewRowLongK && rows > 32);
 }
@@ -528,7 +530,7 @@ PyObject *op_linear(PyObject *const *a, Py_ssize_t n) {
                                    (M > 64 && r.strides[0] < (1 << 22) && kernl_linear_mid_kind(M, N, K, 0) != 0));
     const at::Tensor out = output_for(*x, N);
     const int64_t os[2] = {N, 1};
-    if (!small && vectors && K % 64 == 0 && act_in == nullptr && few_row_rule(M, N, K)) {
+    if (!small && vectors && K % 64 == 0 && act_in == nullptr && few_row_rule(M, N, K, false)) {
         PyObject *x2d = x->dim() == 2 ? (Py_INCREF(a[0]), a[0]) : THPVariable_Wrap(rows_view(*x, r));
         PyObject *y = THPVariable_Wrap(out);
         PyObject *y2d = out.dim() == 2 ? (Py_INCREF(y), y) : THPVariable_Wrap(out.view({M, N}));
@@ -559,7 +561,7 @@ PyObject *plan_few_rows(PyObject *const *a, Py_ssize_t n) {
         Py_RETURN_NONE;
     if (K % 64 != 0 || !r.vectors() || !aligned16(*x) || (gated && rows % 64 != 0)) Py_RETURN_NONE;
     if (!vector_of(bias, *x, rows) || !vector_of(g, *x, K)) Py_RETURN_NONE;
-    const bool stream_k = few_row_rule(M, rows, K) && (cos == nullptr || head_dim == 32 || head_dim == 64 || head_dim == 128);
+    const bool stream_k = few_row_rule(M, rows, K, g != nullptr) && (cos == nullptr || head_dim == 32 || head_dim == 64 || head_dim == 128);
     if (!stream_k && M > 64) Py_RETURN_NONE;
     const int64_t per_batch = x->dim() == 3 ? x->size(1) : M;
     if ((cos == nullptr) != (sin == nullptr)) Py_RETURN_NONE;

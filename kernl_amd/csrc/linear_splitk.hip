@@ -20,7 +20,10 @@
 // A workgroup of 8 waves walks its run: the x rows of two (16 rows: four) units at a time go through LDS (16-byte pieces,
 // XOR-swizzled for the MFMA operand reads; two stages, one barrier per group) and every wave feeds the 16 weight rows it owns
 // of the unit's tile from global memory straight into v_mfma_f32_16x16x32 — weights on the A side, x on the B side,
-// lane (r = lane % 16, g = lane / 16) supplying k = 16 g + 8 s .. + 7 of the chunk in step s on both sides.  The
+// lane (r = lane % 16, g = lane / 16) supplying k = 16 g + 8 s .. + 7 of the chunk in step s on both sides.  Up to 32 rows a load takes
+// eight whole lines (LINES): read with a non-temporal hint they come faster from HBM, and 2 KB of LDS a wave turn them into operands (us, weights
+// from HBM, 24 rows: 12288 x 4096 28.4 -> 25.4, 11008 x 4096 gated 45.2 -> 38.9, 4096 x 11008 25.7 -> 23.4, 32000 x 4096 64.0 -> 54.8; from the memory-side cache
+// within 5 % either way).  More rows are bound by LDS as well: 64 rows from the cache 28.2 -> 31.6, from HBM 33.7 -> 32.6.  The
 // prefetch depth is in registers: a ring of 4 (8) units of weight fragments per wave and the thread's share of the next
 // group of x.
 //
@@ -133,6 +136,7 @@ template <typename T, int MB, int WAVES, int GC, int RING, bool RMS, bool W8 = f
 __global__ void __launch_bounds__(64 * WAVES) linear_fewrow_kernel(const FewRowArgs a) {
     typedef typename Vec8<T>::type vec8;
     static_assert(RING % (2 * GC) == 0, "a round of RING units is a whole number of stage pairs");
+    constexpr bool LINES = !W8 && MB <= 2;  // weights in whole lines
     constexpr int THREADS = 64 * WAVES;
     typedef FewRowStageMap<MB, GC, THREADS> StageMap;   // index_math.h: shared with the host-side replay
     constexpr int MP = StageMap::MP;                    // rows of x, padded to whole MFMA blocks
@@ -142,6 +146,7 @@ __global__ void __launch_bounds__(64 * WAVES) linear_fewrow_kernel(const FewRowA
     static_assert(2 * GC * CHUNK_BYTES >= RPT * THREADS * 4, "the stages double as the buffer of the row sums");
     __shared__ __attribute__((aligned(16))) unsigned char xs[2][GC * CHUNK_BYTES];
     __shared__ float rstd_s[MP];
+    __shared__ __attribute__((aligned(16))) unsigned char wt[LINES ? WAVES : 1][LINES ? 2048 : 16];  // a wave's unit of weights
 
     static_assert(!W8 || std::is_same<T, f16>::value, "one-byte weights are decoded to fp16");
     typedef typename std::conditional<W8, unsigned char, T>::type WT;   // what a weight element is stored as
@@ -166,20 +171,31 @@ __global__ void __launch_bounds__(64 * WAVES) linear_fewrow_kernel(const FewRowA
     auto weight_row = [&](int tile) __attribute__((always_inline)) -> const WT * {
         return W + (int64_t)min(tile * (16 * WAVES) + 16 * wave + r, N - 1) * K + 16 * g;
     };
-    const WT *wrow = weight_row(rq_tile);
+    // LINES: lane l of load `half` takes chunk l % 8 of row 8 half + l / 8
+    auto line_row = [&](int tile, int half) __attribute__((always_inline)) -> const WT * {
+        return W + (int64_t)min(tile * (16 * WAVES) + 16 * wave + 8 * half + (lane >> 3), N - 1) * K + 8 * (lane & 7);
+    };
+    const WT *wrow = LINES ? line_row(rq_tile, 0) : weight_row(rq_tile), *wrow_b = line_row(rq_tile, 1);
+    // ... and the wave turns them in LDS of its own (chunks swizzled by the row; a wave's LDS accesses keep their order)
+    const int wt_to[2] = {swz_offset<128>(lane >> 3, lane & 7), swz_offset<128>(8 + (lane >> 3), lane & 7)}, wt_from[2] = {swz_offset<128>(r, 2 * g), swz_offset<128>(r, 2 * g + 1)};
     auto request_w = [&](int slot) __attribute__((always_inline)) {
         const WT *src = wrow + (int64_t)rq_chunk * 64;
         if constexpr (W8) {
             wraw[slot] = *reinterpret_cast<const u32x4 *>(src);
-        } else {
+        } else if constexpr (!LINES) {
             wf[slot][0] = *reinterpret_cast<const vec8 *>(src);
             wf[slot][1] = *reinterpret_cast<const vec8 *>(src + 8);
+        } else {
+            wf[slot][0] = __builtin_nontemporal_load(reinterpret_cast<const vec8 *>(src));
+            wf[slot][1] = __builtin_nontemporal_load(reinterpret_cast<const vec8 *>(wrow_b + (int64_t)rq_chunk * 64));
         }
         if (rq_left > 0) {      // uniform; address arithmetic only
             --rq_left;
             if (++rq_chunk == nch) {
                 rq_chunk = 0;
-                wrow = weight_row(++rq_tile);
+                ++rq_tile;
+                if constexpr (!LINES) wrow = weight_row(rq_tile);
+                else wrow = line_row(rq_tile, 0), wrow_b = line_row(rq_tile, 1);
             }
         }
     };
@@ -278,9 +294,18 @@ __global__ void __launch_bounds__(64 * WAVES) linear_fewrow_kernel(const FewRowA
                 }
                 w0 = __builtin_bit_cast(vec8, lo);
                 w1 = __builtin_bit_cast(vec8, hi);
-            } else {
+            } else if constexpr (!LINES) {
                 w0 = wf[slot][0];
                 w1 = wf[slot][1];
+            } else {
+                unsigned char *mine = wt[wave];
+                *reinterpret_cast<vec8 *>(mine + wt_to[0]) = wf[slot][0];
+                *reinterpret_cast<vec8 *>(mine + wt_to[1]) = wf[slot][1];
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_wave_barrier();
+                w0 = *reinterpret_cast<const vec8 *>(mine + wt_from[0]);
+                w1 = *reinterpret_cast<const vec8 *>(mine + wt_from[1]);
+                __builtin_amdgcn_wave_barrier();
             }
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) {

@@ -25,21 +25,30 @@ ACTIVATIONS = {
 ONE_BYTE_WEIGHT_DTYPES = (torch.int8, torch.uint8, torch.float8_e5m2)
 
 
-FEW_ROW_MIN_ROWS = 17          # up to 16 rows the kernel that gives a workgroup 16 columns and all of K is as fast or faster
+FEW_ROW_MIN_ROWS = 17          # up to 16 rows the kernel that gives a workgroup 16 columns and all of K is as fast or faster ...
 FEW_ROW_MAX_ROWS = 128         # what `kernl_linear_fewrow_fwd` takes
 SPLIT_K_MAX_ROWS = 2048        # beyond that the tiled kernels always have tiles enough
 FEW_ROW_MIN_WEIGHT = 1 << 22   # elements: below that (2048 x 2048) launch latency decides and one launch beats two ...
 
 
 FEW_ROW_LONG_K = 1536          # ... unless K is long and there are more than 32 rows
+FEW_ROW_LARGE_WEIGHT = 24 << 20  # ... unless the weight is large and there are more than four (which run on csrc/linear_stream.h)
 
 
-def few_row_rule(rows: int, n: int, k: int) -> bool:
+def few_row_rule(rows: int, n: int, k: int, normed: bool = False) -> bool:
     """Where the stream-K kernel is the faster one (measured, graph replay): 17 to 128 rows against a weight of 4 M
     elements or more (5120 x 5120 at 32 / 64 rows: 18 / 21 us against 34 / 35 on the weight-streaming kernel of
     `kernl_linear_fwd`; 4096 x 11008: 25 / 30 against 35 / 53; at 128 rows 28 against 63 and 38 against 130 on its tile
     kernels), and 33 rows or more against smaller weights with a long K (768 x 3072 at 48 / 128 rows: 11 / 14 us against
-    15 / 27).  Short K and few rows stay where they were (3072 x 768 at 48 rows: 8.9 against 7.2)."""
+    15 / 27).  Short K and few rows stay where they were (3072 x 768 at 48 rows: 8.9 against 7.2).
+
+    5 to 16 rows against 24 M elements or more behind an RMSNorm (`normed`), weights from HBM, this / the weight-streaming kernel at 5 and 16 rows: 12288 x
+    4096 rotated 23.0 / 26.0 and 24.3 / 30.1 us, 11008 x 4096 gated 36.1 / 39.9 and 37.4 / 44.9, 32000 x 4096 53.7 / 59.6 and 54.7 / 74.6.  Without a norm
+    from twelve rows and a long K on: 4096 x 11008 22.4 / 25.0, 5120 x 5120 16.7 / 20.5; but 12288 x 4096 22.8 / 22.5, and with eight rows 4096 x 11008
+    21.9 / 19.8 where the weight stays in the memory-side cache.  Smaller weights: 4096 x 4096 at 16 rows 13.5 / 11.4, 5504 x 2048 gated 16.6 / 17.8
+    (at 5 rows 15.7 / 15.3)."""
+    if 4 < rows < FEW_ROW_MIN_ROWS and k % 64 == 0 and k >= 256:
+        return n * k >= FEW_ROW_LARGE_WEIGHT and ((rows >= 8 or k <= 8192) if normed else (rows >= 12 and k >= 5120))
     if not FEW_ROW_MIN_ROWS <= rows <= FEW_ROW_MAX_ROWS or k < 256 or k % 64 != 0:
         return False
     return n * k >= FEW_ROW_MIN_WEIGHT or (k >= FEW_ROW_LONG_K and rows > 32)
@@ -89,8 +98,10 @@ def split_pays_bytes(x2d: torch.Tensor, weight: torch.Tensor) -> int:
     return _lib.linear_split_workspace_bytes(x2d.shape[0], weight.shape[0], x2d.shape[1])
 
 
-def takes_few_row_kernel(x2d: torch.Tensor, weight: torch.Tensor) -> bool:
-    return few_row_rule(x2d.shape[0], weight.shape[0], weight.shape[1]) and _lib.linear_fewrow_supported(x2d, weight)
+def takes_few_row_kernel(x2d: torch.Tensor, weight: torch.Tensor, normed: bool = False) -> bool:
+    if x2d.shape[0] < FEW_ROW_MIN_ROWS and weight.dtype != x2d.dtype:
+        return False  # (one-byte weights are not read in whole lines)
+    return few_row_rule(x2d.shape[0], weight.shape[0], weight.shape[1], normed) and _lib.linear_fewrow_supported(x2d, weight)
 
 
 class LinearLayer(torch.autograd.Function):
@@ -264,7 +275,7 @@ def rms_linear_layer(
     n_out = weight.shape[0] // 2 if gated else weight.shape[0]
     if x.dtype == torch.float16:
         eps = max(eps, 1.6e-5)  # the fp16 policy of the RMSNorm operator (reference: layer_norm.py:295-296)
-    if takes_few_row_kernel(x_, weight) and (not gated or n_out % GLU_BLOCK == 0):
+    if takes_few_row_kernel(x_, weight, True) and (not gated or n_out % GLU_BLOCK == 0):
         out = torch.empty((x_.shape[0], n_out), device=x.device, dtype=x.dtype)
         _lib.linear_fewrow_fwd(x_, weight, bias, None, out, ACTIVATIONS.get(activation, _lib.ACT_NONE),
                                rms_weight=rms_weight, eps=eps, gated=gated)
@@ -448,7 +459,7 @@ def decode_linear_layer(
         assert residual.dtype == x.dtype and residual.numel() == x_.shape[0] * N
         res_ = residual.reshape(-1, N)
     out = torch.empty((x_.shape[0], N), device=x.device, dtype=x.dtype)
-    if takes_few_row_kernel(x_, weight) and (cos is None or head_dim in (32, 64, 128)):
+    if takes_few_row_kernel(x_, weight, rms_weight is not None) and (cos is None or head_dim in (32, 64, 128)):
         _lib.linear_fewrow_fwd(x_, weight, bias, res_, out, _lib.ACT_NONE, rms_weight=rms_weight, eps=eps, cos=cos, sin=sin,
                                head_dim=head_dim, rope_cols=rope_cols, rows_per_batch=rows_per_batch)
     else:

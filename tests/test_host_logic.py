@@ -828,6 +828,18 @@ def test_few_row_kernel_routing_rule():
     assert takes_few_row_kernel(rows(32).to(torch.bfloat16), w.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("rows, n, k, normed, plain", [(4, 12288, 4096, False, False), (5, 12288, 4096, True, False), (16, 6144, 4096, True, False),
+                                                       (16, 6143, 4096, False, False), (7, 4096, 11008, False, False), (8, 4096, 11008, True, False),
+                                                       (12, 4096, 11008, True, True), (11, 5120, 5120, True, False), (12, 5120, 5120, True, True),
+                                                       (16, 12288, 4104, False, False), (16, 1 << 20, 192, False, False)])
+def test_five_to_sixteen_rows_of_a_large_weight_take_the_few_row_kernel(rows, n, k, normed, plain):
+    from kernl_amd.implementations.linear_layer import few_row_rule, takes_few_row_kernel
+
+    assert (few_row_rule(rows, n, k, True), few_row_rule(rows, n, k)) == (normed, plain)
+    one_byte = torch.zeros(1, dtype=torch.uint8).expand(n, k)
+    assert not takes_few_row_kernel(torch.zeros((rows, k), dtype=torch.float16), one_byte)
+
+
 def test_small_problem_rule_of_the_library():
     """`kernl_linear_small_kind` (no GPU needed): which shapes the linear entry point runs on its small-problem kernels.
     One round of workgroups is the condition throughout; big weights, single rows and long K with many rows are not
