@@ -37,7 +37,8 @@ layernorm_rows_kernel(const T *__restrict__ x, const T *__restrict__ res, const 
     static_assert(!HALF || GROUP_WAVES == 1, "half-wave groups are single-wave groups split in two");
     constexpr int G = HALF ? 32 : 64 * GROUP_WAVES;
     typedef Row16<T> chunk_t;
-    __shared__ float red[2][4];
+    __shared__ f32x4 red[2][4];
+    __shared__ float sums[2][4];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int t = HALF ? (lane & 31) : GROUP_WAVES == 1 ? lane : (int)threadIdx.x;  // index inside the group
@@ -46,20 +47,39 @@ layernorm_rows_kernel(const T *__restrict__ x, const T *__restrict__ res, const 
     const int nchunks = N / E;
     const float inv_n = 1.0f / (float)N;
 
-    // sum over the group: wave reduction, then (4-wave groups) a round trip through LDS
-    auto group_sum = [&](float v, int slot) -> float {
+    // sum over the group
+    auto group_sum = [&](float v) -> float {
         if (HALF) {
             float lo, hi;
             half_wave_sums(v, lo, hi);
             return lane < 32 ? lo : hi;
         }
-        v = wave_sum(v);
-        if (GROUP_WAVES == 1) return v;
-        __syncthreads();  // the previous use of this slot has been read by everyone
-        if (lane == 0) red[slot][wave] = v;
-        __syncthreads();
-        return (red[slot][0] + red[slot][1]) + (red[slot][2] + red[slot][3]);
+        return wave_sum(v);
     };
+    // 4-wave groups: every wave leaves what its part of the row gave in LDS, by rows in turn in one half of `red` or the other, so that one barrier a row is
+    // enough (sum and squared deviations each with a round of their own take four: 8192 x 4096 25.5 -> 24.0 us, RMSNorm of 4096 x 4096 13.2 -> 12.6) ...
+    int turn = 0;
+    auto exchange = [&](const f32x4 &part) -> const f32x4 * {
+        if (lane == 0) red[turn][wave] = part;
+        __syncthreads();
+        turn ^= 1;
+        return red[turn ^ 1];
+    };
+    // ... but where a wave has four chunks, which leave no registers for it (8192 x 8192 45.7 -> 46.9, RMSNorm 45.5 -> 47.9)
+    constexpr bool ONE_BARRIER = CHUNKS < 4;
+    auto block_sum = [&](float v, int slot) {
+        __syncthreads();  // the previous use of this slot has been read by everyone
+        if (lane == 0) sums[slot][wave] = v;
+        __syncthreads();
+        return (sums[slot][0] + sums[slot][1]) + (sums[slot][2] + sums[slot][3]);
+    };
+    // values of the row that the wave holds
+    float held = 0.0f, inv_held = 0.0f;
+    if (GROUP_WAVES > 1 && ONE_BARRIER) {
+#pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) held += (float)(E * (FULL ? 64 : min(max(nchunks - (wave * 64 + c * G), 0), 64)));
+        inv_held = held > 0.0f ? 1.0f / held : 0.0f;
+    }
 
     // gamma / beta stay in registers (as 16-bit values; FULL: as fp32) for every row this group visits.
     chunk_t wv[CHUNKS], bv[CHUNKS];
@@ -126,20 +146,7 @@ layernorm_rows_kernel(const T *__restrict__ x, const T *__restrict__ res, const 
         if (FULL ? lead + row_step < M : row + row_step < M) fetch(row + row_step);
 
         float mean = 0.0f, var;
-        if (RMS) {
-            float ss = 0.0f;
-#pragma unroll
-            for (int c = 0; c < CHUNKS; ++c)
-#pragma unroll
-                for (int e = 0; e < E; ++e) ss += v[c][e] * v[c][e];
-            var = group_sum(ss, 0) * inv_n;
-        } else {
-            float s = 0.0f;
-#pragma unroll
-            for (int c = 0; c < CHUNKS; ++c)
-#pragma unroll
-                for (int e = 0; e < E; ++e) s += v[c][e];
-            mean = group_sum(s, 0) * inv_n;
+        auto deviations = [&](float from) {
             float ss = 0.0f;
 #pragma unroll
             for (int c = 0; c < CHUNKS; ++c) {
@@ -147,12 +154,55 @@ layernorm_rows_kernel(const T *__restrict__ x, const T *__restrict__ res, const 
                 if (FULL || ci < nchunks) {
 #pragma unroll
                     for (int e = 0; e < E; ++e) {
-                        const float d = v[c][e] - mean;
+                        const float d = v[c][e] - from;
                         ss += d * d;
                     }
                 }
             }
-            var = group_sum(ss, 1) * inv_n;
+            return group_sum(ss);
+        };
+        if (RMS) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+                for (int e = 0; e < E; ++e) ss += v[c][e] * v[c][e];
+            ss = group_sum(ss);
+            if (GROUP_WAVES > 1) {
+                if (ONE_BARRIER) {
+                    const f32x4 *r = exchange(f32x4{ss, 0.0f, 0.0f, 0.0f});
+                    ss = (r[0][0] + r[1][0]) + (r[2][0] + r[3][0]);
+                } else {
+                    ss = block_sum(ss, 0);
+                }
+            }
+            var = ss * inv_n;
+        } else {
+            float s = 0.0f;
+#pragma unroll
+            for (int c = 0; c < CHUNKS; ++c)
+#pragma unroll
+                for (int e = 0; e < E; ++e) s += v[c][e];
+            s = group_sum(s);
+            if (GROUP_WAVES == 1) {
+                mean = s * inv_n;
+                var = deviations(mean) * inv_n;
+            } else if (!ONE_BARRIER) {
+                mean = block_sum(s, 0) * inv_n;
+                var = block_sum(deviations(mean), 1) * inv_n;
+            } else {
+                // deviations from the wave's own mean, merged around the row's
+                const float own = s * inv_held;
+                const f32x4 *r = exchange(f32x4{s, deviations(own), own, held});
+                mean = ((r[0][0] + r[1][0]) + (r[2][0] + r[3][0])) * inv_n;
+                float m2 = 0.0f;
+#pragma unroll
+                for (int w = 0; w < GROUP_WAVES; ++w) {
+                    const float d = r[w][2] - mean;
+                    m2 += fmaf(r[w][3] * d, d, r[w][1]);
+                }
+                var = m2 * inv_n;
+            }
         }
         const float rstd = 1.0f / sqrtf(var + eps);
         if (t == 0 && live) {
@@ -247,8 +297,8 @@ static void launch_rows(bool rms, bool has_res, dim3 grid, hipStream_t st, const
                         int64_t res_rs, int64_t out_rs, float eps) {
     // rows that fill every lane's chunks exactly take the form without bounds tests (single-wave groups of up to 4
     // chunks: gamma and beta are kept as fp32 there)
-    if constexpr (!FULL && GROUP_WAVES == 1 && CHUNKS <= 4) {
-        if (N == CHUNKS * (HALF ? 32 : 64) * (int)(16 / sizeof(T))) {
+    if constexpr (!FULL && CHUNKS * GROUP_WAVES <= 8 && CHUNKS <= 4) {
+        if (N == CHUNKS * (HALF ? 32 : 64 * GROUP_WAVES) * (int)(16 / sizeof(T))) {
             launch_rows<T, CHUNKS, GROUP_WAVES, HALF, true>(rms, has_res, grid, st, x, res, w, b, out, mean, rstd, M, N, x_rs,
                                                             res_rs, out_rs, eps);
             return;
@@ -290,7 +340,10 @@ static int layernorm_dispatch(const void *x_, const void *res_, const void *w_, 
         // block (more loads in flight per row); otherwise a wave per row, 4 rows per block.  The grid is capped at
         // 8 waves per SIMD (4 where a wave takes two rows) so that every group walks several rows and gamma/beta loads
         // amortise.
-        const bool block_per_row = row_chunks > 128 && M < 16384;
+        // How far the block form goes with 16-bit rows (us, LayerNorm, a block / a wave per row): 16384 x 4096 46.4 / 52.4, 20000 x 4096 54.5 / 56.4, 30000 x 4096 83.0 /
+        // 82.1, 65536 x 4096 217 / 199; 24576 x 2048 37.4 / 33.6; 20000 x 5120 79.8 / 105.8, 20000 x 8192 120 / 157 and 187 / 498 with a residual (a wave
+        // has no registers for such rows).  fp32 rows: 40000 x 4096 243 / 231, 20000 x 2048 52.1 / 50.9.
+        const bool block_per_row = row_chunks > 128 && (M < 16384 || (E == 8 && (row_chunks > 512 || (row_chunks > 256 && M <= 20480))));
         // Two rows per wave, 32 lanes each, where that leaves fewer lanes idle than a wave per row (rows of up to 32
         // or of 65..96 chunks).
         const bool half_wave = !block_per_row && (row_chunks <= 32 || (row_chunks > 64 && row_chunks <= 96));

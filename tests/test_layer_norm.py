@@ -224,3 +224,27 @@ def test_embedding_ids_outside_the_table_are_clamped():
     out = embedding_layer_norm([table], [ids], w, None, 1e-5)
     want = embedding_layer_norm([table], [ids.clamp(0, 9)], w, None, 1e-5)
     assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+@pytest.mark.parametrize("rms", [False, True], ids=["ln", "rms"])
+@pytest.mark.parametrize("rows, n", [(5, 1032), (3, 1544), (2, 2048), (2100, 2056), (7, 3584), (4200, 4096), (16384, 4096), (9, 4104), (6, 6152), (16384, 5120), (3, 8192)])
+def test_rows_shared_by_four_waves(rows, n, rms, dtype, close):
+    """Waves with all, some and none of their chunks inside the row, several rows a workgroup (its exchange alternates between two places), rows far from zero."""
+    from kernl_amd.implementations.layer_norm import layer_norm
+    from oracle import layer_norm_oracle, rms_norm_oracle
+
+    gen = torch.Generator().manual_seed(rows + n)
+    x = (torch.randn((rows, n), generator=gen) + torch.linspace(-3, 3, n)).to(dtype)
+    w, b = (1 + 0.1 * torch.randn((n,), generator=gen)).to(dtype), torch.randn((n,), generator=gen).to(dtype)
+    out = layer_norm(x.cuda(), w.cuda(), None if rms else b.cuda(), 1.6e-5, use_rms_norm=rms)
+    torch.cuda.synchronize()
+    some = torch.cat((torch.arange(min(rows, 40)), torch.arange(max(rows - 40, 0), rows)))
+    expect = rms_norm_oracle(x[some], w, 1.6e-5) if rms else layer_norm_oracle(x[some], w, b, 1.6e-5)
+    close(out[some.cuda()], expect, dtype, what=f"{rows} x {n}")
+    exact = x.cuda().double()
+    exact = exact * torch.rsqrt(exact.pow(2).mean(-1, keepdim=True) + 1.6e-5) * w.cuda().double() if rms else torch.nn.functional.layer_norm(
+        exact, (n,), w.cuda().double(), b.cuda().double(), 1.6e-5)
+    # every row: half a unit of the last place of a 16-bit result, and sums of fp32
+    assert ((out.double() - exact).norm(dim=-1) / exact.norm(dim=-1)).max() < (4e-4 if dtype == torch.float16 else 3.2e-3)
